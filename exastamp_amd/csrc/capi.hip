@@ -14,6 +14,7 @@ namespace xsmd {
 Ctx::~Ctx()
 {
   if (hscalar) (void)hipHostFree(hscalar);
+  if (hthermo) (void)hipHostFree(hthermo);
   if (flag_event) (void)hipEventDestroy(flag_event);
   if (own_stream) (void)hipStreamDestroy(own_stream);
 }
@@ -174,6 +175,7 @@ xs_status xs_ctx_create(int device, xs_ctx** out)
     c->stream = c->own_stream;
     XS_HIP(hipEventCreateWithFlags(&c->flag_event, hipEventDisableTiming));
     XS_HIP(hipHostMalloc((void**)&c->hscalar, 8 * sizeof(unsigned long long), hipHostMallocDefault));
+    XS_HIP(hipHostMalloc((void**)&c->hthermo, 27 * sizeof(double), hipHostMallocDefault));
     c->dscalar.reserve(8);
     XS_HIP(hipMemsetAsync(c->dscalar.p, 0, 8 * sizeof(unsigned long long), c->stream));  // flags start clear
     XS_HIP(hipStreamSynchronize(c->stream));

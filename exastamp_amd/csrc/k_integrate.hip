@@ -117,24 +117,45 @@ __global__ void __launch_bounds__(256) k_stream_copy(int64_t n16, const double2*
 constexpr int kThermoBlocks = 1024;
 constexpr int kThermoQ = 26;
 
-template <class T>
-__device__ __forceinline__ T wave_sum(T v)
+// Sums over the 64 lanes of a wave of 32 quantities per lane: at each halving of the
+// lane distance a lane keeps one half of the quantities it still holds and hands the
+// other half to its partner, so the whole reduction is 32 exchanges instead of 6 per
+// quantity.  Lane l ends with the total of quantity bitrev5(l >> 1), in a fixed order.
+__device__ __forceinline__ double wave_sum32(double (&v)[32], int lane)
 {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
+#pragma unroll
+  for (int half = 16, off = 32; half >= 1; half >>= 1, off >>= 1) {
+    const bool hi = lane & off;
+#pragma unroll
+    for (int q = 0; q < half; q++) {
+      const double keep = hi ? v[half + q] : v[q];
+      const double send = hi ? v[q] : v[half + q];
+      v[q] = keep + __shfl_xor(send, off);
+    }
+  }
+  return v[0] + __shfl_xor(v[0], 1);
+}
+
+// the quantity whose total lane l holds after wave_sum32
+__device__ __forceinline__ int wave_sum32_index(int lane)
+{
+  return ((lane >> 5) & 1) << 4 | ((lane >> 4) & 1) << 3 | ((lane >> 3) & 1) << 2 | ((lane >> 2) & 1) << 1 |
+         ((lane >> 1) & 1);
 }
 
 // Per-block partial sums of the 26 quantities of simulation_thermodynamic_state
 // (virial 9, v(x)v m 9, m v 3, m v^2 3, ep, m) over a fixed grid, so the
-// summation order -- and the result -- does not depend on timing.
+// summation order -- and the result -- does not depend on timing.  Small systems are
+// bound by the reduction's lane exchanges (8.6 us with 6 exchanges per quantity at 864
+// atoms), large ones by the 106 bytes read per atom.
 __global__ void __launch_bounds__(256) k_thermo_partial(
     int64_t n, int64_t npad, const double* __restrict__ vx, const double* __restrict__ vy,
     const double* __restrict__ vz, const double* __restrict__ ep, const double* __restrict__ vir,
     const uint8_t* __restrict__ type, const double* __restrict__ mass, double* __restrict__ part)
 {
-  double acc[kThermoQ];
+  double acc[32];
 #pragma unroll
-  for (int q = 0; q < kThermoQ; q++) acc[q] = 0.0;
+  for (int q = 0; q < 32; q++) acc[q] = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     const double m = mass[type[i]];
@@ -152,13 +173,10 @@ __global__ void __launch_bounds__(256) k_thermo_partial(
     acc[24] += ep[i];
     acc[25] += m;
   }
-  __shared__ double sh[4][kThermoQ];
+  __shared__ double sh[4][32];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-  for (int q = 0; q < kThermoQ; q++) {
-    const double s = wave_sum(acc[q]);
-    if (lane == 0) sh[w][q] = s;
-  }
+  const double s = wave_sum32(acc, lane);
+  if ((lane & 1) == 0) sh[w][wave_sum32_index(lane)] = s;
   __syncthreads();
   if (threadIdx.x < kThermoQ) {
     const int q = threadIdx.x;
@@ -166,29 +184,30 @@ __global__ void __launch_bounds__(256) k_thermo_partial(
   }
 }
 
-__global__ void k_thermo_final(int nblocks, const double* __restrict__ part, double* __restrict__ out)
+// The partial sums added up and written in the 27-double layout of xs_thermo (kinetic
+// tensor and kinetic energy halved, particle count last).  Up to 1024 partials per
+// quantity: 32 threads per quantity each add a fixed stride of them, their sums are
+// added in order.  One thread per quantity adding them all is a chain of dependent
+// loads: 242 us at 1024 partials, 48 us at 200, against about 5 us.
+constexpr int kThermoFinal = 1024;
+__global__ void __launch_bounds__(kThermoFinal) k_thermo_final27(int nblocks, const double* __restrict__ part,
+                                                                 int64_t n, double* __restrict__ out27)
 {
-  const int q = threadIdx.x;
-  if (q >= kThermoQ) return;
+  __shared__ double sh[32][33];
+  const int q = threadIdx.x & 31, g = threadIdx.x >> 5;
   double s = 0.0;
-  for (int b = 0; b < nblocks; b++) s += part[(int64_t)b * kThermoQ + q];
-  out[q] = s;
-}
-
-// The same sums in the same order as k_thermo_final, finished on the device into the
-// 27-double layout of xs_thermo (kinetic tensor and kinetic energy halved, particle
-// count last), so the result never leaves device memory.
-__global__ void k_thermo_final27(int nblocks, const double* __restrict__ part, int64_t n,
-                                 double* __restrict__ out27)
-{
-  const int q = threadIdx.x;
-  if (q >= 27) return;
-  if (q == 26) {
+  if (q < kThermoQ)
+    for (int b = g; b < nblocks; b += 32) s += part[(int64_t)b * kThermoQ + q];
+  sh[g][q] = s;
+  __syncthreads();
+  if (threadIdx.x >= 27) return;
+  if (threadIdx.x == 26) {
     out27[26] = (double)n;
     return;
   }
-  double s = 0.0;
-  for (int b = 0; b < nblocks; b++) s += part[(int64_t)b * kThermoQ + q];
+  s = sh[0][q];
+#pragma unroll
+  for (int k = 1; k < 32; k++) s += sh[k][q];
   const bool half = (q >= 9 && q < 18) || (q >= 21 && q < 24);
   out27[q] = half ? 0.5 * s : s;
 }
@@ -256,26 +275,21 @@ void launch_drift_kick(Ctx& c, double dt)
 void launch_thermo(Ctx& c, double out[27])
 {
   c.red_part.reserve((size_t)kThermoBlocks * kThermoQ);
-  c.red_out.reserve(kThermoQ);
-  double s[kThermoQ] = {0};
-  if (c.n > 0) {
+  c.red_out.reserve(27);
+  const int nb = c.n > 0 ? (int)std::min<int64_t>(kThermoBlocks, grid_for(c.n)) : 0;
+  {
     ProfScope prof(c.prof, c.stream, XS_PROF_THERMO);
-    const int nb = (int)std::min<int64_t>(kThermoBlocks, grid_for(c.n));
-    k_thermo_partial<<<nb, kBlock, 0, c.stream>>>(c.n, c.npad, c.vx.p, c.vy.p, c.vz.p, c.ep.p, c.vir.p,
-                                                  c.type.p, c.mass_d.p, c.red_part.p);
+    if (nb > 0) {
+      k_thermo_partial<<<nb, kBlock, 0, c.stream>>>(c.n, c.npad, c.vx.p, c.vy.p, c.vz.p, c.ep.p, c.vir.p,
+                                                    c.type.p, c.mass_d.p, c.red_part.p);
+      XS_HIP(hipGetLastError());
+    }
+    k_thermo_final27<<<1, kThermoFinal, 0, c.stream>>>(nb, c.red_part.p, c.n, c.red_out.p);
     XS_HIP(hipGetLastError());
-    k_thermo_final<<<1, 64, 0, c.stream>>>(nb, c.red_part.p, c.red_out.p);
-    XS_HIP(hipGetLastError());
-    XS_HIP(hipMemcpyAsync(s, c.red_out.p, sizeof(s), hipMemcpyDeviceToHost, c.stream));
-    XS_HIP(hipStreamSynchronize(c.stream));
   }
-  for (int q = 0; q < 9; q++) out[q] = s[q];
-  for (int q = 9; q < 18; q++) out[q] = 0.5 * s[q];
-  for (int q = 18; q < 21; q++) out[q] = s[q];
-  for (int q = 21; q < 24; q++) out[q] = 0.5 * s[q];
-  out[24] = s[24];
-  out[25] = s[25];
-  out[26] = (double)c.n;
+  XS_HIP(hipMemcpyAsync(c.hthermo, c.red_out.p, 27 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  XS_HIP(hipStreamSynchronize(c.stream));
+  std::memcpy(out, c.hthermo, 27 * sizeof(double));
 }
 
 void thermo_scratch_init(int device)
@@ -305,7 +319,7 @@ void launch_thermo_noalloc(Ctx& c, double* out27_dev)
                                                   c.mass_d.p, part);
     XS_HIP(hipGetLastError());
   }
-  k_thermo_final27<<<1, 64, 0, c.stream>>>(nb, part, c.n, out27_dev);
+  k_thermo_final27<<<1, kThermoFinal, 0, c.stream>>>(nb, part, c.n, out27_dev);
   XS_HIP(hipGetLastError());
 }
 

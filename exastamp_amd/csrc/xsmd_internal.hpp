@@ -340,6 +340,7 @@ struct Ctx {
   bool flag_pending = false;
   DBuf<double> red_part;  // thermo partial sums
   DBuf<double> red_out;
+  double* hthermo = nullptr;  // pinned host copy of the 27 results
 
   bool has_lj = false;
   double lj_eps = 0, lj_sigma = 0, lj_rcut = 0;
