@@ -190,10 +190,6 @@ xs_status xs_ctx_create(int device, xs_ctx** out)
                                                                        : prop.sharedMemPerBlock;
     if (const char* ls = std::getenv("XSMD_LIST_SORT")) c->list_sort_disabled = std::strcmp(ls, "0") == 0;
     if (const char* st = std::getenv("XSMD_EAM_S_TABLE")) c->s_table_disabled = std::strcmp(st, "0") == 0;
-    if (const char* sb = std::getenv("XSMD_SORT_BITS")) {
-      const int v = std::atoi(sb);
-      if (v >= 1 && v <= 8) c->sort_bits = v;
-    }
     if (const char* ba = std::getenv("XSMD_BLOCK_ATOMS")) {
       const double v = std::atof(ba);
       if (v >= 1.0 && v <= 4096.0) {

@@ -364,19 +364,6 @@ __device__ __forceinline__ int pass_half() { return (threadIdx.x >> 5) & 1; }
 // ---------------------------------------------------------------------------
 // list build
 // ---------------------------------------------------------------------------
-// number of central atoms of a brick (the row walk of central_atom)
-__device__ __forceinline__ int central_count(const BlockShape& s, const HaloCell* hc)
-{
-  int n = 0;
-  for (int iz = 1; iz <= s.ez; iz++)
-    for (int iy = 1; iy <= s.ey; iy++) {
-      const int h0 = (iz * s.hy + iy) * s.hx + 1;
-      const int h1 = h0 + s.ex - 1;
-      n += hc[h1].lstart + hc[h1].count - hc[h0].lstart;
-    }
-  return n;
-}
-
 // Destination lane of this lane's key in one stable split pass: keys with a 0 bit
 // first (in lane order), then those with a 1.  zeros = ballot of the 0 keys; mbcnt
 // counts the 0 keys below this lane, so the 1 keys below it are lane minus that.
@@ -404,21 +391,7 @@ __device__ __forceinline__ uint32_t wave_radix_sort(uint32_t key, int lo, int nb
   return key;
 }
 
-// two independent sorts interleaved (the permutes of one wait on the LDS crossbar
-// while the other's ballots issue)
-__device__ __forceinline__ void wave_radix_sort2(uint32_t& k0, uint32_t& k1, int lo, int nbits)
-{
-  const int lane = threadIdx.x & 63;
-  for (int bit = lo; bit < lo + nbits; bit++) {
-    const bool one0 = (k0 >> bit) & 1u, one1 = (k1 >> bit) & 1u;
-    const int d0 = split_dest(one0, __ballot(!one0), lane);
-    const int d1 = split_dest(one1, __ballot(!one1), lane);
-    k0 = (uint32_t)__builtin_amdgcn_ds_permute(d0 << 2, (int)k0);
-    k1 = (uint32_t)__builtin_amdgcn_ds_permute(d1 << 2, (int)k1);
-  }
-}
-
-// Lists of at most 64 entries are kept sorted by distance (see k_list_sort).
+// Lists of at most 64 entries are kept sorted by distance (see k_block_build).
 constexpr int kSortRows = 64;
 
 // Block-list storage.  The entries of atom i come in groups of 8: group q holds
@@ -432,30 +405,6 @@ __device__ __forceinline__ int64_t bl_index(int64_t npad, int64_t i, int k)
   return (((int64_t)(k >> 3) * npad + i) << 3) + ((k & 1) << 2) + ((k & 7) >> 1);
 }
 
-// Block list: stencil order dz, dy, dx, in-cell order ascending (the order of the
-// global build, ascending halo slot).  One lane per central atom walks the
-// candidates itself, two at a time (their LDS reads overlap), and packs its hits
-// into the current 8-entry group in registers; a full group goes out as one
-// 16-byte store.  A neighbour cell whose box (widened by a margin that covers the
-// rounding of cell assignment; unbounded on the outer side of a non-periodic edge
-// cell, which also holds the atoms clamped into it) lies beyond rl is trimmed from
-// the walk (its atoms would all fail the exact test), unless some atom sits outside
-// its cell's box (nocull, set by the cell-key kernel).  Entries past nmax are counted, not
-// stored (the host grows nmax and builds again).
-constexpr int kBuildThreads = 256;
-
-// The current 8-entry group of a lane is a 128-bit FIFO of 16-bit slots in w[0..3]:
-// a new entry enters at the top and the others move down one place (a funnel
-// shift per word), so after eight entries w holds them in list order, two per
-// word, the first in the low half of w[0].
-__device__ __forceinline__ void fifo_push(uint32_t (&w)[4], uint32_t c)
-{
-  w[0] = __builtin_amdgcn_alignbit(w[1], w[0], 16);
-  w[1] = __builtin_amdgcn_alignbit(w[2], w[1], 16);
-  w[2] = __builtin_amdgcn_alignbit(w[3], w[2], 16);
-  w[3] = __builtin_amdgcn_alignbit(c, w[3], 16);
-}
-
 // list order (0, 1), (2, 3), (4, 5), (6, 7) -> the bl_index order (0, 2), (4, 6),
 // (1, 3), (5, 7)
 __device__ __forceinline__ uint4 group_interleave(const uint32_t (&o)[4])
@@ -464,235 +413,352 @@ __device__ __forceinline__ uint4 group_interleave(const uint32_t (&o)[4])
                     (o[0] >> 16) | (o[1] & 0xffff0000u), (o[2] >> 16) | (o[3] & 0xffff0000u));
 }
 
+// Smallest value over the 16 lanes of a row (lane order reversed in ever larger
+// groups, so four steps reach every lane).
+__device__ __forceinline__ double row16_min(double v)
+{
+#define XS_DPP_MIN(ctrl)                                                                                            \
+  {                                                                                                                 \
+    const long long b = __double_as_longlong(v);                                                                    \
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, ctrl, 0xf, 0xf, true);                 \
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), ctrl, 0xf, 0xf, true);         \
+    v = fmin(v, __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo)));                            \
+  }
+  XS_DPP_MIN(0xB1)   // quad_perm [1, 0, 3, 2]
+  XS_DPP_MIN(0x4E)   // quad_perm [2, 3, 0, 1]
+  XS_DPP_MIN(0x141)  // row_half_mirror
+  XS_DPP_MIN(0x140)  // row_mirror
+#undef XS_DPP_MIN
+  return v;
+}
+
+// Sorts, ascending, the 64 values that each group of 8 consecutive lanes holds, 8 per
+// lane; lane j of the group ends with places 8 j .. 8 j + 7.  A sorting network in
+// registers: each lane sorts its own 8 (19 exchanges), then lists of 8, 16 and 32 merge
+// pairwise -- the first exchange of a merge pairs mirrored places, the later ones places
+// at a fixed distance -- with the partner lane's values as DPP operands.  A wave sorts
+// eight lists at once, about 260 instructions; a bitwise radix sort of one list per wave
+// needs about 60 for each list and a pass through LDS for every bit.
+template <int CTRL>
+__device__ __forceinline__ uint32_t lane_swap(uint32_t v)
+{
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+}
+__device__ __forceinline__ void order2(uint32_t& a, uint32_t& b)
+{
+  const uint32_t lo = min(a, b), hi = max(a, b);
+  a = lo;
+  b = hi;
+}
+// the lower places of both partners keep the smaller values; MIRROR: place r against 7 - r
+template <int CTRL, bool MIRROR>
+__device__ __forceinline__ void order_lanes(uint32_t (&v)[8], bool lower)
+{
+  uint32_t o[8];
+#pragma unroll
+  for (int r = 0; r < 8; r++) {
+    const uint32_t t = lane_swap<CTRL>(v[MIRROR ? 7 - r : r]);
+    o[r] = lower ? min(v[r], t) : max(v[r], t);
+  }
+#pragma unroll
+  for (int r = 0; r < 8; r++) v[r] = o[r];
+}
+__device__ __forceinline__ void merge8(uint32_t (&v)[8])
+{
+#pragma unroll
+  for (int d = 4; d >= 1; d >>= 1)
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+      if ((r & d) == 0) order2(v[r], v[r + d]);
+}
+__device__ __forceinline__ void sort64(uint32_t (&v)[8])
+{
+  const int net[19][2] = {{0, 2}, {1, 3}, {4, 6}, {5, 7}, {0, 4}, {1, 5}, {2, 6}, {3, 7}, {0, 1}, {2, 3},
+                          {4, 5}, {6, 7}, {2, 4}, {3, 5}, {1, 4}, {3, 6}, {1, 2}, {3, 4}, {5, 6}};
+#pragma unroll
+  for (int k = 0; k < 19; k++) order2(v[net[k][0]], v[net[k][1]]);
+  const int j = threadIdx.x & 7;
+  order_lanes<0xB1, true>(v, (j & 1) == 0);   // lanes 0-1, quad_perm [1, 0, 3, 2]
+  merge8(v);
+  order_lanes<0x1B, true>(v, (j & 2) == 0);   // lanes 0-3 mirrored, quad_perm [3, 2, 1, 0]
+  order_lanes<0xB1, false>(v, (j & 1) == 0);
+  merge8(v);
+  order_lanes<0x141, true>(v, (j & 4) == 0);  // lanes 0-7 mirrored, row_half_mirror
+  order_lanes<0x4E, false>(v, (j & 2) == 0);  // quad_perm [2, 3, 0, 1]
+  order_lanes<0xB1, false>(v, (j & 1) == 0);
+  merge8(v);
+}
+
+// base plus the number of set bits of m below this lane
+__device__ __forceinline__ int wave_rank(unsigned long long m, int base)
+{
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
+}
+
+// LDS written by some lanes of a wave and read by others of the same wave
+__device__ __forceinline__ void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Block list: stencil order dz, dy, dx, in-cell order ascending (the order of the
+// global build, ascending halo slot), then ordered by distance.
+//
+// One wave takes one central cell.  All its atoms share the candidates of the 27
+// cells around it, so the wave collects them once -- dropping those farther than rl
+// from the bounding box of the cell's atoms -- holds them in registers, up to kBuildTile
+// at a time, and tests each central atom (the same
+// for every lane) against 64 candidates at a time.  A ballot gives each hit its place
+// in the atom's list, so no lane waits for another's trip count and only hits are
+// stored.  The lists of kBuildAtoms atoms are collected in LDS, sorted together in
+// registers and written as whole 8-entry groups, 128 contiguous bytes per group.
+//
+// The dropped candidates would fail the exact test: for an atom inside the box every
+// component of its displacement is at least the gap to the box in magnitude, and
+// rounding (subtraction, fma) is monotonic, so d2 >= the box's d2 >= rl2 in floating
+// point as well.
+//
+// The sort orders lists of at most kSortRows entries by d^2 (FP32, cut to 8 significant
+// bits), then slot.  At a given list position the atoms of a wave then look up nearby
+// spline rows, which cuts the cache lines each table gather of the EAM passes touches
+// by about 40 %.
+//
+// Bound by vector instruction issue (about 130 vector instructions per atom at 53
+// entries, the tests of 197 candidates, the sort and the candidate search in equal
+// parts) at the three 4-wave workgroups per CU its LDS leaves.  One lane per atom
+// walking its own candidates, with the sort as a second kernel, issued twice as many on
+// diverging lanes.  8.39 M EAM atoms (53 entries): 4.04 -> 2.57 ms, 1.05 M argon atoms
+// (79 entries, unsorted) 0.79 -> 0.38 ms, 4000 argon atoms 112 -> 26 us.  Workgroups of
+// 5, 6 or 8 waves measured slower (4.86, 2.84 and 3.70 ms: their waves share the SIMDs
+// unevenly or leave LDS for two workgroups).
+//
+// XF: a non-identity domain xform.  The halo stays in grid space and each candidate's
+// displacement is mapped by xf->m before the test, in the operation order of the
+// global build (so the lists stay bit-identical); grid-space boxes do not bound
+// physical distances, so no candidate is dropped.
+constexpr int kBuildThreads = 256;
+constexpr int kBuildWaves = kBuildThreads / 64;
+constexpr int kBuildAtoms = 8;
+constexpr int kBuildTile = 512;  // candidates held in registers
+
 // LDS of the list build: cap + 1 position records of 24 bytes, 16-byte aligned
 __host__ __device__ inline size_t build_rec_bytes(int cap) { return ((size_t)(cap + 1) * 24 + 15) / 16 * 16; }
 
-// 8-bit distance keys of a group, list order (byte j of b[0..1] = entry j) -> the
-// bl_index order (0, 2, 4, 6 | 1, 3, 5, 7)
-__device__ __forceinline__ uint2 bins_interleave(const uint32_t (&b)[2])
+struct BuildArgs {
+  BlockGeom g;
+  const int* __restrict__ cell_off;
+  const Pos4* __restrict__ pos;
+  const BoxDev* __restrict__ box;
+  const XformDev* __restrict__ xf;
+  double rl2;
+  uint16_t* __restrict__ nbr16;
+  int* __restrict__ nnb;
+  int64_t npad;
+  int nmax;      // list capacity (a multiple of 8)
+  int cap;       // halo slots
+  int cand_cap;  // most atoms in the 27 cells of a central cell
+  int atoms;     // lists collected per wave, at most kBuildAtoms
+  bool sort;     // false: lists stay in stencil order
+  unsigned long long* __restrict__ flags;  // [0] longest list beyond nmax, [1] halo beyond cap
+};
+
+// candidate slots of each wave (the staging uses the same bytes first) and the list rows
+__host__ __device__ inline size_t build_cand_bytes(int cap, int cand_cap)
 {
-  const uint32_t e0 = b[0] & 0xffu, e1 = (b[0] >> 8) & 0xffu, e2 = (b[0] >> 16) & 0xffu, e3 = b[0] >> 24;
-  const uint32_t e4 = b[1] & 0xffu, e5 = (b[1] >> 8) & 0xffu, e6 = (b[1] >> 16) & 0xffu, e7 = b[1] >> 24;
-  return make_uint2(e0 | (e2 << 8) | (e4 << 16) | (e6 << 24), e1 | (e3 << 8) | (e5 << 16) | (e7 << 24));
+  const size_t a = (size_t)cap, b = (size_t)kBuildWaves * cand_cap;
+  return ((a > b ? a : b) * sizeof(uint16_t) + 3) / 4 * 4;
 }
 
-// BINS: each entry also gets its distance key for the sort, min(2^nbits - 1,
-// floor(d2 * bin_scale)) with bin_scale = 2^nbits / rl^2 (bins uniform in d^2), in
-// bins8, grouped like the list.
-// XF: a non-identity domain xform.  The halo stays in grid space and each candidate's
-// displacement is mapped by xf->m before the test, in the operation order of the
-// global build (so the lists stay bit-identical); grid-space cell boxes do not
-// bound physical distances, so no cell is culled.
-template <bool BINS, bool XF>
-__global__ void __launch_bounds__(kBuildThreads) k_block_build(BlockGeom g, const int* __restrict__ cell_off,
-                                                               const Pos4* __restrict__ pos,
-                                                               const BoxDev* __restrict__ box, double rl2,
-                                                               uint16_t* __restrict__ nbr16, int* __restrict__ nnb,
-                                                               int nmax, int64_t npad, int cap, int ccap, int nh_max,
-                                                               const unsigned long long* __restrict__ nocull,
-                                                               int* __restrict__ brick_rows,
-                                                               unsigned long long* __restrict__ flags,
-                                                               uint8_t* __restrict__ bins8, float bin_scale,
-                                                               int bin_max, const XformDev* __restrict__ xf)
+template <bool XF>
+__global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
 {
   const int64_t b = lblock();
-  if (b >= g.nblocks) return;
-  // LDS: cap + 1 position records {x, y, z} (24 bytes; the extra one pads the
-  // second read of a candidate pair), then the halo table
+  if (b >= a.g.nblocks) return;
   extern __shared__ __align__(32) unsigned char smem[];
   double3* P = reinterpret_cast<double3*>(smem);
-  struct {
-    HaloCell* hc;
-    int* total;
-    uint16_t* slot_cell;
-    uint16_t* central_local;
-  } l;
-  l.hc = reinterpret_cast<HaloCell*>(smem + build_rec_bytes(cap));
-  l.total = reinterpret_cast<int*>(l.hc + nh_max);
-  l.slot_cell = reinterpret_cast<uint16_t*>(l.total + 4);
-  l.central_local = l.slot_cell + cap;
-  const BlockShape s = block_shape(g, b);
-  const int total = build_halo(g, s, cell_off, l.hc, l.total);
-  if (total > cap) {  // cannot happen when cap = measured maximum; never write past LDS
-    if (threadIdx.x == 0) atomicMax(flags + 1, (unsigned long long)total);
+  HaloCell* hc = reinterpret_cast<HaloCell*>(smem + build_rec_bytes(a.cap));
+  int* total_p = reinterpret_cast<int*>(hc + a.g.nh_max);  // [0] halo atoms, [1] next central cell
+  uint16_t* cand_all = reinterpret_cast<uint16_t*>(total_p + 4);
+  uint32_t* rows_all = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(cand_all) +
+                                                   build_cand_bytes(a.cap, a.cand_cap));
+  const BlockShape s = block_shape(a.g, b);
+  const int total = build_halo(a.g, s, a.cell_off, hc, total_p);
+  if (total > a.cap) {  // cannot happen when cap = measured maximum; never write past LDS
+    if (threadIdx.x == 0) atomicMax(a.flags + 1, (unsigned long long)total);
     return;
   }
-  const BoxDev bx = box[s.r];
-  const bool cull = !XF && *nocull == 0ull;
-  if (threadIdx.x == 0) l.total[1] = 0;  // longest list of the brick (made visible by stage's barrier)
-  central_table(s, l.hc, l.central_local, ccap, l.total + 2);
-  stage_each<false>(s, l.hc, total, pos, bx.L, nullptr, l.slot_cell,
+  if (threadIdx.x == 0) total_p[1] = 0;
+  const BoxDev bx = a.box[s.r];
+  stage_each<false>(s, hc, total, a.pos, bx.L, nullptr, cand_all,
                     [&](int c, const Pos4& p, int) { P[c] = double3{p.x, p.y, p.z}; });
-  const int ncentral = l.total[2];
-  if (ncentral > ccap) {  // cannot happen when ccap = measured maximum
-    if (threadIdx.x == 0) atomicMax(flags + 1, (unsigned long long)ncentral);
-    return;
-  }
-  for (int q = threadIdx.x;; q += blockDim.x) {
-    Central a;
-    if (!central_at(l.hc, l.slot_cell, l.central_local, ncentral, q, a)) break;
-    const double xi = P[a.local].x, yi = P[a.local].y, zi = P[a.local].z;
-    const Pos4 pi = {xi, yi, zi, 0.0};
-    const int ix = a.h % s.hx, iy = (a.h / s.hx) % s.hy, iz = a.h / (s.hx * s.hy);
-    int cnt = 0;
-    uint32_t w[4] = {0u, 0u, 0u, 0u};
-    // A hit at slot c goes into the group FIFO w; a full group moves to r and is
-    // stored (when it fits in nmax) after the current stencil row, so that the
-    // wave issues one store per row rather than one per candidate pair.
-    // gp is the atom's next group (bl_index(npad, i, 8 q)); gq its index q.
-    uint32_t r[4] = {0u, 0u, 0u, 0u};
-    uint32_t bw[2] = {0u, 0u}, br[2] = {0u, 0u};  // distance keys of w and r (BINS)
-    bool ready = false;
-    uint16_t* gp = nbr16 + bl_index(npad, a.global, 0);
-    uint8_t* bp = BINS ? bins8 + bl_index(npad, a.global, 0) : nullptr;
-    const int64_t gstep = npad * 8;
-    const int gmax = nmax >> 3;  // groups that fit
-    int gq = 0;
-    auto flush = [&]() {
-      if (gq < gmax) {
-        *reinterpret_cast<uint4*>(gp) = group_interleave(r);
-        if constexpr (BINS) *reinterpret_cast<uint2*>(bp) = bins_interleave(br);
-      }
-      gp += gstep;
-      if constexpr (BINS) bp += gstep;
-      gq++;
-      ready = false;
-    };
-    auto hit = [&](int c, double d2) {
-      fifo_push(w, (uint32_t)c);
-      if constexpr (BINS) {
-        const uint32_t bin = (uint32_t)min(bin_max, (int)((float)d2 * bin_scale));
-        bw[0] = __builtin_amdgcn_alignbit(bw[1], bw[0], 8);
-        bw[1] = __builtin_amdgcn_alignbit(bin, bw[1], 8);
-      }
-      cnt++;
-      if ((cnt & 7) == 0) {
-        if (ready) flush();  // a second full group within one row
-        r[0] = w[0];
-        r[1] = w[1];
-        r[2] = w[2];
-        r[3] = w[3];
-        br[0] = bw[0];
-        br[1] = bw[1];
-        ready = true;
-      }
-    };
-    // The three cells dx = -1, 0, 1 of one (dy, dz) row of the stencil hold
-    // consecutive halo slots, so a row is walked as one slot range: from the first
-    // to the last of its cells that the box test keeps (a culled cell between them
-    // is walked, and its atoms fail the exact test).  Nine walks of about three
-    // cells each, rather than 27 of one, even out the trip counts of the wave's
-    // lanes and halve the odd-count tails of the pairwise walk.
-    for (int dz = -1; dz <= 1; dz++)
-      for (int dy = -1; dy <= 1; dy++) {
-        const int h0 = ((iz + dz) * s.hy + (iy + dy)) * s.hx + ix - 1;
-        int beg = l.hc[h0].lstart;
-        int end = l.hc[h0 + 2].lstart + l.hc[h0 + 2].count;
-        if (cull) {
-          const int gx = s.cx0 - 2 + ix, gy = s.cy0 - 1 + iy + dy, gz = s.cz0 - 1 + iz + dz;
-          const double uy = xsmd_cell_gap(pi.y, bx.lo[1], bx.L[1], g.ny, gy, g.py);
-          const double uz = xsmd_cell_gap(pi.z, bx.lo[2], bx.L[2], g.nz, gz, g.pz);
-          bool keep[3];
-#pragma unroll
-          for (int k = 0; k < 3; k++)
-            keep[k] = xsmd_d2(xsmd_cell_gap(pi.x, bx.lo[0], bx.L[0], g.nx, gx + k, g.px), uy, uz) < rl2;
-          if (!keep[0]) beg = keep[1] ? l.hc[h0 + 1].lstart : l.hc[h0 + 2].lstart;
-          if (!keep[2]) end = keep[1] ? l.hc[h0 + 2].lstart : l.hc[h0 + 1].lstart;
-        }
-        for (int c = beg; c < end; c += 2) {
-          // record c + 1 <= cap exists (the next cell's first atom, or padding)
-          const double3 p0 = P[c], p1 = P[c + 1];
-          double u0 = p0.x - xi, v0 = p0.y - yi, w0 = p0.z - zi;
-          double u1 = p1.x - xi, v1 = p1.y - yi, w1 = p1.z - zi;
-          if constexpr (XF) {
-            xsmd_xform_apply(xf->m, &u0, &v0, &w0);
-            xsmd_xform_apply(xf->m, &u1, &v1, &w1);
-          }
-          const double d0 = xsmd_d2(u0, v0, w0);
-          const double d1 = xsmd_d2(u1, v1, w1);
-          if (d0 < rl2 && c != a.local) hit(c, d0);
-          if (c + 1 < end && d1 < rl2 && c + 1 != a.local) hit(c + 1, d1);
-        }
-        if (ready) flush();
-      }
-    if ((cnt & 7) != 0) {  // the last, partial group: move it down (unused places hold slot 0)
-      for (int k = cnt & 7; k < 8; k++) {
-        fifo_push(w, 0u);
-        bw[0] = __builtin_amdgcn_alignbit(bw[1], bw[0], 8);
-        bw[1] = __builtin_amdgcn_alignbit(0u, bw[1], 8);
-      }
-      r[0] = w[0];
-      r[1] = w[1];
-      r[2] = w[2];
-      r[3] = w[3];
-      br[0] = bw[0];
-      br[1] = bw[1];
-      flush();
-    }
-    nnb[a.global] = cnt;
-    atomicMax(l.total + 1, cnt);
-    if (cnt > nmax) atomicMax(flags, (unsigned long long)cnt);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) brick_rows[b] = l.total[1];
-}
 
-// Orders each atom's block-list entries by their distance keys (written by the
-// build; stable, so equal keys keep ascending slot order), for lists of at most
-// kSortRows entries.  At a given list position the atoms of a wave then look up
-// nearby spline rows, which cuts the cache lines each table gather of the EAM
-// passes touches by about 40 %.  One wave takes eight atoms: each lane loads one
-// 8-entry group (slots and keys) of one atom, the groups go through LDS to one row
-// per atom, and the wave sorts two rows at a time (ballot, popcount, ds_permute).
-constexpr int kSortThreads = 256;
-constexpr int kSortWaveAtoms = 8;
-constexpr int kSortRowWords = 65;  // 64 keys + 1: the lanes of a group load start in distinct banks
-
-__global__ void __launch_bounds__(kSortThreads) k_list_sort(int64_t n, uint16_t* __restrict__ nbr16,
-                                                            const uint8_t* __restrict__ bins8,
-                                                            const int* __restrict__ nnb, int64_t npad, int nbits)
-{
-  __shared__ uint32_t keys[kSortThreads / 64][kSortWaveAtoms][kSortRowWords];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t a0 = ((int64_t)blockIdx.x * (kSortThreads / 64) + w) * kSortWaveAtoms;
-  const int la = lane >> 3, grp = lane & 7;
-  const int64_t a = a0 + la;
-  const int cnt = a < n ? nnb[a] : 0;
-  const bool sorts = cnt >= 2 && cnt <= kSortRows;
-  uint32_t* row = keys[w][la];
-  if (sorts && 8 * grp < cnt) {
-    const int64_t at = bl_index(npad, a, 8 * grp);
-    const uint4 sl = *reinterpret_cast<const uint4*>(nbr16 + at);
-    const uint2 bn = *reinterpret_cast<const uint2*>(bins8 + at);
-    const uint32_t h[4] = {sl.x, sl.y, sl.z, sl.w};
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  uint16_t* cand = cand_all + (size_t)wave * a.cand_cap;
+  const int stride = a.nmax + 1;  // odd, so the group loads of 8 rows start in distinct banks
+  uint32_t* rows = rows_all + (size_t)wave * a.atoms * stride;
+  const int ncell = s.ex * s.ey * s.ez;
+  int nrow = 0;         // lists in the rows
+  int cnt = 0, gi = 0;  // lane k: entries and atom of row k
+  // the collected lists out: counts, then whole groups, 8 lanes per atom and one group
+  // each (places past the count hold whatever the row held; readers stop at the count)
+  const auto flush = [&]() {
+    wave_lds_sync();
+    if (lane < nrow) {
+      a.nnb[gi] = cnt;
+      if (cnt > a.nmax) atomicMax(a.flags, (unsigned long long)cnt);
+    }
+    const int la = lane >> 3, j = lane & 7;
+    const int ca = la < nrow ? min(__shfl(cnt, la), a.nmax) : 0;
+    const int64_t ga = __shfl(gi, la);
+    const uint32_t* row = rows + (la < nrow ? la : 0) * stride;
+    const auto put = [&](int grp, const uint32_t (&e)[8]) {
+      uint32_t o[4];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {  // storage order (0, 2, 4, 6, 1, 3, 5, 7)
-      const int k = 8 * grp + (j < 4 ? 2 * j : 2 * (j - 4) + 1);
-      const uint32_t slot = (h[j >> 1] >> (16 * (j & 1))) & 0xffffu;
-      const uint32_t bin = ((j < 4 ? bn.x : bn.y) >> (8 * (j & 3))) & 0xffu;
-      row[k] = (bin << 16) | slot;
+      for (int k = 0; k < 4; k++) o[k] = (e[2 * k] & 0xffffu) | (e[2 * k + 1] << 16);
+      *reinterpret_cast<uint4*>(a.nbr16 + bl_index(a.npad, ga, 8 * grp)) = group_interleave(o);
+    };
+    const bool sorts = a.sort && ca <= kSortRows;
+    if (__any(sorts)) {
+      uint32_t v[8];
+#pragma unroll
+      for (int r = 0; r < 8; r++) v[r] = j + 8 * r < (sorts ? ca : 0) ? row[j + 8 * r] : 0xffffffffu;
+      sort64(v);
+      if (sorts && 8 * j < ca) put(j, v);
+    }
+    if (!sorts)
+      for (int grp = j; 8 * grp < ca; grp += 8) {
+        uint32_t v[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) v[r] = row[8 * grp + r];
+        put(grp, v);
+      }
+    wave_lds_sync();
+    nrow = 0;
+    cnt = 0;
+  };
+  for (;;) {
+    int cc = 0;
+    if (lane == 0) cc = atomicAdd(total_p + 1, 1);
+    cc = __builtin_amdgcn_readfirstlane(cc);
+    if (cc >= ncell) break;
+    const int ix = 1 + cc % s.ex, iy = 1 + (cc / s.ex) % s.ey, iz = 1 + cc / (s.ex * s.ey);
+    const int h = (iz * s.hy + iy) * s.hx + ix;
+    const int nat = __builtin_amdgcn_readfirstlane(hc[h].count);
+    const int l0 = __builtin_amdgcn_readfirstlane(hc[h].lstart);
+    const int g0 = __builtin_amdgcn_readfirstlane(hc[h].gstart);
+    if (nat == 0) continue;
+    double lx = 1e300, ly = 1e300, lz = 1e300, ux = -1e300, uy = -1e300, uz = -1e300;
+    if constexpr (!XF) {
+      for (int k = lane & 15; k < nat; k += 16) {
+        const double3 p = P[l0 + k];
+        lx = fmin(lx, p.x);
+        ly = fmin(ly, p.y);
+        lz = fmin(lz, p.z);
+        ux = fmax(ux, p.x);
+        uy = fmax(uy, p.y);
+        uz = fmax(uz, p.z);
+      }
+      lx = row16_min(lx);
+      ly = row16_min(ly);
+      lz = row16_min(lz);
+      ux = -row16_min(-ux);
+      uy = -row16_min(-uy);
+      uz = -row16_min(-uz);
+    }
+    // candidates, in ascending slot order; lane k < 9 holds the slots of stencil row k
+    const int rk = min(lane, 8);
+    const int rh = h + ((rk / 3 - 1) * s.hy + (rk % 3 - 1)) * s.hx - 1;
+    const int row_beg = hc[rh].lstart, row_end = hc[rh + 2].lstart + hc[rh + 2].count;
+    int nc = 0;
+    for (int row = 0; row < 9; row++) {
+      const int beg = __builtin_amdgcn_readlane(row_beg, row), end = __builtin_amdgcn_readlane(row_end, row);
+      for (int c0 = beg; c0 < end; c0 += 64) {
+        const int c = c0 + lane;
+        bool keep = c < end;
+        if constexpr (!XF) {
+          const double3 p = P[min(c, a.cap)];
+          const double gx = fmax(fmax(lx - p.x, p.x - ux), 0.0);
+          const double gy = fmax(fmax(ly - p.y, p.y - uy), 0.0);
+          const double gz = fmax(fmax(lz - p.z, p.z - uz), 0.0);
+          keep = keep && xsmd_d2(gx, gy, gz) < a.rl2;
+        }
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
+        const int at = wave_rank(m, nc);
+        if (keep) cand[at] = (uint16_t)c;
+        nc += __popcll(m);
+      }
+    }
+    wave_lds_sync();
+    // T x 64 candidates from t0 on against atoms a0 .. a0 + nb - 1, lists into rows nrow,
+    // nrow + 1, ...; with ALL (every candidate of the cell fits) the full rows go out
+    // between atoms, so the candidates are loaded once per cell
+    const auto test = [&](auto tiles, auto all, int t0, int a0, int nb) {
+      constexpr int T = decltype(tiles)::value;
+      constexpr bool ALL = decltype(all)::value;
+      double cx[T], cy[T], cz[T];
+      int cs[T];
+#pragma unroll
+      for (int t = 0; t < T; t++) {
+        const int k = t0 + 64 * t + lane;
+        cs[t] = k < nc ? (int)cand[k] : a.cap;
+        const double3 p = P[cs[t]];
+        cx[t] = k < nc ? p.x : 1e200;  // no candidate: its d2 is infinite
+        cy[t] = p.y;
+        cz[t] = p.z;
+      }
+      for (int k = 0; k < nb; k++) {
+        const int local = l0 + a0 + k, to_row = ALL ? nrow : nrow + k;
+        const double3 pi = P[local];
+        uint32_t* row = rows + to_row * stride;
+        int base = ALL ? 0 : __builtin_amdgcn_readlane(cnt, to_row);
+        double d2[T];
+        bool in[T];
+        uint32_t* to[T];
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+          double dx = cx[t] - pi.x, dy = cy[t] - pi.y, dz = cz[t] - pi.z;
+          if constexpr (XF) xsmd_xform_apply(a.xf->m, &dx, &dy, &dz);
+          d2[t] = xsmd_d2(dx, dy, dz);
+          in[t] = d2[t] < a.rl2 && cs[t] != local;
+          const unsigned long long m = __builtin_amdgcn_ballot_w64(d2[t] < a.rl2) &
+                                       ~__builtin_amdgcn_ballot_w64(cs[t] == local);
+          to[t] = row + base + min(wave_rank(m, 0), a.nmax - base);  // past the capacity: the row's spare word
+          base += __popcll(m);
+        }
+#pragma unroll
+        for (int t = 0; t < T; t++)
+          if (in[t]) *to[t] = (__float_as_uint((float)d2[t]) & 0xffff0000u) | (uint32_t)cs[t];
+        cnt = lane == to_row ? base : cnt;
+        if constexpr (ALL) {
+          gi = lane == to_row ? g0 + k : gi;
+          if (++nrow == a.atoms) flush();
+        }
+      }
+    };
+    const auto pick = [&](int t0, auto all, int a0, int nb) {
+      const int left = nc - t0;
+      if (left > 384) test(std::integral_constant<int, 8>{}, all, t0, a0, nb);
+      else if (left > 256) test(std::integral_constant<int, 6>{}, all, t0, a0, nb);
+      else if (left > 192) test(std::integral_constant<int, 4>{}, all, t0, a0, nb);
+      else if (left > 128) test(std::integral_constant<int, 3>{}, all, t0, a0, nb);
+      else test(std::integral_constant<int, 2>{}, all, t0, a0, nb);
+    };
+    if (nc <= kBuildTile) {
+      pick(0, std::true_type{}, 0, nat);
+      continue;
+    }
+    for (int a0 = 0; a0 < nat;) {
+      const int nb = min(a.atoms - nrow, nat - a0);
+      for (int t0 = 0; t0 < nc; t0 += kBuildTile) pick(t0, std::false_type{}, a0, nb);
+      if (lane >= nrow && lane < nrow + nb) gi = g0 + a0 + lane - nrow;
+      nrow += nb;
+      a0 += nb;
+      if (nrow == a.atoms) flush();
     }
   }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < kSortWaveAtoms; r += 2) {
-    const int c0 = __shfl(cnt, 8 * r), c1 = __shfl(cnt, 8 * (r + 1));
-    const bool s0 = c0 >= 2 && c0 <= kSortRows, s1 = c1 >= 2 && c1 <= kSortRows;
-    if (!s0 && !s1) continue;  // uniform across the wave
-    uint32_t k0 = (s0 && lane < c0) ? keys[w][r][lane] : 0xffffffffu;
-    uint32_t k1 = (s1 && lane < c1) ? keys[w][r + 1][lane] : 0xffffffffu;
-    wave_radix_sort2(k0, k1, 16, nbits);
-    if (s0 && lane < c0) keys[w][r][lane] = k0;
-    if (s1 && lane < c1) keys[w][r + 1][lane] = k1;
-  }
-  __syncthreads();
-  if (sorts && 8 * grp < cnt) {
-    uint32_t o[4];
-#pragma unroll
-    for (int j2 = 0; j2 < 4; j2++)  // list order (2 j2, 2 j2 + 1)
-      o[j2] = (row[8 * grp + 2 * j2] & 0xffffu) | (row[8 * grp + 2 * j2 + 1] << 16);
-    *reinterpret_cast<uint4*>(nbr16 + bl_index(npad, a, 8 * grp)) = group_interleave(o);
-  }
+  if (nrow > 0) flush();
 }
 
 // Block-local entries -> global (index, image) entries of the same list, in the
@@ -735,28 +801,68 @@ __global__ void __launch_bounds__(256) k_block_to_global(BlockGeom g, const int*
   }
 }
 
-// per-block halo atom count (sizes the LDS of the block kernels)
-__global__ void k_block_halo_max(BlockGeom g, const int* __restrict__ cell_off,
-                                 unsigned long long* __restrict__ out)
+// Sizes the LDS of the block kernels: the most halo atoms and central atoms of a brick,
+// and the most atoms in the 27 cells of a central cell.  One wave per brick, one lane
+// per halo cell (a thread per brick reads its cells one after the other: 33 us for a
+// single brick of 125 cells, against 4 us).
+constexpr int kHaloMaxWaves = 4;
+__global__ void __launch_bounds__(64 * kHaloMaxWaves) k_block_halo_max(BlockGeom g, const int* __restrict__ cell_off,
+                                                                       unsigned long long* __restrict__ out)
 {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= g.nblocks) return;
-  const BlockShape s = block_shape(g, b);
-  int total = 0, central = 0;
-  for (int iz = 0; iz < s.hz; iz++)
-    for (int iy = 0; iy < s.hy; iy++)
-      for (int ix = 0; ix < s.hx; ix++) {
-        int wx, wy, wz, kx, ky, kz;
-        if (!wrap_axis(s.cx0 - 1 + ix, g.nx, g.px, wx, kx) || !wrap_axis(s.cy0 - 1 + iy, g.ny, g.py, wy, ky) ||
-            !wrap_axis(s.cz0 - 1 + iz, g.nz, g.pz, wz, kz))
-          continue;
+  __shared__ int cnt_all[kHaloMaxWaves][kMaxHaloCells];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  int* cnt = cnt_all[wave];
+  int m_total = 0, m_central = 0, m_cand = 0;
+  for (int64_t b = (int64_t)blockIdx.x * kHaloMaxWaves + wave; b < g.nblocks; b += (int64_t)gridDim.x * kHaloMaxWaves) {
+    const BlockShape s = block_shape(g, b);
+    const int nh = s.hx * s.hy * s.hz;
+    int total = 0, central = 0;
+    for (int h = lane; h < nh; h += 64) {
+      const int ix = h % s.hx, iy = (h / s.hx) % s.hy, iz = h / (s.hx * s.hy);
+      int wx, wy, wz, kx, ky, kz, n = 0;
+      if (wrap_axis(s.cx0 - 1 + ix, g.nx, g.px, wx, kx) && wrap_axis(s.cy0 - 1 + iy, g.ny, g.py, wy, ky) &&
+          wrap_axis(s.cz0 - 1 + iz, g.nz, g.pz, wz, kz)) {
         const int64_t c = (int64_t)s.r * g.ncell_rep + ((int64_t)wz * g.ny + wy) * g.nx + wx;
-        const int n = cell_off[c + 1] - cell_off[c];
-        total += n;
-        if (ix >= 1 && ix <= s.ex && iy >= 1 && iy <= s.ey && iz >= 1 && iz <= s.ez) central += n;
+        n = cell_off[c + 1] - cell_off[c];
       }
-  atomicMax(out, (unsigned long long)total);
-  atomicMax(out + 1, (unsigned long long)central);
+      cnt[h] = n;
+      total += n;
+      if (ix >= 1 && ix <= s.ex && iy >= 1 && iy <= s.ey && iz >= 1 && iz <= s.ez) central += n;
+    }
+    wave_lds_sync();
+    const int ncell = s.ex * s.ey * s.ez;
+    for (int cc = lane; cc < ncell; cc += 64) {
+      const int h = ((1 + cc / (s.ex * s.ey)) * s.hy + 1 + (cc / s.ex) % s.ey) * s.hx + 1 + cc % s.ex;
+      int n = 0;
+      for (int row = 0; row < 9; row++) {
+        const int h0 = h + ((row / 3 - 1) * s.hy + (row % 3 - 1)) * s.hx;
+        n += cnt[h0 - 1] + cnt[h0] + cnt[h0 + 1];
+      }
+      m_cand = max(m_cand, n);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      total += __shfl_xor(total, off);
+      central += __shfl_xor(central, off);
+    }
+    m_total = max(m_total, total);
+    m_central = max(m_central, central);
+    wave_lds_sync();
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) m_cand = max(m_cand, __shfl_xor(m_cand, off));
+  __shared__ int best[kHaloMaxWaves][3];
+  if (lane == 0) {
+    best[wave][0] = m_total;
+    best[wave][1] = m_central;
+    best[wave][2] = m_cand;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    int v = best[0][threadIdx.x];
+    for (int w = 1; w < kHaloMaxWaves; w++) v = max(v, best[w][threadIdx.x]);
+    atomicMax(out + threadIdx.x, (unsigned long long)v);
+  }
 }
 
 __global__ void k_cell_offsets(int64_t n, int64_t ncell, const uint32_t* __restrict__ keys, int* __restrict__ off)
@@ -1410,14 +1516,16 @@ void block_setup(Ctx& c)
   double bound = c.block_atoms;
   for (int attempt = 0;; attempt++) {
     block_shape_choose(c, g, bound, per_cell);
-    XS_HIP(hipMemsetAsync(c.dscalar.p + 2, 0, 2 * sizeof(unsigned long long), c.stream));
-    k_block_halo_max<<<grid_for(g.nblocks), kBlock, 0, c.stream>>>(g, c.cell_off.p, c.dscalar.p + 2);
+    XS_HIP(hipMemsetAsync(c.dscalar.p + 2, 0, 3 * sizeof(unsigned long long), c.stream));
+    k_block_halo_max<<<(unsigned)std::min<int64_t>(512, (g.nblocks + kHaloMaxWaves - 1) / kHaloMaxWaves),
+                       64 * kHaloMaxWaves, 0, c.stream>>>(g, c.cell_off.p, c.dscalar.p + 2);
     XS_HIP(hipGetLastError());
-    XS_HIP(hipMemcpyAsync(c.hscalar + 2, c.dscalar.p + 2, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+    XS_HIP(hipMemcpyAsync(c.hscalar + 2, c.dscalar.p + 2, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                           c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
     c.bcap = (int)((c.hscalar[2] + 63) / 64 * 64);
     c.bcentral = (int)c.hscalar[3];
+    c.bcand = (int)c.hscalar[4];
     const size_t budget = c.block_atoms_set ? kBlockLdsLimit : std::min(kBlockLdsLimit, kLdsPerCu / 3);
     if (block_lds_bytes(c, true, true) <= budget || g.nh_max == 27 || attempt == 6) break;
     // the densest halo set the capacity: size the next shape for that density
@@ -1444,47 +1552,56 @@ unsigned block_grid(const Ctx& c)
   return (unsigned)((c.bgeom.nblocks + 7) / 8 * 8);
 }
 
-// Block list build, then (unless XSMD_LIST_SORT=0) the distance order of each list
-// of at most 64 entries: the build writes an 8-bit distance key per entry
-// (2^bits bins uniform in d^2 over [0, rl^2)), k_list_sort orders by it.
-void block_build(Ctx& c, double rl2)
+// LDS of a build launch that collects `atoms` lists per wave
+static size_t build_lds_bytes(const Ctx& c, int atoms)
 {
-  const size_t lds = build_rec_bytes(c.bcap) + (size_t)c.bgeom.nh_max * sizeof(HaloCell) + 4 * sizeof(int) +
-                     (size_t)(c.bcap + c.bcentral) * sizeof(uint16_t);
-  const bool sorted = !c.list_sort_disabled;
-  const int bits = std::max(1, std::min(c.sort_bits, 8));
-  const float bin_scale = (float)((double)(1 << bits) / rl2);
+  return build_rec_bytes(c.bcap) + (size_t)c.bgeom.nh_max * sizeof(HaloCell) + 4 * sizeof(int) +
+         build_cand_bytes(c.bcap, c.bcand) + (size_t)kBuildWaves * atoms * (c.nmax + 1) * sizeof(uint32_t);
+}
+
+// Block list build; false when its LDS does not fit a workgroup (then nothing was
+// built).  The lists of fewer atoms are collected at once where long lists need it.
+bool block_build(Ctx& c, double rl2)
+{
+  BuildArgs a;
+  a.g = c.bgeom;
+  a.cell_off = c.cell_off.p;
+  a.pos = c.pos.p;
+  a.box = c.box_d.p;
+  a.xf = c.xf_dev();
+  a.rl2 = rl2;
+  a.npad = c.npad;
+  a.cap = c.bcap;
+  a.cand_cap = c.bcand;
+  a.sort = !c.list_sort_disabled;
+  a.flags = c.dscalar.p;
   for (int attempt = 0; attempt < 2; attempt++) {
+    a.atoms = kBuildAtoms;
+    while (a.atoms > 1 && build_lds_bytes(c, a.atoms) > kBlockLdsLimit) a.atoms /= 2;
+    const size_t lds = build_lds_bytes(c, a.atoms);
+    if (lds > c.lds_max) return false;
     c.nbr16.reserve((size_t)c.nmax * c.npad);
-    if (sorted) c.bins8.reserve((size_t)c.nmax * c.npad);
     c.nnb.reserve(c.npad);
-    c.brick_rows.reserve(c.bgeom.nblocks);
+    a.nbr16 = c.nbr16.p;
+    a.nnb = c.nnb.p;
+    a.nmax = c.nmax;
+    const auto k = a.xf ? k_block_build<true> : k_block_build<false>;
+    if (lds > kBlockLdsLimit)
+      XS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)lds));
     XS_HIP(hipMemsetAsync(c.dscalar.p, 0, 2 * sizeof(unsigned long long), c.stream));
-    auto k = c.xf_dev() ? (sorted ? k_block_build<true, true> : k_block_build<false, true>)
-                     : (sorted ? k_block_build<true, false> : k_block_build<false, false>);
-    k<<<block_grid(c), kBuildThreads, lds, c.stream>>>(c.bgeom, c.cell_off.p, c.pos.p, c.box_d.p, rl2, c.nbr16.p,
-                                                       c.nnb.p, c.nmax, c.npad, c.bcap, c.bcentral, c.bgeom.nh_max,
-                                                       c.dscalar.p + 4, c.brick_rows.p, c.dscalar.p,
-                                                       sorted ? c.bins8.p : nullptr, bin_scale, (1 << bits) - 1,
-                                                       c.xf_dev());
+    k<<<block_grid(c), kBuildThreads, lds, c.stream>>>(a);
     XS_HIP(hipGetLastError());
     XS_HIP(hipMemcpyAsync(c.hscalar, c.dscalar.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                           c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
-    if (c.hscalar[1] != 0) throw Error(XS_E_STATE, "block halo or central atoms exceed their measured capacity");
+    if (c.hscalar[1] != 0) throw Error(XS_E_STATE, "block halo exceeds its measured capacity");
     const unsigned long long need = c.hscalar[0];
-    if (need == 0) {
-      if (sorted && c.n > 0) {
-        const int64_t per_block = (int64_t)(kSortThreads / 64) * kSortWaveAtoms;
-        const unsigned grid = (unsigned)((c.n + per_block - 1) / per_block);
-        k_list_sort<<<grid, kSortThreads, 0, c.stream>>>(c.n, c.nbr16.p, c.bins8.p, c.nnb.p, c.npad, bits);
-        XS_HIP(hipGetLastError());
-      }
-      return;
-    }
+    if (need == 0) return true;
     if (attempt == 1) throw Error(XS_E_STATE, "neighbour list overflow after resize");
     c.nmax = (int)((need + 7) / 8 * 8 + 8);
   }
+  return false;
 }
 
 void block_to_global(Ctx& c)

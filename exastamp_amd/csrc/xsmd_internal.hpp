@@ -318,22 +318,20 @@ struct Ctx {
   DBuf<int> nnb_half;
   bool half_valid = false;
   DBuf<uint16_t> nbr16;
-  DBuf<uint8_t> bins8;  // distance keys of the block-list entries (for the sort)
   DBuf<int> cell_off;              // first atom of each cell, ncell_tot + 1
   BlockGeom bgeom{};
   int bcap = 0;                    // LDS slots per block (max halo atoms, rounded)
   int bcentral = 0;                // max central atoms per block
-  DBuf<int> brick_rows;            // longest list of each block
+  int bcand = 0;                   // max atoms in the 27 cells of a central cell
   int num_cu = 0;           // CUs of the device (persistent grids)
   size_t lds_max = 65536;   // dynamic LDS one workgroup may use
   bool list_sort_disabled = false;  // XSMD_LIST_SORT=0: block lists stay in stencil order
-  int sort_bits = 7;                // distance keys of the list sort: 2^sort_bits bins over [0, rl^2), <= 8
   bool s_table_disabled = false;    // XSMD_EAM_S_TABLE=0: the FP32 passes read the knot rows
   bool drift_done = false;  // the last force launch applied ForceEpilogue::drift
 
   // small device scalars + pinned host mirror
-  DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..3] halo maxima,
-                                     // [4] atom outside its cell, [5] fused-drift rebuild flag,
+  DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..4] halo maxima,
+                                     // [5] fused-drift rebuild flag,
                                      // [6] block-pass capacity exceeded
   unsigned long long* hscalar = nullptr;
   hipEvent_t flag_event = nullptr;  // the deferred copy of dscalar[6] to hscalar[6] (check_or_defer_overflow)
@@ -384,7 +382,7 @@ void block_setup(Ctx& c);
 bool block_feasible(const Ctx& c);
 size_t block_lds_bytes(const Ctx& c, bool with_type, bool with_w);
 unsigned block_grid(const Ctx& c);
-void block_build(Ctx& c, double rl2);
+bool block_build(Ctx& c, double rl2);
 void block_to_global(Ctx& c);
 void ensure_global_list(Ctx& c);
 // the half list (nbr_half / nnb_half) of the current list
