@@ -829,7 +829,7 @@ xs_status xs_md_run(xs_ctx* h, int potential, int nsteps, double dt, double rcut
       }
       if (c.prof.on) c.prof.flush();
       if (over) {
-        build_neighbor_list(c, rcut, skin, true);
+        build_neighbor_list(c, rcut, skin, true, false);  // forces() writes new accelerations
         rebuilds++;
       }
       drifted = forces(step, 0.5 * dt, step < nsteps);

@@ -865,15 +865,6 @@ __global__ void __launch_bounds__(64 * kHaloMaxWaves) k_block_halo_max(BlockGeom
   }
 }
 
-__global__ void k_cell_offsets(int64_t n, int64_t ncell, const uint32_t* __restrict__ keys, int* __restrict__ off)
-{
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i > n) return;
-  const int64_t hi = (i == n) ? ncell : (int64_t)keys[i];
-  const int64_t lo = (i == 0) ? -1 : (int64_t)keys[i - 1];
-  for (int64_t c = lo + 1; c <= hi; c++) off[c] = (int)i;
-}
-
 // ---------------------------------------------------------------------------
 // EAM passes on the block list
 // ---------------------------------------------------------------------------
@@ -1454,14 +1445,6 @@ double gather_ceiling(Ctx& c, double rcut, bool force, int level, int reps)
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// cell offsets: off[k] = first atom with cell key >= k, off[ncell] = n
-void cell_offsets(Ctx& c)
-{
-  c.cell_off.reserve(c.ncell_tot + 1);
-  k_cell_offsets<<<grid_for(c.n + 1), kBlock, 0, c.stream>>>(c.n, c.ncell_tot, c.keys2.p, c.cell_off.p);
-  XS_HIP(hipGetLastError());
-}
-
 // Brick shape: the one that stages the fewest halo cells per grid cell (partial
 // bricks at the grid edge count as whole ones) among the shapes whose expected
 // central atoms stay within `bound` (one round of the 256 atom slots of a pass

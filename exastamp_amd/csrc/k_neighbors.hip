@@ -1,7 +1,7 @@
 // k_neighbors.hip -- cell binning, atom re-sort and full neighbour-list build.
 //
 // A rebuild is: wrap atoms into their periodic box, compute each atom's cell,
-// stable radix sort by cell (so the in-cell order is deterministic and equal to
+// stable counting sort by cell (so the in-cell order is deterministic and equal to
 // a stable CPU sort), gather every per-atom array into the new order, find the
 // cell ranges, then one thread per atom scans the 27 surrounding cells and
 // writes the (atom, image) entries within rcut+skin into an ELL list stored
@@ -9,35 +9,149 @@
 // it with coalesced loads.
 #include "xsmd_internal.hpp"
 
-#include <hipcub/hipcub.hpp>
-
 #include <algorithm>
 #include <cmath>
 
 namespace xsmd {
 namespace {
 
-__global__ void k_wrap_cellkey(int64_t n, Pos4* __restrict__ pos, const uint16_t* __restrict__ rep,
-                               const BoxDev* __restrict__ box, int px, int py, int pz, int nx, int ny,
-                               int nz, int64_t ncell_rep, uint32_t* __restrict__ keys,
-                               uint32_t* __restrict__ vals)
+// Re-sort by cell.  A counting sort: the atoms of each cell are counted and numbered in
+// the order the counting happened to take them (k_cell_count), an exclusive sum over the
+// cells gives each cell its range (k_cell_sums, k_cell_offsets), k_cell_place writes the
+// atom indices into the ranges, and k_cell_order puts each at the number of smaller
+// indices in its cell, so the result is the stable sort by cell whatever order the
+// counts were taken in.  That last step reads a cell's members once per atom, which is a
+// small part of the list build's own work per cell.  Four or five launches; a library
+// radix sort of (cell, index) pairs took 8 launches at 4 k atoms and 20 at 1 M
+// (about 150 us there against 57, and 90 against 17 at 4 k).  Leaving the order to k_permute, each atom written to its place,
+// cost more than the launch it saved: its writes lose their coalescing (340 us
+// against 237 + 75 at 8.39 M atoms, 48 against 34 + 16 at 1.05 M).
+
+// Wraps atom i into its box, finds its cell, counts it there: num[i] = its number among
+// the atoms of the cell so far.  Consecutive atoms mostly share a cell (they were sorted
+// at the last build), so a run of equal cells in a wave takes one atomic.
+__global__ void __launch_bounds__(256) k_cell_count(int64_t n, Pos4* __restrict__ pos, const uint16_t* __restrict__ rep,
+                                                    const BoxDev* __restrict__ box, int px, int py, int pz, int nx,
+                                                    int ny, int nz, int64_t ncell_rep, uint32_t* __restrict__ keys,
+                                                    uint32_t* __restrict__ num, uint32_t* __restrict__ count)
 {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int r = rep ? rep[i] : 0;
-  const BoxDev& b = box[r];
-  Pos4 p = load_pos(pos, i);
-  if (px || py || pz) {
-    if (px) p.x = xsmd_wrap(p.x, b.lo[0], b.L[0]);
-    if (py) p.y = xsmd_wrap(p.y, b.lo[1], b.L[1]);
-    if (pz) p.z = xsmd_wrap(p.z, b.lo[2], b.L[2]);
-    store_pos(pos, i, p);
+  const bool live = i < n;
+  uint32_t key = 0xffffffffu;  // no cell has it (fewer than 2^32 cells)
+  if (live) {
+    const int r = rep ? rep[i] : 0;
+    const BoxDev& b = box[r];
+    Pos4 p = load_pos(pos, i);
+    if (px || py || pz) {
+      if (px) p.x = xsmd_wrap(p.x, b.lo[0], b.L[0]);
+      if (py) p.y = xsmd_wrap(p.y, b.lo[1], b.L[1]);
+      if (pz) p.z = xsmd_wrap(p.z, b.lo[2], b.L[2]);
+      store_pos(pos, i, p);
+    }
+    const int cx = xsmd_cell_coord(p.x, b.lo[0], b.inv_cs[0], nx);
+    const int cy = xsmd_cell_coord(p.y, b.lo[1], b.inv_cs[1], ny);
+    const int cz = xsmd_cell_coord(p.z, b.lo[2], b.inv_cs[2], nz);
+    key = (uint32_t)((int64_t)r * ncell_rep + ((int64_t)cz * ny + cy) * nx + cx);
+    keys[i] = key;
   }
-  const int cx = xsmd_cell_coord(p.x, b.lo[0], b.inv_cs[0], nx);
-  const int cy = xsmd_cell_coord(p.y, b.lo[1], b.inv_cs[1], ny);
-  const int cz = xsmd_cell_coord(p.z, b.lo[2], b.inv_cs[2], nz);
-  keys[i] = (uint32_t)((int64_t)r * ncell_rep + ((int64_t)cz * ny + cy) * nx + cx);
-  vals[i] = (uint32_t)i;
+  const int lane = threadIdx.x & 63;
+  const uint32_t before = __shfl_up(key, 1);
+  const unsigned long long heads = __ballot(lane == 0 || key != before);
+  const unsigned long long upto = heads & (~0ull >> (63 - lane));
+  const int head = 63 - __clzll((long long)upto);
+  const unsigned long long after = lane == 63 ? 0ull : heads >> (lane + 1) << (lane + 1);
+  uint32_t base = 0;
+  if (live && lane == head) {
+    const int end = after ? __ffsll((unsigned long long)after) - 1 : 64;
+    base = atomicAdd(count + key, (uint32_t)(end - lane));
+  }
+  base = __shfl(base, head);
+  if (live) num[i] = base + (uint32_t)(lane - head);
+}
+
+constexpr int kScanThreads = 256;
+
+// sum of v over the threads below this one (and the workgroup's total)
+__device__ __forceinline__ uint32_t block_exclusive(uint32_t v, uint32_t& total)
+{
+  __shared__ uint32_t wsum[kScanThreads / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t s = v;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t t = __shfl_up(s, off);
+    if (lane >= off) s += t;
+  }
+  __syncthreads();  // the sums of an earlier call are read
+  if (lane == 63) wsum[w] = s;
+  __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (int k = 0; k < kScanThreads / 64; k++) {
+    if (k < w) before += wsum[k];
+    total += wsum[k];
+  }
+  return before + s - v;
+}
+
+// atoms in each run of `items` cells
+__global__ void __launch_bounds__(kScanThreads) k_cell_sums(int64_t ncell, int64_t items,
+                                                            const uint32_t* __restrict__ count,
+                                                            uint32_t* __restrict__ sums)
+{
+  const int64_t c0 = (int64_t)blockIdx.x * items, c1 = min(c0 + items, ncell);
+  uint32_t v = 0, total;
+  for (int64_t c = c0 + threadIdx.x; c < c1; c += kScanThreads) v += count[c];
+  block_exclusive(v, total);
+  if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+// first atom of each cell, off[ncell] = n; clears the counts for the next sort
+__global__ void __launch_bounds__(kScanThreads) k_cell_offsets(int64_t ncell, int64_t items,
+                                                               uint32_t* __restrict__ count,
+                                                               const uint32_t* __restrict__ sums,
+                                                               int* __restrict__ off)
+{
+  const int64_t c0 = (int64_t)blockIdx.x * items, c1 = min(c0 + items, ncell);
+  uint32_t v = 0, base, total;
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += kScanThreads) v += sums[b];
+  block_exclusive(v, base);
+  for (int64_t c = c0; c < c1; c += kScanThreads) {
+    const int64_t k = c + threadIdx.x;
+    v = 0;
+    if (k < c1) {
+      v = count[k];
+      count[k] = 0;
+    }
+    const uint32_t ex = block_exclusive(v, total);
+    if (k < c1) off[k] = (int)(base + ex);
+    base += total;
+  }
+  if (c1 == ncell && threadIdx.x == 0) off[ncell] = (int)base;
+}
+
+__global__ void k_cell_place(int64_t n, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ num,
+                             const int* __restrict__ off, uint32_t* __restrict__ members)
+{
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) members[off[keys[i]] + num[i]] = (uint32_t)i;
+}
+
+// perm[k] = atom at place k of the stable order, and its cell
+__global__ void k_cell_order(int64_t n, const uint32_t* __restrict__ members, const uint32_t* __restrict__ keys,
+                             const int* __restrict__ off, uint32_t* __restrict__ perm,
+                             uint32_t* __restrict__ keys_out)
+{
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const uint32_t p = members[k];
+  const uint32_t key = keys[p];
+  const int o0 = off[key], o1 = off[key + 1];
+  int64_t i = o0;
+  for (int o = o0; o < o1; o++) i += members[o] < p;
+  perm[i] = p;
+  keys_out[k] = key;  // places k and i are in the same cell
 }
 
 struct PermuteArgs {
@@ -56,9 +170,11 @@ struct PermuteArgs {
   uint16_t* rep_dst;
 };
 
-// Gather every per-atom array into the new order; the new positions also become
-// the reference positions of the displacement check.
-__global__ void k_permute(int64_t n, const uint32_t* __restrict__ perm, PermuteArgs a)
+// Gather every per-atom array into the new order (ND of the six velocity and
+// acceleration components; a caller about to overwrite the accelerations leaves them
+// out); the new positions also become the reference positions of the displacement check.
+template <int ND>
+__global__ void __launch_bounds__(256) k_permute(int64_t n, const uint32_t* __restrict__ perm, PermuteArgs a)
 {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -69,7 +185,7 @@ __global__ void k_permute(int64_t n, const uint32_t* __restrict__ perm, PermuteA
   a.rry[i] = q.y;
   a.rrz[i] = q.z;
 #pragma unroll
-  for (int d = 0; d < 6; d++) a.dst[d][i] = a.src[d][p];
+  for (int d = 0; d < ND; d++) a.dst[d][i] = a.src[d][p];
   a.type_dst[i] = a.type_src[p];
   a.id_dst[i] = a.id_src[p];
   if (a.rep_src) a.rep_dst[i] = a.rep_src[p];
@@ -195,7 +311,7 @@ __global__ void k_pair_count(int64_t n, int64_t npad, const Pos4* __restrict__ p
 
 }  // namespace
 
-void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block)
+void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block, bool keep_accel)
 {
   ProfScope prof(c.prof, c.stream, XS_PROF_NEIGHBORS);
   const int64_t n = c.n;
@@ -229,19 +345,32 @@ void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block)
   if (c.ncell_tot >= (int64_t)1 << 32) throw Error(XS_E_LIMIT, "too many cells");
 
   const unsigned g = grid_for(n);
-  k_wrap_cellkey<<<g, kBlock, 0, c.stream>>>(n, c.pos.p, c.has_rep ? c.rep.p : nullptr, c.box_d.p,
-                                             c.periodic[0], c.periodic[1], c.periodic[2], c.nc[0], c.nc[1],
-                                             c.nc[2], c.ncell_rep, c.keys.p, c.vals.p);
+  c.cell_off.reserve(c.ncell_tot + 1);
+  if (c.cell_count.n < (size_t)c.ncell_tot || !c.counts_clear) {
+    c.cell_count.reserve(c.ncell_tot);
+    XS_HIP(hipMemsetAsync(c.cell_count.p, 0, sizeof(uint32_t) * c.cell_count.n, c.stream));
+  }
+  c.counts_clear = false;  // until k_cell_offsets, which clears them, is queued
+  k_cell_count<<<g, kBlock, 0, c.stream>>>(n, c.pos.p, c.has_rep ? c.rep.p : nullptr, c.box_d.p, c.periodic[0],
+                                           c.periodic[1], c.periodic[2], c.nc[0], c.nc[1], c.nc[2], c.ncell_rep,
+                                           c.keys.p, c.vals.p, c.cell_count.p);
   XS_HIP(hipGetLastError());
-
-  int nbits = 1;
-  while (((int64_t)1 << nbits) < c.ncell_tot) nbits++;
-  size_t tmp_bytes = 0;
-  XS_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, c.keys.p, c.keys2.p, c.vals.p,
-                                            c.vals2.p, (int)n, 0, nbits, c.stream));
-  c.sort_tmp.reserve(tmp_bytes);
-  XS_HIP(hipcub::DeviceRadixSort::SortPairs(c.sort_tmp.p, tmp_bytes, c.keys.p, c.keys2.p, c.vals.p,
-                                            c.vals2.p, (int)n, 0, nbits, c.stream));
+  // runs of at least 2048 cells, at most 1024 of them (each workgroup adds up the sums
+  // of the runs before its own)
+  const int64_t items = std::max<int64_t>(2048, (c.ncell_tot + 1023) / 1024);
+  const unsigned runs = (unsigned)((c.ncell_tot + items - 1) / items);
+  c.cell_sums.reserve(1024);
+  if (runs > 1) {
+    k_cell_sums<<<runs, kScanThreads, 0, c.stream>>>(c.ncell_tot, items, c.cell_count.p, c.cell_sums.p);
+    XS_HIP(hipGetLastError());
+  }
+  k_cell_offsets<<<runs, kScanThreads, 0, c.stream>>>(c.ncell_tot, items, c.cell_count.p, c.cell_sums.p, c.cell_off.p);
+  XS_HIP(hipGetLastError());
+  c.counts_clear = true;
+  k_cell_place<<<g, kBlock, 0, c.stream>>>(n, c.keys.p, c.vals.p, c.cell_off.p, c.vals2.p);
+  XS_HIP(hipGetLastError());
+  k_cell_order<<<g, kBlock, 0, c.stream>>>(n, c.vals2.p, c.keys.p, c.cell_off.p, c.vals.p, c.keys2.p);
+  XS_HIP(hipGetLastError());
 
   PermuteArgs pa{};
   pa.pos_src = c.pos.p;
@@ -261,22 +390,22 @@ void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block)
   pa.id_dst = c.id2.p;
   pa.rep_src = c.has_rep ? c.rep.p : nullptr;
   pa.rep_dst = c.has_rep ? c.rep2.p : nullptr;
-  k_permute<<<g, kBlock, 0, c.stream>>>(n, c.vals2.p, pa);
+  (keep_accel ? k_permute<6> : k_permute<3>)<<<g, kBlock, 0, c.stream>>>(n, c.vals.p, pa);
   XS_HIP(hipGetLastError());
   c.pos.swap(c.pos2);
   c.vx.swap(c.vx2);
   c.vy.swap(c.vy2);
   c.vz.swap(c.vz2);
-  c.ax.swap(c.ax2);
-  c.ay.swap(c.ay2);
-  c.az.swap(c.az2);
+  if (keep_accel) {
+    c.ax.swap(c.ax2);
+    c.ay.swap(c.ay2);
+    c.az.swap(c.az2);
+  }
   c.type.swap(c.type2);
   c.id.swap(c.id2);
   if (c.has_rep) c.rep.swap(c.rep2);
   c.rho_state = RhoState::None;  // per-atom EAM state is in the old order
   c.rho_ckpt = false;
-
-  cell_offsets(c);
 
   // list capacity: estimate from the density, grow to the measured maximum on overflow
   if (c.nmax == 0) {

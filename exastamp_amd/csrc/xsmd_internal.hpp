@@ -298,7 +298,8 @@ struct Ctx {
   int nc[3] = {1, 1, 1};
   int64_t ncell_rep = 1, ncell_tot = 1;
   DBuf<uint32_t> keys, keys2, vals, vals2;
-  DBuf<uint8_t> sort_tmp;
+  DBuf<uint32_t> cell_count, cell_sums;  // atoms per cell (all 0 between builds) and per run of cells
+  bool counts_clear = false;
 
   // neighbour list, ELL column-major: nbr[k*npad + i], k < nnb[i] <= nmax
   DBuf<uint32_t> nbr;
@@ -374,10 +375,10 @@ inline bool eam_multi(const Ctx& c) { return c.eam.nel > 1 || (c.eam_types & 1u)
 
 // ---- launches (k_neighbors.hip) ----
 // prefer_block: build the cell-block list when its LDS footprint allows
-void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block = false);
+// keep_accel = false: the accelerations are about to be overwritten and stay behind
+void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block = false, bool keep_accel = true);
 
 // ---- cell blocks (k_block.hip) ----
-void cell_offsets(Ctx& c);
 void block_setup(Ctx& c);
 bool block_feasible(const Ctx& c);
 size_t block_lds_bytes(const Ctx& c, bool with_type, bool with_w);
