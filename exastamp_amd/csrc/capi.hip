@@ -15,7 +15,6 @@ Ctx::~Ctx()
 {
   if (hscalar) (void)hipHostFree(hscalar);
   if (hthermo) (void)hipHostFree(hthermo);
-  if (flag_event) (void)hipEventDestroy(flag_event);
   if (own_stream) (void)hipStreamDestroy(own_stream);
 }
 
@@ -28,7 +27,6 @@ xs_status guarded(xs_ctx* h, F&& f)
   if (!c) return XS_E_ARG;
   try {
     XS_HIP(hipSetDevice(c->device));
-    poll_pass_overflow(*c, false);
     f(*c);
     c->err.clear();
     return XS_OK;
@@ -173,7 +171,6 @@ xs_status xs_ctx_create(int device, xs_ctx** out)
     thermo_scratch_init(device);
     XS_HIP(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
     c->stream = c->own_stream;
-    XS_HIP(hipEventCreateWithFlags(&c->flag_event, hipEventDisableTiming));
     XS_HIP(hipHostMalloc((void**)&c->hscalar, 8 * sizeof(unsigned long long), hipHostMallocDefault));
     XS_HIP(hipHostMalloc((void**)&c->hthermo, 27 * sizeof(double), hipHostMallocDefault));
     c->dscalar.reserve(8);
@@ -229,7 +226,6 @@ void switch_stream(Ctx& c, hipStream_t next)
   // work queued so far stays ahead of what comes next
   XS_HIP(hipStreamSynchronize(c.stream));
   c.stream = next;
-  poll_pass_overflow(c, true);
 }
 }  // namespace
 
@@ -247,8 +243,7 @@ xs_status xs_synchronize(xs_ctx* h)
 {
   return guarded(h, [&](Ctx& c) {
     XS_HIP(hipStreamSynchronize(c.stream));
-    poll_pass_overflow(c, true);
-  });
+    });
 }
 
 xs_status xs_device_memory(xs_ctx* h, size_t* free_bytes, size_t* total_bytes)
@@ -506,7 +501,6 @@ xs_status xs_lj_compute_force(xs_ctx* h, double epsilon, double sigma, double rc
     require_list(c);
     require(rcut <= c.list_rcut + c.list_skin, XS_E_ARG, "rcut exceeds the neighbour-list radius");
     launch_lj(c, epsilon, sigma, rcut, flags, ForceEpilogue{});
-    check_or_defer_overflow(c);
   });
 }
 
@@ -554,7 +548,6 @@ xs_status xs_lj_multi_force(xs_ctx* h, int ntypes, const double* epsilon, const 
     c.ljm_ntypes = ntypes;
     c.ljm_rcmax = rcmax;
     launch_lj_multi(c, flags);
-    check_or_defer_overflow(c);
   });
 }
 
@@ -588,7 +581,6 @@ xs_status xs_eam_alloy_force(xs_ctx* h, double rcut, int eam_rho, int eam_rho2em
       require(rcut <= c.list_rcut + c.list_skin, XS_E_ARG, "rcut exceeds the neighbour-list radius");
     }
     launch_eam(c, rcut, eam_rho != 0, eam_rho2emb != 0, eam_force != 0, flags, ForceEpilogue{});
-    check_or_defer_overflow(c);
   });
 }
 
@@ -820,12 +812,10 @@ xs_status xs_md_run(xs_ctx* h, int potential, int nsteps, double dt, double rcut
         std::memcpy(&d2, &c.hscalar[1], sizeof(double));
         over = d2 > thr2;
       } else {  // the force pass of the previous step moved the atoms and tested them
-        // the rebuild flag and the block passes' capacity flag in one copy
-        XS_HIP(hipMemcpyAsync(c.hscalar + 5, c.dscalar.p + 5, 2 * sizeof(unsigned long long),
-                              hipMemcpyDeviceToHost, c.stream));
+        XS_HIP(hipMemcpyAsync(c.hscalar + 5, c.dscalar.p + 5, sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                              c.stream));
         XS_HIP(hipStreamSynchronize(c.stream));
         over = c.hscalar[5] != 0;
-        if (c.hscalar[6] != 0) check_pass_overflow(c);
       }
       if (c.prof.on) c.prof.flush();
       if (over) {
@@ -836,7 +826,6 @@ xs_status xs_md_run(xs_ctx* h, int potential, int nsteps, double dt, double rcut
     }
     XS_HIP(hipStreamSynchronize(c.stream));
     const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    check_pass_overflow(c);
     if (c.prof.on) c.prof.flush();
     if (stats) {
       stats->steps = nsteps;

@@ -154,31 +154,14 @@ __device__ int build_halo(const BlockGeom& g, const BlockShape& s, const int* __
   return *total_out;
 }
 
-// halo cell holding local slot c (binary search over lstart)
-__device__ __forceinline__ int find_cell(const HaloCell* hc, int nh, int c)
-{
-  int lo = 0, hi = nh - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (hc[mid].lstart <= c) lo = mid;
-    else hi = mid - 1;
-  }
-  // the last cell starting at or before c: among cells sharing one lstart only the
-  // last can be non-empty, so this is the cell that holds slot c
-  return lo;
-}
-
-// Stage halo atoms: f(c, p, j) for slot c, position p (+ image shift; under a
-// non-identity xform mapped to physical space, so that the passes' displacements
-// are physical) and, with WITH_W, w (else 0: the 24 bytes of x, y, z are read, not
-// the whole record), global index j; ends with __syncthreads().  slot_cell (total <= its capacity)
-// first receives the halo cell of every slot, so that a thread finds the cell of
-// a slot with one LDS read instead of a binary search over the halo table.
-// (Issuing several slots' position loads per thread before using them measured
-// slower: the force pass lost 4 %.)
-template <bool WITH_W, class F>
-__device__ void stage_each(const BlockShape& s, const HaloCell* hc, int total, const Pos4* __restrict__ pos,
-                           const double* L, const XformDev* xf, uint16_t* slot_cell, F f)
+// Halo atoms of a brick for the list build: f(c, p, e) for slot c, position p (+ image
+// shift) and staging entry e (global index and image, encoded like a neighbour entry);
+// ends with __syncthreads().  slot_cell (total <= its capacity) first receives the halo
+// cell of every slot, so that a thread finds the cell of a slot with one LDS read
+// instead of a binary search over the halo table.
+template <class F>
+__device__ void stage_cells(const BlockShape& s, const HaloCell* hc, int total, const Pos4* __restrict__ pos,
+                            const double* L, uint16_t* slot_cell, F f)
 {
   const int nh = s.hx * s.hy * s.hz;
   for (int h = threadIdx.x; h < nh; h += blockDim.x) {
@@ -188,134 +171,19 @@ __device__ void stage_each(const BlockShape& s, const HaloCell* hc, int total, c
   __syncthreads();
   for (int c = threadIdx.x; c < total; c += blockDim.x) {
     const HaloCell e = hc[slot_cell[c]];
-    const int j = e.gstart + (c - e.lstart);
-    Pos4 p;
-    if constexpr (WITH_W) {
-      p = load_pos(pos, j);
-    } else {
-      const double* q = reinterpret_cast<const double*>(pos + j);
-      const double2 a = *reinterpret_cast<const double2*>(q);
-      p = {a.x, a.y, q[2], 0.0};
-    }
+    const uint32_t j = (uint32_t)(e.gstart + (c - e.lstart));
+    const double* q = reinterpret_cast<const double*>(pos + j);
+    const double2 xy = *reinterpret_cast<const double2*>(q);
+    Pos4 p = {xy.x, xy.y, q[2], 0.0};
+    const uint32_t code = (uint32_t)e.img << XSMD_NBR_INDEX_BITS;
     if (e.img) {
-      const uint32_t code = (uint32_t)e.img << XSMD_NBR_INDEX_BITS;
       p.x = xsmd_image(p.x, xsmd_nbr_img_x(code), L[0]);
       p.y = xsmd_image(p.y, xsmd_nbr_img_y(code), L[1]);
       p.z = xsmd_image(p.z, xsmd_nbr_img_z(code), L[2]);
     }
-    if (xf) xsmd_xform_apply(xf->m, &p.x, &p.y, &p.z);
-    f(c, p, j);
+    f(c, p, j | code);
   }
   __syncthreads();
-}
-
-// Stage halo atoms into the records (and types when requested), and the far record
-// at slot cap: list entries past an atom's count point there (lslots), so their
-// displacement is finite and longer than any cutoff, and the passes mask them by
-// d2 <= rc2 alone.  It lies at least 10^4 A from every staged position (which are
-// within the box and its images) and close enough that its knot index fits an int.
-__device__ void stage(const BlockShape& s, const HaloCell* hc, int total, const Pos4* __restrict__ pos,
-                      const BoxDev& box, const XformDev* xf, const uint8_t* __restrict__ type, const LRec& rec,
-                      uint8_t* ltype, uint16_t* slot_cell, int cap)
-{
-  const double* L = box.L;
-  if (threadIdx.x == 0) {  // visible after stage_each's barriers
-    const double far = 4.0 * (fabs(box.lo[0]) + fabs(box.lo[1]) + fabs(box.lo[2]) + L[0] + L[1] + L[2]) + 1e4;
-    Pos4 f = {far, far, far, 0.0};
-    if (xf) {
-      xsmd_xform_apply(xf->m, &f.x, &f.y, &f.z);
-      const double g = 1e4 + 4.0 * fabs(f.x - far) + 4.0 * fabs(f.y - far) + 4.0 * fabs(f.z - far);
-      f = {f.x + g, f.y + g, f.z + g, 0.0};  // still far in physical space
-    }
-    double* r = rec.xyz + 3 * cap;
-    r[0] = f.x;
-    r[1] = f.y;
-    r[2] = f.z;
-    if (rec.has_w) rec.w[cap] = 0.0;
-    if (ltype) ltype[cap] = 0;
-  }
-  const auto put = [&](int c, const Pos4& p, int j) {
-    rec.put(c, p);
-    if (ltype) ltype[c] = type[j];
-  };
-  if (rec.has_w) stage_each<true>(s, hc, total, pos, L, xf, slot_cell, put);
-  else stage_each<false>(s, hc, total, pos, L, xf, slot_cell, put);
-}
-
-// Central atom q of the block: its halo cell h, local slot and global index.
-struct Central {
-  int h, local;
-  int64_t global;
-};
-
-__device__ __forceinline__ bool central_atom(const BlockShape& s, const HaloCell* hc, int q, Central& out)
-{
-  // central cells are ix in [1, ex], iy in [1, ey], iz in [1, ez]; walk rows
-  for (int iz = 1; iz <= s.ez; iz++)
-    for (int iy = 1; iy <= s.ey; iy++) {
-      const int h0 = (iz * s.hy + iy) * s.hx + 1;
-      const int h1 = h0 + s.ex - 1;
-      const int n = hc[h1].lstart + hc[h1].count - hc[h0].lstart;
-      if (q < n) {
-        const int local = hc[h0].lstart + q;
-        int h = h0;
-        while (hc[h].lstart + hc[h].count <= local) h++;
-        out.h = h;
-        out.local = local;
-        out.global = (int64_t)hc[h0].gstart + q;
-        return true;
-      }
-      q -= n;
-    }
-  return false;
-}
-
-// Local slots of the central atoms in q order (the order of central_atom):
-// central_local[q] for q < count, count in *count_out.  Wave 0 takes one central
-// row (iz, iy) per lane, scans the row lengths with shuffles and writes the rows'
-// slots; entries beyond ccap are not written (the caller checks count <= ccap).
-// The caller's next __syncthreads publishes the table.
-__device__ void central_table(const BlockShape& s, const HaloCell* hc, uint16_t* central_local, int ccap,
-                              int* count_out)
-{
-  if (threadIdx.x >= 64) return;
-  const int lane = threadIdx.x;
-  const int nrows = s.ez * s.ey;
-  int carry = 0;
-  for (int base = 0; base < nrows; base += 64) {
-    const int r = base + lane;
-    int len = 0, l0 = 0;
-    if (r < nrows) {
-      const int iz = 1 + r / s.ey, iy = 1 + r % s.ey;
-      const int h0 = (iz * s.hy + iy) * s.hx + 1;
-      const int h1 = h0 + s.ex - 1;
-      l0 = hc[h0].lstart;
-      len = hc[h1].lstart + hc[h1].count - l0;
-    }
-    int v = len;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int t = __shfl_up(v, off);
-      if (lane >= off) v += t;
-    }
-    const int q0 = carry + v - len;
-    for (int k = 0; k < len && q0 + k < ccap; k++) central_local[q0 + k] = (uint16_t)(l0 + k);
-    carry += __shfl(v, 63);
-  }
-  if (lane == 0) *count_out = carry;
-}
-
-// central atom q from the tables (slot_cell and central_local filled)
-__device__ __forceinline__ bool central_at(const HaloCell* hc, const uint16_t* slot_cell,
-                                           const uint16_t* central_local, int count, int q, Central& out)
-{
-  if (q >= count) return false;
-  const int local = central_local[q];
-  const int h = slot_cell[local];
-  out.h = h;
-  out.local = local;
-  out.global = (int64_t)hc[h].gstart + (local - hc[h].lstart);
-  return true;
 }
 
 __device__ __forceinline__ int64_t lblock()
@@ -324,35 +192,94 @@ __device__ __forceinline__ int64_t lblock()
   return (int64_t)(b & 7u) * (g >> 3) + (b >> 3);
 }
 
-struct LdsLayout {
-  LRec rec;
-  HaloCell* hc;
-  uint8_t* ltype;
-  int* total;
-  uint16_t* slot_cell;      // halo cell of each slot (staging)
-  uint16_t* central_local;  // local slots of the central atoms
-};
-
-// LDS of the block kernels: records, halo table, counters (total[0] halo atoms,
-// total[2] central atoms), slot cells, central slots, per-record types
-// (block_lds_bytes on the host adds up the same sizes)
-__device__ __forceinline__ LdsLayout lds_layout(int cap, int ccap, int nh_max, bool with_type, bool with_w)
-{
-  extern __shared__ __align__(32) unsigned char smem[];
-  LdsLayout l;
-  const size_t rb = lrec_at(smem, cap, with_w, l.rec);
-  l.hc = reinterpret_cast<HaloCell*>(smem + rb);
-  l.total = reinterpret_cast<int*>(l.hc + nh_max);
-  l.slot_cell = reinterpret_cast<uint16_t*>(l.total + 4);
-  l.central_local = l.slot_cell + cap;
-  l.ltype = with_type ? reinterpret_cast<uint8_t*>(l.central_local + ccap) : nullptr;
-  return l;
-}
-
 // Two lanes per central atom: the two halves of a wave take the same 32 atoms
 // (list build: alternate candidates; EAM passes: even and odd list entries).
 constexpr int kPassThreads = 512;
 constexpr int kPassAtoms = kPassThreads / 2;
+
+// What the block kernels read.  The build leaves each brick's halo as a staging table, so
+// that a pass reaches the positions with one table read instead of rebuilding the halo
+// from the cells (cell ranges, a prefix sum, a slot table, three barriers), and holds
+// nothing but the records in LDS.  The table costs 4 bytes per halo atom (about 24 per
+// atom at 220-atom bricks) written at the build and read by each pass; the chain of
+// waits it removes was longer: 8.39 M EAM atoms, mixed: density pass 0.907 -> 0.761 ms,
+// force pass 1.350 -> 1.258 ms; 1.05 M argon atoms 0.171 -> 0.141 ms per pass.
+struct BlockArgs {
+  const int4* __restrict__ head;       // per brick: halo atoms, central atoms, replica
+  const uint32_t* __restrict__ stage;  // per brick cap entries: global index and image of each slot
+  const uint32_t* __restrict__ cen;    // per brick ccap entries: central atoms (global index)
+  const uint16_t* __restrict__ cen_slot;  // and their slots
+  const Pos4* __restrict__ pos;
+  const uint8_t* __restrict__ type;
+  const BoxDev* __restrict__ box;
+  const uint16_t* __restrict__ nbr16;
+  const int* __restrict__ nnb;
+  int64_t npad;
+  int64_t nblocks;
+  int cap;   // halo slots (LDS records)
+  int ccap;  // central atoms per brick at most
+  double rc2;
+  const XformDev* xf;  // the staging maps positions to physical space when not NULL
+};
+
+// LDS of the block passes: records, then per-record types (block_lds_bytes on the host
+// adds up the same sizes)
+__device__ __forceinline__ LRec pass_lds(const BlockArgs& a, bool with_type, bool with_w, uint8_t*& ltype)
+{
+  extern __shared__ __align__(32) unsigned char smem[];
+  LRec rec;
+  const size_t rb = lrec_at(smem, a.cap, with_w, rec);
+  ltype = with_type ? smem + rb : nullptr;
+  return rec;
+}
+
+// Stages the halo of brick b (head hd) into the records (and types when asked for):
+// position + image shift, under a non-identity xform mapped to physical space, so that
+// the passes' displacements are physical; w with WITH_W (else the 24 bytes of x, y, z
+// are read, not the whole record).  The far record goes to slot cap: list entries past
+// an atom's count point there (lslots), so their displacement is finite and longer than
+// any cutoff, and the passes mask them by d2 <= rc2 alone.  It lies at least 10^4 A from
+// every staged position (which are within the box and its images) and close enough that
+// its knot index fits an int.  Ends with __syncthreads().
+template <bool WITH_W>
+__device__ __forceinline__ void stage(const BlockArgs& a, int64_t b, const int4& hd, const LRec& rec, uint8_t* ltype)
+{
+  const BoxDev& box = a.box[hd.z];
+  const double* L = box.L;
+  if (threadIdx.x == 0) {
+    const double far = 4.0 * (fabs(box.lo[0]) + fabs(box.lo[1]) + fabs(box.lo[2]) + L[0] + L[1] + L[2]) + 1e4;
+    Pos4 f = {far, far, far, 0.0};
+    if (a.xf) {
+      xsmd_xform_apply(a.xf->m, &f.x, &f.y, &f.z);
+      const double g = 1e4 + 4.0 * fabs(f.x - far) + 4.0 * fabs(f.y - far) + 4.0 * fabs(f.z - far);
+      f = {f.x + g, f.y + g, f.z + g, 0.0};  // still far in physical space
+    }
+    rec.put(a.cap, f);
+    if (ltype) ltype[a.cap] = 0;
+  }
+  const uint32_t* st = a.stage + b * a.cap;
+  for (int c = threadIdx.x; c < hd.x; c += kPassThreads) {
+    const uint32_t e = st[c];
+    const uint32_t j = xsmd_nbr_index(e);
+    Pos4 p;
+    if constexpr (WITH_W) {
+      p = load_pos(a.pos, j);
+    } else {
+      const double* q = reinterpret_cast<const double*>(a.pos + j);
+      const double2 xy = *reinterpret_cast<const double2*>(q);
+      p = {xy.x, xy.y, q[2], 0.0};
+    }
+    if (e >> XSMD_NBR_INDEX_BITS) {
+      p.x = xsmd_image(p.x, xsmd_nbr_img_x(e), L[0]);
+      p.y = xsmd_image(p.y, xsmd_nbr_img_y(e), L[1]);
+      p.z = xsmd_image(p.z, xsmd_nbr_img_z(e), L[2]);
+    }
+    if (a.xf) xsmd_xform_apply(a.xf->m, &p.x, &p.y, &p.z);
+    rec.put(c, p);
+    if (ltype) ltype[c] = a.type[j];
+  }
+  __syncthreads();
+}
 
 // sum of v over the two halves of the wave (lanes l and l ^ 32)
 __device__ __forceinline__ double half_sum(double v) { return v + __shfl_xor(v, 32); }
@@ -561,6 +488,12 @@ struct BuildArgs {
   int cand_cap;  // most atoms in the 27 cells of a central cell
   int atoms;     // lists collected per wave, at most kBuildAtoms
   bool sort;     // false: lists stay in stencil order
+  // what the passes read instead of the cells (see BlockArgs)
+  int4* __restrict__ head;
+  uint32_t* __restrict__ stage;
+  uint32_t* __restrict__ cen;
+  uint16_t* __restrict__ cen_slot;
+  int ccap;
   unsigned long long* __restrict__ flags;  // [0] longest list beyond nmax, [1] halo beyond cap
 };
 
@@ -580,7 +513,8 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
   double3* P = reinterpret_cast<double3*>(smem);
   HaloCell* hc = reinterpret_cast<HaloCell*>(smem + build_rec_bytes(a.cap));
   int* total_p = reinterpret_cast<int*>(hc + a.g.nh_max);  // [0] halo atoms, [1] next central cell
-  uint16_t* cand_all = reinterpret_cast<uint16_t*>(total_p + 4);
+  int* cell_q = total_p + 4;                                // first central atom of each central cell
+  uint16_t* cand_all = reinterpret_cast<uint16_t*>(cell_q + a.g.bx * a.g.by * a.g.bz);
   uint32_t* rows_all = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(cand_all) +
                                                    build_cand_bytes(a.cap, a.cand_cap));
   const BlockShape s = block_shape(a.g, b);
@@ -589,16 +523,40 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
     if (threadIdx.x == 0) atomicMax(a.flags + 1, (unsigned long long)total);
     return;
   }
-  if (threadIdx.x == 0) total_p[1] = 0;
-  const BoxDev bx = a.box[s.r];
-  stage_each<false>(s, hc, total, a.pos, bx.L, nullptr, cand_all,
-                    [&](int c, const Pos4& p, int) { P[c] = double3{p.x, p.y, p.z}; });
-
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int ncell = s.ex * s.ey * s.ez;
+  const auto central_cell = [&](int cc) {
+    return ((1 + cc / (s.ex * s.ey)) * s.hy + 1 + (cc / s.ex) % s.ey) * s.hx + 1 + cc % s.ex;
+  };
+  if (wave == 0) {  // central atoms before each central cell
+    int carry = 0;
+    for (int c0 = 0; c0 < ncell; c0 += 64) {
+      const int cc = c0 + lane;
+      const int n = cc < ncell ? hc[central_cell(cc)].count : 0;
+      int v = n;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int t = __shfl_up(v, off);
+        if (lane >= off) v += t;
+      }
+      if (cc < ncell) cell_q[cc] = carry + v - n;
+      carry += __shfl(v, 63);
+    }
+    if (lane == 0) {
+      total_p[1] = 0;
+      a.head[b] = make_int4(total, carry, s.r, 0);
+    }
+  }
+  const BoxDev bx = a.box[s.r];
+  uint32_t* stage = a.stage + b * a.cap;
+  stage_cells(s, hc, total, a.pos, bx.L, cand_all, [&](int c, const Pos4& p, uint32_t e) {
+    P[c] = double3{p.x, p.y, p.z};
+    stage[c] = e;
+  });
+
   uint16_t* cand = cand_all + (size_t)wave * a.cand_cap;
   const int stride = a.nmax + 1;  // odd, so the group loads of 8 rows start in distinct banks
   uint32_t* rows = rows_all + (size_t)wave * a.atoms * stride;
-  const int ncell = s.ex * s.ey * s.ez;
   int nrow = 0;         // lists in the rows
   int cnt = 0, gi = 0;  // lane k: entries and atom of row k
   // the collected lists out: counts, then whole groups, 8 lanes per atom and one group
@@ -643,12 +601,16 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
     if (lane == 0) cc = atomicAdd(total_p + 1, 1);
     cc = __builtin_amdgcn_readfirstlane(cc);
     if (cc >= ncell) break;
-    const int ix = 1 + cc % s.ex, iy = 1 + (cc / s.ex) % s.ey, iz = 1 + cc / (s.ex * s.ey);
-    const int h = (iz * s.hy + iy) * s.hx + ix;
+    const int h = central_cell(cc);
     const int nat = __builtin_amdgcn_readfirstlane(hc[h].count);
     const int l0 = __builtin_amdgcn_readfirstlane(hc[h].lstart);
     const int g0 = __builtin_amdgcn_readfirstlane(hc[h].gstart);
     if (nat == 0) continue;
+    const int64_t q0 = b * a.ccap + cell_q[cc];
+    for (int k = lane; k < nat; k += 64) {
+      a.cen[q0 + k] = (uint32_t)(g0 + k);
+      a.cen_slot[q0 + k] = (uint16_t)(l0 + k);
+    }
     double lx = 1e300, ly = 1e300, lz = 1e300, ux = -1e300, uy = -1e300, uz = -1e300;
     if constexpr (!XF) {
       for (int k = lane & 15; k < nat; k += 16) {
@@ -763,40 +725,25 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
 
 // Block-local entries -> global (index, image) entries of the same list, in the
 // stencil order of the global build: a distance-sorted list goes back to ascending
-// halo slot order (the stencil order) first.  One wave per central atom.
-__global__ void __launch_bounds__(256) k_block_to_global(BlockGeom g, const int* __restrict__ cell_off,
-                                                         const uint16_t* __restrict__ nbr16,
-                                                         const int* __restrict__ nnb, uint32_t* __restrict__ nbr,
-                                                         int64_t npad, int nh_max)
+// halo slot order (the stencil order) first.  A slot's staging entry is its global
+// entry.  One wave per central atom.
+__global__ void __launch_bounds__(256) k_block_to_global(BlockArgs a, uint32_t* __restrict__ nbr)
 {
   const int64_t b = lblock();
-  if (b >= g.nblocks) return;
-  LdsLayout l = lds_layout(0, 0, nh_max, false, false);
-  const BlockShape s = block_shape(g, b);
-  const int nh = s.hx * s.hy * s.hz;
-  build_halo(g, s, cell_off, l.hc, l.total);
+  if (b >= a.nblocks) return;
+  const int ncentral = a.head[b].y;
+  const uint32_t* stage = a.stage + b * a.cap;
   const int lane = threadIdx.x & 63;
-  for (int q = threadIdx.x >> 6;; q += blockDim.x >> 6) {
-    Central a;
-    if (!central_atom(s, l.hc, q, a)) break;
-    const int cnt = nnb[a.global];
+  for (int q = threadIdx.x >> 6; q < ncentral; q += blockDim.x >> 6) {
+    const int64_t i = a.cen[b * a.ccap + q];
+    const int cnt = a.nnb[i];
     if (cnt <= kSortRows) {
       uint32_t key = 0xffffu;
-      if (lane < cnt) key = nbr16[bl_index(npad, a.global, lane)];
+      if (lane < cnt) key = a.nbr16[bl_index(a.npad, i, lane)];
       key = wave_radix_sort(key, 0, 16);
-      if (lane < cnt) {
-        const int c = (int)key;
-        const HaloCell e = l.hc[find_cell(l.hc, nh, c)];
-        nbr[(int64_t)lane * npad + a.global] =
-            (uint32_t)(e.gstart + (c - e.lstart)) | ((uint32_t)e.img << XSMD_NBR_INDEX_BITS);
-      }
+      if (lane < cnt) nbr[(int64_t)lane * a.npad + i] = stage[key];
     } else {
-      for (int k = lane; k < cnt; k += 64) {
-        const int c = nbr16[bl_index(npad, a.global, k)];
-        const HaloCell e = l.hc[find_cell(l.hc, nh, c)];
-        nbr[(int64_t)k * npad + a.global] =
-            (uint32_t)(e.gstart + (c - e.lstart)) | ((uint32_t)e.img << XSMD_NBR_INDEX_BITS);
-      }
+      for (int k = lane; k < cnt; k += 64) nbr[(int64_t)k * a.npad + i] = stage[a.nbr16[bl_index(a.npad, i, k)]];
     }
   }
 }
@@ -868,33 +815,6 @@ __global__ void __launch_bounds__(64 * kHaloMaxWaves) k_block_halo_max(BlockGeom
 // ---------------------------------------------------------------------------
 // EAM passes on the block list
 // ---------------------------------------------------------------------------
-struct BlockArgs {
-  BlockGeom g;
-  const int* __restrict__ cell_off;
-  const Pos4* __restrict__ pos;
-  const uint8_t* __restrict__ type;
-  const BoxDev* __restrict__ box;
-  const uint16_t* __restrict__ nbr16;
-  const int* __restrict__ nnb;
-  int64_t npad;
-  int cap;   // halo slots (LDS records)
-  int ccap;  // central atoms per brick at most
-  double rc2;
-  // set to 1 by a brick whose halo or central atoms exceed cap or ccap (the maxima
-  // the host measured at list build, which hold while the cells do not change); such
-  // a brick leaves its atoms unwritten and the host reports the call as failed
-  unsigned long long* overflow;
-  const XformDev* xf;  // the staging maps positions to physical space when not NULL
-};
-
-// a brick beyond the measured capacities: raise the flag, skip the brick
-__device__ __forceinline__ bool over_capacity(const BlockArgs& a, int count, int cap)
-{
-  if (count <= cap) return false;
-  if (threadIdx.x == 0) *a.overflow = 1ull;
-  return true;
-}
-
 constexpr int kBBatch = 4;
 // EAM passes run two lanes per central atom: the two halves of a wave take the
 // even and odd list entries of the same 32 atoms and combine their sums with one
@@ -968,25 +888,21 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
                                                                 double* __restrict__ pos_w, double* __restrict__ ep)
 {
   const int64_t b = lblock();
-  if (b >= a.g.nblocks) return;
-  LdsLayout l = lds_layout(a.cap, a.ccap, a.g.nh_max, MULTI, false);
-  const BlockShape s = block_shape(a.g, b);
-  const int total = build_halo(a.g, s, a.cell_off, l.hc, l.total);
-  if (over_capacity(a, total, a.cap)) return;
-  central_table(s, l.hc, l.central_local, a.ccap, l.total + 2);
-  stage(s, l.hc, total, a.pos, a.box[s.r], a.xf, a.type, l.rec, l.ltype, l.slot_cell, a.cap);
-  const int ncentral = l.total[2];
-  if (over_capacity(a, ncentral, a.ccap)) return;
+  if (b >= a.nblocks) return;
+  uint8_t* ltype;
+  const LRec rec = pass_lds(a, MULTI, false, ltype);
+  const int4 hd = a.head[b];
+  stage<false>(a, b, hd, rec, ltype);
   const int half = pass_half();
-  for (int q = pass_slot();; q += kPassAtoms) {
-    Central ca;
-    if (!central_at(l.hc, l.slot_cell, l.central_local, ncentral, q, ca)) break;
-    const Pos4 pi = l.rec.get(ca.local);
-    const int ti = MULTI ? l.ltype[ca.local] : 0;
+  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+    const int64_t gi = a.cen[b * a.ccap + q];
+    const int slot = a.cen_slot[b * a.ccap + q];
+    const Pos4 pi = rec.get(slot);
+    const int ti = MULTI ? ltype[slot] : 0;
     const bool oni = !MULTI || pm::eam_on(t, ti);
-    const int cnt = oni ? a.nnb[ca.global] : 0;
+    const int cnt = oni ? a.nnb[gi] : 0;
     double rho = 0.0;
-    LWords lw = lwords(a, ca.global, half);
+    LWords lw = lwords(a, gi, half);
     uint2 wnext = lw.get(0);
     for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
       const uint2 w = wnext;
@@ -994,10 +910,10 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
       LNb nb[kBBatch];
-      lgather<kBBatch>(a, l.rec, c, k0, cnt, pi, nb);
+      lgather<kBBatch>(a, rec, c, k0, cnt, pi, nb);
       if constexpr (MULTI) {
 #pragma unroll
-        for (int u = 0; u < kBBatch; u++) nb[u].in = nb[u].in && pm::eam_on(t, l.ltype[nb[u].c]);
+        for (int u = 0; u < kBBatch; u++) nb[u].in = nb[u].in && pm::eam_on(t, ltype[nb[u].c]);
       }
       // a batch with no pair inside rc on any lane of the wave (the tails of the
       // distance-sorted lists) skips the table reads; skipped terms would add 0
@@ -1007,7 +923,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
       if (!__any(any)) continue;
 #pragma unroll
       for (int u = 0; u < kBBatch; u++) {
-        const int tj = MULTI ? l.ltype[nb[u].c] : 0;
+        const int tj = MULTI ? ltype[nb[u].c] : 0;
         // every d2 here is finite and positive (entries past the count read the far
         // record), so the knot index needs no guard value; the sum masks by `in`
         const Real val = pm::eam_rho_knot<Real, MULTI>(t, pair, ti, tj, nb[u].d2, true);
@@ -1016,15 +932,15 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
     }
     rho = half_sum(rho);
     if (half == 0) {
-      rho_io[ca.global] = rho;
+      rho_io[gi] = rho;
       if constexpr (EMB) {
         Real F, Fp;
         pm::embed(t, ti, rho, F, Fp);
         if (!oni) F = Fp = Real(0);  // a disabled species keeps rho_dEmb = 0 and adds no F
-        pos_w[4 * ca.global + 3] = (double)Fp;
+        pos_w[4 * gi + 3] = (double)Fp;
         if constexpr (ENERGY) {
-          if constexpr (SET_EP) ep[ca.global] = (double)F;
-          else ep[ca.global] += (double)F;
+          if constexpr (SET_EP) ep[gi] = (double)F;
+          else ep[gi] += (double)F;
         }
       }
     }
@@ -1038,23 +954,22 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_
 {
   static_assert(!DRIFT || (FUSED && !ENERGY && !VIRIAL), "the drift epilogue is the plain MD-loop step");
   const int64_t b = lblock();
-  if (b >= a.g.nblocks) return;
-  LdsLayout l = lds_layout(a.cap, a.ccap, a.g.nh_max, MULTI, true);
-  const BlockShape s = block_shape(a.g, b);
-  const int total = build_halo(a.g, s, a.cell_off, l.hc, l.total);
-  if (over_capacity(a, total, a.cap)) return;
-  stage(s, l.hc, total, a.pos, a.box[s.r], a.xf, a.type, l.rec, l.ltype, l.slot_cell, a.cap);
+  if (b >= a.nblocks) return;
+  uint8_t* ltype;
+  const LRec rec = pass_lds(a, MULTI, true, ltype);
+  const int4 hd = a.head[b];
+  stage<true>(a, b, hd, rec, ltype);
   const int half = pass_half();
-  for (int q = pass_slot();; q += kPassAtoms) {
-    Central ca;
-    if (!central_atom(s, l.hc, q, ca)) break;
-    const Pos4 pi = l.rec.get(ca.local);
-    const int ti = MULTI ? l.ltype[ca.local] : 0;
+  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+    const int64_t gi = a.cen[b * a.ccap + q];
+    const int slot = a.cen_slot[b * a.ccap + q];
+    const Pos4 pi = rec.get(slot);
+    const int ti = MULTI ? ltype[slot] : 0;
     const Real fpi = (Real)pi.w;
-    const int cnt = (!MULTI || pm::eam_on(t, ti)) ? a.nnb[ca.global] : 0;
+    const int cnt = (!MULTI || pm::eam_on(t, ti)) ? a.nnb[gi] : 0;
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    LWords lw = lwords(a, ca.global, half);
+    LWords lw = lwords(a, gi, half);
     uint2 wnext = lw.get(0);
     for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
       const uint2 w = wnext;
@@ -1067,10 +982,10 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_
 #pragma unroll
       for (int sub = 0; sub < kBBatch; sub += 2) {
         LNb nb[2];
-        lgather<2>(a, l.rec, c + sub, k0 + 2 * sub, cnt, pi, nb);
+        lgather<2>(a, rec, c + sub, k0 + 2 * sub, cnt, pi, nb);
         if constexpr (MULTI) {
-          nb[0].in = nb[0].in && pm::eam_on(t, l.ltype[nb[0].c]);
-          nb[1].in = nb[1].in && pm::eam_on(t, l.ltype[nb[1].c]);
+          nb[0].in = nb[0].in && pm::eam_on(t, ltype[nb[0].c]);
+          nb[1].in = nb[1].in && pm::eam_on(t, ltype[nb[1].c]);
         }
         if (!__any(nb[0].in || nb[1].in)) continue;  // as in the density pass
         auto add = [&](const LNb& q, bool in, Real fp, Real ph) {
@@ -1102,7 +1017,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_
         } else {
 #pragma unroll
           for (int u = 0; u < 2; u++) {
-            const int tj = MULTI ? l.ltype[nb[u].c] : 0;
+            const int tj = MULTI ? ltype[nb[u].c] : 0;
             Real fp_r, phi;
             pm::eam_pair_knot<Real, MULTI>(t, pair, ti, tj, fpi, (Real)nb[u].w, nb[u].d2, true, fp_r, phi);
             add(nb[u], nb[u].in, fp_r, phi);
@@ -1120,8 +1035,8 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_
       for (int k = 0; k < 9; k++) v[k] = half_sum(v[k]);
     }
     if (half == 0) {
-      if constexpr (DRIFT) pm::write_outputs_drift(o, dr, ca.global, pi, fx, fy, fz);
-      else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, ca.global, fx, fy, fz, e, v);
+      if constexpr (DRIFT) pm::write_outputs_drift(o, dr, gi, pi, fx, fy, fz);
+      else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, gi, fx, fy, fz, e, v);
     }
   }
 }
@@ -1143,34 +1058,23 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
                                                                                             double* __restrict__ sink)
 {
   const int64_t b = lblock();
-  if (b >= a.g.nblocks) return;
-  LdsLayout l = lds_layout(a.cap, a.ccap, a.g.nh_max, false, FORCE);
-  const BlockShape s = block_shape(a.g, b);
-  const int total = build_halo(a.g, s, a.cell_off, l.hc, l.total);
-  if (over_capacity(a, total, a.cap)) return;
-  if constexpr (!FORCE) central_table(s, l.hc, l.central_local, a.ccap, l.total + 2);
-  stage(s, l.hc, total, a.pos, a.box[s.r], a.xf, nullptr, l.rec, l.ltype, l.slot_cell, a.cap);
-  int ncentral = 0;
-  if constexpr (!FORCE) {
-    ncentral = l.total[2];
-    if (over_capacity(a, ncentral, a.ccap)) return;
-  }
+  if (b >= a.nblocks) return;
+  uint8_t* ltype;
+  const LRec rec = pass_lds(a, false, FORCE, ltype);
+  const int4 hd = a.head[b];
+  stage<FORCE>(a, b, hd, rec, ltype);
   const int half = pass_half();
-  for (int q = pass_slot();; q += kPassAtoms) {
-    Central ca;
-    if constexpr (FORCE) {
-      if (!central_atom(s, l.hc, q, ca)) break;
-    } else {
-      if (!central_at(l.hc, l.slot_cell, l.central_local, ncentral, q, ca)) break;
-    }
-    const Pos4 pi = l.rec.get(ca.local);
-    const int cnt = a.nnb[ca.global];
+  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+    const int64_t gi = a.cen[b * a.ccap + q];
+    const int slot = a.cen_slot[b * a.ccap + q];
+    const Pos4 pi = rec.get(slot);
+    const int cnt = a.nnb[gi];
     float acc = 0.0f;
     if constexpr (LEVEL == 3) {
-      if (half == 0) sink[ca.global] = pi.x + cnt;
+      if (half == 0) sink[gi] = pi.x + cnt;
       continue;
     }
-    LWords lw = lwords(a, ca.global, half);
+    LWords lw = lwords(a, gi, half);
     uint2 wnext = lw.get(0);
     for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
       const uint2 w = wnext;
@@ -1182,7 +1086,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
         continue;
       }
       LNb nb[kBBatch];
-      lgather<kBBatch>(a, l.rec, c, k0, cnt, pi, nb);
+      lgather<kBBatch>(a, rec, c, k0, cnt, pi, nb);
       bool any = false;
 #pragma unroll
       for (int u = 0; u < kBBatch; u++) any |= nb[u].in;
@@ -1219,7 +1123,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
       }
     }
     const double sum = half_sum((double)acc);
-    if (half == 0) sink[ca.global] = sum;
+    if (half == 0) sink[gi] = sum;
   }
 }
 
@@ -1235,26 +1139,21 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
 {
   static_assert(!DRIFT || (FUSED && !ENERGY && !VIRIAL), "the drift epilogue is the plain MD-loop step");
   const int64_t b = lblock();
-  if (b >= a.g.nblocks) return;
-  LdsLayout l = lds_layout(a.cap, a.ccap, a.g.nh_max, MULTI, false);
-  const BlockShape s = block_shape(a.g, b);
-  const int total = build_halo(a.g, s, a.cell_off, l.hc, l.total);
-  if (over_capacity(a, total, a.cap)) return;
-  central_table(s, l.hc, l.central_local, a.ccap, l.total + 2);
-  stage(s, l.hc, total, a.pos, a.box[s.r], a.xf, MULTI ? a.type : nullptr, l.rec, l.ltype, l.slot_cell,
-        a.cap);
-  const int ncentral = l.total[2];
-  if (over_capacity(a, ncentral, a.ccap)) return;
+  if (b >= a.nblocks) return;
+  uint8_t* ltype;
+  const LRec rec = pass_lds(a, MULTI, false, ltype);
+  const int4 hd = a.head[b];
+  stage<false>(a, b, hd, rec, ltype);
   const int half = pass_half();
-  for (int q = pass_slot();; q += kPassAtoms) {
-    Central ca;
-    if (!central_at(l.hc, l.slot_cell, l.central_local, ncentral, q, ca)) break;
-    const Pos4 pi = l.rec.get(ca.local);
-    const int ti = MULTI ? l.ltype[ca.local] : 0;
-    const int cnt = a.nnb[ca.global];
+  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+    const int64_t gi = a.cen[b * a.ccap + q];
+    const int slot = a.cen_slot[b * a.ccap + q];
+    const Pos4 pi = rec.get(slot);
+    const int ti = MULTI ? ltype[slot] : 0;
+    const int cnt = a.nnb[gi];
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    LWords lw = lwords(a, ca.global, half);
+    LWords lw = lwords(a, gi, half);
     uint2 wnext = lw.get(0);
     for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
       const uint2 w = wnext;
@@ -1262,12 +1161,12 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
       LNb nb[kBBatch];
-      lgather<kBBatch>(a, l.rec, c, k0, cnt, pi, nb);
+      lgather<kBBatch>(a, rec, c, k0, cnt, pi, nb);
 #pragma unroll
       for (int u = 0; u < kBBatch; u++) {
         double de_r, eh;
         if constexpr (MULTI) {
-          const int pid = pm::type_pair(ti, l.ltype[nb[u].c]);
+          const int pid = pm::type_pair(ti, ltype[nb[u].c]);
           pm::lj_pair(pm::lj_multi_row<Real>(lm, pid), nb[u].d2, nb[u].in && pm::lj_multi_in(lm, pid, nb[u].d2),
                       de_r, eh);
         } else {
@@ -1290,10 +1189,31 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
       for (int k = 0; k < 9; k++) v[k] = half_sum(v[k]);
     }
     if (half == 0) {
-      if constexpr (DRIFT) pm::write_outputs_drift(o, dr, ca.global, pi, fx, fy, fz);
-      else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, ca.global, fx, fy, fz, e, v);
+      if constexpr (DRIFT) pm::write_outputs_drift(o, dr, gi, pi, fx, fy, fz);
+      else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, gi, fx, fy, fz, e, v);
     }
   }
+}
+
+BlockArgs block_args(const Ctx& c, double rcut)
+{
+  BlockArgs a;
+  a.head = c.brick_head.p;
+  a.stage = c.brick_stage.p;
+  a.cen = c.brick_cen.p;
+  a.cen_slot = c.brick_cen_slot.p;
+  a.pos = c.pos.p;
+  a.type = c.type.p;
+  a.box = c.box_d.p;
+  a.nbr16 = c.nbr16.p;
+  a.nnb = c.nnb.p;
+  a.npad = c.npad;
+  a.nblocks = c.bgeom.nblocks;
+  a.cap = c.bcap;
+  a.ccap = c.bcentral;
+  a.rc2 = rcut * rcut;
+  a.xf = c.xf_dev();
+  return a;
 }
 
 // Fused next-step drift of the MD loop (ForceEpilogue::drift) for a force launch
@@ -1332,20 +1252,7 @@ void block_eam_dispatch(Ctx& c, double rcut, bool do_rho, bool do_emb, bool do_f
 {
   const EamTabDev<Real> t = make_eam_tab<Real>(c);
   const Real* pair = eam_pair_table<Real>(c);
-  BlockArgs a;
-  a.g = c.bgeom;
-  a.cell_off = c.cell_off.p;
-  a.pos = c.pos.p;
-  a.type = c.type.p;
-  a.box = c.box_d.p;
-  a.xf = c.xf_dev();
-  a.nbr16 = c.nbr16.p;
-  a.nnb = c.nnb.p;
-  a.npad = c.npad;
-  a.cap = c.bcap;
-  a.ccap = c.bcentral;
-  a.overflow = c.dscalar.p + 6;
-  a.rc2 = rcut * rcut;
+  const BlockArgs a = block_args(c, rcut);
   const size_t lds_rho = block_lds_bytes(c, MULTI, false);
   const size_t lds = block_lds_bytes(c, MULTI, true);
   const unsigned g = block_grid(c);
@@ -1402,20 +1309,7 @@ double gather_ceiling(Ctx& c, double rcut, bool force, int level, int reps)
   if (reps < 1) throw Error(XS_E_ARG, "reps must be >= 1");
   const EamTabDev<float> t = make_eam_tab<float>(c);
   if (force && c.eam.s_pieces == 0) throw Error(XS_E_STATE, "gather ceiling of the force pass needs the s-table");
-  BlockArgs a;
-  a.g = c.bgeom;
-  a.cell_off = c.cell_off.p;
-  a.pos = c.pos.p;
-  a.type = c.type.p;
-  a.box = c.box_d.p;
-  a.xf = c.xf_dev();
-  a.nbr16 = c.nbr16.p;
-  a.nnb = c.nnb.p;
-  a.npad = c.npad;
-  a.cap = c.bcap;
-  a.ccap = c.bcentral;
-  a.overflow = c.dscalar.p + 6;
-  a.rc2 = rcut * rcut;
+  const BlockArgs a = block_args(c, rcut);
   DBuf<double> sink;
   sink.reserve(c.npad);
   const unsigned g = block_grid(c);
@@ -1438,7 +1332,6 @@ double gather_ceiling(Ctx& c, double rcut, bool force, int level, int reps)
   XS_HIP(hipEventElapsedTime(&ms, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  check_pass_overflow(c);
   return ms / reps;
 }
 
@@ -1519,10 +1412,8 @@ void block_setup(Ctx& c)
 
 size_t block_lds_bytes(const Ctx& c, bool with_type, bool with_w)
 {
-  // bcap records and the far record, halo table, counters, slot cells, central slots,
-  // per-record types (lds_layout)
-  return (size_t)(c.bcap + 1) * sizeof(double) * (with_w ? 4 : 3) + (size_t)c.bgeom.nh_max * sizeof(HaloCell) +
-         4 * sizeof(int) + (size_t)(c.bcap + c.bcentral) * sizeof(uint16_t) + (with_type ? (size_t)c.bcap + 1 : 0);
+  // bcap records and the far record, and their types (pass_lds)
+  return ((size_t)c.bcap + 1) * (sizeof(double) * (with_w ? 4 : 3) + (with_type ? 1 : 0));
 }
 
 bool block_feasible(const Ctx& c)
@@ -1538,8 +1429,8 @@ unsigned block_grid(const Ctx& c)
 // LDS of a build launch that collects `atoms` lists per wave
 static size_t build_lds_bytes(const Ctx& c, int atoms)
 {
-  return build_rec_bytes(c.bcap) + (size_t)c.bgeom.nh_max * sizeof(HaloCell) + 4 * sizeof(int) +
-         build_cand_bytes(c.bcap, c.bcand) + (size_t)kBuildWaves * atoms * (c.nmax + 1) * sizeof(uint32_t);
+  return build_rec_bytes(c.bcap) + (size_t)c.bgeom.nh_max * sizeof(HaloCell) +
+         (4 + (size_t)c.bgeom.bx * c.bgeom.by * c.bgeom.bz) * sizeof(int) + build_cand_bytes(c.bcap, c.bcand) + (size_t)kBuildWaves * atoms * (c.nmax + 1) * sizeof(uint32_t);
 }
 
 // Block list build; false when its LDS does not fit a workgroup (then nothing was
@@ -1558,6 +1449,15 @@ bool block_build(Ctx& c, double rl2)
   a.cand_cap = c.bcand;
   a.sort = !c.list_sort_disabled;
   a.flags = c.dscalar.p;
+  c.brick_head.reserve(c.bgeom.nblocks);
+  c.brick_stage.reserve((size_t)c.bgeom.nblocks * c.bcap);
+  c.brick_cen.reserve((size_t)c.bgeom.nblocks * c.bcentral);
+  c.brick_cen_slot.reserve((size_t)c.bgeom.nblocks * c.bcentral);
+  a.head = c.brick_head.p;
+  a.stage = c.brick_stage.p;
+  a.cen = c.brick_cen.p;
+  a.cen_slot = c.brick_cen_slot.p;
+  a.ccap = c.bcentral;
   for (int attempt = 0; attempt < 2; attempt++) {
     a.atoms = kBuildAtoms;
     while (a.atoms > 1 && build_lds_bytes(c, a.atoms) > kBlockLdsLimit) a.atoms /= 2;
@@ -1590,9 +1490,7 @@ bool block_build(Ctx& c, double rl2)
 void block_to_global(Ctx& c)
 {
   c.nbr.reserve((size_t)c.nmax * c.npad);
-  const size_t lds = block_lds_bytes(c, false, false) - (size_t)c.bcap * 3 * sizeof(double);
-  k_block_to_global<<<block_grid(c), kBlock, lds, c.stream>>>(c.bgeom, c.cell_off.p, c.nbr16.p, c.nnb.p, c.nbr.p,
-                                                              c.npad, c.bgeom.nh_max);
+  k_block_to_global<<<block_grid(c), kBlock, 0, c.stream>>>(block_args(c, 0.0), c.nbr.p);
   XS_HIP(hipGetLastError());
 }
 
@@ -1633,20 +1531,7 @@ void launch_eam_block(Ctx& c, double rcut, bool do_rho, bool do_emb, bool do_for
 void launch_lj_block(Ctx& c, double eps, double sigma, double rcut, unsigned flags, const ForceEpilogue& epi)
 {
   const double ecut = lj_energy_cutoff(eps, sigma, rcut);
-  BlockArgs a;
-  a.g = c.bgeom;
-  a.cell_off = c.cell_off.p;
-  a.pos = c.pos.p;
-  a.type = c.type.p;
-  a.box = c.box_d.p;
-  a.xf = c.xf_dev();
-  a.nbr16 = c.nbr16.p;
-  a.nnb = c.nnb.p;
-  a.npad = c.npad;
-  a.cap = c.bcap;
-  a.ccap = c.bcentral;
-  a.overflow = c.dscalar.p + 6;
-  a.rc2 = rcut * rcut;
+  const BlockArgs a = block_args(c, rcut);
   const size_t lds = block_lds_bytes(c, false, false);
   const unsigned g = block_grid(c);
   const pm::Outputs o = make_outputs(c, epi);
@@ -1681,20 +1566,7 @@ void launch_lj_block(Ctx& c, double eps, double sigma, double rcut, unsigned fla
 
 void launch_lj_multi_block(Ctx& c, unsigned flags)
 {
-  BlockArgs a;
-  a.g = c.bgeom;
-  a.cell_off = c.cell_off.p;
-  a.pos = c.pos.p;
-  a.type = c.type.p;
-  a.box = c.box_d.p;
-  a.xf = c.xf_dev();
-  a.nbr16 = c.nbr16.p;
-  a.nnb = c.nnb.p;
-  a.npad = c.npad;
-  a.cap = c.bcap;
-  a.ccap = c.bcentral;
-  a.overflow = c.dscalar.p + 6;
-  a.rc2 = c.ljm_rcmax * c.ljm_rcmax;
+  const BlockArgs a = block_args(c, c.ljm_rcmax);
   const size_t lds = block_lds_bytes(c, true, false);
   const unsigned g = block_grid(c);
   const pm::Outputs o = make_outputs(c, ForceEpilogue{});
@@ -1723,49 +1595,6 @@ void ensure_global_list(Ctx& c)
   if (c.list_kind == ListKind::Global || c.global_from_block) return;
   block_to_global(c);
   c.global_from_block = true;
-}
-
-void check_pass_overflow(Ctx& c)
-{
-  XS_HIP(hipMemcpyAsync(c.hscalar + 6, c.dscalar.p + 6, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                        c.stream));
-  XS_HIP(hipStreamSynchronize(c.stream));
-  if (c.hscalar[6] == 0) return;
-  c.hscalar[6] = 0;
-  XS_HIP(hipMemsetAsync(c.dscalar.p + 6, 0, sizeof(unsigned long long), c.stream));
-  XS_HIP(hipStreamSynchronize(c.stream));
-  throw Error(XS_E_STATE, "block pass: a brick holds more halo or central atoms than measured at the list build "
-                          "(cells changed without a rebuild); its atoms were not computed");
-}
-
-void check_or_defer_overflow(Ctx& c)
-{
-  if (c.stream == c.own_stream) {
-    check_pass_overflow(c);
-    return;
-  }
-  XS_HIP(hipMemcpyAsync(c.hscalar + 6, c.dscalar.p + 6, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                        c.stream));
-  XS_HIP(hipEventRecord(c.flag_event, c.stream));
-  c.flag_pending = true;
-}
-
-void poll_pass_overflow(Ctx& c, bool wait)
-{
-  if (!c.flag_pending) return;
-  if (!wait) {
-    const hipError_t q = hipEventQuery(c.flag_event);
-    if (q == hipErrorNotReady) return;
-    XS_HIP(q);
-  } else {
-    XS_HIP(hipEventSynchronize(c.flag_event));
-  }
-  c.flag_pending = false;
-  if (c.hscalar[6] == 0) return;
-  c.hscalar[6] = 0;
-  XS_HIP(hipMemsetAsync(c.dscalar.p + 6, 0, sizeof(unsigned long long), c.stream));
-  throw Error(XS_E_STATE, "block pass (an earlier call): a brick holds more halo or central atoms than measured at "
-                          "the list build (cells changed without a rebuild); its atoms were not computed");
 }
 
 }  // namespace xsmd

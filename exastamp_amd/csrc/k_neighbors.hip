@@ -324,6 +324,7 @@ void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block, bo
     c.global_from_block = false;
     return;
   }
+  c.list_valid = false;  // until the new list is complete
   const double rl = rcut + skin;
   if (!(rl > 0)) throw Error(XS_E_ARG, "rcut + skin must be positive");
 

@@ -321,6 +321,10 @@ struct Ctx {
   DBuf<uint16_t> nbr16;
   DBuf<int> cell_off;              // first atom of each cell, ncell_tot + 1
   BlockGeom bgeom{};
+  // staging tables of the bricks, written by the block build (k_block.hip, BlockArgs)
+  DBuf<int4> brick_head;
+  DBuf<uint32_t> brick_stage, brick_cen;
+  DBuf<uint16_t> brick_cen_slot;
   int bcap = 0;                    // LDS slots per block (max halo atoms, rounded)
   int bcentral = 0;                // max central atoms per block
   int bcand = 0;                   // max atoms in the 27 cells of a central cell
@@ -332,11 +336,8 @@ struct Ctx {
 
   // small device scalars + pinned host mirror
   DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..4] halo maxima,
-                                     // [5] fused-drift rebuild flag,
-                                     // [6] block-pass capacity exceeded
+                                     // [5] fused-drift rebuild flag
   unsigned long long* hscalar = nullptr;
-  hipEvent_t flag_event = nullptr;  // the deferred copy of dscalar[6] to hscalar[6] (check_or_defer_overflow)
-  bool flag_pending = false;
   DBuf<double> red_part;  // thermo partial sums
   DBuf<double> red_out;
   double* hthermo = nullptr;  // pinned host copy of the 27 results
@@ -389,16 +390,6 @@ void ensure_global_list(Ctx& c);
 // the half list (nbr_half / nnb_half) of the current list
 void ensure_half_list(Ctx& c);
 double max_displacement2(Ctx& c);
-// raises XS_E_STATE (and clears the flag) when a block pass found a brick beyond the
-// capacities measured at list build (dscalar[6]); synchronises the stream
-void check_pass_overflow(Ctx& c);
-// The operators' form: on the context's own stream, check_pass_overflow; on a stream
-// the caller set (xs_ctx_set_stream), the flag is copied to the host asynchronously
-// and checked by poll_pass_overflow at the next call (no synchronisation mid-step).
-void check_or_defer_overflow(Ctx& c);
-// raises XS_E_STATE when a deferred flag copy has arrived (wait: wait for it) and
-// found the flag set
-void poll_pass_overflow(Ctx& c, bool wait);
 // average ms of the gather-ceiling kernel of the density (force = false) or force pass
 double gather_ceiling(Ctx& c, double rcut, bool force, int level, int reps);
 void pair_count(Ctx& c, double rcut, int64_t& entries, int64_t& within);

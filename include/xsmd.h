@@ -80,10 +80,7 @@ xs_status xs_synchronize(xs_ctx* ctx);
  * device's null stream), so that device buffers the caller's own kernels write or read
  * (the *_dev arguments) need no further synchronisation.  Waits for the work already
  * queued on the current stream first.  The caller keeps `stream` alive while the
- * context uses it.  On such a stream the force operators do not wait for their block
- * passes' capacity flag (a brick beyond the capacity measured at the list build,
- * XS_E_STATE): the flag travels to the host with the work, and the first later call
- * that finds it arrived (xs_synchronize waits for it) returns XS_E_STATE. */
+ * context uses it. */
 xs_status xs_ctx_set_stream(xs_ctx* ctx, void* stream);
 /* Back to the context's own stream (the one xs_ctx_create made), after waiting for
  * the work queued on the current one. */
