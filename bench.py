@@ -428,15 +428,14 @@ def cpu_baseline(cfg, tab, steps, threads, dt, rc, skin):
 
 def operator_forms(sim, rc, reps=5):
     """The eam_alloy_force operator (density, embedding and force passes, mixed) in
-    its full-list form and in its Newton-symmetric form (half list, FP64 atomics):
-    GPU time per call of each pass class, and the symmetric form's force deviation."""
+    its plain and its Newton-symmetric form: GPU time per call of each pass class, and the symmetric form's force deviation."""
     from exastamp_amd import _lib
     import ctypes as C
     out = {}
     forces = {}
     for name, sym in (("full_list", False), ("symmetric", True)):
         sim.zero_force_energy()
-        sim.eam_alloy_force(rcut=rc, mixed=True, eam_symmetry=sym)   # untimed: builds the half list
+        sim.eam_alloy_force(rcut=rc, mixed=True, eam_symmetry=sym)   # untimed
         forces[name] = sim.accelerations()
         sim.ctx.xs_synchronize()
         sim.ctx.xs_profile_enable(1)
@@ -454,8 +453,8 @@ def operator_forms(sim, rc, reps=5):
     f0, f1 = forces["full_list"], forces["symmetric"]
     rms = float(np.sqrt((f0 ** 2).sum(1).mean()))
     out["symmetric_max_dev_over_rms"] = float(np.sqrt(((f1 - f0) ** 2).sum(1)).max() / rms)
-    out["note"] = ("operator calls outside the timed MD loop; symmetric = each pair once from a half list, "
-                   "partner share by FP64 atomics on the global list")
+    out["note"] = ("operator calls outside the timed MD loop; symmetric = the Newton-symmetric operators, which "
+                   "evaluate every pair from both atoms with a symmetric pair scalar")
     return out
 
 

@@ -305,7 +305,6 @@ xs_status xs_system_set(xs_ctx* h, int64_t n, const double* rx, const double* ry
     c.n = n;
     allocate_atoms(c, n);
     c.list_valid = false;
-    c.half_valid = false;
     c.rho_state = RhoState::None;
     c.rho_ckpt = false;
     if (n > 0) {

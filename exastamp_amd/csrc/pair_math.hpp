@@ -393,7 +393,9 @@ __device__ __forceinline__ void eam_pair_knot(const EamTabDev<Real>& t, const Re
     Real phip, psip;
     if constexpr (sizeof(Real) == 4) {
       phip = fmaf(z2p, rinv, -(phi * rinv)) * t.conv;
-      psip = fmaf(fpi, rhojp, fmaf(fpj, rhoip, phip));
+      // in an order that both atoms of the pair agree on, so that their forces cancel
+      const bool first = fpi <= fpj;
+      psip = fmaf(first ? fpi : fpj, first ? rhojp : rhoip, fmaf(first ? fpj : fpi, first ? rhoip : rhojp, phip));
     } else {
       phip = (z2p * rinv - phi * rinv) * t.conv;
       psip = fpi * rhojp + fpj * rhoip + phip;

@@ -217,7 +217,7 @@ class Simulation:
 
     def lj_compute_force_symetric(self, parameters, rcut, **kw):
         """lj_compute_force_symetric (pair_potential_singlemat_symetric.cpp:101-332):
-        the same forces, each pair evaluated once with Newton's third law."""
+        the same forces, a pair's opposite by Newton's third law."""
         self.lj_compute_force(parameters, rcut, symmetric=True, **kw)
 
     def lj_multi_force(self, rcut, parameters=(), common_parameters=None, compute_virial=True,
@@ -335,9 +335,8 @@ class Simulation:
                         mixed=False, types=None, **_slots):
         """eam_alloy_force (eam_potential_multimat.cu:88-109 slots).  eam_ghost is
         accepted and has no effect (one GPU holds every atom; images are resolved in
-        the pair kernels).  eam_symmetry selects the Newton-symmetric evaluation
-        (each pair once from a half list, the partner's share added atomically):
-        the same quantities up to FP64 summation order.  types (eam_potential_multimat.cu:90,
+        the pair kernels).  eam_symmetry selects the Newton-symmetric operator: the
+        same quantities, the forces of a pair's atoms opposite.  types (eam_potential_multimat.cu:90,
         154-166): an empty list means every species; otherwise only pairs of two listed
         species contribute, and atoms of an unlisted species get rho = F' = 0 and no force."""
         mask = self._types_mask(types)

@@ -51,10 +51,9 @@ typedef enum {
 #define XS_CONTINUE 8u /* xs_md_run: continue a previous run (valid list and current
                           accelerations): skip the initial build and force step */
 #define XS_SYMMETRIC 16u /* Newton-symmetric evaluation (eam_symmetry: true,
-                            lj_compute_force_symetric): each pair once, from a half of
-                            the neighbour list, the partner's share added with FP64
-                            atomics.  Operators only (not xs_md_run); the order of the
-                            atomic sums, hence the last bits, varies from run to run. */
+                            lj_compute_force_symetric): the two atoms of a pair get
+                            opposite forces from the same pair scalar.  Operators only
+                            (not xs_md_run). */
 
 /* potentials for xs_md_run */
 #define XS_POT_LJ 0
