@@ -528,7 +528,16 @@ xs_status xs_lj_multi_force(xs_ctx* h, int ntypes, const double* epsilon, const 
     require(rcmax <= c.list_rcut + c.list_skin, XS_E_ARG, "rcut exceeds the neighbour-list radius");
     std::vector<double> d(4 * (size_t)np);
     std::vector<float> f(4 * (size_t)np);
+    std::vector<double> rc2(np, -1.0);
+    double reach = 0.0;
     for (int k = 0; k < np; k++) {
+      if (epsilon[k] != 0.0) {  // the largest number whose square root is at most rcut
+        double x = rcut[k] * rcut[k];
+        while (std::sqrt(x) > rcut[k]) x = std::nextafter(x, 0.0);
+        for (double y; std::sqrt(y = std::nextafter(x, HUGE_VAL)) <= rcut[k];) x = y;
+        rc2[k] = x;
+        reach = std::max(reach, rcut[k]);
+      }
       const double row[4] = {sigma[k] * sigma[k], 4.0 * epsilon[k], 24.0 * epsilon[k],
                              lj_energy_cutoff(epsilon[k], sigma[k], rcut[k])};
       for (int q = 0; q < 4; q++) {
@@ -538,14 +547,14 @@ xs_status xs_lj_multi_force(xs_ctx* h, int ntypes, const double* epsilon, const 
     }
     c.ljm_d.reserve(d.size());
     c.ljm_f.reserve(f.size());
-    c.ljm_rcut.reserve(np);
+    c.ljm_rcut2.reserve(np);
     to_device(c, c.ljm_d, d.data(), (int64_t)d.size());
     to_device(c, c.ljm_f, f.data(), (int64_t)f.size());
-    to_device(c, c.ljm_rcut, rcut, np);
+    to_device(c, c.ljm_rcut2, rc2.data(), np);
     XS_HIP(hipStreamSynchronize(c.stream));  // the host rows go out of scope
     c.has_ljm = true;
     c.ljm_ntypes = ntypes;
-    c.ljm_rcmax = rcmax;
+    c.ljm_reach = reach;
     launch_lj_multi(c, flags);
   });
 }

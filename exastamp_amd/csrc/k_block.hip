@@ -1143,6 +1143,17 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, false, ltype);
   const int4 hd = a.head[b];
+  // MULTI: the pairs' parameters and squared cutoffs (at most 28 pairs of 7 species), so
+  // that a pair's lookup is an LDS read rather than two gathers through the texture path
+  // (136 k atoms, FP64, energy and virial: 90 -> 66 us)
+  __shared__ pm::LJ<Real> lrow[MULTI ? 28 : 1];
+  __shared__ double lrc2[MULTI ? 28 : 1];
+  if constexpr (MULTI) {
+    if ((int)threadIdx.x < lm.npair) {
+      lrow[threadIdx.x] = pm::lj_multi_row<Real>(lm, threadIdx.x);
+      lrc2[threadIdx.x] = lm.rcut2[threadIdx.x];
+    }
+  }
   stage<false>(a, b, hd, rec, ltype);
   const int half = pass_half();
   for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
@@ -1167,17 +1178,16 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
         double de_r, eh;
         if constexpr (MULTI) {
           const int pid = pm::type_pair(ti, ltype[nb[u].c]);
-          pm::lj_pair(pm::lj_multi_row<Real>(lm, pid), nb[u].d2, nb[u].in && pm::lj_multi_in(lm, pid, nb[u].d2),
-                      de_r, eh);
+          pm::lj_pair(lrow[pid], nb[u].d2, nb[u].in && nb[u].d2 <= lrc2[pid], de_r, eh);
         } else {
           pm::lj_pair(lp, nb[u].d2, nb[u].in, de_r, eh);
         }
-        const double fe0 = nb[u].x * de_r, fe1 = nb[u].y * de_r, fe2 = nb[u].z * de_r;
-        fx += fe0;
-        fy += fe1;
-        fz += fe2;
+        fx = fma(nb[u].x, de_r, fx);
+        fy = fma(nb[u].y, de_r, fy);
+        fz = fma(nb[u].z, de_r, fz);
         if constexpr (ENERGY) e += eh;
-        if constexpr (VIRIAL) pm::add_virial(v, fe0, fe1, fe2, nb[u].x, nb[u].y, nb[u].z);
+        if constexpr (VIRIAL)
+          pm::add_virial(v, nb[u].x * de_r, nb[u].y * de_r, nb[u].z * de_r, nb[u].x, nb[u].y, nb[u].z);
       }
     }
     fx = half_sum(fx);
@@ -1192,6 +1202,111 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
       if constexpr (DRIFT) pm::write_outputs_drift(o, dr, gi, pi, fx, fy, fz);
       else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, gi, fx, fy, fz, e, v);
     }
+  }
+}
+
+// Analytic Johnson EAM on the block list (FP64): pass 1 (EmbOp, eam_force_op_singlemat.h:39-171),
+// rho_i, F'(rho_i) into the position record's w and F(rho_i) added to ep.
+// Bound by the FP64 arithmetic of the pairs (one or two exponentials, divisions and a
+// square root each).  128 k Ta atoms (83 entries, 53 in rc), both passes with energy and
+// virial: 134 us, against 338 us, and 115 us to convert the list, on the global list with
+// the general power function and every term evaluated for itself.
+__global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs a, JohnsonParams jp,
+                                                                       double* __restrict__ rho_out,
+                                                                       double* __restrict__ pos_w,
+                                                                       double* __restrict__ ep)
+{
+  const int64_t b = lblock();
+  if (b >= a.nblocks) return;
+  uint8_t* ltype;
+  const LRec rec = pass_lds(a, false, false, ltype);
+  const int4 hd = a.head[b];
+  stage<false>(a, b, hd, rec, ltype);
+  const int half = pass_half();
+  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+    const int64_t gi = a.cen[b * a.ccap + q];
+    const int slot = a.cen_slot[b * a.ccap + q];
+    const Pos4 pi = rec.get(slot);
+    const int cnt = a.nnb[gi];
+    double rho = 0.0;
+    LWords lw = lwords(a, gi, half);
+    uint2 wnext = lw.get(0);
+    for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
+      const uint2 w = wnext;
+      if (k0 + 8 < cnt) wnext = lw.get(q + 1);
+      int c[kBBatch];
+      lslots(w, a.cap, k0, cnt, c);
+#pragma unroll
+      for (int u = 0; u < kBBatch; u++) {
+        LNb nb[1];
+        lgather<1>(a, rec, c + u, k0 + 2 * u, cnt, pi, nb);
+        if (!__any(nb[0].in)) continue;
+        const double v = pm::johnson_rho(jp, nb[0].in ? nb[0].d2 : jp.re * jp.re);
+        rho += nb[0].in ? v : 0.0;
+      }
+    }
+    rho = half_sum(rho);
+    if (half == 0) {
+      rho_out[gi] = rho;
+      double F, Fp;
+      pm::johnson_embed(jp, rho, F, Fp);
+      pos_w[4 * gi + 3] = Fp;
+      ep[gi] += F;
+    }
+  }
+}
+
+// Pass 2 (ForceOp): f_i += (rho'(r) (F'_i + F'_j) + phi'(r)) / r (r_j - r_i), ep += phi / 2,
+// virial -1/2 f (x) dr.
+template <bool VIRIAL>
+__global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_force(BlockArgs a, JohnsonParams jp, pm::Outputs o)
+{
+  const int64_t b = lblock();
+  if (b >= a.nblocks) return;
+  uint8_t* ltype;
+  const LRec rec = pass_lds(a, false, true, ltype);
+  const int4 hd = a.head[b];
+  stage<true>(a, b, hd, rec, ltype);
+  const int half = pass_half();
+  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+    const int64_t gi = a.cen[b * a.ccap + q];
+    const int slot = a.cen_slot[b * a.ccap + q];
+    const Pos4 pi = rec.get(slot);
+    const int cnt = a.nnb[gi];
+    double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
+    double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    LWords lw = lwords(a, gi, half);
+    uint2 wnext = lw.get(0);
+    for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
+      const uint2 w = wnext;
+      if (k0 + 8 < cnt) wnext = lw.get(q + 1);
+      int c[kBBatch];
+      lslots(w, a.cap, k0, cnt, c);
+#pragma unroll
+      for (int u = 0; u < kBBatch; u++) {
+        LNb nb[1];
+        lgather<1>(a, rec, c + u, k0 + 2 * u, cnt, pi, nb);
+        if (!__any(nb[0].in)) continue;
+        double de, phi;
+        pm::johnson_pair(jp, nb[0].in ? nb[0].d2 : jp.re * jp.re, pi.w + nb[0].w, de, phi);
+        de = nb[0].in ? de : 0.0;
+        const double fe0 = de * nb[0].x, fe1 = de * nb[0].y, fe2 = de * nb[0].z;
+        fx += fe0;
+        fy += fe1;
+        fz += fe2;
+        e += nb[0].in ? 0.5 * phi : 0.0;
+        if constexpr (VIRIAL) pm::add_virial(v, fe0, fe1, fe2, nb[0].x, nb[0].y, nb[0].z);
+      }
+    }
+    fx = half_sum(fx);
+    fy = half_sum(fy);
+    fz = half_sum(fz);
+    e = half_sum(e);
+    if constexpr (VIRIAL) {
+#pragma unroll
+      for (int k = 0; k < 9; k++) v[k] = half_sum(v[k]);
+    }
+    if (half == 0) pm::write_outputs<true, VIRIAL, false>(o, gi, fx, fy, fz, e, v);
   }
 }
 
@@ -1566,7 +1681,7 @@ void launch_lj_block(Ctx& c, double eps, double sigma, double rcut, unsigned fla
 
 void launch_lj_multi_block(Ctx& c, unsigned flags)
 {
-  const BlockArgs a = block_args(c, c.ljm_rcmax);
+  const BlockArgs a = block_args(c, c.ljm_reach);
   const size_t lds = block_lds_bytes(c, true, false);
   const unsigned g = block_grid(c);
   const pm::Outputs o = make_outputs(c, ForceEpilogue{});
@@ -1587,6 +1702,25 @@ void launch_lj_multi_block(Ctx& c, unsigned flags)
   };
   if (flags & XS_MIXED) run(0.0f);
   else run(0.0);
+  XS_HIP(hipGetLastError());
+}
+
+void launch_johnson_block(Ctx& c, const JohnsonParams& p, double rcut, bool do_emb, bool do_force, unsigned flags)
+{
+  const BlockArgs a = block_args(c, rcut);
+  const unsigned g = block_grid(c);
+  if (do_emb) {
+    ProfScope prof(c.prof, c.stream, XS_PROF_EAM_RHO);
+    k_block_johnson_rho<<<g, kPassThreads, block_lds_bytes(c, false, false), c.stream>>>(
+        a, p, c.rho.p, reinterpret_cast<double*>(c.pos.p), c.ep.p);
+    XS_HIP(hipGetLastError());
+  }
+  if (!do_force) return;
+  const pm::Outputs o = make_outputs(c, ForceEpilogue{});
+  ProfScope prof(c.prof, c.stream, XS_PROF_EAM_FORCE);
+  const size_t lds = block_lds_bytes(c, false, true);
+  if (flags & XS_VIRIAL) k_block_johnson_force<true><<<g, kPassThreads, lds, c.stream>>>(a, p, o);
+  else k_block_johnson_force<false><<<g, kPassThreads, lds, c.stream>>>(a, p, o);
   XS_HIP(hipGetLastError());
 }
 

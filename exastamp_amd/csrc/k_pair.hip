@@ -101,17 +101,17 @@ __global__ void __launch_bounds__(256) k_lj(PairCommon pc, LJParams<Real> lp, Ou
       double de_r, eh;
       if constexpr (MULTI) {
         const int pid = pm::type_pair(ti, pc.type[nb[u].j]);
-        pm::lj_pair(pm::lj_multi_row<Real>(lm, pid), nb[u].d2, nb[u].in && pm::lj_multi_in(lm, pid, nb[u].d2),
+        pm::lj_pair(pm::lj_multi_row<Real>(lm, pid), nb[u].d2, nb[u].in && nb[u].d2 <= lm.rcut2[pid],
                     de_r, eh);
       } else {
         pm::lj_pair(lp, nb[u].d2, nb[u].in, de_r, eh);
       }
-      const double fe0 = de_r * nb[u].x, fe1 = de_r * nb[u].y, fe2 = de_r * nb[u].z;
-      fx += fe0;
-      fy += fe1;
-      fz += fe2;
+      fx = fma(nb[u].x, de_r, fx);
+      fy = fma(nb[u].y, de_r, fy);
+      fz = fma(nb[u].z, de_r, fz);
       if constexpr (ENERGY) e += eh;
-      if constexpr (VIRIAL) add_virial(v, fe0, fe1, fe2, nb[u].x, nb[u].y, nb[u].z);
+      if constexpr (VIRIAL)
+        add_virial(v, nb[u].x * de_r, nb[u].y * de_r, nb[u].z * de_r, nb[u].x, nb[u].y, nb[u].z);
     }
   }
   write_outputs<ENERGY, VIRIAL, FUSED>(o, i, fx, fy, fz, e, v);
@@ -220,60 +220,6 @@ __global__ void __launch_bounds__(256) k_eam_force(PairCommon pc, EamTabDev<Real
 // accumulated, as EmbOp and ForceOp do.
 // ------------------------------------------------------------------------------
 
-// One screened exponential c exp(-a (x - 1)) / (1 + (x - k)^20) of x = r / re and its
-// r-derivative by the quotient rule: phi is the sum of two such terms (johnson.h:59-99),
-// rho(r) is one (johnson.h:105-124).
-__device__ __forceinline__ void johnson_term(double c, double a, double k, double x, double ire, double& v,
-                                             double& dv)
-{
-  const double num = c * exp(-a * (x - 1.0));
-  const double s = x - k;
-  const double s20 = pow(s, 20.0);
-  const double den = 1.0 + s20;
-  const double dnum = -a * num;
-  const double dden = 20.0 * s20 / s;
-  v = num / den;
-  dv = ire * (dnum * den - num * dden) / (den * den);
-}
-
-__device__ __forceinline__ void johnson_rho(const JohnsonParams& p, double r, double& rho, double& drho)
-{
-  johnson_term(p.fe, p.beta, p.lambda, r / p.re, 1.0 / p.re, rho, drho);
-}
-
-__device__ __forceinline__ void johnson_phi(const JohnsonParams& p, double r, double& phi, double& dphi)
-{
-  const double x = r / p.re, ire = 1.0 / p.re;
-  double v2, d2;
-  johnson_term(p.A, p.alpha, p.kappa, x, ire, phi, dphi);
-  johnson_term(-p.B, p.beta, p.lambda, x, ire, v2, d2);
-  phi += v2;
-  dphi += d2;
-}
-
-// F(rho) and F'(rho) (johnson.h:131-167): cubic in rho / (0.85 rhoe) - 1 below
-// 0.85 rhoe, cubic in rho / rhoe - 1 below 1.15 rhoe, Fo (1 - ln q^eta) q^eta above.
-__device__ __forceinline__ void johnson_embed(const JohnsonParams& p, double rho, double& f, double& df)
-{
-  const double rhon = 0.85 * p.rhoe, rho0 = 1.15 * p.rhoe;
-  const double irhoe = 1.0 / p.rhoe;
-  if (rho < rhon) {
-    const double t = rho / rhon - 1.0, t2 = t * t, t3 = t * t2;
-    f = p.Fn0 + p.Fn1 * t + p.Fn2 * t2 + p.Fn3 * t3;
-    df = (p.Fn1 + 2.0 * p.Fn2 * t + 3.0 * p.Fn3 * t2) * (1.0 / rhon);
-  } else if (rho < rho0) {
-    const double t = rho * irhoe - 1.0, t2 = t * t, t3 = t * t2;
-    f = p.F0 + p.F1 * t + p.F2 * t2 + p.F3 * t3;
-    df = (p.F1 + 2.0 * p.F2 * t + 3.0 * p.F3 * t2) * irhoe;
-  } else {
-    const double q = rho * irhoe;
-    const double qe = pow(q, p.eta);
-    const double lq = log(qe);
-    f = p.Fo * (1.0 - lq) * qe;
-    df = (-p.eta * qe + (1.0 - lq) * p.eta * qe) * (p.Fo * irhoe / q);
-  }
-}
-
 // Pass 1 (EmbOp): rho_i over the pairs inside rc, then F'(rho_i) into the position
 // record's w and F(rho_i) added to ep.
 __global__ void __launch_bounds__(256) k_johnson_rho(PairCommon pc, JohnsonParams jp, double* __restrict__ rho_out,
@@ -290,8 +236,7 @@ __global__ void __launch_bounds__(256) k_johnson_rho(PairCommon pc, JohnsonParam
     fetch<kBatch>(pc, i, k0, cnt, pi, L, nb);
 #pragma unroll
     for (int u = 0; u < kBatch; u++) {
-      double v, dv;
-      johnson_rho(jp, nb[u].in ? sqrt(nb[u].d2) : jp.re, v, dv);
+      const double v = johnson_rho(jp, nb[u].in ? nb[u].d2 : jp.re * jp.re);
       rho += nb[u].in ? v : 0.0;
     }
   }
@@ -319,11 +264,9 @@ __global__ void __launch_bounds__(256) k_johnson_force(PairCommon pc, JohnsonPar
     fetch<kBatch>(pc, i, k0, cnt, pi, L, nb);
 #pragma unroll
     for (int u = 0; u < kBatch; u++) {
-      const double r = nb[u].in ? sqrt(nb[u].d2) : jp.re;
-      double rho, drho, phi, dphi;
-      johnson_rho(jp, r, rho, drho);
-      johnson_phi(jp, r, phi, dphi);
-      const double de = nb[u].in ? (drho * (pi.w + nb[u].w) + dphi) / r : 0.0;
+      double de, phi;
+      johnson_pair(jp, nb[u].in ? nb[u].d2 : jp.re * jp.re, pi.w + nb[u].w, de, phi);
+      de = nb[u].in ? de : 0.0;
       const double fe0 = de * nb[u].x, fe1 = de * nb[u].y, fe2 = de * nb[u].z;
       fx += fe0;
       fy += fe1;
@@ -435,7 +378,7 @@ void lj_dispatch(Ctx& c, double eps, double sigma, double rcut, unsigned flags, 
 template <class Real>
 void lj_multi_dispatch(Ctx& c, unsigned flags)
 {
-  const PairCommon pc = make_common(c, c.ljm_rcmax);
+  const PairCommon pc = make_common(c, c.ljm_reach);
   const Outputs o = make_outputs(c, ForceEpilogue{});
   const pm::LJMultiDev lm = ljm_dev<Real>(c);
   const unsigned g = pair_grid(c.n);
@@ -585,7 +528,10 @@ void launch_johnson(Ctx& c, const JohnsonParams& p, double rcut, bool do_emb, bo
   c.rho_ckpt = false;
   if (do_emb) c.rho_state = RhoState::FpJohnson;
   if (c.n == 0 || !(do_emb || do_force)) return;
-  ensure_global_list(c);
+  if (c.list_kind == ListKind::Block) {
+    launch_johnson_block(c, p, rcut, do_emb, do_force, flags);
+    return;
+  }
   const PairCommon pc = make_common(c, rcut);
   const unsigned g = pair_grid(c.n);
   if (do_emb) {

@@ -37,6 +37,8 @@ __device__ __forceinline__ void dist(double d2, double& r, double& rinv)
 }
 __device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double recip(double x) { return 1.0 / x; }
+__device__ __forceinline__ float fma_r(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_r(double a, double b, double c) { return fma(a, b, c); }
 
 // XCD-aware block order: hardware hands workgroup b to XCD b % 8, so map it to
 // logical block (b % 8) * (G/8) + b / 8 and each XCD's L2 sees one contiguous
@@ -141,7 +143,7 @@ __device__ __forceinline__ void add_virial(double* v, double fe0, double fe1, do
 #pragma unroll
   for (int a = 0; a < 3; a++)
 #pragma unroll
-    for (int b = 0; b < 3; b++) v[3 * a + b] += (fe[a] * dr[b]) * -0.5;
+    for (int b = 0; b < 3; b++) v[3 * a + b] = fma(fe[a] * dr[b], -0.5, v[3 * a + b]);
 }
 
 template <class Real>
@@ -441,6 +443,65 @@ __device__ __forceinline__ void eam_pair_batch(const EamTabDev<Real>& t, const R
   }
 }
 
+// ---------------------------------------------------------------------------
+// Analytic Johnson EAM (johnson.h:59-167), FP64
+// ---------------------------------------------------------------------------
+// Its functions of r are sums of screened exponentials t(x) = exp(-a (x - 1)) / (1 + (x - k)^20)
+// of x = r / re (johnson.h:59-124); t and its x-derivative -t (a + 20 (x - k)^19 / (1 + (x - k)^20)).
+// The power is five squarings and products (the general power function cost more than
+// the two exponentials of a pair), and rho and the second term of phi share one t.
+__device__ __forceinline__ void johnson_term(double a, double k, double x, double& t, double& dt)
+{
+  const double s = x - k, s2 = s * s, s4 = s2 * s2, s8 = s4 * s4;
+  const double s19 = s8 * s8 * (s2 * s);
+  const double inv = 1.0 / fma(s19, s, 1.0);
+  t = exp(-a * (x - 1.0)) * inv;
+  dt = -t * fma(20.0 * s19, inv, a);
+}
+
+// rho(r) at d2 = r^2
+__device__ __forceinline__ double johnson_rho(const JohnsonParams& p, double d2)
+{
+  double t, dt;
+  johnson_term(p.beta, p.lambda, sqrt(d2) / p.re, t, dt);
+  return p.fe * t;
+}
+
+// (rho'(r) fsum + phi'(r)) / r and phi(r) at d2 = r^2, fsum = F'_i + F'_j
+__device__ __forceinline__ void johnson_pair(const JohnsonParams& p, double d2, double fsum, double& de_r,
+                                             double& phi)
+{
+  const double r = sqrt(d2), ire = 1.0 / p.re, x = r * ire;
+  double t1, d1, t2, d2x;
+  johnson_term(p.alpha, p.kappa, x, t1, d1);
+  johnson_term(p.beta, p.lambda, x, t2, d2x);
+  phi = p.A * t1 - p.B * t2;
+  de_r = (fma(p.fe, fsum, -p.B) * d2x + p.A * d1) * ire / r;
+}
+
+// F(rho) and F'(rho) (johnson.h:131-167): cubic in rho / (0.85 rhoe) - 1 below
+// 0.85 rhoe, cubic in rho / rhoe - 1 below 1.15 rhoe, Fo (1 - ln q^eta) q^eta above.
+__device__ __forceinline__ void johnson_embed(const JohnsonParams& p, double rho, double& f, double& df)
+{
+  const double rhon = 0.85 * p.rhoe, rho0 = 1.15 * p.rhoe;
+  const double irhoe = 1.0 / p.rhoe;
+  if (rho < rhon) {
+    const double t = rho / rhon - 1.0, t2 = t * t, t3 = t * t2;
+    f = p.Fn0 + p.Fn1 * t + p.Fn2 * t2 + p.Fn3 * t3;
+    df = (p.Fn1 + 2.0 * p.Fn2 * t + 3.0 * p.Fn3 * t2) * (1.0 / rhon);
+  } else if (rho < rho0) {
+    const double t = rho * irhoe - 1.0, t2 = t * t, t3 = t * t2;
+    f = p.F0 + p.F1 * t + p.F2 * t2 + p.F3 * t3;
+    df = (p.F1 + 2.0 * p.F2 * t + 3.0 * p.F3 * t2) * irhoe;
+  } else {
+    const double q = rho * irhoe;
+    const double qe = pow(q, p.eta);
+    const double lq = log(qe);
+    f = p.Fo * (1.0 - lq) * qe;
+    df = (-p.eta * qe + (1.0 - lq) * p.eta * qe) * (p.Fo * irhoe / q);
+  }
+}
+
 // Lennard-Jones pair (lennard_jones.h:40-50, force_op_impl2.hxx:33-78) written in
 // r^2 only: (sigma/r)^2 = sigma^2 / d2, de/r = -24 eps (2 s^12 - s^6) / d2, e shifted
 // by E(rcut) (pair_potential_impl.hxx:487-498).  Pair math in Real, FP64 out.
@@ -450,11 +511,13 @@ struct LJ {
 };
 
 // lj_multi_force: parameters per unordered pair of species (packed triangle,
-// entry b*(b+1)/2 + a for a <= b) and each pair's cutoff radius; a pair counts
-// when r <= its rcut (pair_potential_force_op_multiparam.h:82-84).
+// entry b*(b+1)/2 + a for a <= b) and each pair's squared cutoff; a pair counts when
+// r <= its rcut (pair_potential_force_op_multiparam.h:82-84), i.e. when d2 is at most the
+// largest number whose square root is (the host's rcut2; below 0: no interaction).
 struct LJMultiDev {
   const void* rows;          // LJ<Real> per type pair
-  const double* __restrict__ rcut;
+  const double* __restrict__ rcut2;
+  int npair;
 };
 __device__ __forceinline__ int type_pair(int a, int b)
 {
@@ -466,10 +529,6 @@ __device__ __forceinline__ LJ<Real> lj_multi_row(const LJMultiDev& m, int pid)
 {
   return reinterpret_cast<const LJ<Real>*>(m.rows)[pid];
 }
-__device__ __forceinline__ bool lj_multi_in(const LJMultiDev& m, int pid, double d2)
-{
-  return sqrt(d2) <= m.rcut[pid];
-}
 
 template <class Real>
 __device__ __forceinline__ void lj_pair(const LJ<Real>& lp, double d2, bool in, double& de_r, double& e)
@@ -478,8 +537,9 @@ __device__ __forceinline__ void lj_pair(const LJ<Real>& lp, double d2, bool in, 
   const Real s2 = lp.sigma2 * ir2;
   const Real s6 = s2 * s2 * s2;
   const Real s12 = s6 * s6;
-  de_r = in ? (double)(-lp.eps24 * (Real(2) * s12 - s6) * ir2) : 0.0;
-  e = in ? 0.5 * (double)(lp.eps4 * (s12 - s6) - lp.ecut) : 0.0;
+  // fused multiply-adds spelled out, so that every kernel rounds a pair alike
+  de_r = in ? (double)(-lp.eps24 * fma_r(Real(2), s12, -s6) * ir2) : 0.0;
+  e = in ? 0.5 * (double)fma_r(lp.eps4, s12 - s6, -lp.ecut) : 0.0;
 }
 
 }  // namespace pm
@@ -493,7 +553,8 @@ inline pm::LJMultiDev ljm_dev(const Ctx& c)
   pm::LJMultiDev m;
   if constexpr (sizeof(Real) == 4) m.rows = c.ljm_f.p;
   else m.rows = c.ljm_d.p;
-  m.rcut = c.ljm_rcut.p;
+  m.rcut2 = c.ljm_rcut2.p;
+  m.npair = c.ljm_ntypes * (c.ljm_ntypes + 1) / 2;
   return m;
 }
 

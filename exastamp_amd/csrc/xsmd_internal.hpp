@@ -156,6 +156,12 @@ struct EamHost {
   double s_err[3] = {0, 0, 0};
 };
 
+// EamJohnsonParameters (johnson.h:30-51) in internal units, in the order of
+// xs_johnson_force's parameter array
+struct JohnsonParams {
+  double re, fe, rhoe, alpha, beta, A, B, kappa, lambda, Fn0, Fn1, Fn2, Fn3, F0, F1, F2, F3, Fo, eta;
+};
+
 // What the per-atom EAM scalar currently holds: rho (c.rho) after the density
 // pass alone, or F'(rho) (pos[i].w) after the embedding step.
 enum class RhoState { None, Rho, FpDouble, FpFloat, FpJohnson };
@@ -340,12 +346,12 @@ struct Ctx {
   bool has_lj = false;
   double lj_eps = 0, lj_sigma = 0, lj_rcut = 0;
   // lj_multi_force: per type pair (packed triangle) FP32 and FP64 rows
-  // {sigma^2, 4 eps, 24 eps, E(rcut)} and the pairs' cutoffs
+  // {sigma^2, 4 eps, 24 eps, E(rcut)} and the pairs' squared cutoffs
   bool has_ljm = false;
   int ljm_ntypes = 0;
-  double ljm_rcmax = 0;
+  double ljm_reach = 0;  // largest cutoff of a pair that interacts
   DBuf<float> ljm_f;
-  DBuf<double> ljm_d, ljm_rcut;
+  DBuf<double> ljm_d, ljm_rcut2;
   bool has_eam = false;
   EamHost eam;
   // types slot of eam_alloy_force (eam_potential_multimat.cu:90,154-166) as enable
@@ -428,14 +434,10 @@ inline double lj_energy_cutoff(double eps, double sigma, double rcut)
 void launch_lj(Ctx& c, double eps, double sigma, double rcut, unsigned flags, const ForceEpilogue& ep);
 // lj_multi_force (operator form) on the current list; tables set by xs_lj_multi_force
 void launch_lj_multi(Ctx& c, unsigned flags);
-// EamJohnsonParameters (johnson.h:30-51) in internal units, in the order of
-// xs_johnson_force's parameter array
-struct JohnsonParams {
-  double re, fe, rhoe, alpha, beta, A, B, kappa, lambda, Fn0, Fn1, Fn2, Fn3, F0, F1, F2, F3, Fo, eta;
-};
 // johnson_force / johnson_emb / johnson_force_reuse_emb: the passes of the
-// single-material EAM template, FP64, global list
+// single-material EAM template, FP64
 void launch_johnson(Ctx& c, const JohnsonParams& p, double rcut, bool do_emb, bool do_force, unsigned flags);
+void launch_johnson_block(Ctx& c, const JohnsonParams& p, double rcut, bool do_emb, bool do_force, unsigned flags);
 void launch_lj_multi_block(Ctx& c, unsigned flags);
 // LJ on the cell-block list (k_block.hip)
 void launch_lj_block(Ctx& c, double eps, double sigma, double rcut, unsigned flags, const ForceEpilogue& ep);
