@@ -282,7 +282,12 @@ __device__ __forceinline__ void stage(const BlockArgs& a, int64_t b, const int4&
 }
 
 // sum of v over the two halves of the wave (lanes l and l ^ 32)
-__device__ __forceinline__ double half_sum(double v) { return v + __shfl_xor(v, 32); }
+__device__ __forceinline__ double half_sum(double v)
+{
+  double a = v, b = v;
+  swap_halves<false>(a, b);
+  return a + b;
+}
 
 // this lane's atom slot and which half of the wave it is in
 __device__ __forceinline__ int pass_slot() { return (threadIdx.x >> 6) * 32 + (threadIdx.x & 31); }
@@ -344,18 +349,10 @@ __device__ __forceinline__ uint4 group_interleave(const uint32_t (&o)[4])
 // groups, so four steps reach every lane).
 __device__ __forceinline__ double row16_min(double v)
 {
-#define XS_DPP_MIN(ctrl)                                                                                            \
-  {                                                                                                                 \
-    const long long b = __double_as_longlong(v);                                                                    \
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, ctrl, 0xf, 0xf, true);                 \
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), ctrl, 0xf, 0xf, true);         \
-    v = fmin(v, __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo)));                            \
-  }
-  XS_DPP_MIN(0xB1)   // quad_perm [1, 0, 3, 2]
-  XS_DPP_MIN(0x4E)   // quad_perm [2, 3, 0, 1]
-  XS_DPP_MIN(0x141)  // row_half_mirror
-  XS_DPP_MIN(0x140)  // row_mirror
-#undef XS_DPP_MIN
+  v = fmin(v, dpp_double<kDppXor1>(v));
+  v = fmin(v, dpp_double<kDppXor2>(v));
+  v = fmin(v, dpp_double<kDppHalfMirror>(v));
+  v = fmin(v, dpp_double<kDppMirror>(v));
   return v;
 }
 
@@ -405,14 +402,14 @@ __device__ __forceinline__ void sort64(uint32_t (&v)[8])
 #pragma unroll
   for (int k = 0; k < 19; k++) order2(v[net[k][0]], v[net[k][1]]);
   const int j = threadIdx.x & 7;
-  order_lanes<0xB1, true>(v, (j & 1) == 0);   // lanes 0-1, quad_perm [1, 0, 3, 2]
+  order_lanes<kDppXor1, true>(v, (j & 1) == 0);  // lanes 0-1
   merge8(v);
-  order_lanes<0x1B, true>(v, (j & 2) == 0);   // lanes 0-3 mirrored, quad_perm [3, 2, 1, 0]
-  order_lanes<0xB1, false>(v, (j & 1) == 0);
+  order_lanes<0x1B, true>(v, (j & 2) == 0);      // lanes 0-3 mirrored, quad_perm [3, 2, 1, 0]
+  order_lanes<kDppXor1, false>(v, (j & 1) == 0);
   merge8(v);
-  order_lanes<0x141, true>(v, (j & 4) == 0);  // lanes 0-7 mirrored, row_half_mirror
-  order_lanes<0x4E, false>(v, (j & 2) == 0);  // quad_perm [2, 3, 0, 1]
-  order_lanes<0xB1, false>(v, (j & 1) == 0);
+  order_lanes<kDppHalfMirror, true>(v, (j & 4) == 0);  // lanes 0-7 mirrored
+  order_lanes<kDppXor2, false>(v, (j & 2) == 0);
+  order_lanes<kDppXor1, false>(v, (j & 1) == 0);
   merge8(v);
 }
 

@@ -117,23 +117,38 @@ __global__ void __launch_bounds__(256) k_stream_copy(int64_t n16, const double2*
 constexpr int kThermoBlocks = 1024;
 constexpr int kThermoQ = 26;
 
+// one halving of wave_sum32 between the lanes whose bit `hi` differs
+template <int CTRL, int HALF>
+__device__ __forceinline__ void halve(double (&v)[32], bool hi)
+{
+#pragma unroll
+  for (int q = 0; q < HALF; q++) {
+    const double keep = hi ? v[HALF + q] : v[q];
+    const double send = hi ? v[q] : v[HALF + q];
+    v[q] = keep + dpp_double<CTRL>(send);
+  }
+}
+
 // Sums over the 64 lanes of a wave of 32 quantities per lane: at each halving of the
 // lane distance a lane keeps one half of the quantities it still holds and hands the
 // other half to its partner, so the whole reduction is 32 exchanges instead of 6 per
-// quantity.  Lane l ends with the total of quantity bitrev5(l >> 1), in a fixed order.
+// quantity.  Lane l ends with the total of quantity wave_sum32_index(l), in a fixed order.
 __device__ __forceinline__ double wave_sum32(double (&v)[32], int lane)
 {
 #pragma unroll
-  for (int half = 16, off = 32; half >= 1; half >>= 1, off >>= 1) {
-    const bool hi = lane & off;
-#pragma unroll
-    for (int q = 0; q < half; q++) {
-      const double keep = hi ? v[half + q] : v[q];
-      const double send = hi ? v[q] : v[half + q];
-      v[q] = keep + __shfl_xor(send, off);
-    }
+  for (int q = 0; q < 16; q++) {
+    swap_halves<false>(v[q], v[16 + q]);
+    v[q] += v[16 + q];
   }
-  return v[0] + __shfl_xor(v[0], 1);
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    swap_halves<true>(v[q], v[8 + q]);
+    v[q] += v[8 + q];
+  }
+  halve<kDppXor8, 4>(v, lane & 8);
+  halve<kDppHalfMirror, 2>(v, lane & 4);
+  halve<kDppXor2, 1>(v, lane & 2);
+  return v[0] + dpp_double<kDppXor1>(v[0]);
 }
 
 // the quantity whose total lane l holds after wave_sum32

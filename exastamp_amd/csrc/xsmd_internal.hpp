@@ -84,6 +84,43 @@ __device__ __forceinline__ void store_pos(Pos4* __restrict__ p, int64_t j, const
   q[1] = make_double2(v.z, v.w);
 }
 
+// Lane exchanges of doubles in vector registers (no LDS permutes).
+// The value of the lane that DPP control CTRL names:
+template <int CTRL>
+__device__ __forceinline__ double dpp_double(double v)
+{
+  const long long b = __double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+constexpr int kDppXor1 = 0xB1;         // quad_perm [1, 0, 3, 2]
+constexpr int kDppXor2 = 0x4E;         // quad_perm [2, 3, 0, 1]
+constexpr int kDppHalfMirror = 0x141;  // lane 7 - i within each 8
+constexpr int kDppMirror = 0x140;      // lane 15 - i within each 16
+constexpr int kDppXor8 = 0x128;        // row_ror:8
+
+// the upper half of the wave in a (ROW16: the odd rows of 16 lanes) trades places with
+// the lower half (the even rows) in b
+template <bool ROW16>
+__device__ __forceinline__ void swap_halves(double& a, double& b)
+{
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a);
+  const unsigned long long y = (unsigned long long)__double_as_longlong(b);
+  uint32_t x0 = (uint32_t)x, x1 = (uint32_t)(x >> 32), y0 = (uint32_t)y, y1 = (uint32_t)(y >> 32);
+  if constexpr (ROW16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
+    const auto t = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
+    x0 = r[0], y0 = r[1], x1 = t[0], y1 = t[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(x0, y0, false, false);
+    const auto t = __builtin_amdgcn_permlane32_swap(x1, y1, false, false);
+    x0 = r[0], y0 = r[1], x1 = t[0], y1 = t[1];
+  }
+  a = __longlong_as_double((long long)(((unsigned long long)x1 << 32) | x0));
+  b = __longlong_as_double((long long)(((unsigned long long)y1 << 32) | y0));
+}
+
 // Box of one replica, as kernels read it: lo[3], L[3], n/L[3].
 struct BoxDev {
   double lo[3];
