@@ -220,6 +220,7 @@ struct BlockArgs {
   int ccap;  // central atoms per brick at most
   double rc2;
   const XformDev* xf;  // the staging maps positions to physical space when not NULL
+  StepGate gate;       // MD loop
 };
 
 // LDS of the block passes: records, then per-record types (block_lds_bytes on the host
@@ -885,7 +886,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
                                                                 double* __restrict__ pos_w, double* __restrict__ ep)
 {
   const int64_t b = lblock();
-  if (b >= a.nblocks) return;
+  if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, false, ltype);
   const int4 hd = a.head[b];
@@ -951,7 +952,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_
 {
   static_assert(!DRIFT || (FUSED && !ENERGY && !VIRIAL), "the drift epilogue is the plain MD-loop step");
   const int64_t b = lblock();
-  if (b >= a.nblocks) return;
+  if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, true, ltype);
   const int4 hd = a.head[b];
@@ -1136,7 +1137,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
 {
   static_assert(!DRIFT || (FUSED && !ENERGY && !VIRIAL), "the drift epilogue is the plain MD-loop step");
   const int64_t b = lblock();
-  if (b >= a.nblocks) return;
+  if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, false, ltype);
   const int4 hd = a.head[b];
@@ -1307,9 +1308,10 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_force(BlockAr
   }
 }
 
-BlockArgs block_args(const Ctx& c, double rcut)
+BlockArgs block_args(const Ctx& c, double rcut, const StepGate& gate = {})
 {
   BlockArgs a;
+  a.gate = gate;
   a.head = c.brick_head.p;
   a.stage = c.brick_stage.p;
   a.cen = c.brick_cen.p;
@@ -1345,8 +1347,7 @@ bool drift_setup(Ctx& c, const ForceEpilogue& epi, unsigned flags, pm::Drift& dr
   dr.dt2 = epi.drift_dt * epi.drift_dt * 0.5;
   dr.hdt = epi.drift_dt * 0.5;
   dr.thr2 = epi.drift_thr2;
-  dr.over = c.dscalar.p + 5;
-  XS_HIP(hipMemsetAsync(c.dscalar.p + 5, 0, sizeof(unsigned long long), c.stream));
+  dr.over = StepFlag{c.dscalar.p + 5, c.hflag, epi.step + 1};
   return true;
 }
 
@@ -1364,7 +1365,7 @@ void block_eam_dispatch(Ctx& c, double rcut, bool do_rho, bool do_emb, bool do_f
 {
   const EamTabDev<Real> t = make_eam_tab<Real>(c);
   const Real* pair = eam_pair_table<Real>(c);
-  const BlockArgs a = block_args(c, rcut);
+  const BlockArgs a = block_args(c, rcut, step_gate(c, epi));
   const size_t lds_rho = block_lds_bytes(c, MULTI, false);
   const size_t lds = block_lds_bytes(c, MULTI, true);
   const unsigned g = block_grid(c);
@@ -1643,10 +1644,11 @@ void launch_eam_block(Ctx& c, double rcut, bool do_rho, bool do_emb, bool do_for
 void launch_lj_block(Ctx& c, double eps, double sigma, double rcut, unsigned flags, const ForceEpilogue& epi)
 {
   const double ecut = lj_energy_cutoff(eps, sigma, rcut);
-  const BlockArgs a = block_args(c, rcut);
+  const BlockArgs a = block_args(c, rcut, step_gate(c, epi));
   const size_t lds = block_lds_bytes(c, false, false);
   const unsigned g = block_grid(c);
-  const pm::Outputs o = make_outputs(c, epi);
+  pm::Outputs o = make_outputs(c, epi);
+  o.set_ep = epi.fused;
   const bool energy = flags & XS_ENERGY, vir = flags & XS_VIRIAL;
   pm::Drift dr{};
   const bool drift = drift_setup(c, epi, flags, dr);

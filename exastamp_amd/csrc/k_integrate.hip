@@ -64,18 +64,18 @@ __global__ void k_push_f_v(int64_t n, double dt, double* vx, double* vy, double*
   vz[i] = fma(az[i], dt, vz[i]);
 }
 
-// push_f_v_r(dt) then push_f_v(dt/2), plus the largest squared displacement
-// since the last list build (as bits of a non-negative double, which order
-// like the doubles themselves): reduced per block, one atomic per block.  Under a
-// non-identity xform the step is mapped by mi (INV_XFORM) and the displacement is
-// measured in physical space.
+// push_f_v_r(dt) then push_f_v(dt/2), raising the loop's flag when an atom is further
+// than sqrt(thr2) from its position at the last list build.  Under a non-identity xform
+// the step is mapped by mi (INV_XFORM) and the displacement is measured in physical
+// space.
 __global__ void __launch_bounds__(256) k_drift_kick(
     int64_t n, double dt, double dt2, double hdt, Pos4* __restrict__ pos, double* vx, double* vy,
     double* vz, const double* __restrict__ ax, const double* __restrict__ ay,
     const double* __restrict__ az, const double* __restrict__ rrx, const double* __restrict__ rry,
-    const double* __restrict__ rrz, unsigned long long* __restrict__ maxd2, const XformDev* __restrict__ xf)
+    const double* __restrict__ rrz, double thr2, StepFlag over, StepGate gate, const XformDev* __restrict__ xf)
 {
-  double d2 = 0.0;
+  if (gate.closed()) return;
+  bool far = false;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     const double a0 = ax[i], a1 = ay[i], a2 = az[i];
@@ -92,17 +92,9 @@ __global__ void __launch_bounds__(256) k_drift_kick(
     vz[i] = fma(a2, hdt, v2);
     double ux = p.x - rrx[i], uy = p.y - rry[i], uz = p.z - rrz[i];
     if (xf) xsmd_xform_apply(xf->m, &ux, &uy, &uz);
-    d2 = fmax(d2, xsmd_d2(ux, uy, uz));
+    far |= xsmd_d2(ux, uy, uz) > thr2;
   }
-  for (int off = 32; off > 0; off >>= 1) d2 = fmax(d2, __shfl_xor(d2, off));
-  __shared__ double sh[kBlock / 64];
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = d2;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = sh[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); w++) m = fmax(m, sh[w]);
-    if (m > 0.0) atomicMax(maxd2, (unsigned long long)__double_as_longlong(m));
-  }
+  if (far) over.raise();
 }
 
 // Plain streaming copy, 16 bytes per lane per iteration.
@@ -166,8 +158,9 @@ __device__ __forceinline__ int wave_sum32_index(int lane)
 __global__ void __launch_bounds__(256) k_thermo_partial(
     int64_t n, int64_t npad, const double* __restrict__ vx, const double* __restrict__ vy,
     const double* __restrict__ vz, const double* __restrict__ ep, const double* __restrict__ vir,
-    const uint8_t* __restrict__ type, const double* __restrict__ mass, double* __restrict__ part)
+    const uint8_t* __restrict__ type, const double* __restrict__ mass, double* __restrict__ part, StepGate gate)
 {
+  if (gate.closed()) return;
   double acc[32];
 #pragma unroll
   for (int q = 0; q < 32; q++) acc[q] = 0.0;
@@ -206,8 +199,9 @@ __global__ void __launch_bounds__(256) k_thermo_partial(
 // loads: 242 us at 1024 partials, 48 us at 200, against about 5 us.
 constexpr int kThermoFinal = 1024;
 __global__ void __launch_bounds__(kThermoFinal) k_thermo_final27(int nblocks, const double* __restrict__ part,
-                                                                 int64_t n, double* __restrict__ out27)
+                                                                 int64_t n, double* __restrict__ out27, StepGate gate)
 {
+  if (gate.closed()) return;
   __shared__ double sh[32][33];
   const int q = threadIdx.x & 31, g = threadIdx.x >> 5;
   double s = 0.0;
@@ -275,33 +269,38 @@ void launch_push_f_v(Ctx& c, double dt)
   XS_HIP(hipGetLastError());
 }
 
-void launch_drift_kick(Ctx& c, double dt)
+void launch_drift_kick(Ctx& c, double dt, double thr2, unsigned long long step, bool gated)
 {
   if (c.n == 0) return;
   c.rho_ckpt = false;
   const double dt2 = dt * dt * 0.5;
   ProfScope prof(c.prof, c.stream, XS_PROF_DRIFT);
   const unsigned g = std::min<unsigned>(grid_for(c.n), 4096);
+  const StepGate gate = gated ? StepGate{c.dscalar.p + 5, step - 1} : StepGate{};
   k_drift_kick<<<g, kBlock, 0, c.stream>>>(c.n, dt, dt2, dt * 0.5, c.pos.p, c.vx.p, c.vy.p, c.vz.p, c.ax.p,
-                                           c.ay.p, c.az.p, c.rrx.p, c.rry.p, c.rrz.p, c.dscalar.p + 1, c.xf_dev());
+                                           c.ay.p, c.az.p, c.rrx.p, c.rry.p, c.rrz.p, thr2,
+                                           StepFlag{c.dscalar.p + 5, c.hflag, step}, gate, c.xf_dev());
+  XS_HIP(hipGetLastError());
+}
+
+void launch_thermo_dev(Ctx& c, double* out27_dev, const StepGate& gate)
+{
+  c.red_part.reserve((size_t)kThermoBlocks * kThermoQ);
+  ProfScope prof(c.prof, c.stream, XS_PROF_THERMO);
+  const int nb = c.n > 0 ? (int)std::min<int64_t>(kThermoBlocks, grid_for(c.n)) : 0;
+  if (nb > 0) {
+    k_thermo_partial<<<nb, kBlock, 0, c.stream>>>(c.n, c.npad, c.vx.p, c.vy.p, c.vz.p, c.ep.p, c.vir.p,
+                                                  c.type.p, c.mass_d.p, c.red_part.p, gate);
+    XS_HIP(hipGetLastError());
+  }
+  k_thermo_final27<<<1, kThermoFinal, 0, c.stream>>>(nb, c.red_part.p, c.n, out27_dev, gate);
   XS_HIP(hipGetLastError());
 }
 
 void launch_thermo(Ctx& c, double out[27])
 {
-  c.red_part.reserve((size_t)kThermoBlocks * kThermoQ);
   c.red_out.reserve(27);
-  const int nb = c.n > 0 ? (int)std::min<int64_t>(kThermoBlocks, grid_for(c.n)) : 0;
-  {
-    ProfScope prof(c.prof, c.stream, XS_PROF_THERMO);
-    if (nb > 0) {
-      k_thermo_partial<<<nb, kBlock, 0, c.stream>>>(c.n, c.npad, c.vx.p, c.vy.p, c.vz.p, c.ep.p, c.vir.p,
-                                                    c.type.p, c.mass_d.p, c.red_part.p);
-      XS_HIP(hipGetLastError());
-    }
-    k_thermo_final27<<<1, kThermoFinal, 0, c.stream>>>(nb, c.red_part.p, c.n, c.red_out.p);
-    XS_HIP(hipGetLastError());
-  }
+  launch_thermo_dev(c, c.red_out.p, StepGate{});
   XS_HIP(hipMemcpyAsync(c.hthermo, c.red_out.p, 27 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
   XS_HIP(hipStreamSynchronize(c.stream));
   std::memcpy(out, c.hthermo, 27 * sizeof(double));
@@ -331,10 +330,10 @@ void launch_thermo_noalloc(Ctx& c, double* out27_dev)
                                 " doubles)");
   if (nb > 0) {
     k_thermo_partial<<<nb, kBlock, 0, c.stream>>>(c.n, c.npad, c.vx.p, c.vy.p, c.vz.p, c.ep.p, c.vir.p, c.type.p,
-                                                  c.mass_d.p, part);
+                                                  c.mass_d.p, part, StepGate{});
     XS_HIP(hipGetLastError());
   }
-  k_thermo_final27<<<1, kThermoFinal, 0, c.stream>>>(nb, part, c.n, out27_dev);
+  k_thermo_final27<<<1, kThermoFinal, 0, c.stream>>>(nb, part, c.n, out27_dev, StepGate{});
   XS_HIP(hipGetLastError());
 }
 

@@ -30,6 +30,7 @@ struct PairCommon {
   const int* __restrict__ nnb;
   double rc2;
   const XformDev* xf;  // displacements m * (r_j(image) - r_i) when not NULL
+  StepGate gate;       // MD loop
 };
 
 constexpr int kBatch = 4;
@@ -86,7 +87,7 @@ template <class Real, bool ENERGY, bool VIRIAL, bool FUSED, bool MULTI = false>
 __global__ void __launch_bounds__(256) k_lj(PairCommon pc, LJParams<Real> lp, Outputs o, pm::LJMultiDev lm = {})
 {
   const int64_t i = logical_block() * blockDim.x + threadIdx.x;
-  if (i >= pc.n) return;
+  if (i >= pc.n || pc.gate.closed()) return;
   const double* L = pc.box[pc.rep ? pc.rep[i] : 0].L;
   const Pos4 pi = load_pos(pc.pos, i);
   const int ti = MULTI ? pc.type[i] : 0;
@@ -131,7 +132,7 @@ __global__ void __launch_bounds__(256) k_eam_rho(PairCommon pc, EamTabDev<Real> 
                                                  double* __restrict__ ep)
 {
   const int64_t i = logical_block() * blockDim.x + threadIdx.x;
-  if (i >= pc.n) return;
+  if (i >= pc.n || pc.gate.closed()) return;
   const int ti = MULTI ? pc.type[i] : 0;
   const bool oni = !MULTI || eam_on(t, ti);
   double rho = 0.0;
@@ -172,7 +173,7 @@ __global__ void __launch_bounds__(256) k_eam_force(PairCommon pc, EamTabDev<Real
                                                    Outputs o)
 {
   const int64_t i = logical_block() * blockDim.x + threadIdx.x;
-  if (i >= pc.n) return;
+  if (i >= pc.n || pc.gate.closed()) return;
   const int ti = MULTI ? pc.type[i] : 0;
   const double* L = pc.box[pc.rep ? pc.rep[i] : 0].L;
   const Pos4 pi = load_pos(pc.pos, i);
@@ -278,9 +279,10 @@ __global__ void __launch_bounds__(256) k_johnson_force(PairCommon pc, JohnsonPar
   write_outputs<true, VIRIAL, false>(o, i, fx, fy, fz, e, v);
 }
 
-PairCommon make_common(Ctx& c, double rcut)
+PairCommon make_common(Ctx& c, double rcut, const StepGate& gate = {})
 {
   PairCommon pc;
+  pc.gate = gate;
   pc.n = c.n;
   pc.npad = c.npad;
   pc.pos = c.pos.p;
@@ -306,7 +308,7 @@ void eam_dispatch(Ctx& c, double rcut, bool do_rho, bool do_emb, bool do_force, 
 {
   const EamTabDev<Real> t = make_eam_tab<Real>(c);
   const Real* pair = eam_pair_table<Real>(c);
-  const PairCommon pc = make_common(c, rcut);
+  const PairCommon pc = make_common(c, rcut, step_gate(c, epi));
   const unsigned g = pair_grid(c.n);
   const bool energy = flags & XS_ENERGY;
   double* pos_w = reinterpret_cast<double*>(c.pos.p);
@@ -354,8 +356,9 @@ void lj_dispatch(Ctx& c, double eps, double sigma, double rcut, unsigned flags, 
 {
   const double ecut = lj_energy_cutoff(eps, sigma, rcut);
   LJParams<Real> lp{(Real)(sigma * sigma), (Real)(4.0 * eps), (Real)(24.0 * eps), (Real)ecut};
-  const PairCommon pc = make_common(c, rcut);
-  const Outputs o = make_outputs(c, epi);
+  const PairCommon pc = make_common(c, rcut, step_gate(c, epi));
+  Outputs o = make_outputs(c, epi);
+  o.set_ep = epi.fused;
   const unsigned g = pair_grid(c.n);
   const bool energy = flags & XS_ENERGY, vir = flags & XS_VIRIAL;
   ProfScope prof(c.prof, c.stream, XS_PROF_LJ);
@@ -482,6 +485,7 @@ Outputs make_outputs(Ctx& c, const ForceEpilogue& ep)
   o.vz = c.vz.p;
   o.kick_dt = ep.kick_dt;
   o.npad = c.npad;
+  o.set_ep = false;
   return o;
 }
 

@@ -62,6 +62,7 @@ struct Outputs {
   double* vz;
   double kick_dt;
   int64_t npad;
+  bool set_ep;  // ep is written, not added to
 };
 
 // Per-atom epilogue: add the force (operator form) or write a = f/m and kick v
@@ -84,7 +85,7 @@ __device__ __forceinline__ void write_outputs(const Outputs& o, int64_t i, doubl
     o.ay[i] += fy;
     o.az[i] += fz;
   }
-  if constexpr (ENERGY) o.ep[i] += e;
+  if constexpr (ENERGY) o.ep[i] = o.set_ep ? e : o.ep[i] + e;
   if constexpr (VIRIAL) {
 #pragma unroll
     for (int q = 0; q < 9; q++) {
@@ -96,8 +97,8 @@ __device__ __forceinline__ void write_outputs(const Outputs& o, int64_t i, doubl
 
 // Next-step drift fused into the MD-loop epilogue: the arithmetic of k_drift_kick
 // applied to the velocity this step's kick produced.  The loop only needs to know
-// whether some atom moved more than the rebuild threshold, so an atom past it
-// stores 1 to *over (every writer stores the same value).
+// whether some atom moved more than the rebuild threshold, so an atom past it raises
+// the loop's flag (see StepGate).
 struct Drift {
   Pos4* pos_out;
   const double* rrx;
@@ -105,7 +106,7 @@ struct Drift {
   const double* rrz;
   double dt, dt2, hdt;
   double thr2;
-  unsigned long long* over;
+  StepFlag over;
 };
 
 // Fused epilogue with drift: a = f/m, v += a*kick_dt (this step), then
@@ -131,7 +132,7 @@ __device__ __forceinline__ void write_outputs_drift(const Outputs& o, const Drif
   o.vx[i] = fma(a0, d.hdt, v0);
   o.vy[i] = fma(a1, d.hdt, v1);
   o.vz[i] = fma(a2, d.hdt, v2);
-  if (xsmd_d2(q.x - d.rrx[i], q.y - d.rry[i], q.z - d.rrz[i]) > d.thr2) *d.over = 1ull;
+  if (xsmd_d2(q.x - d.rrx[i], q.y - d.rry[i], q.z - d.rrz[i]) > d.thr2) d.over.raise();
 }
 
 // onika tensor(fe, dr) * -0.5 added to v (row-major m11 m12 ... m33)

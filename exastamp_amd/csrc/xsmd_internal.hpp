@@ -121,6 +121,34 @@ __device__ __forceinline__ void swap_halves(double& a, double& b)
   b = __longlong_as_double((long long)(((unsigned long long)y1 << 32) | y0));
 }
 
+// The MD loop queues steps before it knows whether an earlier one moved an atom far
+// enough to need a new list.  A kernel that moves atoms to their positions of step s
+// raises the loop's flag with value s when some atom passed the threshold; kernels that
+// need the list at step t, or move atoms on from it, do nothing once the flag holds a
+// step <= t (StepGate), so the state waits there for the rebuild.  The host reads its own
+// copy of the flag, in pinned memory, when it waits for the queued work.
+struct StepFlag {
+  unsigned long long* dev = nullptr;
+  unsigned long long* host = nullptr;
+  unsigned long long step = 0;
+  // every writer of a launch stores the same value
+  __device__ __forceinline__ void raise() const
+  {
+    *dev = step;
+    __hip_atomic_store(host, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
+struct StepGate {
+  const unsigned long long* flag = nullptr;  // NULL: always open
+  unsigned long long step = 0;
+  __device__ __forceinline__ bool closed() const
+  {
+    if (!flag) return false;
+    const unsigned long long f = *flag;
+    return f != 0 && f <= step;
+  }
+};
+
 // Box of one replica, as kernels read it: lo[3], L[3], n/L[3].
 struct BoxDev {
   double lo[3];
@@ -371,10 +399,13 @@ struct Ctx {
   bool list_sort_disabled = false;  // XSMD_LIST_SORT=0: block lists stay in stencil order
   bool s_table_disabled = false;    // XSMD_EAM_S_TABLE=0: the FP32 passes read the knot rows
   bool drift_done = false;  // the last force launch applied ForceEpilogue::drift
+  unsigned long long* hflag = nullptr;  // pinned host copy of the loop's flag dscalar[5] (StepFlag)
+  hipEvent_t step_event[2] = {nullptr, nullptr};  // ends of the MD loop's queued steps
+  DBuf<double> thermo_log;              // the loop's thermodynamic samples
 
   // small device scalars + pinned host mirror
   DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..4] halo maxima,
-                                     // [5] fused-drift rebuild flag
+                                     // [5] the MD loop's rebuild flag (StepFlag)
   unsigned long long* hscalar = nullptr;
   DBuf<double> red_part;  // thermo partial sums
   DBuf<double> red_out;
@@ -437,8 +468,11 @@ void launch_force_to_accel(Ctx& c);
 // inverse); false: IDENTITY
 void launch_push_f_v_r(Ctx& c, double dt, bool inv_xform);
 void launch_push_f_v(Ctx& c, double dt);
-// fused first half of a step: r += v dt + a dt^2/2 ; v += a dt/2 ; max |r - r_ref|^2
-void launch_drift_kick(Ctx& c, double dt);
+// fused first half of step `step`: r += v dt + a dt^2/2 ; v += a dt/2 ; the loop's flag
+// raised if some |r - r_ref|^2 > thr2; gated: nothing if the flag holds an earlier step
+void launch_drift_kick(Ctx& c, double dt, double thr2, unsigned long long step, bool gated);
+// the 27 values of xs_thermo at out27_dev (device memory) on the context's partial-sum buffer
+void launch_thermo_dev(Ctx& c, double* out27_dev, const StepGate& gate);
 void launch_thermo(Ctx& c, double out[27]);
 // once per device, with that device current: address of the fixed partial-sum array
 // of launch_thermo_noalloc on that device
@@ -453,14 +487,20 @@ struct ForceEpilogue {
   bool fused = false;   // overwrite a with f/m and kick v by a*kick_dt (MD loop)
   double kick_dt = 0;
   // MD loop, fused form only: also apply the next step's push_f_v_r(drift_dt) and
-  // push_f_v(drift_dt/2), writing the new positions to pos2 (then made current),
-  // and set dscalar[5] to 1 if some atom moved more than sqrt(drift_thr2) since the
-  // last build.  A launcher that can do this sets Ctx::drift_done; otherwise the
-  // loop runs k_drift_kick itself.
+  // push_f_v(drift_dt/2), writing the new positions to pos2 (then made current), and
+  // raise the loop's flag (value step + 1) if some atom moved more than
+  // sqrt(drift_thr2) since the last build.  A launcher that can do this sets
+  // Ctx::drift_done; otherwise the loop runs k_drift_kick itself.
   bool drift = false;
   double drift_dt = 0;
   double drift_thr2 = 0;
+  unsigned long long step = 0;  // MD loop: the step these forces belong to
+  bool gated = false;           // its kernels check the loop's flag (StepGate)
 };
+inline StepGate step_gate(const Ctx& c, const ForceEpilogue& e)
+{
+  return e.gated ? StepGate{c.dscalar.p + 5, e.step} : StepGate{};
+}
 // energy_cutoff (pair_potential_impl.hxx:487-498): E_LJ(rcut) in FP64, 0 for rcut <= 0
 inline double lj_energy_cutoff(double eps, double sigma, double rcut)
 {
