@@ -219,6 +219,7 @@ struct BlockArgs {
   int cap;   // halo slots (LDS records)
   int ccap;  // central atoms per brick at most
   double rc2;
+  int split;           // SPLIT passes: log2 of the parts an atom's list is walked in
   const XformDev* xf;  // the staging maps positions to physical space when not NULL
   StepGate gate;       // MD loop
 };
@@ -290,9 +291,35 @@ __device__ __forceinline__ double half_sum(double v)
   return a + b;
 }
 
-// this lane's atom slot and which half of the wave it is in
-__device__ __forceinline__ int pass_slot() { return (threadIdx.x >> 6) * 32 + (threadIdx.x & 31); }
-__device__ __forceinline__ int pass_half() { return (threadIdx.x >> 5) & 1; }
+// The lanes of a pass.  Two lanes take an atom, the even and the odd entries of its
+// list.  SPLIT (bricks of at most 128 atoms, which small systems are cut into): 2 parts
+// lanes, each taking every parts-th group of 8 entries, so that a workgroup's 512 lanes
+// are busy whatever its atom count.  4000 argon atoms: 27 bricks of 148 atoms, 9.2 us a
+// pass -> 125 bricks of 32 atoms, 16 lanes each, 7.0 us.
+template <bool SPLIT>
+struct PassLanes {
+  int half, slot, part, log;
+  __device__ __forceinline__ explicit PassLanes(const BlockArgs& a)
+  {
+    const int l = threadIdx.x & 31, w = threadIdx.x >> 6;
+    half = (threadIdx.x >> 5) & 1;
+    log = SPLIT ? a.split : 0;
+    slot = (w << (5 - log)) + (SPLIT ? l & ((32 >> log) - 1) : l);
+    part = SPLIT ? l >> (5 - log) : 0;
+  }
+  __device__ __forceinline__ int atoms() const { return kPassAtoms >> log; }
+  __device__ __forceinline__ int first() const { return half + 8 * part; }  // first entry
+  __device__ __forceinline__ int step() const { return 8 << log; }          // to the next group
+  __device__ __forceinline__ bool writes() const { return half == 0 && part == 0; }
+  // sum over the atom's lanes
+  __device__ __forceinline__ double sum(double v) const
+  {
+    v = half_sum(v);
+    if constexpr (SPLIT)
+      for (int off = 16; off >= (32 >> log); off >>= 1) v += __shfl_xor(v, off);
+    return v;
+  }
+};
 
 // ---------------------------------------------------------------------------
 // list build
@@ -555,6 +582,8 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
   uint16_t* cand = cand_all + (size_t)wave * a.cand_cap;
   const int stride = a.nmax + 1;  // odd, so the group loads of 8 rows start in distinct banks
   uint32_t* rows = rows_all + (size_t)wave * a.atoms * stride;
+  // bricks of fewer cells than waves: several waves share a cell's atoms
+  const int parts = ncell >= kBuildWaves ? 1 : kBuildWaves / ncell;
   int nrow = 0;         // lists in the rows
   int cnt = 0, gi = 0;  // lane k: entries and atom of row k
   // the collected lists out: counts, then whole groups, 8 lanes per atom and one group
@@ -598,13 +627,16 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
     int cc = 0;
     if (lane == 0) cc = atomicAdd(total_p + 1, 1);
     cc = __builtin_amdgcn_readfirstlane(cc);
-    if (cc >= ncell) break;
+    if (cc >= ncell * parts) break;
+    const int part = cc % parts;
+    cc /= parts;
     const int h = central_cell(cc);
-    const int nat = __builtin_amdgcn_readfirstlane(hc[h].count);
-    const int l0 = __builtin_amdgcn_readfirstlane(hc[h].lstart);
-    const int g0 = __builtin_amdgcn_readfirstlane(hc[h].gstart);
+    const int all = __builtin_amdgcn_readfirstlane(hc[h].count);
+    const int skip = all * part / parts, nat = all * (part + 1) / parts - skip;
     if (nat == 0) continue;
-    const int64_t q0 = b * a.ccap + cell_q[cc];
+    const int l0 = __builtin_amdgcn_readfirstlane(hc[h].lstart) + skip;
+    const int g0 = __builtin_amdgcn_readfirstlane(hc[h].gstart) + skip;
+    const int64_t q0 = b * a.ccap + cell_q[cc] + skip;
     for (int k = lane; k < nat; k += 64) {
       a.cen[q0 + k] = (uint32_t)(g0 + k);
       a.cen_slot[q0 + k] = (uint16_t)(l0 + k);
@@ -840,16 +872,31 @@ struct LNb {
 // into the array.  Every lane of a wave is at the same q in a given iteration, so
 // the group's start is one scalar address and each lane adds its own fixed 32-bit
 // offset (the list holds at most 2^26 atoms x 64 entries = 2^30 words).
+template <bool SPLIT>
 struct LWords {
   const uint2* base;
   uint32_t lane;  // this lane's word within a group
-  int64_t step;   // words per group
-  __device__ __forceinline__ uint2 get(int q) const { return (base + q * step)[lane]; }
+  int64_t step;   // words to the lane's next group
+  int q = 0;
+  __device__ __forceinline__ LWords(const BlockArgs& a, int64_t gi, const PassLanes<SPLIT>& ln)
+      : base(reinterpret_cast<const uint2*>(a.nbr16)), lane((uint32_t)(2 * gi + ln.half)), step(2 * a.npad)
+  {
+    if constexpr (SPLIT) {
+      base += ln.part * step;
+      step <<= ln.log;
+    }
+  }
+  // the first word (SPLIT: only where the list reaches the part's first group, which may
+  // lie beyond the list's capacity)
+  __device__ __forceinline__ uint2 first(const PassLanes<SPLIT>& ln, int cnt) const
+  {
+    if constexpr (SPLIT) {
+      if (ln.first() >= cnt) return make_uint2(0u, 0u);
+    }
+    return base[lane];
+  }
+  __device__ __forceinline__ uint2 next() { return (base + ++q * step)[lane]; }
 };
-__device__ __forceinline__ LWords lwords(const BlockArgs& a, int64_t gi, int half)
-{
-  return {reinterpret_cast<const uint2*>(a.nbr16), (uint32_t)(2 * gi + half), 2 * a.npad};
-}
 __device__ __forceinline__ void lslots(uint2 w, int far_slot, int k0, int cnt, int (&c)[4])
 {
   const int raw[4] = {(int)(w.x & 0xffffu), (int)(w.x >> 16), (int)(w.y & 0xffffu), (int)(w.y >> 16)};
@@ -879,8 +926,8 @@ __device__ __forceinline__ void lgather(const BlockArgs& a, const LRec& rec, con
 }
 
 // rho_i, then (EMB) F(rho_i) and F'(rho_i) for the central atoms of one brick
-template <class Real, bool MULTI, bool EMB, bool ENERGY, bool SET_EP>
-__global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_rho(BlockArgs a, EamTabDev<Real> t,
+template <class Real, bool MULTI, bool EMB, bool ENERGY, bool SET_EP, bool SPLIT>
+__global__ void __launch_bounds__(kPassThreads, kPassWaves<SPLIT>) k_block_eam_rho(BlockArgs a, EamTabDev<Real> t,
                                                                 const Real* __restrict__ pair,
                                                                 double* __restrict__ rho_io,
                                                                 double* __restrict__ pos_w, double* __restrict__ ep)
@@ -891,8 +938,8 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
   const LRec rec = pass_lds(a, MULTI, false, ltype);
   const int4 hd = a.head[b];
   stage<false>(a, b, hd, rec, ltype);
-  const int half = pass_half();
-  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+  const PassLanes<SPLIT> ln(a);
+  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
     const int64_t gi = a.cen[b * a.ccap + q];
     const int slot = a.cen_slot[b * a.ccap + q];
     const Pos4 pi = rec.get(slot);
@@ -900,11 +947,11 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
     const bool oni = !MULTI || pm::eam_on(t, ti);
     const int cnt = oni ? a.nnb[gi] : 0;
     double rho = 0.0;
-    LWords lw = lwords(a, gi, half);
-    uint2 wnext = lw.get(0);
-    for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
+    LWords<SPLIT> lw(a, gi, ln);
+    uint2 wnext = lw.first(ln, cnt);
+    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
-      if (k0 + 8 < cnt) wnext = lw.get(q + 1);
+      if (k0 + ln.step() < cnt) wnext = lw.next();
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
       LNb nb[kBBatch];
@@ -928,8 +975,8 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
         rho += (double)(nb[u].in ? val : Real(0));
       }
     }
-    rho = half_sum(rho);
-    if (half == 0) {
+    rho = ln.sum(rho);
+    if (ln.writes()) {
       rho_io[gi] = rho;
       if constexpr (EMB) {
         Real F, Fp;
@@ -945,8 +992,8 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_eam_r
   }
 }
 
-template <class Real, bool MULTI, bool ENERGY, bool VIRIAL, bool FUSED, bool DRIFT>
-__global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_force(BlockArgs a, EamTabDev<Real> t,
+template <class Real, bool MULTI, bool ENERGY, bool VIRIAL, bool FUSED, bool DRIFT, bool SPLIT>
+__global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_block_eam_force(BlockArgs a, EamTabDev<Real> t,
                                                                   const Real* __restrict__ pair, pm::Outputs o,
                                                                   pm::Drift dr)
 {
@@ -957,8 +1004,8 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_
   const LRec rec = pass_lds(a, MULTI, true, ltype);
   const int4 hd = a.head[b];
   stage<true>(a, b, hd, rec, ltype);
-  const int half = pass_half();
-  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+  const PassLanes<SPLIT> ln(a);
+  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
     const int64_t gi = a.cen[b * a.ccap + q];
     const int slot = a.cen_slot[b * a.ccap + q];
     const Pos4 pi = rec.get(slot);
@@ -967,11 +1014,11 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_
     const int cnt = (!MULTI || pm::eam_on(t, ti)) ? a.nnb[gi] : 0;
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    LWords lw = lwords(a, gi, half);
-    uint2 wnext = lw.get(0);
-    for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
+    LWords<SPLIT> lw(a, gi, ln);
+    uint2 wnext = lw.first(ln, cnt);
+    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
-      if (k0 + 8 < cnt) wnext = lw.get(q + 1);
+      if (k0 + ln.step() < cnt) wnext = lw.next();
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
       // two entries at a time: their four table rows stay in flight together within
@@ -1024,15 +1071,15 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_eam_
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    fx = half_sum(fx);
-    fy = half_sum(fy);
-    fz = half_sum(fz);
-    if constexpr (ENERGY) e = half_sum(e);
+    fx = ln.sum(fx);
+    fy = ln.sum(fy);
+    fz = ln.sum(fz);
+    if constexpr (ENERGY) e = ln.sum(e);
     if constexpr (VIRIAL) {
 #pragma unroll
-      for (int k = 0; k < 9; k++) v[k] = half_sum(v[k]);
+      for (int k = 0; k < 9; k++) v[k] = ln.sum(v[k]);
     }
-    if (half == 0) {
+    if (ln.writes()) {
       if constexpr (DRIFT) pm::write_outputs_drift(o, dr, gi, pi, fx, fy, fz);
       else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, gi, fx, fy, fz, e, v);
     }
@@ -1061,22 +1108,22 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
   const LRec rec = pass_lds(a, false, FORCE, ltype);
   const int4 hd = a.head[b];
   stage<FORCE>(a, b, hd, rec, ltype);
-  const int half = pass_half();
-  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+  const PassLanes<false> ln(a);
+  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
     const int64_t gi = a.cen[b * a.ccap + q];
     const int slot = a.cen_slot[b * a.ccap + q];
     const Pos4 pi = rec.get(slot);
     const int cnt = a.nnb[gi];
     float acc = 0.0f;
     if constexpr (LEVEL == 3) {
-      if (half == 0) sink[gi] = pi.x + cnt;
+      if (ln.writes()) sink[gi] = pi.x + cnt;
       continue;
     }
-    LWords lw = lwords(a, gi, half);
-    uint2 wnext = lw.get(0);
-    for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
+    LWords<false> lw(a, gi, ln);
+    uint2 wnext = lw.first(ln, cnt);
+    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
-      if (k0 + 8 < cnt) wnext = lw.get(q + 1);
+      if (k0 + ln.step() < cnt) wnext = lw.next();
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
       if constexpr (LEVEL == 2) {
@@ -1120,8 +1167,8 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
         }
       }
     }
-    const double sum = half_sum((double)acc);
-    if (half == 0) sink[gi] = sum;
+    const double sum = ln.sum((double)acc);
+    if (ln.writes()) sink[gi] = sum;
   }
 }
 
@@ -1130,8 +1177,8 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
 // pair math of the global-list kernel (pm::lj_pair).
 // MULTI (lj_multi_force): types staged with the records; each pair takes the
 // parameters and cutoff of its two species.
-template <class Real, bool ENERGY, bool VIRIAL, bool FUSED, bool DRIFT, bool MULTI = false>
-__global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(BlockArgs a, pm::LJ<Real> lp,
+template <class Real, bool ENERGY, bool VIRIAL, bool FUSED, bool DRIFT, bool SPLIT, bool MULTI = false>
+__global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_block_lj(BlockArgs a, pm::LJ<Real> lp,
                                                                            pm::Outputs o, pm::Drift dr,
                                                                            pm::LJMultiDev lm = {})
 {
@@ -1153,8 +1200,8 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
     }
   }
   stage<false>(a, b, hd, rec, ltype);
-  const int half = pass_half();
-  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+  const PassLanes<SPLIT> ln(a);
+  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
     const int64_t gi = a.cen[b * a.ccap + q];
     const int slot = a.cen_slot[b * a.ccap + q];
     const Pos4 pi = rec.get(slot);
@@ -1162,11 +1209,11 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
     const int cnt = a.nnb[gi];
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    LWords lw = lwords(a, gi, half);
-    uint2 wnext = lw.get(0);
-    for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
+    LWords<SPLIT> lw(a, gi, ln);
+    uint2 wnext = lw.first(ln, cnt);
+    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
-      if (k0 + 8 < cnt) wnext = lw.get(q + 1);
+      if (k0 + ln.step() < cnt) wnext = lw.next();
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
       LNb nb[kBBatch];
@@ -1188,15 +1235,15 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
           pm::add_virial(v, nb[u].x * de_r, nb[u].y * de_r, nb[u].z * de_r, nb[u].x, nb[u].y, nb[u].z);
       }
     }
-    fx = half_sum(fx);
-    fy = half_sum(fy);
-    fz = half_sum(fz);
-    if constexpr (ENERGY) e = half_sum(e);
+    fx = ln.sum(fx);
+    fy = ln.sum(fy);
+    fz = ln.sum(fz);
+    if constexpr (ENERGY) e = ln.sum(e);
     if constexpr (VIRIAL) {
 #pragma unroll
-      for (int k = 0; k < 9; k++) v[k] = half_sum(v[k]);
+      for (int k = 0; k < 9; k++) v[k] = ln.sum(v[k]);
     }
-    if (half == 0) {
+    if (ln.writes()) {
       if constexpr (DRIFT) pm::write_outputs_drift(o, dr, gi, pi, fx, fy, fz);
       else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, gi, fx, fy, fz, e, v);
     }
@@ -1209,6 +1256,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL>) k_block_lj(B
 // square root each).  128 k Ta atoms (83 entries, 53 in rc), both passes with energy and
 // virial: 134 us, against 338 us, and 115 us to convert the list, on the global list with
 // the general power function and every term evaluated for itself.
+template <bool SPLIT>
 __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs a, JohnsonParams jp,
                                                                        double* __restrict__ rho_out,
                                                                        double* __restrict__ pos_w,
@@ -1220,18 +1268,18 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs
   const LRec rec = pass_lds(a, false, false, ltype);
   const int4 hd = a.head[b];
   stage<false>(a, b, hd, rec, ltype);
-  const int half = pass_half();
-  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+  const PassLanes<SPLIT> ln(a);
+  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
     const int64_t gi = a.cen[b * a.ccap + q];
     const int slot = a.cen_slot[b * a.ccap + q];
     const Pos4 pi = rec.get(slot);
     const int cnt = a.nnb[gi];
     double rho = 0.0;
-    LWords lw = lwords(a, gi, half);
-    uint2 wnext = lw.get(0);
-    for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
+    LWords<SPLIT> lw(a, gi, ln);
+    uint2 wnext = lw.first(ln, cnt);
+    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
-      if (k0 + 8 < cnt) wnext = lw.get(q + 1);
+      if (k0 + ln.step() < cnt) wnext = lw.next();
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
 #pragma unroll
@@ -1243,8 +1291,8 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs
         rho += nb[0].in ? v : 0.0;
       }
     }
-    rho = half_sum(rho);
-    if (half == 0) {
+    rho = ln.sum(rho);
+    if (ln.writes()) {
       rho_out[gi] = rho;
       double F, Fp;
       pm::johnson_embed(jp, rho, F, Fp);
@@ -1256,7 +1304,7 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs
 
 // Pass 2 (ForceOp): f_i += (rho'(r) (F'_i + F'_j) + phi'(r)) / r (r_j - r_i), ep += phi / 2,
 // virial -1/2 f (x) dr.
-template <bool VIRIAL>
+template <bool VIRIAL, bool SPLIT>
 __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_force(BlockArgs a, JohnsonParams jp, pm::Outputs o)
 {
   const int64_t b = lblock();
@@ -1265,19 +1313,19 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_force(BlockAr
   const LRec rec = pass_lds(a, false, true, ltype);
   const int4 hd = a.head[b];
   stage<true>(a, b, hd, rec, ltype);
-  const int half = pass_half();
-  for (int q = pass_slot(); q < hd.y; q += kPassAtoms) {
+  const PassLanes<SPLIT> ln(a);
+  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
     const int64_t gi = a.cen[b * a.ccap + q];
     const int slot = a.cen_slot[b * a.ccap + q];
     const Pos4 pi = rec.get(slot);
     const int cnt = a.nnb[gi];
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    LWords lw = lwords(a, gi, half);
-    uint2 wnext = lw.get(0);
-    for (int k0 = half, q = 0; k0 < cnt; k0 += 2 * kBBatch, q++) {
+    LWords<SPLIT> lw(a, gi, ln);
+    uint2 wnext = lw.first(ln, cnt);
+    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
-      if (k0 + 8 < cnt) wnext = lw.get(q + 1);
+      if (k0 + ln.step() < cnt) wnext = lw.next();
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
 #pragma unroll
@@ -1296,15 +1344,15 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_force(BlockAr
         if constexpr (VIRIAL) pm::add_virial(v, fe0, fe1, fe2, nb[0].x, nb[0].y, nb[0].z);
       }
     }
-    fx = half_sum(fx);
-    fy = half_sum(fy);
-    fz = half_sum(fz);
-    e = half_sum(e);
+    fx = ln.sum(fx);
+    fy = ln.sum(fy);
+    fz = ln.sum(fz);
+    e = ln.sum(e);
     if constexpr (VIRIAL) {
 #pragma unroll
-      for (int k = 0; k < 9; k++) v[k] = half_sum(v[k]);
+      for (int k = 0; k < 9; k++) v[k] = ln.sum(v[k]);
     }
-    if (half == 0) pm::write_outputs<true, VIRIAL, false>(o, gi, fx, fy, fz, e, v);
+    if (ln.writes()) pm::write_outputs<true, VIRIAL, false>(o, gi, fx, fy, fz, e, v);
   }
 }
 
@@ -1327,6 +1375,8 @@ BlockArgs block_args(const Ctx& c, double rcut, const StepGate& gate = {})
   a.ccap = c.bcentral;
   a.rc2 = rcut * rcut;
   a.xf = c.xf_dev();
+  a.split = 0;
+  while (a.split < 3 && (c.bcentral << (a.split + 1)) <= kPassAtoms) a.split++;
   return a;
 }
 
@@ -1374,7 +1424,8 @@ void block_eam_dispatch(Ctx& c, double rcut, bool do_rho, bool do_emb, bool do_f
   if (do_rho) {
     ProfScope prof(c.prof, c.stream, XS_PROF_EAM_RHO);
 #define XS_BRHO(EMB, EN, SET) \
-  k_block_eam_rho<Real, MULTI, EMB, EN, SET><<<g, kPassThreads, lds_rho, c.stream>>>(a, t, pair, c.rho.p, pos_w, c.ep.p)
+  (a.split ? k_block_eam_rho<Real, MULTI, EMB, EN, SET, true> : k_block_eam_rho<Real, MULTI, EMB, EN, SET, false>) \
+      <<<g, kPassThreads, lds_rho, c.stream>>>(a, t, pair, c.rho.p, pos_w, c.ep.p)
     if (!do_emb) XS_BRHO(false, false, false);
     else if (energy && epi.fused) XS_BRHO(true, true, true);
     else if (energy) XS_BRHO(true, true, false);
@@ -1389,7 +1440,8 @@ void block_eam_dispatch(Ctx& c, double rcut, bool do_rho, bool do_emb, bool do_f
     const bool drift = drift_setup(c, epi, flags, dr);
     ProfScope prof(c.prof, c.stream, XS_PROF_EAM_FORCE);
 #define XS_BF(EN, VI, FU, DR) \
-  k_block_eam_force<Real, MULTI, EN, VI, FU, DR><<<g, kPassThreads, lds, c.stream>>>(a, t, pair, o, dr)
+  (a.split ? k_block_eam_force<Real, MULTI, EN, VI, FU, DR, true>                                       \
+           : k_block_eam_force<Real, MULTI, EN, VI, FU, DR, false>)<<<g, kPassThreads, lds, c.stream>>>(a, t, pair, o, dr)
     if (drift) {
       XS_BF(false, false, true, true);
     } else if (epi.fused) {
@@ -1502,7 +1554,10 @@ void block_setup(Ctx& c)
   // of the grid (slabs, clusters) the measured halo can exceed the LDS budget, and
   // the bound shrinks until it fits (or the bricks are single cells).
   double per_cell = std::max((double)c.n / (double)c.ncell_tot, 1e-3);
+  // Systems that 230-atom bricks would not spread over the CUs three workgroups deep are
+  // cut into smaller ones, whose passes walk each list with more lanes (PassLanes).
   double bound = c.block_atoms;
+  if (!c.block_atoms_set) bound = std::min(bound, std::max(8.0, (double)c.n / (3.0 * std::max(c.num_cu, 1))));
   for (int attempt = 0;; attempt++) {
     block_shape_choose(c, g, bound, per_cell);
     XS_HIP(hipMemsetAsync(c.dscalar.p + 2, 0, 3 * sizeof(unsigned long long), c.stream));
@@ -1656,7 +1711,9 @@ void launch_lj_block(Ctx& c, double eps, double sigma, double rcut, unsigned fla
   auto run = [&](auto zero) {
     using Real = decltype(zero);
     const pm::LJ<Real> lp{(Real)(sigma * sigma), (Real)(4.0 * eps), (Real)(24.0 * eps), (Real)ecut};
-#define XS_BL(EN, VI, FU, DR) k_block_lj<Real, EN, VI, FU, DR><<<g, kPassThreads, lds, c.stream>>>(a, lp, o, dr)
+#define XS_BL(EN, VI, FU, DR)                                                                                \
+  (a.split ? k_block_lj<Real, EN, VI, FU, DR, true> : k_block_lj<Real, EN, VI, FU, DR, false>)               \
+      <<<g, kPassThreads, lds, c.stream>>>(a, lp, o, dr, pm::LJMultiDev{})
     if (drift) {
       XS_BL(false, false, true, true);
     } else if (epi.fused) {
@@ -1692,7 +1749,8 @@ void launch_lj_multi_block(Ctx& c, unsigned flags)
     const pm::LJ<Real> none{};
     const pm::LJMultiDev lm = ljm_dev<Real>(c);
 #define XS_BLM(EN, VI) \
-  k_block_lj<Real, EN, VI, false, false, true><<<g, kPassThreads, lds, c.stream>>>(a, none, o, dr, lm)
+  (a.split ? k_block_lj<Real, EN, VI, false, false, true, true>                                              \
+           : k_block_lj<Real, EN, VI, false, false, false, true>)<<<g, kPassThreads, lds, c.stream>>>(a, none, o, dr, lm)
     if (energy && vir) XS_BLM(true, true);
     else if (energy) XS_BLM(true, false);
     else if (vir) XS_BLM(false, true);
@@ -1710,16 +1768,18 @@ void launch_johnson_block(Ctx& c, const JohnsonParams& p, double rcut, bool do_e
   const unsigned g = block_grid(c);
   if (do_emb) {
     ProfScope prof(c.prof, c.stream, XS_PROF_EAM_RHO);
-    k_block_johnson_rho<<<g, kPassThreads, block_lds_bytes(c, false, false), c.stream>>>(
-        a, p, c.rho.p, reinterpret_cast<double*>(c.pos.p), c.ep.p);
+    (a.split ? k_block_johnson_rho<true> : k_block_johnson_rho<false>)
+        <<<g, kPassThreads, block_lds_bytes(c, false, false), c.stream>>>(a, p, c.rho.p, reinterpret_cast<double*>(c.pos.p), c.ep.p);
     XS_HIP(hipGetLastError());
   }
   if (!do_force) return;
   const pm::Outputs o = make_outputs(c, ForceEpilogue{});
   ProfScope prof(c.prof, c.stream, XS_PROF_EAM_FORCE);
   const size_t lds = block_lds_bytes(c, false, true);
-  if (flags & XS_VIRIAL) k_block_johnson_force<true><<<g, kPassThreads, lds, c.stream>>>(a, p, o);
-  else k_block_johnson_force<false><<<g, kPassThreads, lds, c.stream>>>(a, p, o);
+  const bool vir = flags & XS_VIRIAL;
+  const auto k = a.split ? (vir ? k_block_johnson_force<true, true> : k_block_johnson_force<false, true>)
+                         : (vir ? k_block_johnson_force<true, false> : k_block_johnson_force<false, false>);
+  k<<<g, kPassThreads, lds, c.stream>>>(a, p, o);
   XS_HIP(hipGetLastError());
 }
 
