@@ -219,6 +219,7 @@ struct BlockArgs {
   int cap;   // halo slots (LDS records)
   int ccap;  // central atoms per brick at most
   double rc2;
+  int nmax;            // list capacity
   int split;           // SPLIT passes: log2 of the parts an atom's list is walked in
   const XformDev* xf;  // the staging maps positions to physical space when not NULL
   StepGate gate;       // MD loop
@@ -242,7 +243,7 @@ __device__ __forceinline__ LRec pass_lds(const BlockArgs& a, bool with_type, boo
 // an atom's count point there (lslots), so their displacement is finite and longer than
 // any cutoff, and the passes mask them by d2 <= rc2 alone.  It lies at least 10^4 A from
 // every staged position (which are within the box and its images) and close enough that
-// its knot index fits an int.  Ends with __syncthreads().
+// its knot index fits an int.  The caller's __syncthreads() follows.
 template <bool WITH_W>
 __device__ __forceinline__ void stage(const BlockArgs& a, int64_t b, const int4& hd, const LRec& rec, uint8_t* ltype)
 {
@@ -260,8 +261,11 @@ __device__ __forceinline__ void stage(const BlockArgs& a, int64_t b, const int4&
     if (ltype) ltype[a.cap] = 0;
   }
   const uint32_t* st = a.stage + b * a.cap;
-  for (int c = threadIdx.x; c < hd.x; c += kPassThreads) {
-    const uint32_t e = st[c];
+  int c = threadIdx.x;
+  uint32_t ahead = c < hd.x ? st[c] : 0u;  // the next entry is on its way while a record is staged
+  while (c < hd.x) {
+    const uint32_t e = ahead;
+    if (c + kPassThreads < hd.x) ahead = st[c + kPassThreads];
     const uint32_t j = xsmd_nbr_index(e);
     Pos4 p;
     if constexpr (WITH_W) {
@@ -279,8 +283,8 @@ __device__ __forceinline__ void stage(const BlockArgs& a, int64_t b, const int4&
     if (a.xf) xsmd_xform_apply(a.xf->m, &p.x, &p.y, &p.z);
     rec.put(c, p);
     if (ltype) ltype[c] = a.type[j];
+    c += kPassThreads;
   }
-  __syncthreads();
 }
 
 // sum of v over the two halves of the wave (lanes l and l ^ 32)
@@ -886,16 +890,35 @@ struct LWords {
       step <<= ln.log;
     }
   }
-  // the first word (SPLIT: only where the list reaches the part's first group, which may
-  // lie beyond the list's capacity)
-  __device__ __forceinline__ uint2 first(const PassLanes<SPLIT>& ln, int cnt) const
-  {
-    if constexpr (SPLIT) {
-      if (ln.first() >= cnt) return make_uint2(0u, 0u);
-    }
-    return base[lane];
-  }
+  __device__ __forceinline__ uint2 first() const { return base[lane]; }
   __device__ __forceinline__ uint2 next() { return (base + ++q * step)[lane]; }
+};
+// A central atom on its way: its index and slot, then the length of its list and the
+// lane's first list word.  The first atom of each lane is fetched while the halo is
+// staged, so that the passes do not wait for these loads one after the other behind the
+// barrier.
+template <bool SPLIT>
+struct PassAtom {
+  int64_t gi = 0;
+  int slot = 0, cnt = 0;
+  uint2 w = {0u, 0u};
+  __device__ __forceinline__ void index(const BlockArgs& a, int64_t b, int q)
+  {
+    gi = a.cen[b * a.ccap + q];
+    slot = a.cen_slot[b * a.ccap + q];
+  }
+  __device__ __forceinline__ void list(const BlockArgs& a, const PassLanes<SPLIT>& ln)
+  {
+    cnt = a.nnb[gi];
+    // a part's first group may lie beyond the lists' capacity
+    if (!SPLIT || 8 * ln.part < a.nmax) w = LWords<SPLIT>(a, gi, ln).first();
+  }
+  __device__ __forceinline__ void fetch(const BlockArgs& a, int64_t b, int n, int q, const PassLanes<SPLIT>& ln)
+  {
+    if (q >= n) return;
+    index(a, b, q);
+    list(a, ln);
+  }
 };
 __device__ __forceinline__ void lslots(uint2 w, int far_slot, int k0, int cnt, int (&c)[4])
 {
@@ -937,18 +960,22 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<SPLIT>) k_block_eam_r
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, false, ltype);
   const int4 hd = a.head[b];
-  stage<false>(a, b, hd, rec, ltype);
   const PassLanes<SPLIT> ln(a);
-  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
-    const int64_t gi = a.cen[b * a.ccap + q];
-    const int slot = a.cen_slot[b * a.ccap + q];
+  PassAtom<SPLIT> at;
+  if (ln.slot < hd.y) at.index(a, b, ln.slot);
+  stage<false>(a, b, hd, rec, ltype);
+  if (ln.slot < hd.y) at.list(a, ln);
+  __syncthreads();
+  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+    const int64_t gi = at.gi;
+    const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
     const int ti = MULTI ? ltype[slot] : 0;
     const bool oni = !MULTI || pm::eam_on(t, ti);
-    const int cnt = oni ? a.nnb[gi] : 0;
+    const int cnt = oni ? at.cnt : 0;
     double rho = 0.0;
     LWords<SPLIT> lw(a, gi, ln);
-    uint2 wnext = lw.first(ln, cnt);
+    uint2 wnext = at.w;
     for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
       if (k0 + ln.step() < cnt) wnext = lw.next();
@@ -1003,19 +1030,23 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, true, ltype);
   const int4 hd = a.head[b];
-  stage<true>(a, b, hd, rec, ltype);
   const PassLanes<SPLIT> ln(a);
-  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
-    const int64_t gi = a.cen[b * a.ccap + q];
-    const int slot = a.cen_slot[b * a.ccap + q];
+  PassAtom<SPLIT> at;
+  if (ln.slot < hd.y) at.index(a, b, ln.slot);
+  stage<true>(a, b, hd, rec, ltype);
+  if (ln.slot < hd.y) at.list(a, ln);
+  __syncthreads();
+  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+    const int64_t gi = at.gi;
+    const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
     const int ti = MULTI ? ltype[slot] : 0;
     const Real fpi = (Real)pi.w;
-    const int cnt = (!MULTI || pm::eam_on(t, ti)) ? a.nnb[gi] : 0;
+    const int cnt = (!MULTI || pm::eam_on(t, ti)) ? at.cnt : 0;
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     LWords<SPLIT> lw(a, gi, ln);
-    uint2 wnext = lw.first(ln, cnt);
+    uint2 wnext = at.w;
     for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
       if (k0 + ln.step() < cnt) wnext = lw.next();
@@ -1107,20 +1138,24 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, FORCE, ltype);
   const int4 hd = a.head[b];
-  stage<FORCE>(a, b, hd, rec, ltype);
   const PassLanes<false> ln(a);
-  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
-    const int64_t gi = a.cen[b * a.ccap + q];
-    const int slot = a.cen_slot[b * a.ccap + q];
+  PassAtom<false> at;
+  if (ln.slot < hd.y) at.index(a, b, ln.slot);
+  stage<FORCE>(a, b, hd, rec, ltype);
+  if (ln.slot < hd.y) at.list(a, ln);
+  __syncthreads();
+  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+    const int64_t gi = at.gi;
+    const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
-    const int cnt = a.nnb[gi];
+    const int cnt = at.cnt;
     float acc = 0.0f;
     if constexpr (LEVEL == 3) {
       if (ln.writes()) sink[gi] = pi.x + cnt;
       continue;
     }
     LWords<false> lw(a, gi, ln);
-    uint2 wnext = lw.first(ln, cnt);
+    uint2 wnext = at.w;
     for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
       if (k0 + ln.step() < cnt) wnext = lw.next();
@@ -1199,18 +1234,22 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
       lrc2[threadIdx.x] = lm.rcut2[threadIdx.x];
     }
   }
-  stage<false>(a, b, hd, rec, ltype);
   const PassLanes<SPLIT> ln(a);
-  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
-    const int64_t gi = a.cen[b * a.ccap + q];
-    const int slot = a.cen_slot[b * a.ccap + q];
+  PassAtom<SPLIT> at;
+  if (ln.slot < hd.y) at.index(a, b, ln.slot);
+  stage<false>(a, b, hd, rec, ltype);
+  if (ln.slot < hd.y) at.list(a, ln);
+  __syncthreads();
+  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+    const int64_t gi = at.gi;
+    const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
     const int ti = MULTI ? ltype[slot] : 0;
-    const int cnt = a.nnb[gi];
+    const int cnt = at.cnt;
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     LWords<SPLIT> lw(a, gi, ln);
-    uint2 wnext = lw.first(ln, cnt);
+    uint2 wnext = at.w;
     for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
       if (k0 + ln.step() < cnt) wnext = lw.next();
@@ -1267,16 +1306,20 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, false, ltype);
   const int4 hd = a.head[b];
-  stage<false>(a, b, hd, rec, ltype);
   const PassLanes<SPLIT> ln(a);
-  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
-    const int64_t gi = a.cen[b * a.ccap + q];
-    const int slot = a.cen_slot[b * a.ccap + q];
+  PassAtom<SPLIT> at;
+  if (ln.slot < hd.y) at.index(a, b, ln.slot);
+  stage<false>(a, b, hd, rec, ltype);
+  if (ln.slot < hd.y) at.list(a, ln);
+  __syncthreads();
+  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+    const int64_t gi = at.gi;
+    const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
-    const int cnt = a.nnb[gi];
+    const int cnt = at.cnt;
     double rho = 0.0;
     LWords<SPLIT> lw(a, gi, ln);
-    uint2 wnext = lw.first(ln, cnt);
+    uint2 wnext = at.w;
     for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
       if (k0 + ln.step() < cnt) wnext = lw.next();
@@ -1312,17 +1355,21 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_force(BlockAr
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, true, ltype);
   const int4 hd = a.head[b];
-  stage<true>(a, b, hd, rec, ltype);
   const PassLanes<SPLIT> ln(a);
-  for (int q = ln.slot; q < hd.y; q += ln.atoms()) {
-    const int64_t gi = a.cen[b * a.ccap + q];
-    const int slot = a.cen_slot[b * a.ccap + q];
+  PassAtom<SPLIT> at;
+  if (ln.slot < hd.y) at.index(a, b, ln.slot);
+  stage<true>(a, b, hd, rec, ltype);
+  if (ln.slot < hd.y) at.list(a, ln);
+  __syncthreads();
+  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+    const int64_t gi = at.gi;
+    const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
-    const int cnt = a.nnb[gi];
+    const int cnt = at.cnt;
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     LWords<SPLIT> lw(a, gi, ln);
-    uint2 wnext = lw.first(ln, cnt);
+    uint2 wnext = at.w;
     for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
       const uint2 w = wnext;
       if (k0 + ln.step() < cnt) wnext = lw.next();
@@ -1375,6 +1422,7 @@ BlockArgs block_args(const Ctx& c, double rcut, const StepGate& gate = {})
   a.ccap = c.bcentral;
   a.rc2 = rcut * rcut;
   a.xf = c.xf_dev();
+  a.nmax = c.nmax;
   a.split = 0;
   while (a.split < 3 && (c.bcentral << (a.split + 1)) <= kPassAtoms) a.split++;
   return a;
