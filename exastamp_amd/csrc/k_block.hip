@@ -1602,10 +1602,13 @@ void block_setup(Ctx& c)
   // of the grid (slabs, clusters) the measured halo can exceed the LDS budget, and
   // the bound shrinks until it fits (or the bricks are single cells).
   double per_cell = std::max((double)c.n / (double)c.ncell_tot, 1e-3);
-  // Systems that 230-atom bricks would not spread over the CUs three workgroups deep are
-  // cut into smaller ones, whose passes walk each list with more lanes (PassLanes).
+  // Systems that 230-atom bricks would not spread over the CUs are cut into smaller ones,
+  // whose passes walk each list with more lanes (PassLanes).  One and a half workgroups
+  // per CU measured best at 50 k EAM atoms (density and force pass, mixed: bricks of at
+  // most 60 atoms 11.4 + 15.8 us, 85: 10.6 + 16.0, 128: 11.0 + 12.8, 170: 12.3 + 14.6,
+  // 230: 12.9 + 18.2); 4000 argon atoms end at one cell per brick either way.
   double bound = c.block_atoms;
-  if (!c.block_atoms_set) bound = std::min(bound, std::max(8.0, (double)c.n / (3.0 * std::max(c.num_cu, 1))));
+  if (!c.block_atoms_set) bound = std::min(bound, std::max(8.0, (double)c.n / (1.5 * std::max(c.num_cu, 1))));
   for (int attempt = 0;; attempt++) {
     block_shape_choose(c, g, bound, per_cell);
     XS_HIP(hipMemsetAsync(c.dscalar.p + 2, 0, 3 * sizeof(unsigned long long), c.stream));
