@@ -65,6 +65,7 @@ SIGNATURES = {
                                 C.POINTER(C.c_int)]),
     "xs_system_size": (C.c_int64, [_CTX]),
     "xs_system_get": (C.c_int, [_CTX, _D, _D, _D, _D, _D, _D]),
+    "xs_state_get": (C.c_int, [_CTX, _D, _D]),
     "xs_field_get": (C.c_int, [_CTX, C.c_int, _D]),
     "xs_velocity_set": (C.c_int, [_CTX, _D, _D, _D]),
     "xs_chunk_neighbors": (C.c_int, [_CTX, C.c_double, C.c_double, C.c_int]),

@@ -16,6 +16,7 @@ Ctx::~Ctx()
   if (hscalar) (void)hipHostFree(hscalar);
   if (hthermo) (void)hipHostFree(hthermo);
   if (hflag) (void)hipHostFree(hflag);
+  if (pinned) (void)hipHostFree(pinned);
   for (hipEvent_t e : step_event)
     if (e) (void)hipEventDestroy(e);
   if (own_stream) (void)hipStreamDestroy(own_stream);
@@ -65,20 +66,53 @@ std::vector<T> from_device(Ctx& c, const DBuf<T>& d, int64_t n)
   return h;
 }
 
-// gather a device array in cell order back to id order
-void to_id_order(Ctx& c, const DBuf<double>& d, double* out, int64_t stride = 0)
+char* pinned_buffer(Ctx& c)
 {
-  if (!out) return;
-  const std::vector<int64_t> id = from_device(c, c.id, c.n);
-  if (stride == 0) {
-    const std::vector<double> v = from_device(c, d, c.n);
-    for (int64_t k = 0; k < c.n; k++) out[id[k]] = v[k];
-  } else {
-    // 9 components stored as vir[q*npad + k]
-    const std::vector<double> v = from_device(c, d, 9 * c.npad);
-    for (int64_t k = 0; k < c.n; k++)
-      for (int q = 0; q < 9; q++) out[9 * id[k] + q] = v[q * c.npad + k];
+  if (!c.pinned) XS_HIP(hipHostMalloc((void**)&c.pinned, kPinnedBytes, hipHostMallocDefault));
+  return c.pinned;
+}
+
+// Rows of the device's cell order to the caller's arrays, in id order: the order is
+// restored on the device, and the host copies what it asked for.  `out` receives the
+// rows one after the other, row q at out[q] (NULL: not wanted); with one array of all
+// rows (interleaved), out[0].  Small results cross in one transfer through pinned memory.
+void to_id_order(Ctx& c, const double* const* src, int64_t stride, int rows, bool interleaved, double* const* out)
+{
+  if (c.n == 0) return;
+  IdRows r{};
+  double* to[9];
+  for (int q = 0; q < rows; q++)
+    if (interleaved || out[q]) {
+      to[r.rows] = interleaved ? nullptr : out[q];
+      r.src[r.rows++] = src[q];
+    }
+  if (r.rows == 0) return;
+  r.stride = stride;
+  r.atom_step = interleaved ? r.rows : 1;
+  r.row_step = interleaved ? 1 : c.n;
+  const size_t row = sizeof(double) * (size_t)c.n, all = row * r.rows;
+  c.io_d.reserve((size_t)c.n * r.rows);
+  launch_to_id_order(c, r, c.io_d.p);
+  if (all <= kPinnedBytes) {
+    char* h = pinned_buffer(c);
+    XS_HIP(hipMemcpyAsync(h, c.io_d.p, all, hipMemcpyDeviceToHost, c.stream));
+    XS_HIP(hipStreamSynchronize(c.stream));
+    if (interleaved) std::memcpy(out[0], h, all);
+    else
+      for (int q = 0; q < r.rows; q++) std::memcpy(to[q], h + q * row, row);
+    return;
   }
+  if (interleaved) XS_HIP(hipMemcpyAsync(out[0], c.io_d.p, all, hipMemcpyDeviceToHost, c.stream));
+  else
+    for (int q = 0; q < r.rows; q++)
+      XS_HIP(hipMemcpyAsync(to[q], c.io_d.p + (size_t)q * c.n, row, hipMemcpyDeviceToHost, c.stream));
+  XS_HIP(hipStreamSynchronize(c.stream));
+}
+
+void to_id_order(Ctx& c, const DBuf<double>& d, double* out)
+{
+  const double* src[1] = {d.p};
+  to_id_order(c, src, 1, 1, false, &out);
 }
 
 void allocate_atoms(Ctx& c, int64_t n)
@@ -305,7 +339,6 @@ xs_status xs_system_set(xs_ctx* h, int64_t n, const double* rx, const double* ry
       }
     for (int a = 0; a < 3; a++) c.periodic[a] = periodic[a] ? 1 : 0;
     c.box_d.reserve(nrep);
-    XS_HIP(hipMemcpyAsync(c.box_d.p, c.box_h.data(), sizeof(BoxDev) * nrep, hipMemcpyHostToDevice, c.stream));
     c.nrep = nrep;
     c.has_rep = nrep > 1;
     c.n = n;
@@ -313,22 +346,32 @@ xs_status xs_system_set(xs_ctx* h, int64_t n, const double* rx, const double* ry
     c.list_valid = false;
     c.rho_state = RhoState::None;
     c.rho_ckpt = false;
+    // the boxes reach the device with each list build, which sets their cell size
     if (n > 0) {
-      std::vector<Pos4> p4(n);
-      for (int64_t i = 0; i < n; i++) p4[i] = Pos4{rx[i], ry[i], rz[i], 0.0};
-      to_device(c, c.pos, p4.data(), n);
-      to_device(c, c.rrx, rx, n);
-      to_device(c, c.rry, ry, n);
-      to_device(c, c.rrz, rz, n);
-      to_device(c, c.vx, vx, n);
-      to_device(c, c.vy, vy, n);
-      to_device(c, c.vz, vz, n);
-      to_device(c, c.type, type, n);
-      std::vector<int64_t> id(n);
-      for (int64_t i = 0; i < n; i++) id[i] = i;
-      to_device(c, c.id, id.data(), n);
-      if (c.has_rep) to_device(c, c.rep, rep, n);
-      launch_zero(c);
+      const double* rows[6] = {rx, ry, rz, vx, vy, vz};
+      const size_t row = sizeof(double) * (size_t)n, rep_at = 6 * row, type_at = rep_at + (c.has_rep ? 2 * (size_t)n : 0);
+      const size_t all = type_at + (size_t)n;
+      if (all <= kPinnedBytes) {  // one transfer
+        c.io_d.reserve((all + 7) / 8);
+        char* h = pinned_buffer(c);
+        for (int q = 0; q < 6; q++) std::memcpy(h + q * row, rows[q], row);
+        if (c.has_rep) std::memcpy(h + rep_at, rep, 2 * (size_t)n);
+        std::memcpy(h + type_at, type, (size_t)n);
+        XS_HIP(hipMemcpyAsync(c.io_d.p, h, all, hipMemcpyHostToDevice, c.stream));
+        char* d = reinterpret_cast<char*>(c.io_d.p);
+        launch_unpack_atoms(c, c.io_d.p, reinterpret_cast<uint8_t*>(d + type_at), reinterpret_cast<uint16_t*>(d + rep_at));
+      } else {
+        c.io_d.reserve(6 * (size_t)n);
+        c.io_type.reserve(n);
+        for (int q = 0; q < 6; q++)
+          XS_HIP(hipMemcpyAsync(c.io_d.p + (size_t)q * n, rows[q], row, hipMemcpyHostToDevice, c.stream));
+        to_device(c, c.io_type, type, n);
+        if (c.has_rep) {
+          c.io_rep.reserve(n);
+          to_device(c, c.io_rep, rep, n);
+        }
+        launch_unpack_atoms(c, c.io_d.p, c.io_type.p, c.io_rep.p);
+      }
     }
     XS_HIP(hipStreamSynchronize(c.stream));
   });
@@ -343,18 +386,24 @@ int64_t xs_system_size(const xs_ctx* h)
 xs_status xs_system_get(xs_ctx* h, double* rx, double* ry, double* rz, double* vx, double* vy, double* vz)
 {
   return guarded(h, [&](Ctx& c) {
-    if (rx || ry || rz) {
-      const std::vector<int64_t> id = from_device(c, c.id, c.n);
-      const std::vector<Pos4> p = from_device(c, c.pos, c.n);
-      for (int64_t k = 0; k < c.n; k++) {
-        if (rx) rx[id[k]] = p[k].x;
-        if (ry) ry[id[k]] = p[k].y;
-        if (rz) rz[id[k]] = p[k].z;
-      }
-    }
-    to_id_order(c, c.vx, vx);
-    to_id_order(c, c.vy, vy);
-    to_id_order(c, c.vz, vz);
+    const double* p = reinterpret_cast<const double*>(c.pos.p);
+    const double* pos[3] = {p, p + 1, p + 2};
+    double* const to_r[3] = {rx, ry, rz};
+    to_id_order(c, pos, 4, 3, false, to_r);
+    const double* vel[3] = {c.vx.p, c.vy.p, c.vz.p};
+    double* const to_v[3] = {vx, vy, vz};
+    to_id_order(c, vel, 1, 3, false, to_v);
+  });
+}
+
+xs_status xs_state_get(xs_ctx* h, double* r, double* v)
+{
+  return guarded(h, [&](Ctx& c) {
+    const double* p = reinterpret_cast<const double*>(c.pos.p);
+    const double* pos[3] = {p, p + 1, p + 2};
+    if (r) to_id_order(c, pos, 4, 3, true, &r);
+    const double* vel[3] = {c.vx.p, c.vy.p, c.vz.p};
+    if (v) to_id_order(c, vel, 1, 3, true, &v);
   });
 }
 
@@ -362,13 +411,13 @@ xs_status xs_velocity_set(xs_ctx* h, const double* vx, const double* vy, const d
 {
   return guarded(h, [&](Ctx& c) {
     require(vx && vy && vz, XS_E_ARG, "null velocity array");
-    const std::vector<int64_t> id = from_device(c, c.id, c.n);
-    std::vector<double> t(c.n);
-    for (auto [src, dst] : {std::pair<const double*, DBuf<double>*>{vx, &c.vx}, {vy, &c.vy}, {vz, &c.vz}}) {
-      for (int64_t k = 0; k < c.n; k++) t[k] = src[id[k]];
-      to_device(c, *dst, t.data(), c.n);
-      XS_HIP(hipStreamSynchronize(c.stream));
-    }
+    if (c.n == 0) return;
+    c.io_d.reserve(3 * (size_t)c.n);
+    const double* rows[3] = {vx, vy, vz};
+    for (int q = 0; q < 3; q++)
+      XS_HIP(hipMemcpyAsync(c.io_d.p + (size_t)q * c.n, rows[q], sizeof(double) * c.n, hipMemcpyHostToDevice, c.stream));
+    launch_velocities_in(c, c.io_d.p);
+    XS_HIP(hipStreamSynchronize(c.stream));
   });
 }
 
@@ -378,22 +427,27 @@ xs_status xs_field_get(xs_ctx* h, int field, double* out)
     require(out != nullptr, XS_E_ARG, "null output");
     switch (field) {
       case XS_FIELD_EP: to_id_order(c, c.ep, out); break;
-      case XS_FIELD_VIRIAL: to_id_order(c, c.vir, out, 9); break;
+      case XS_FIELD_VIRIAL: {  // 9 components stored as vir[q*npad + k]
+        const double* src[9];
+        for (int q = 0; q < 9; q++) src[q] = c.vir.p + (size_t)q * c.npad;
+        to_id_order(c, src, 1, 9, true, &out);
+        break;
+      }
       case XS_FIELD_RHO_DEMB:
         if (c.rho_state == RhoState::FpFloat || c.rho_state == RhoState::FpDouble ||
             c.rho_state == RhoState::FpJohnson) {
-          const std::vector<int64_t> id = from_device(c, c.id, c.n);
-          const std::vector<Pos4> p = from_device(c, c.pos, c.n);
-          for (int64_t k = 0; k < c.n; k++) out[id[k]] = p[k].w;
+          const double* src[1] = {reinterpret_cast<const double*>(c.pos.p) + 3};
+          to_id_order(c, src, 4, 1, false, &out);
         } else {
           to_id_order(c, c.rho, out);
         }
         break;
-      case XS_FIELD_ACCEL:
-        to_id_order(c, c.ax, out);
-        to_id_order(c, c.ay, out + c.n);
-        to_id_order(c, c.az, out + 2 * c.n);
+      case XS_FIELD_ACCEL: {
+        const double* src[3] = {c.ax.p, c.ay.p, c.az.p};
+        double* const to[3] = {out, out + c.n, out + 2 * c.n};
+        to_id_order(c, src, 1, 3, false, to);
         break;
+      }
       default: throw Error(XS_E_ARG, "unknown field");
     }
   });

@@ -97,6 +97,56 @@ __global__ void __launch_bounds__(256) k_drift_kick(
   if (far) over.raise();
 }
 
+// Atoms as the caller gave them -- x, y, z, vx, vy, vz in rows of n, types, replicas --
+// into the per-atom arrays, accelerations, energies and virials zeroed
+__global__ void k_unpack_atoms(int64_t n, int64_t npad, const double* __restrict__ in,
+                               const uint8_t* __restrict__ type_in, const uint16_t* __restrict__ rep_in,
+                               Pos4* __restrict__ pos, double* __restrict__ rrx, double* __restrict__ rry,
+                               double* __restrict__ rrz, double* __restrict__ vx, double* __restrict__ vy,
+                               double* __restrict__ vz, double* __restrict__ ax, double* __restrict__ ay,
+                               double* __restrict__ az, double* __restrict__ ep, double* __restrict__ vir,
+                               uint8_t* __restrict__ type, uint16_t* __restrict__ rep, int64_t* __restrict__ id)
+{
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double x = in[i], y = in[n + i], z = in[2 * n + i];
+  store_pos(pos, i, Pos4{x, y, z, 0.0});
+  rrx[i] = x;
+  rry[i] = y;
+  rrz[i] = z;
+  vx[i] = in[3 * n + i];
+  vy[i] = in[4 * n + i];
+  vz[i] = in[5 * n + i];
+  ax[i] = ay[i] = az[i] = ep[i] = 0.0;
+#pragma unroll
+  for (int q = 0; q < 9; q++) vir[q * npad + i] = 0.0;
+  type[i] = type_in[i];
+  if (rep) rep[i] = rep_in[i];
+  id[i] = i;
+}
+
+// `rows` per-atom arrays in id order: row q of atom k from src[q][stride k] to
+// out[os id[k] + oq q] (os, oq: the caller's layout)
+__global__ void k_to_id_order(int64_t n, const int64_t* __restrict__ id, IdRows r, double* __restrict__ out)
+{
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  double* o = out + r.atom_step * id[k];
+  for (int q = 0; q < r.rows; q++) o[q * r.row_step] = r.src[q][r.stride * k];
+}
+
+// v (id order, rows of n) into the cell order
+__global__ void k_velocities_in(int64_t n, const int64_t* __restrict__ id, const double* __restrict__ in,
+                                double* __restrict__ vx, double* __restrict__ vy, double* __restrict__ vz)
+{
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const int64_t i = id[k];
+  vx[k] = in[i];
+  vy[k] = in[n + i];
+  vz[k] = in[2 * n + i];
+}
+
 // Plain streaming copy, 16 bytes per lane per iteration.
 __global__ void __launch_bounds__(256) k_stream_copy(int64_t n16, const double2* __restrict__ src,
                                                      double2* __restrict__ dst)
@@ -234,6 +284,26 @@ std::mutex g_scratch_mu;
 double* g_scratch_ptr[kMaxDevices] = {};
 
 }  // namespace
+
+void launch_unpack_atoms(Ctx& c, const double* in, const uint8_t* type, const uint16_t* rep)
+{
+  k_unpack_atoms<<<grid_for(c.n), kBlock, 0, c.stream>>>(
+      c.n, c.npad, in, type, rep, c.pos.p, c.rrx.p, c.rry.p, c.rrz.p, c.vx.p, c.vy.p, c.vz.p, c.ax.p, c.ay.p, c.az.p,
+      c.ep.p, c.vir.p, c.type.p, c.has_rep ? c.rep.p : nullptr, c.id.p);
+  XS_HIP(hipGetLastError());
+}
+
+void launch_to_id_order(Ctx& c, const IdRows& r, double* out)
+{
+  k_to_id_order<<<grid_for(c.n), kBlock, 0, c.stream>>>(c.n, c.id.p, r, out);
+  XS_HIP(hipGetLastError());
+}
+
+void launch_velocities_in(Ctx& c, const double* in)
+{
+  k_velocities_in<<<grid_for(c.n), kBlock, 0, c.stream>>>(c.n, c.id.p, in, c.vx.p, c.vy.p, c.vz.p);
+  XS_HIP(hipGetLastError());
+}
 
 void launch_zero(Ctx& c)
 {

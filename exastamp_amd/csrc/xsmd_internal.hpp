@@ -402,6 +402,12 @@ struct Ctx {
   unsigned long long* hflag = nullptr;  // pinned host copy of the loop's flag dscalar[5] (StepFlag)
   hipEvent_t step_event[2] = {nullptr, nullptr};  // ends of the MD loop's queued steps
   DBuf<double> thermo_log;              // the loop's thermodynamic samples
+  // atoms on their way in and out: device buffers, and pinned host memory that small
+  // transfers go through in one piece (kPinnedBytes)
+  DBuf<double> io_d;
+  DBuf<uint8_t> io_type;
+  DBuf<uint16_t> io_rep;
+  char* pinned = nullptr;
 
   // small device scalars + pinned host mirror
   DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..4] halo maxima,
@@ -462,6 +468,17 @@ double gather_ceiling(Ctx& c, double rcut, bool force, int level, int reps);
 void pair_count(Ctx& c, double rcut, int64_t& entries, int64_t& within);
 
 // ---- launches (k_integrate.hip) ----
+// x, y, z, vx, vy, vz (rows of n), types and replicas in device memory into the context
+void launch_unpack_atoms(Ctx& c, const double* in, const uint8_t* type, const uint16_t* rep);
+// per-atom rows of the cell order, element k of row q at src[q][stride k], and where they
+// go in id order: atom i, row q at atom_step i + row_step q
+struct IdRows {
+  const double* src[9];
+  int rows;
+  int64_t stride, atom_step, row_step;
+};
+void launch_to_id_order(Ctx& c, const IdRows& r, double* out);
+void launch_velocities_in(Ctx& c, const double* in);
 void launch_zero(Ctx& c);
 void launch_force_to_accel(Ctx& c);
 // inv_xform: xform_mode INV_XFORM (the step is mapped to grid space by the xform's
@@ -554,6 +571,7 @@ void eam_theta_dev(Ctx& c, const double* theta);
 void forces_energies_dev(Ctx& c, double* F, double* E, double scale);
 
 // ---- helpers ----
+constexpr size_t kPinnedBytes = 4 << 20;
 constexpr int kBlock = 256;
 inline unsigned grid_for(int64_t n, int block = kBlock)
 {

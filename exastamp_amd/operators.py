@@ -421,10 +421,9 @@ class Simulation:
 
     # --- read back (id order) --------------------------------------------------
     def state(self):
-        n = self.n
-        arrs = [np.zeros(n) for _ in range(6)]
-        self.ctx.xs_system_get(*[_lib.dptr(a) for a in arrs])
-        return np.stack(arrs[:3], axis=1), np.stack(arrs[3:], axis=1)
+        r, v = np.empty((self.n, 3)), np.empty((self.n, 3))
+        self.ctx.xs_state_get(_lib.dptr(r), _lib.dptr(v))
+        return r, v
 
     def set_velocities(self, v):
         cols = [np.ascontiguousarray(v[:, a], dtype=np.float64) for a in range(3)]

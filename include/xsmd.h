@@ -105,6 +105,8 @@ int64_t xs_system_size(const xs_ctx* ctx);
 /* Copy state back in id order; any pointer may be NULL. */
 xs_status xs_system_get(xs_ctx* ctx, double* rx, double* ry, double* rz, double* vx,
                         double* vy, double* vz);
+/* The same state as two arrays of 3n doubles, x y z per atom; either may be NULL. */
+xs_status xs_state_get(xs_ctx* ctx, double* r, double* v);
 xs_status xs_field_get(xs_ctx* ctx, int field, double* out);
 /* Domain xform of a deformed domain (exaNBody's Domain::xform / set_xform; read by
  * the pair operators at pair_potential_impl.hxx:388-413, which switch to the
