@@ -847,7 +847,7 @@ xs_status xs_md_run(xs_ctx* h, int potential, int nsteps, double dt, double rcut
     const size_t nlog = thermo_every > 0 ? (size_t)(nsteps / thermo_every) + 1 : 0;
     if (nlog) c.thermo_log.reserve(27 * nlog);
     const auto clear_flag = [&]() {
-      XS_HIP(hipMemsetAsync(c.dscalar.p + 5, 0, sizeof(unsigned long long), c.stream));
+      XS_HIP(hipMemsetAsync(c.dscalar.p + 6, 0, sizeof(unsigned long long), c.stream));
       __atomic_store_n(c.hflag, 0ull, __ATOMIC_RELAXED);
     };
     XS_HIP(hipStreamSynchronize(c.stream));  // no queued kernel still writes the host's flag
@@ -948,8 +948,10 @@ xs_status xs_md_run(xs_ctx* h, int potential, int nsteps, double dt, double rcut
         queue_step();
       }
     }
-    if (nlog)
-      XS_HIP(hipMemcpyAsync(thermo_out, c.thermo_log.p, 27 * nlog * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+    const size_t log0 = cont ? 27 : 0;  // a continued run has no step 0
+    if (27 * nlog > log0)
+      XS_HIP(hipMemcpyAsync(thermo_out + log0, c.thermo_log.p + log0, (27 * nlog - log0) * sizeof(double),
+                            hipMemcpyDeviceToHost, c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
     const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     if (c.prof.on) c.prof.flush();

@@ -204,10 +204,14 @@ constexpr int kPassAtoms = kPassThreads / 2;
 // atom at 220-atom bricks) written at the build and read by each pass; the chain of
 // waits it removes was longer: 8.39 M EAM atoms, mixed: density pass 0.907 -> 0.761 ms,
 // force pass 1.350 -> 1.258 ms; 1.05 M argon atoms 0.171 -> 0.141 ms per pass.
+// The bricks' parts of the tables follow one another in the order the build's workgroups
+// took them, so their size goes with the atoms, not with the number of bricks times the
+// densest one.
+constexpr uint32_t kStageAlign = 16;  // a brick's staging entries start on 64 bytes
 struct BlockArgs {
-  const int4* __restrict__ head;       // per brick: halo atoms, central atoms, replica
-  const uint32_t* __restrict__ stage;  // per brick cap entries: global index and image of each slot
-  const uint32_t* __restrict__ cen;    // per brick ccap entries: central atoms (global index)
+  const uint4* __restrict__ head;      // per brick: BrickHead
+  const uint32_t* __restrict__ stage;  // global index and image of each halo slot
+  const uint32_t* __restrict__ cen;    // central atoms (global index)
   const uint16_t* __restrict__ cen_slot;  // and their slots
   const Pos4* __restrict__ pos;
   const uint8_t* __restrict__ type;
@@ -216,13 +220,26 @@ struct BlockArgs {
   const int* __restrict__ nnb;
   int64_t npad;
   int64_t nblocks;
-  int cap;   // halo slots (LDS records)
-  int ccap;  // central atoms per brick at most
+  int cap;  // halo slots (LDS records)
   double rc2;
   int nmax;            // list capacity
   int split;           // SPLIT passes: log2 of the parts an atom's list is walked in
   const XformDev* xf;  // the staging maps positions to physical space when not NULL
   StepGate gate;       // MD loop
+};
+
+// What a brick holds and where its parts of the tables start
+struct BrickHead {
+  int halo, central, replica;
+  uint32_t stage, cen;
+  __device__ __forceinline__ static uint4 pack(int halo, int central, int replica, uint32_t stage16, uint32_t cen)
+  {
+    return make_uint4((uint32_t)halo | (uint32_t)central << 16, (uint32_t)replica, stage16, cen);
+  }
+  __device__ __forceinline__ explicit BrickHead(const uint4& h)
+      : halo((int)(h.x & 0xffffu)), central((int)(h.x >> 16)), replica((int)h.y), stage(h.z * kStageAlign), cen(h.w)
+  {
+  }
 };
 
 // LDS of the block passes: records, then per-record types (block_lds_bytes on the host
@@ -245,9 +262,9 @@ __device__ __forceinline__ LRec pass_lds(const BlockArgs& a, bool with_type, boo
 // every staged position (which are within the box and its images) and close enough that
 // its knot index fits an int.  The caller's __syncthreads() follows.
 template <bool WITH_W>
-__device__ __forceinline__ void stage(const BlockArgs& a, int64_t b, const int4& hd, const LRec& rec, uint8_t* ltype)
+__device__ __forceinline__ void stage(const BlockArgs& a, const BrickHead& hd, const LRec& rec, uint8_t* ltype)
 {
-  const BoxDev& box = a.box[hd.z];
+  const BoxDev& box = a.box[hd.replica];
   const double* L = box.L;
   if (threadIdx.x == 0) {
     const double far = 4.0 * (fabs(box.lo[0]) + fabs(box.lo[1]) + fabs(box.lo[2]) + L[0] + L[1] + L[2]) + 1e4;
@@ -260,12 +277,12 @@ __device__ __forceinline__ void stage(const BlockArgs& a, int64_t b, const int4&
     rec.put(a.cap, f);
     if (ltype) ltype[a.cap] = 0;
   }
-  const uint32_t* st = a.stage + b * a.cap;
+  const uint32_t* st = a.stage + hd.stage;
   int c = threadIdx.x;
-  uint32_t ahead = c < hd.x ? st[c] : 0u;  // the next entry is on its way while a record is staged
-  while (c < hd.x) {
+  uint32_t ahead = c < hd.halo ? st[c] : 0u;  // the next entry is on its way while a record is staged
+  while (c < hd.halo) {
     const uint32_t e = ahead;
-    if (c + kPassThreads < hd.x) ahead = st[c + kPassThreads];
+    if (c + kPassThreads < hd.halo) ahead = st[c + kPassThreads];
     const uint32_t j = xsmd_nbr_index(e);
     Pos4 p;
     if constexpr (WITH_W) {
@@ -518,12 +535,13 @@ struct BuildArgs {
   int atoms;     // lists collected per wave, at most kBuildAtoms
   bool sort;     // false: lists stay in stencil order
   // what the passes read instead of the cells (see BlockArgs)
-  int4* __restrict__ head;
+  uint4* __restrict__ head;
   uint32_t* __restrict__ stage;
   uint32_t* __restrict__ cen;
   uint16_t* __restrict__ cen_slot;
-  int ccap;
-  unsigned long long* __restrict__ flags;  // [0] longest list beyond nmax, [1] halo beyond cap
+  // [0] longest list beyond nmax, [1] halo beyond cap, [2] table space taken (staging
+  // entries in units of kStageAlign, central atoms in the lower half)
+  unsigned long long* __restrict__ flags;
 };
 
 // candidate slots of each wave (the staging uses the same bytes first) and the list rows
@@ -541,7 +559,9 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
   extern __shared__ __align__(32) unsigned char smem[];
   double3* P = reinterpret_cast<double3*>(smem);
   HaloCell* hc = reinterpret_cast<HaloCell*>(smem + build_rec_bytes(a.cap));
-  int* total_p = reinterpret_cast<int*>(hc + a.g.nh_max);  // [0] halo atoms, [1] next central cell
+  // [0] halo atoms, [1] next central cell, [2] the brick's staging entries / kStageAlign,
+  // (-1: no central atoms), [3] its central atoms in the tables
+  int* total_p = reinterpret_cast<int*>(hc + a.g.nh_max);
   int* cell_q = total_p + 4;                                // first central atom of each central cell
   uint16_t* cand_all = reinterpret_cast<uint16_t*>(cell_q + a.g.bx * a.g.by * a.g.bz);
   uint32_t* rows_all = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(cand_all) +
@@ -573,15 +593,24 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
     }
     if (lane == 0) {
       total_p[1] = 0;
-      a.head[b] = make_int4(total, carry, s.r, 0);
+      total_p[2] = -1;
+      uint4 head = BrickHead::pack(0, 0, s.r, 0, 0);  // no central atom: nothing to stage
+      if (carry > 0) {
+        const unsigned long long need = (unsigned long long)((total + kStageAlign - 1) / kStageAlign) << 32;
+        const unsigned long long at = atomicAdd(a.flags + 2, need | (unsigned long long)carry);
+        total_p[2] = (int)(at >> 32);
+        total_p[3] = (int)(uint32_t)at;
+        head = BrickHead::pack(total, carry, s.r, (uint32_t)(at >> 32), (uint32_t)at);
+      }
+      a.head[b] = head;
     }
   }
   const BoxDev bx = a.box[s.r];
-  uint32_t* stage = a.stage + b * a.cap;
   stage_cells(s, hc, total, a.pos, bx.L, cand_all, [&](int c, const Pos4& p, uint32_t e) {
     P[c] = double3{p.x, p.y, p.z};
-    stage[c] = e;
+    if (total_p[2] >= 0) a.stage[(uint32_t)total_p[2] * kStageAlign + (uint32_t)c] = e;
   });
+  const uint32_t cen0 = (uint32_t)__builtin_amdgcn_readfirstlane(total_p[3]);
 
   uint16_t* cand = cand_all + (size_t)wave * a.cand_cap;
   const int stride = a.nmax + 1;  // odd, so the group loads of 8 rows start in distinct banks
@@ -640,7 +669,7 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
     if (nat == 0) continue;
     const int l0 = __builtin_amdgcn_readfirstlane(hc[h].lstart) + skip;
     const int g0 = __builtin_amdgcn_readfirstlane(hc[h].gstart) + skip;
-    const int64_t q0 = b * a.ccap + cell_q[cc] + skip;
+    const uint32_t q0 = cen0 + (uint32_t)(cell_q[cc] + skip);
     for (int k = lane; k < nat; k += 64) {
       a.cen[q0 + k] = (uint32_t)(g0 + k);
       a.cen_slot[q0 + k] = (uint16_t)(l0 + k);
@@ -765,11 +794,11 @@ __global__ void __launch_bounds__(256) k_block_to_global(BlockArgs a, uint32_t* 
 {
   const int64_t b = lblock();
   if (b >= a.nblocks) return;
-  const int ncentral = a.head[b].y;
-  const uint32_t* stage = a.stage + b * a.cap;
+  const BrickHead hd(a.head[b]);
+  const uint32_t* stage = a.stage + hd.stage;
   const int lane = threadIdx.x & 63;
-  for (int q = threadIdx.x >> 6; q < ncentral; q += blockDim.x >> 6) {
-    const int64_t i = a.cen[b * a.ccap + q];
+  for (int q = threadIdx.x >> 6; q < hd.central; q += blockDim.x >> 6) {
+    const int64_t i = a.cen[hd.cen + (uint32_t)q];
     const int cnt = a.nnb[i];
     if (cnt <= kSortRows) {
       uint32_t key = 0xffffu;
@@ -782,8 +811,9 @@ __global__ void __launch_bounds__(256) k_block_to_global(BlockArgs a, uint32_t* 
   }
 }
 
-// Sizes the LDS of the block kernels: the most halo atoms and central atoms of a brick,
-// and the most atoms in the 27 cells of a central cell.  One wave per brick, one lane
+// Sizes the LDS of the block kernels and the staging table: out[0..2] the most halo atoms
+// and central atoms of a brick and the most atoms in the 27 cells of a central cell,
+// out[3] the staging entries of the bricks that hold atoms, in units of kStageAlign.  One wave per brick, one lane
 // per halo cell (a thread per brick reads its cells one after the other: 33 us for a
 // single brick of 125 cells, against 4 us).
 constexpr int kHaloMaxWaves = 4;
@@ -794,6 +824,7 @@ __global__ void __launch_bounds__(64 * kHaloMaxWaves) k_block_halo_max(BlockGeom
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   int* cnt = cnt_all[wave];
   int m_total = 0, m_central = 0, m_cand = 0;
+  unsigned long long entries = 0;
   for (int64_t b = (int64_t)blockIdx.x * kHaloMaxWaves + wave; b < g.nblocks; b += (int64_t)gridDim.x * kHaloMaxWaves) {
     const BlockShape s = block_shape(g, b);
     const int nh = s.hx * s.hy * s.hz;
@@ -827,6 +858,7 @@ __global__ void __launch_bounds__(64 * kHaloMaxWaves) k_block_halo_max(BlockGeom
       central += __shfl_xor(central, off);
     }
     m_total = max(m_total, total);
+    if (central > 0) entries += (unsigned long long)((total + kStageAlign - 1) / kStageAlign);
     m_central = max(m_central, central);
     wave_lds_sync();
   }
@@ -834,6 +866,7 @@ __global__ void __launch_bounds__(64 * kHaloMaxWaves) k_block_halo_max(BlockGeom
   for (int off = 32; off >= 1; off >>= 1) m_cand = max(m_cand, __shfl_xor(m_cand, off));
   __shared__ int best[kHaloMaxWaves][3];
   if (lane == 0) {
+    if (entries) atomicAdd(out + 3, entries);
     best[wave][0] = m_total;
     best[wave][1] = m_central;
     best[wave][2] = m_cand;
@@ -902,10 +935,10 @@ struct PassAtom {
   int64_t gi = 0;
   int slot = 0, cnt = 0;
   uint2 w = {0u, 0u};
-  __device__ __forceinline__ void index(const BlockArgs& a, int64_t b, int q)
+  __device__ __forceinline__ void index(const BlockArgs& a, const BrickHead& hd, int q)
   {
-    gi = a.cen[b * a.ccap + q];
-    slot = a.cen_slot[b * a.ccap + q];
+    gi = a.cen[hd.cen + (uint32_t)q];
+    slot = a.cen_slot[hd.cen + (uint32_t)q];
   }
   __device__ __forceinline__ void list(const BlockArgs& a, const PassLanes<SPLIT>& ln)
   {
@@ -913,10 +946,10 @@ struct PassAtom {
     // a part's first group may lie beyond the lists' capacity
     if (!SPLIT || 8 * ln.part < a.nmax) w = LWords<SPLIT>(a, gi, ln).first();
   }
-  __device__ __forceinline__ void fetch(const BlockArgs& a, int64_t b, int n, int q, const PassLanes<SPLIT>& ln)
+  __device__ __forceinline__ void fetch(const BlockArgs& a, const BrickHead& hd, int q, const PassLanes<SPLIT>& ln)
   {
-    if (q >= n) return;
-    index(a, b, q);
+    if (q >= hd.central) return;
+    index(a, hd, q);
     list(a, ln);
   }
 };
@@ -959,14 +992,14 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<SPLIT>) k_block_eam_r
   if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, false, ltype);
-  const int4 hd = a.head[b];
+  const BrickHead hd(a.head[b]);
   const PassLanes<SPLIT> ln(a);
   PassAtom<SPLIT> at;
-  if (ln.slot < hd.y) at.index(a, b, ln.slot);
-  stage<false>(a, b, hd, rec, ltype);
-  if (ln.slot < hd.y) at.list(a, ln);
+  if (ln.slot < hd.central) at.index(a, hd, ln.slot);
+  stage<false>(a, hd, rec, ltype);
+  if (ln.slot < hd.central) at.list(a, ln);
   __syncthreads();
-  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
     const int64_t gi = at.gi;
     const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
@@ -1029,14 +1062,14 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
   if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, true, ltype);
-  const int4 hd = a.head[b];
+  const BrickHead hd(a.head[b]);
   const PassLanes<SPLIT> ln(a);
   PassAtom<SPLIT> at;
-  if (ln.slot < hd.y) at.index(a, b, ln.slot);
-  stage<true>(a, b, hd, rec, ltype);
-  if (ln.slot < hd.y) at.list(a, ln);
+  if (ln.slot < hd.central) at.index(a, hd, ln.slot);
+  stage<true>(a, hd, rec, ltype);
+  if (ln.slot < hd.central) at.list(a, ln);
   __syncthreads();
-  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
     const int64_t gi = at.gi;
     const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
@@ -1137,14 +1170,14 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
   if (b >= a.nblocks) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, FORCE, ltype);
-  const int4 hd = a.head[b];
+  const BrickHead hd(a.head[b]);
   const PassLanes<false> ln(a);
   PassAtom<false> at;
-  if (ln.slot < hd.y) at.index(a, b, ln.slot);
-  stage<FORCE>(a, b, hd, rec, ltype);
-  if (ln.slot < hd.y) at.list(a, ln);
+  if (ln.slot < hd.central) at.index(a, hd, ln.slot);
+  stage<FORCE>(a, hd, rec, ltype);
+  if (ln.slot < hd.central) at.list(a, ln);
   __syncthreads();
-  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
     const int64_t gi = at.gi;
     const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
@@ -1222,7 +1255,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
   if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, false, ltype);
-  const int4 hd = a.head[b];
+  const BrickHead hd(a.head[b]);
   // MULTI: the pairs' parameters and squared cutoffs (at most 28 pairs of 7 species), so
   // that a pair's lookup is an LDS read rather than two gathers through the texture path
   // (136 k atoms, FP64, energy and virial: 90 -> 66 us)
@@ -1236,11 +1269,11 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
   }
   const PassLanes<SPLIT> ln(a);
   PassAtom<SPLIT> at;
-  if (ln.slot < hd.y) at.index(a, b, ln.slot);
-  stage<false>(a, b, hd, rec, ltype);
-  if (ln.slot < hd.y) at.list(a, ln);
+  if (ln.slot < hd.central) at.index(a, hd, ln.slot);
+  stage<false>(a, hd, rec, ltype);
+  if (ln.slot < hd.central) at.list(a, ln);
   __syncthreads();
-  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
     const int64_t gi = at.gi;
     const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
@@ -1305,14 +1338,14 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs
   if (b >= a.nblocks) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, false, ltype);
-  const int4 hd = a.head[b];
+  const BrickHead hd(a.head[b]);
   const PassLanes<SPLIT> ln(a);
   PassAtom<SPLIT> at;
-  if (ln.slot < hd.y) at.index(a, b, ln.slot);
-  stage<false>(a, b, hd, rec, ltype);
-  if (ln.slot < hd.y) at.list(a, ln);
+  if (ln.slot < hd.central) at.index(a, hd, ln.slot);
+  stage<false>(a, hd, rec, ltype);
+  if (ln.slot < hd.central) at.list(a, ln);
   __syncthreads();
-  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
     const int64_t gi = at.gi;
     const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
@@ -1354,14 +1387,14 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_force(BlockAr
   if (b >= a.nblocks) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, true, ltype);
-  const int4 hd = a.head[b];
+  const BrickHead hd(a.head[b]);
   const PassLanes<SPLIT> ln(a);
   PassAtom<SPLIT> at;
-  if (ln.slot < hd.y) at.index(a, b, ln.slot);
-  stage<true>(a, b, hd, rec, ltype);
-  if (ln.slot < hd.y) at.list(a, ln);
+  if (ln.slot < hd.central) at.index(a, hd, ln.slot);
+  stage<true>(a, hd, rec, ltype);
+  if (ln.slot < hd.central) at.list(a, ln);
   __syncthreads();
-  for (int q = ln.slot; q < hd.y; q += ln.atoms(), at.fetch(a, b, hd.y, q, ln)) {
+  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
     const int64_t gi = at.gi;
     const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
@@ -1419,7 +1452,6 @@ BlockArgs block_args(const Ctx& c, double rcut, const StepGate& gate = {})
   a.npad = c.npad;
   a.nblocks = c.bgeom.nblocks;
   a.cap = c.bcap;
-  a.ccap = c.bcentral;
   a.rc2 = rcut * rcut;
   a.xf = c.xf_dev();
   a.nmax = c.nmax;
@@ -1445,7 +1477,7 @@ bool drift_setup(Ctx& c, const ForceEpilogue& epi, unsigned flags, pm::Drift& dr
   dr.dt2 = epi.drift_dt * epi.drift_dt * 0.5;
   dr.hdt = epi.drift_dt * 0.5;
   dr.thr2 = epi.drift_thr2;
-  dr.over = StepFlag{c.dscalar.p + 5, c.hflag, epi.step + 1};
+  dr.over = StepFlag{c.dscalar.p + 6, c.hflag, epi.step + 1};
   return true;
 }
 
@@ -1611,16 +1643,17 @@ void block_setup(Ctx& c)
   if (!c.block_atoms_set) bound = std::min(bound, std::max(8.0, (double)c.n / (1.5 * std::max(c.num_cu, 1))));
   for (int attempt = 0;; attempt++) {
     block_shape_choose(c, g, bound, per_cell);
-    XS_HIP(hipMemsetAsync(c.dscalar.p + 2, 0, 3 * sizeof(unsigned long long), c.stream));
+    XS_HIP(hipMemsetAsync(c.dscalar.p + 2, 0, 4 * sizeof(unsigned long long), c.stream));
     k_block_halo_max<<<(unsigned)std::min<int64_t>(512, (g.nblocks + kHaloMaxWaves - 1) / kHaloMaxWaves),
                        64 * kHaloMaxWaves, 0, c.stream>>>(g, c.cell_off.p, c.dscalar.p + 2);
     XS_HIP(hipGetLastError());
-    XS_HIP(hipMemcpyAsync(c.hscalar + 2, c.dscalar.p + 2, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+    XS_HIP(hipMemcpyAsync(c.hscalar + 2, c.dscalar.p + 2, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                           c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
     c.bcap = (int)((c.hscalar[2] + 63) / 64 * 64);
     c.bcentral = (int)c.hscalar[3];
     c.bcand = (int)c.hscalar[4];
+    c.bstage = (size_t)c.hscalar[5] * kStageAlign;
     const size_t budget = c.block_atoms_set ? kBlockLdsLimit : std::min(kBlockLdsLimit, kLdsPerCu / 3);
     if (block_lds_bytes(c, true, true) <= budget || g.nh_max == 27 || attempt == 6) break;
     // the densest halo set the capacity: size the next shape for that density
@@ -1637,7 +1670,7 @@ size_t block_lds_bytes(const Ctx& c, bool with_type, bool with_w)
 
 bool block_feasible(const Ctx& c)
 {
-  return c.bcap > 0 && c.bcap < 65536 && block_lds_bytes(c, true, true) <= kBlockLdsLimit;
+  return c.bcap > 0 && c.bcap < 65536 && c.bstage < (size_t)1 << 32 && block_lds_bytes(c, true, true) <= kBlockLdsLimit;
 }
 
 unsigned block_grid(const Ctx& c)
@@ -1669,14 +1702,13 @@ bool block_build(Ctx& c, double rl2)
   a.sort = !c.list_sort_disabled;
   a.flags = c.dscalar.p;
   c.brick_head.reserve(c.bgeom.nblocks);
-  c.brick_stage.reserve((size_t)c.bgeom.nblocks * c.bcap);
-  c.brick_cen.reserve((size_t)c.bgeom.nblocks * c.bcentral);
-  c.brick_cen_slot.reserve((size_t)c.bgeom.nblocks * c.bcentral);
+  c.brick_stage.reserve(c.bstage);
+  c.brick_cen.reserve(c.n);
+  c.brick_cen_slot.reserve(c.n);
   a.head = c.brick_head.p;
   a.stage = c.brick_stage.p;
   a.cen = c.brick_cen.p;
   a.cen_slot = c.brick_cen_slot.p;
-  a.ccap = c.bcentral;
   for (int attempt = 0; attempt < 2; attempt++) {
     a.atoms = kBuildAtoms;
     while (a.atoms > 1 && build_lds_bytes(c, a.atoms) > kBlockLdsLimit) a.atoms /= 2;
@@ -1691,7 +1723,7 @@ bool block_build(Ctx& c, double rl2)
     if (lds > kBlockLdsLimit)
       XS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)lds));
-    XS_HIP(hipMemsetAsync(c.dscalar.p, 0, 2 * sizeof(unsigned long long), c.stream));
+    XS_HIP(hipMemsetAsync(c.dscalar.p, 0, 3 * sizeof(unsigned long long), c.stream));
     k<<<block_grid(c), kBuildThreads, lds, c.stream>>>(a);
     XS_HIP(hipGetLastError());
     XS_HIP(hipMemcpyAsync(c.hscalar, c.dscalar.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,

@@ -346,10 +346,10 @@ void launch_drift_kick(Ctx& c, double dt, double thr2, unsigned long long step, 
   const double dt2 = dt * dt * 0.5;
   ProfScope prof(c.prof, c.stream, XS_PROF_DRIFT);
   const unsigned g = std::min<unsigned>(grid_for(c.n), 4096);
-  const StepGate gate = gated ? StepGate{c.dscalar.p + 5, step - 1} : StepGate{};
+  const StepGate gate = gated ? StepGate{c.dscalar.p + 6, step - 1} : StepGate{};
   k_drift_kick<<<g, kBlock, 0, c.stream>>>(c.n, dt, dt2, dt * 0.5, c.pos.p, c.vx.p, c.vy.p, c.vz.p, c.ax.p,
                                            c.ay.p, c.az.p, c.rrx.p, c.rry.p, c.rrz.p, thr2,
-                                           StepFlag{c.dscalar.p + 5, c.hflag, step}, gate, c.xf_dev());
+                                           StepFlag{c.dscalar.p + 6, c.hflag, step}, gate, c.xf_dev());
   XS_HIP(hipGetLastError());
 }
 

@@ -131,10 +131,13 @@ struct StepFlag {
   unsigned long long* dev = nullptr;
   unsigned long long* host = nullptr;
   unsigned long long step = 0;
-  // every writer of a launch stores the same value
+  // Every writer of a launch stores the same value; those that find it there leave the
+  // host's copy alone (with no skin every atom of every step passes the threshold, and each
+  // store to the host crosses the bus).
   __device__ __forceinline__ void raise() const
   {
-    *dev = step;
+    if (__hip_atomic_load(dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == step) return;
+    __hip_atomic_store(dev, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(host, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 };
@@ -388,18 +391,19 @@ struct Ctx {
   DBuf<int> cell_off;              // first atom of each cell, ncell_tot + 1
   BlockGeom bgeom{};
   // staging tables of the bricks, written by the block build (k_block.hip, BlockArgs)
-  DBuf<int4> brick_head;
+  DBuf<uint4> brick_head;
   DBuf<uint32_t> brick_stage, brick_cen;
   DBuf<uint16_t> brick_cen_slot;
   int bcap = 0;                    // LDS slots per block (max halo atoms, rounded)
   int bcentral = 0;                // max central atoms per block
   int bcand = 0;                   // max atoms in the 27 cells of a central cell
+  size_t bstage = 0;               // entries of brick_stage in use
   int num_cu = 0;           // CUs of the device (persistent grids)
   size_t lds_max = 65536;   // dynamic LDS one workgroup may use
   bool list_sort_disabled = false;  // XSMD_LIST_SORT=0: block lists stay in stencil order
   bool s_table_disabled = false;    // XSMD_EAM_S_TABLE=0: the FP32 passes read the knot rows
   bool drift_done = false;  // the last force launch applied ForceEpilogue::drift
-  unsigned long long* hflag = nullptr;  // pinned host copy of the loop's flag dscalar[5] (StepFlag)
+  unsigned long long* hflag = nullptr;  // pinned host copy of the loop's flag dscalar[6] (StepFlag)
   hipEvent_t step_event[2] = {nullptr, nullptr};  // ends of the MD loop's queued steps
   DBuf<double> thermo_log;              // the loop's thermodynamic samples
   // atoms on their way in and out: device buffers, and pinned host memory that small
@@ -410,8 +414,8 @@ struct Ctx {
   char* pinned = nullptr;
 
   // small device scalars + pinned host mirror
-  DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..4] halo maxima,
-                                     // [5] the MD loop's rebuild flag (StepFlag)
+  DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..5] halo sizes,
+                                     // [6] the MD loop's rebuild flag (StepFlag)
   unsigned long long* hscalar = nullptr;
   DBuf<double> red_part;  // thermo partial sums
   DBuf<double> red_out;
@@ -516,7 +520,7 @@ struct ForceEpilogue {
 };
 inline StepGate step_gate(const Ctx& c, const ForceEpilogue& e)
 {
-  return e.gated ? StepGate{c.dscalar.p + 5, e.step} : StepGate{};
+  return e.gated ? StepGate{c.dscalar.p + 6, e.step} : StepGate{};
 }
 // energy_cutoff (pair_potential_impl.hxx:487-498): E_LJ(rcut) in FP64, 0 for rcut <= 0
 inline double lj_energy_cutoff(double eps, double sigma, double rcut)

@@ -60,3 +60,28 @@ def test_block_lists_equal_global(monkeypatch, n, box, rcut, cluster):
     print(f"{n} atoms: longest list {glob[0].max()}, brick {info['brick']}, halo {info['halo_capacity']}")
     for x, y in zip(blk, glob):
         assert np.array_equal(x, y)
+
+
+def test_tables_of_a_cluster_in_a_large_box(monkeypatch):
+    """A dense cluster in a box of 600 k cells: the bricks' tables go with the atoms (3000
+    atoms, at most 27 staging entries each and their padding), not with the number of
+    bricks times the densest one (gigabytes here).  200 MB covers the per-cell arrays."""
+    from exastamp_amd.operators import Simulation
+    import ctypes as C
+    cfg = _config(3000, (370.0, 365.0, 360.0), seed=7, cluster=13.0)
+    glob, _ = _lists(monkeypatch, "global", cfg, 4.0)
+    monkeypatch.delenv("XSMD_LIST", raising=False)
+    sim = Simulation(0)
+    sim.species([("Ar", 39.948)])
+    sim.set_config(cfg)
+    free = [C.c_size_t(0), C.c_size_t(0)]
+    total = C.c_size_t(0)
+    sim.ctx.xs_device_memory(C.byref(free[0]), C.byref(total))
+    sim.chunk_neighbors(rcut_max=4.0, rcut_inc=0.3)
+    sim.ctx.xs_device_memory(C.byref(free[1]), C.byref(total))
+    assert sim.list_info()["kind"] == "block"
+    blk = sim.neighbors() + (sim.order(),)
+    sim.close()
+    for x, y in zip(blk, glob):
+        assert np.array_equal(x, y)
+    assert free[0].value - free[1].value < 200e6
