@@ -405,8 +405,7 @@ EamTabDev<double> make_eam_tab<double>(Ctx& c)
 {
   EamTabDev<double> t;
   t.frho = c.eam.frho_d.p;
-  t.rhor = c.eam.rhor_d.p;
-  t.z2r = c.eam.z2r_d.p;
+  t.nel = c.eam.nel;
   t.nr = c.eam.nr;
   t.nrho = c.eam.nrho;
   t.rdr = c.eam.rdr;
@@ -414,8 +413,6 @@ EamTabDev<double> make_eam_tab<double>(Ctx& c)
   t.rdrho = c.eam.rdrho;
   t.rhomax = c.eam.rhomax;
   t.conv = kEV;
-  std::memcpy(t.t2rhor, c.eam.t2rhor, sizeof(t.t2rhor));
-  std::memcpy(t.t2z2r, c.eam.t2z2r, sizeof(t.t2z2r));
   std::memcpy(t.t2frho, c.eam.t2frho, sizeof(t.t2frho));
   t.types = c.eam_types;
   return t;
@@ -426,8 +423,7 @@ EamTabDev<float> make_eam_tab<float>(Ctx& c)
 {
   EamTabDev<float> t;
   t.frho = c.eam.frho_f.p;
-  t.rhor = c.eam.rhor_f.p;
-  t.z2r = c.eam.z2r_f.p;
+  t.nel = c.eam.nel;
   t.nr = c.eam.nr;
   t.nrho = c.eam.nrho;
   t.rdr = (float)c.eam.rdr;
@@ -435,10 +431,10 @@ EamTabDev<float> make_eam_tab<float>(Ctx& c)
   t.rdrho = (float)c.eam.rdrho;
   t.rhomax = (float)c.eam.rhomax;
   t.conv = (float)kEV;
-  // s = r^2 tables after the two knot planes of the FP32 pair table (setfl.cpp)
+  // s = r^2 tables after the knot planes of the FP32 pair table (setfl.cpp)
   const EamHost& e = c.eam;
   if (e.s_pieces > 0) {
-    const int knot_planes = 8 * (e.nr + 1);
+    const int knot_planes = 4 * (e.nel + e.nel * (e.nel + 1) / 2) * (e.nr + 1);
     t.sprows = e.s_pieces;
     t.s_force = (knot_planes + 7) / 8 * 8;
     t.s_phi = t.s_force + 8 * e.s_pieces;
@@ -452,8 +448,6 @@ EamTabDev<float> make_eam_tab<float>(Ctx& c)
     t.s_off = -1.0;
     t.s_xmax = 1.0;
   }
-  std::memcpy(t.t2rhor, c.eam.t2rhor, sizeof(t.t2rhor));
-  std::memcpy(t.t2z2r, c.eam.t2z2r, sizeof(t.t2z2r));
   std::memcpy(t.t2frho, c.eam.t2frho, sizeof(t.t2frho));
   t.types = c.eam_types;
   return t;

@@ -196,12 +196,6 @@ __device__ __forceinline__ const T* at32(const T* base, uint32_t i)
 }
 
 template <class Real>
-__device__ __forceinline__ const Real* row_r(const Real* tab, const EamTabDev<Real>& t, int which, int m)
-{
-  return at32(tab, ((uint32_t)which * (uint32_t)(t.nr + 1) + (uint32_t)m) * 8u);
-}
-
-template <class Real>
 __device__ __forceinline__ Real cubic(const Q4<Real>& c, Real p)
 {
   return ((c.a * p + c.b) * p + c.c) * p + c.d;
@@ -262,10 +256,31 @@ __device__ __forceinline__ void embed(const EamTabDev<Real>& t, int ti, double r
   Fp *= t.conv;
 }
 
-// Single-element pair table: two planes of (nr + 1) rows of 4 values, the rho value
-// cubic [c3 c4 c5 c6] of knot m at row m of plane 0 and the z2r value cubic at row m
-// of plane 1.  Rows of 4 values keep 8 (FP32) or 4 (FP64) knots per 128-byte line,
-// so the clustered knots that the lanes of a wave look up touch few lines.
+// Pair table: planes of (nr + 1) rows of 4 values, the value cubic [c3 c4 c5 c6] of knot
+// m at row m; nel planes of rho, then the nel (nel + 1) / 2 planes of z2r (one of each
+// for a single element).  Rows of 4 values keep 8 (FP32) or 4 (FP64) knots per 128-byte
+// line, so the clustered knots that the lanes of a wave look up touch few lines; the
+// derivative quadratics follow from the value cubics.
+template <class Real>
+__device__ __forceinline__ const Real* pair_row(const Real* __restrict__ pair, const EamTabDev<Real>& t, int plane,
+                                                int m)
+{
+  return at32(pair, ((uint32_t)plane * (uint32_t)(t.nr + 1) + (uint32_t)m) * 4u);
+}
+// Planes of the pair of types ti, tj (type t is element t; initialize_types_table,
+// eam_alloy.h:70-133): rho of each and their z2r, in arithmetic.  A type map is one more
+// gather ahead of every row's, and rows that also hold the derivative quadratic cost four
+// 32-byte gathers per pair instead of three: the alloy force pass of 130 k atoms (FP64,
+// energy and virial) took 134 us with both, 80 us without, the density pass 42 and 35.
+// Types past the last element take the first planes.
+__device__ __forceinline__ void pair_planes(int nel, int ti, int tj, int& rho_i, int& rho_j, int& z2r)
+{
+  const int hi = max(ti, tj), lo = min(ti, tj);
+  const bool known = hi < nel;
+  rho_i = known ? ti : 0;
+  rho_j = known ? tj : 0;
+  z2r = nel + (known ? ((hi * (hi + 1)) >> 1) + lo : 0);
+}
 template <class Real>
 __device__ __forceinline__ const Real* pair_rho_row(const Real* __restrict__ pair, int m)
 {
@@ -372,7 +387,7 @@ __device__ __forceinline__ Real eam_rho_knot(const EamTabDev<Real>& t, const Rea
   int m;
   knot_dist(t, in ? d2 : 1.0, m, p, rinv);
   const Real* row;
-  if constexpr (MULTI) row = row_r(t.rhor, t, t.t2rhor[tj + 1][ti + 1], m);
+  if constexpr (MULTI) row = pair_row(pair, t, max(ti, tj) < t.nel ? tj : 0, m);
   else row = pair_rho_row(pair, m);
   return cubic(load4(row), p);
 }
@@ -387,11 +402,13 @@ __device__ __forceinline__ void eam_pair_knot(const EamTabDev<Real>& t, const Re
   int m;
   knot_dist(t, in ? d2 : 1.0, m, p, rinv);
   if constexpr (MULTI) {
-    const Real rhoip = quad(load4(row_r(t.rhor, t, t.t2rhor[ti + 1][tj + 1], m) + 4), p);
-    const Real rhojp = quad(load4(row_r(t.rhor, t, t.t2rhor[tj + 1][ti + 1], m) + 4), p);
-    const Real* zrow = row_r(t.z2r, t, t.t2z2r[ti + 1][tj + 1], m);
-    const Real z2p = quad(load4(zrow + 4), p);
-    const Real z2 = cubic(load4(zrow), p);
+    int pi, pj, pz;
+    pair_planes(t.nel, ti, tj, pi, pj, pz);
+    const Q4<Real> zc = load4(pair_row(pair, t, pz, m));
+    const Real rhoip = dcubic(load4(pair_row(pair, t, pi, m)), p) * t.rdr;
+    const Real rhojp = dcubic(load4(pair_row(pair, t, pj, m)), p) * t.rdr;
+    const Real z2p = dcubic(zc, p) * t.rdr;
+    const Real z2 = cubic(zc, p);
     phi = z2 * rinv;
     Real phip, psip;
     if constexpr (sizeof(Real) == 4) {

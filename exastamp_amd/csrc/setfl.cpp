@@ -262,15 +262,11 @@ void eam_upload(Ctx& c)
   upload(c, e.rhor_f, cr);
   upload(c, e.z2r_f, cz);
 
-  // pair table of element 0 / pair 00 for single-element kernels: plane 0 holds the
-  // rho value cubics [c3 c4 c5 c6] of rows 0..nr, plane 1 the z2r value cubics
-  const size_t rows = (size_t)e.nr + 1;
-  std::vector<double> pair(8 * rows);
-  for (size_t m = 0; m < rows; m++)
-    for (int k = 0; k < 4; k++) {
-      pair[4 * m + k] = cr[8 * m + 3 + k];
-      pair[4 * (rows + m) + k] = cz[8 * m + 3 + k];
-    }
+  // pair table: the value cubics [c3 c4 c5 c6] of the rho rows, then of the z2r rows
+  const size_t rows = (size_t)e.nr + 1, nrows = (nel + nz) * rows;
+  std::vector<double> pair(4 * nrows);
+  for (size_t q = 0; q < nrows; q++)
+    for (int k = 0; k < 4; k++) pair[4 * q + k] = q < nel * rows ? cr[8 * q + 3 + k] : cz[8 * (q - nel * rows) + 3 + k];
   auto up = [&](auto& buf, const auto& tmp) {
     buf.reserve(tmp.size());
     XS_HIP(hipMemcpyAsync(buf.p, tmp.data(), tmp.size() * sizeof(tmp[0]), hipMemcpyHostToDevice, c.stream));
@@ -335,15 +331,15 @@ __global__ void k_spline_rows(int ntab, int n, double delta, const double* __res
   }
 }
 
-// The knot planes of the single-element pair table (rho and z2r value cubics of
-// table 0, eam_upload's layout) from the device rows, both precisions.
-__global__ void k_pair_planes(int64_t rows, const double* __restrict__ rhor, const double* __restrict__ z2r,
+// The knot planes of the pair table (rho and z2r value cubics, eam_upload's layout) from
+// the device rows, both precisions: nr rows of rho tables, nz of z2r tables.
+__global__ void k_pair_planes(int64_t nr, int64_t nz, const double* __restrict__ rhor, const double* __restrict__ z2r,
                               double* __restrict__ pair_d, float* __restrict__ pair_f)
 {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= 8 * rows) return;
-  const int64_t plane = q / (4 * rows), m = (q >> 2) - plane * rows, k = q & 3;
-  const double v = (plane == 0 ? rhor : z2r)[8 * m + k];
+  if (q >= 4 * (nr + nz)) return;
+  const int64_t m = q >> 2, k = q & 3;
+  const double v = m < nr ? rhor[8 * m + k] : z2r[8 * (m - nr) + k];
   pair_d[q] = v;
   pair_f[q] = (float)v;
 }
@@ -369,7 +365,8 @@ void eam_theta_dev(Ctx& c, const double* theta)
   spline_rows_dev(c, nel, e.nr, e.dr, r, e.rhor_d, e.rhor_f);
   spline_rows_dev(c, nz, e.nr, e.dr, z, e.z2r_d, e.z2r_f);
   const int64_t rows = (int64_t)e.nr + 1;
-  k_pair_planes<<<grid_for(8 * rows), kBlock, 0, c.stream>>>(rows, e.rhor_d.p, e.z2r_d.p, e.pair_d.p, e.pair_f.p);
+  k_pair_planes<<<grid_for(4 * (nel + nz) * rows), kBlock, 0, c.stream>>>(nel * rows, nz * rows, e.rhor_d.p,
+                                                                          e.z2r_d.p, e.pair_d.p, e.pair_f.p);
   XS_HIP(hipGetLastError());
   // the s = r^2 tables were built (and checked) from the previous knots on the host
   e.s_pieces = 0;

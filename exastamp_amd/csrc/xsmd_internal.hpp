@@ -184,13 +184,9 @@ inline double xform_det(const XformDev& x)
 template <class Real>
 struct EamTabDev {
   const Real* frho = nullptr;  // nel tables of (nrho+1) rows
-  const Real* rhor = nullptr;  // nel tables of (nr+1) rows
-  const Real* z2r = nullptr;   // nel(nel+1)/2 tables of (nr+1) rows
-  int nr = 0, nrho = 0;
+  int nel = 0, nr = 0, nrho = 0;
   Real rdr = 0, rdrho = 0, rhomax = 0, conv = 0;
   double rdr_d = 0;  // 1/dr in FP64 (the knot of r is found in FP64 in both forms)
-  int8_t t2rhor[8][8] = {};
-  int8_t t2z2r[8][8] = {};
   int8_t t2frho[8] = {};
   // types slot of eam_alloy_force: bit t set = species t takes part (alloy kernels)
   uint32_t types = ~0u;
@@ -211,9 +207,9 @@ struct EamHost {
   int8_t t2frho[8] = {};
   DBuf<double> frho_d, rhor_d, z2r_d;
   DBuf<float> frho_f, rhor_f, z2r_f;
-  // single-element pair table: plane 0 row m = rho [c3 c4 c5 c6], plane 1 row m =
-  // z2r [c3 c4 c5 c6]; the derivative quadratics follow from the value cubics, so
-  // the two planes serve both EAM passes
+  // pair table: nel rho planes, then nel (nel + 1) / 2 z2r planes, row m = [c3 c4 c5 c6]
+  // of knot m; the derivative quadratics follow from the value cubics, so the planes
+  // serve both EAM passes
   DBuf<double> pair_d;
   DBuf<float> pair_f;
   // FP32 s = r^2 tables after the knot planes of pair_f (pair_math.hpp): pieces
