@@ -17,22 +17,32 @@
 // where "slope" multiplies the derivative of the spline with respect to r (or rho).
 // rho_i and F'_i come from the forward pass (checkpointed, not recomputed).
 //
-// Each weight is spread on the four value coefficients c3..c6 of the spline row
-// it falls in (the slope coefficients c0..c2 are 3c3/D, 2c4/D, c5/D), accumulated
-// in FP64; a last kernel applies the transpose of the knot -> coefficient map.
+// Every undirected pair is taken once, from its atom with the smaller index: the two
+// list entries of a pair share r, the knot and s_ij, their z2r weights are equal, and
+// for atoms of one species so are their rho rows, so the second one costs two adds.
+//
+// A spline row is the Hermite cubic of the values f and slopes s at its two knots, so the
+// weights of a pair go to f and s of knots m and m + 1 (FP64); a last kernel applies the
+// transpose of the knot -> slope map.
 //
 // Accumulation.  All pairs of a shell fall on a few hundred rows, and all atoms on
 // a few F rows, so atomics on the gradient rows in HBM serialise.  Instead a
-// launch covers a set of row windows (slots) that fit in LDS: persistent
+// launch covers a set of row windows (one per table) that fit in LDS: persistent
 // workgroups walk all atoms (or pairs), add the contributions that fall in a window
 // into their LDS copy (LDS FP64 atomics), and write it out as a partial; a second
 // kernel sums the partials over the workgroups in a fixed order.  Windows cover
-// every row of every table, one launch per group of windows.  The first launch walks
-// the list for B1 (lambda_i stays in registers) and then B2 per atom; when every row
-// of every table fits in it (small tables) that is the whole sweep, otherwise it
-// stores lambda_i and the F-table weights for the F-row launches and the later B2
-// launches.
-#include "xsmd_internal.hpp"
+// every row of every table, one launch per group of windows.  Two sums per knot (16
+// bytes, against 32 for four coefficients per row) let the five pair tables of two
+// species at 2000 knots share one launch's 160 KB.
+//
+// The first sweep (drho_i, lambda_i) needs no accumulators and runs on the brick lists
+// like the density pass (k_block_adj_b1); the second gathers positions and loss gradients
+// through the list, since the accumulators take the LDS a brick's halo would need.
+// Bound by the LDS atomics (8 to 12 per pair) and the gathers (64 bytes per pair).
+// 1.04 M Cu/Ni atoms, 2000 knots: first sweep 233 us, second 532 us, F rows 11 us; walking
+// every list entry on the global list, with four coefficients per row and so three
+// launches, took 1107 + 2 x 645 us.  55 k atoms, 500 knots: 16 + 36 us against 80.
+#include "pair_math.hpp"
 
 #include <algorithm>
 
@@ -42,212 +52,130 @@ namespace {
 __device__ __forceinline__ int64_t lblock()
 {
   const unsigned b = blockIdx.x, g = gridDim.x;
+  if (g & 7u) return b;
   return (int64_t)(b & 7u) * (g >> 3) + (b >> 3);
-}
-
-// Only the table storage follows Real: distances, knot fractions, weights and
-// accumulations are FP64 (the sweeps are bound by gathers and atomics, and the
-// knot fraction of an FP32 r would carry the rounding of r times the knot count).
-template <class Real>
-struct AdjTab {
-  const Real* frho;  // reference layout rows [c3 c4 c5 c6 | c0 c1 c2 0]
-  const Real* rhor;
-  const Real* z2r;
-  int nr, nrho;
-  double rdr, rdrho, rhomax, conv;
-  int8_t t2rhor[8][8];
-  int8_t t2z2r[8][8];
-  int8_t t2frho[8];
-  uint32_t types;  // types slot of eam_alloy_force: bit t set = species t takes part
-};
-
-template <class Real>
-__device__ __forceinline__ bool adj_on(const AdjTab<Real>& t, int type)
-{
-  return (t.types >> type) & 1u;
 }
 
 struct AdjArgs {
   int64_t n, npad;
   const Pos4* pos;        // x y z F'_i
-  const Pos4* gvec;       // g_i (dL/dF_i) in cell order, w unused
+  Pos4* gvec;             // g_i (dL/dF_i) in cell order, w = lambda_i (first sweep out)
   const double* rho;      // checkpointed rho_i
+  double* drho;           // first sweep out
   const uint8_t* type;
   const uint16_t* rep;
   const BoxDev* box;
-  const uint32_t* nbr;
+  const uint32_t* nbr;    // global list, or
+  const uint16_t* nbr16;  // brick list: slots,
+  const uint32_t* stage;  // the global entry of each slot,
+  const uint32_t* base;   // and where the slots of atom i's brick start
   const int* nnb;
   const double* gE;       // per replica
   double rc2;
-  double* lam;            // lambda_i (B1 out, B2 in)
-  double* fc;             // F-table contribution of atom i (4 coefficients; B1 out)
-  int* fm;                // its F-table row
-  int nel;                // elements: table ids F 0..nel-1, rho nel..2nel-1, z2r 2nel..
+  int nel, nr, nrho;      // table ids: F 0..nel-1, rho nel..2nel-1, z2r 2nel..
+  double rdr, rdrho, rhomax, conv;
+  uint32_t types;         // types slot of eam_alloy_force: bit t set = species t takes part
   const XformDev* xf;     // physical displacements m * (r_j(image) - r_i) when not NULL
 };
 
-// LDS row windows of one launch: rows [lo, lo + rows) of table `table` at LDS
-// rows off .. off + rows - 1
-constexpr int kAdjSlots = 8;
-constexpr int kAdjRowsMax = 5120;  // LDS rows per launch: 32 bytes each, 160 KB at most
-constexpr int kAdjThreads = 1024;
-struct AdjSlot {
-  int table, lo, rows, off;
-  int64_t g0;  // row of the gradient array that holds row lo of the table
-};
-struct AdjSlots {
-  int n, total;
-  int stride;  // rows of one workgroup's partial
-  AdjSlot s[kAdjSlots];
-};
+__device__ __forceinline__ bool adj_on(const AdjArgs& a, int type) { return (a.types >> type) & 1u; }
+__device__ __forceinline__ int f_table(const AdjArgs& a, int type) { return type < a.nel ? type : 0; }
 
-// the four coefficient weights of a value weight wv and a slope weight ws at
-// fraction p: v = c3 p^3 + c4 p^2 + c5 p + c6, dv/dx = (3 c3 p^2 + 2 c4 p + c5) rscale
-__device__ __forceinline__ void coeff4(double wv, double ws, double p, double rscale, double (&o)[4])
+// LDS row windows of one launch: of table T the knots lo + 1 .. lo + rows at LDS rows
+// off .. off + rows - 1 (rows = 0: none)
+struct AdjWin {
+  int lo, rows, off;
+};
+constexpr int kAdjTables = 7 + 7 + 28;
+constexpr int kAdjThreads = 1024;
+struct AdjWindows {
+  int total;  // rows of the launch: as many values, then as many slopes
+  AdjWin w[kAdjTables];
+};
+__host__ __device__ inline size_t adj_lds_bytes(int total)
 {
-  const double s = ws * rscale;
-  o[0] = wv * p * p * p + s * 3.0 * p * p;
-  o[1] = wv * p * p + s * 2.0 * p;
-  o[2] = wv * p + s;
-  o[3] = wv;
+  return (size_t)total * 2 * sizeof(double) + (kAdjTables * sizeof(AdjWin) + 7) / 8 * 8;
 }
 
-// add o to row m of table T if a window of this launch holds it
-__device__ __forceinline__ void lds_add(double* acc, const AdjSlots& S, int T, int m, const double (&o)[4])
+// the accumulators of a workgroup, and the windows beside them: their lookup by table is
+// per lane
+struct AdjAcc {
+  double* f;
+  double* s;
+  const AdjWin* win;
+  int total;
+  __device__ __forceinline__ AdjAcc(double* lds, const AdjWindows& W)
+      : f(lds), s(lds + W.total), win(reinterpret_cast<const AdjWin*>(lds + 2 * W.total)), total(W.total)
+  {
+    AdjWin* w = reinterpret_cast<AdjWin*>(lds + 2 * W.total);
+    for (int k = threadIdx.x; k < kAdjTables; k += blockDim.x) w[k] = W.w[k];
+    for (int q = threadIdx.x; q < 2 * total; q += blockDim.x) lds[q] = 0.0;
+    __syncthreads();
+  }
+  __device__ __forceinline__ void out(double* __restrict__ part) const
+  {
+    __syncthreads();
+    double* dst = part + (int64_t)blockIdx.x * 2 * total;
+    for (int q = threadIdx.x; q < 2 * total; q += blockDim.x) dst[q] = f[q];
+  }
+};
+
+// Hermite basis at fraction p of knots m, m + 1: of a value weight and of the weight of
+// the derivative with respect to p
+struct Hermite {
+  double h01, h10, h11, d01, d10, d11;
+  __device__ __forceinline__ explicit Hermite(double p)
+  {
+    const double q = 1.0 - p, pq = p * q;
+    h01 = p * p * (3.0 - 2.0 * p);
+    h10 = pq * q;
+    h11 = -pq * p;
+    d01 = 6.0 * pq;
+    d10 = q * (1.0 - 3.0 * p);
+    d11 = p * (3.0 * p - 2.0);
+  }
+};
+
+// value weight wv and p-derivative weight ws at knot m (1-based) of table T
+__device__ __forceinline__ void adj_add(const AdjAcc& A, int T, int m, const Hermite& h, double wv, double ws)
 {
-  for (int k = 0; k < S.n; k++) {
-    const AdjSlot& w = S.s[k];
-    if (w.table == T && m >= w.lo && m < w.lo + w.rows) {
-      double* row = acc + 4 * (w.off + m - w.lo);
-      atomicAdd(row + 0, o[0]);
-      atomicAdd(row + 1, o[1]);
-      atomicAdd(row + 2, o[2]);
-      atomicAdd(row + 3, o[3]);
-    }
+  const AdjWin w = A.win[T];
+  const int row = m - 1 - w.lo;
+  const double f1 = wv * h.h01 + ws * h.d01;
+  if ((unsigned)row < (unsigned)w.rows) {
+    atomicAdd(A.f + w.off + row, wv - f1);
+    atomicAdd(A.s + w.off + row, wv * h.h10 + ws * h.d10);
+  }
+  if ((unsigned)(row + 1) < (unsigned)w.rows) {
+    atomicAdd(A.f + w.off + row + 1, f1);
+    atomicAdd(A.s + w.off + row + 1, wv * h.h11 + ws * h.d11);
   }
 }
 
-__device__ __forceinline__ void lds_zero(double* acc, int total)
-{
-  for (int q = threadIdx.x; q < 4 * total; q += blockDim.x) acc[q] = 0.0;
-  __syncthreads();
-}
-
-__device__ __forceinline__ void lds_out(const double* acc, const AdjSlots& S, double* __restrict__ part)
-{
-  __syncthreads();
-  double* dst = part + (int64_t)blockIdx.x * S.stride * 4;
-  for (int q = threadIdx.x; q < 4 * S.total; q += blockDim.x) dst[q] = acc[q];
-}
-
-__device__ __forceinline__ void knot(double x, double rscale, int nmax1, int mmin, int& m, double& p,
-                                     bool& clamped)
+// knot and fraction of x as the spline evaluation finds them (knots 1 .. n - 1)
+__device__ __forceinline__ void adj_knot(double x, double rscale, int n, int& m, double& p)
 {
   p = x * rscale + 1.0;
-  m = (int)p;
-  m = max(mmin, min(m, nmax1));
-  p -= (double)m;
-  clamped = p > 1.0;
-  p = fmin(p, 1.0);
+  m = max(1, min((int)p, n - 1));
+  p = fmin(p - (double)m, 1.0);
 }
 
-template <class Real>
-__device__ __forceinline__ double quad4(const Real* row, double p)
-{
-  return ((double)row[4] * p + (double)row[5]) * p + (double)row[6];
-}
-
-// B1 for atom i: drho_i and lambda_i, and the atom's F-table contribution o (four
-// coefficient weights) at row m of F table T.  L lanes share the atom (consecutive
-// lanes, sub = 0 .. L - 1, entries sub, sub + L, ...); every lane gets the results.
-template <class Real, bool MULTI, int L>
-__device__ __forceinline__ void adj_b1_atom(const AdjArgs& a, const AdjTab<Real>& t, int64_t i, int sub,
-                                            double& lam, double (&o)[4], int& m, int& T)
-{
-  const int ti = MULTI ? a.type[i] : 0;
-  const int rep = a.rep ? a.rep[i] : 0;
-  const double* Lb = a.box[rep].L;
-  const Pos4 pi = load_pos(a.pos, i);
-  const Pos4 gi = load_pos(a.gvec, i);
-  double drho = 0.0;
-  const bool oni = !MULTI || adj_on(t, ti);
-  const int cnt = oni ? a.nnb[i] : 0;
-  for (int k = sub; k < cnt; k += L) {
-    const uint32_t e = a.nbr[(int64_t)k * a.npad + i];
-    const uint32_t j = xsmd_nbr_index(e);
-    const Pos4 pj = load_pos(a.pos, j);
-    double dx = xsmd_image(pj.x, xsmd_nbr_img_x(e), Lb[0]) - pi.x;
-    double dy = xsmd_image(pj.y, xsmd_nbr_img_y(e), Lb[1]) - pi.y;
-    double dz = xsmd_image(pj.z, xsmd_nbr_img_z(e), Lb[2]) - pi.z;
-    if (a.xf) xsmd_xform_apply(a.xf->m, &dx, &dy, &dz);
-    const double d2 = xsmd_d2(dx, dy, dz);
-    if (d2 > a.rc2) continue;
-    const Pos4 gj = load_pos(a.gvec, j);
-    const double r = sqrt(d2);
-    // s_ij = u_ij . (g_i - g_j), u_ij = -(dx,dy,dz)/r
-    const double s = (dx * (gj.x - gi.x) + dy * (gj.y - gi.y) + dz * (gj.z - gi.z)) / r;
-    const int tj = MULTI ? a.type[j] : 0;
-    if (MULTI && !adj_on(t, tj)) continue;
-    int mr;
-    double p;
-    bool cl;
-    knot(r, t.rdr, t.nr - 1, 0, mr, p, cl);
-    const Real* row = t.rhor + ((int64_t)t.t2rhor[tj + 1][ti + 1] * (t.nr + 1) + mr) * 8;
-    drho += quad4(row, p) * s;
-  }
-#pragma unroll
-  for (int off = 1; off < L; off <<= 1) drho += __shfl_xor(drho, off);
-  const double rho = a.rho[i];
-  double p;
-  bool cl;
-  knot(rho, t.rdrho, t.nrho - 1, 1, m, p, cl);
-  T = t.t2frho[ti + 1];
-  const Real* row = t.frho + ((int64_t)T * (t.nrho + 1) + m) * 8;
-  // F'' = d/drho of (c0 p + c1) p + c2, zero where p was clamped
-  const double fpp = cl ? 0.0 : (2.0 * (double)row[4] * p + (double)row[5]) * t.rdrho * t.conv;
-  lam = fpp * drho;
-  const double ge = a.gE[rep];
-  const double conv = t.conv;
-  const double over = rho > t.rhomax ? rho - t.rhomax : 0.0;
-  coeff4(ge * conv, conv * (ge * over - drho), p, t.rdrho, o);
-  if (!oni) {  // a disabled species has no embedding term (lambda and drho are 0 already)
-    o[0] = o[1] = o[2] = o[3] = 0.0;
-    lam = 0.0;
-  }
-}
-
-// F-table rows: the per-atom contributions of B1 into this launch's windows
+// First sweep on the global list: kB1Lanes lanes per atom gather through it.
+constexpr int kB1Lanes = 4;
 template <class Real, bool MULTI>
-__global__ void __launch_bounds__(kAdjThreads) k_adj_fsum(AdjArgs a, AdjTab<Real> t, AdjSlots S,
-                                                          double* __restrict__ part)
+__global__ void __launch_bounds__(256) k_adj_b1(AdjArgs a, EamTabDev<Real> t, const Real* __restrict__ slope)
 {
-  extern __shared__ double acc[];
-  lds_zero(acc, S.total);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * blockDim.x) {
-    const int T = t.t2frho[(MULTI ? a.type[i] : 0) + 1];
-    const Pos4 c = load_pos(reinterpret_cast<const Pos4*>(a.fc), i);
-    const double o[4] = {c.x, c.y, c.z, c.w};
-    lds_add(acc, S, T, a.fm[i], o);
-  }
-  lds_out(acc, S, part);
-}
-
-// B2: per pair, the rho- and z2r-table gradients.
-template <class Real, bool MULTI, int L>
-__device__ __forceinline__ void adj_b2_atom(const AdjArgs& a, const AdjTab<Real>& t, const AdjSlots& S,
-                                            double* acc, int64_t i, int sub, double lam)
-{
+  const int sub = threadIdx.x % kB1Lanes;
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kB1Lanes;
+  if (i >= a.n) return;  // the lanes of an atom leave together (their shuffles)
   const int ti = MULTI ? a.type[i] : 0;
-  const int rep = a.rep ? a.rep[i] : 0;
-  const double* Lb = a.box[rep].L;
+  const double* Lb = a.box[a.rep ? a.rep[i] : 0].L;
   const Pos4 pi = load_pos(a.pos, i);
-  const Pos4 gi = load_pos(a.gvec, i);
-  const double fpi = pi.w;
-  const double ge = a.gE[rep];
-  const double conv = t.conv;
-  const double rdr = t.rdr;
-  const int cnt = (!MULTI || adj_on(t, ti)) ? a.nnb[i] : 0;
-  for (int k = sub; k < cnt; k += L) {
+  const double* gi = reinterpret_cast<const double*>(a.gvec + i);
+  const bool oni = !MULTI || adj_on(a, ti);
+  const int cnt = oni ? a.nnb[i] : 0;
+  double drho = 0.0;
+  for (int k = sub; k < cnt; k += kB1Lanes) {
     const uint32_t e = a.nbr[(int64_t)k * a.npad + i];
     const uint32_t j = xsmd_nbr_index(e);
     const Pos4 pj = load_pos(a.pos, j);
@@ -257,67 +185,164 @@ __device__ __forceinline__ void adj_b2_atom(const AdjArgs& a, const AdjTab<Real>
     if (a.xf) xsmd_xform_apply(a.xf->m, &dx, &dy, &dz);
     const double d2 = xsmd_d2(dx, dy, dz);
     if (d2 > a.rc2) continue;
-    const Pos4 gj = load_pos(a.gvec, j);
-    const double r = sqrt(d2);
-    const double s = (dx * (gj.x - gi.x) + dy * (gj.y - gi.y) + dz * (gj.z - gi.z)) / r;
     const int tj = MULTI ? a.type[j] : 0;
-    if (MULTI && !adj_on(t, tj)) continue;
+    if (MULTI && !adj_on(a, tj)) continue;
+    const double* gj = reinterpret_cast<const double*>(a.gvec + j);
+    const double r = sqrt(d2);
+    const double s = (dx * (gj[0] - gi[0]) + dy * (gj[1] - gi[1]) + dz * (gj[2] - gi[2])) / r;
     int m;
     double p;
-    bool cl;
-    knot(r, t.rdr, t.nr - 1, 0, m, p, cl);
-    double o[4];
-    coeff4(ge * fpi - lam, -fpi * s, p, rdr, o);
-    lds_add(acc, S, a.nel + t.t2rhor[tj + 1][ti + 1], m, o);
-    const double ir = 1.0 / r;
-    coeff4(conv * (0.5 * ge * ir + 0.5 * s * ir * ir), -conv * 0.5 * s * ir, p, rdr, o);
-    lds_add(acc, S, 2 * a.nel + t.t2z2r[ti + 1][tj + 1], m, o);
+    adj_knot(r, a.rdr, a.nr, m, p);
+    const pm::Q4<Real> row = pm::load4(pm::pair_row(slope, t, MULTI && max(ti, tj) < a.nel ? tj : 0, m));
+    drho += (((double)row.a * p + (double)row.b) * p + (double)row.c) * s;
   }
+#pragma unroll
+  for (int off = 1; off < kB1Lanes; off <<= 1) drho += __shfl_xor(drho, off);
+  if (sub != 0) return;
+  // F'' = d/drho of (c0 p + c1) p + c2, zero where p was clamped
+  double p = a.rho[i] * a.rdrho + 1.0;
+  const int m = max(1, min((int)p, a.nrho - 1));
+  p -= (double)m;
+  const Real* row = t.frho + ((int64_t)f_table(a, ti) * (a.nrho + 1) + m) * 8;
+  const double fpp = p > 1.0 ? 0.0 : (2.0 * (double)row[4] * p + (double)row[5]) * a.rdrho * a.conv;
+  a.drho[i] = drho;
+  reinterpret_cast<double*>(a.gvec + i)[3] = oni ? fpp * drho : 0.0;
 }
 
-template <class Real, bool MULTI>
-__global__ void __launch_bounds__(kAdjThreads) k_adj_b2(AdjArgs a, AdjTab<Real> t, AdjSlots S,
-                                                        double* __restrict__ part)
+// The F-table weights of atom i (a disabled species has no embedding term)
+template <bool MULTI>
+__device__ __forceinline__ void adj_embed_add(const AdjArgs& a, const AdjAcc& acc, int64_t i)
 {
-  extern __shared__ double acc[];
-  lds_zero(acc, S.total);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * blockDim.x)
-    adj_b2_atom<Real, MULTI, 1>(a, t, S, acc, i, 0, a.lam[i]);
-  lds_out(acc, S, part);
+  const int ti = MULTI ? a.type[i] : 0;
+  if (MULTI && !adj_on(a, ti)) return;
+  const double rho = a.rho[i], ge = a.gE[a.rep ? a.rep[i] : 0];
+  int m;
+  double p;
+  adj_knot(rho, a.rdrho, a.nrho, m, p);
+  const double over = rho > a.rhomax ? rho - a.rhomax : 0.0;
+  adj_add(acc, f_table(a, ti), m, Hermite(p), ge * a.conv, a.conv * (ge * over - a.drho[i]) * a.rdrho);
 }
 
-// B1 and B2 in one launch, kFusedLanes lanes per atom walking its list twice: B1
-// (lambda_i kept in registers), then B2 into this launch's windows.  When the rows of
-// every table fit the launch (small tables, small systems) the F-table contribution
-// goes into LDS too and this is the whole sweep; with STORE (the first of several
-// launches) lambda_i and the F-table contribution are stored for k_adj_fsum and the
-// later k_adj_b2 launches instead, so the list is walked once less.
-constexpr int kFusedLanes = 4;
-template <class Real, bool MULTI, bool STORE>
-__global__ void __launch_bounds__(kAdjThreads) k_adj_fused(AdjArgs a, AdjTab<Real> t, AdjSlots S,
+// F-table rows where they have launches of their own
+template <bool MULTI>
+__global__ void __launch_bounds__(kAdjThreads) k_adj_fsum(AdjArgs a, AdjWindows W, double* __restrict__ part)
+{
+  extern __shared__ double lds[];
+  const AdjAcc acc(lds, W);
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * blockDim.x)
+    adj_embed_add<MULTI>(a, acc, i);
+  acc.out(part);
+}
+
+// Second sweep: the rho and z2r rows of every pair, from its atom with the smaller index
+// (an atom's own images come as two entries, which take half each), and with FSUM the
+// F-table rows.  1 << lanes_log lanes per atom.  A lane first marks which of its entries
+// are its to take, up to 64 of them, then walks the marked ones, so that lanes whose
+// neighbour had the larger index do not idle through the pair's arithmetic.
+template <bool MULTI, bool BLOCK, bool FSUM>
+__global__ void __launch_bounds__(kAdjThreads) k_adj_pairs(AdjArgs a, AdjWindows W, int lanes_log,
                                                            double* __restrict__ part)
 {
-  extern __shared__ double acc[];
-  lds_zero(acc, S.total);
-  const int sub = threadIdx.x % kFusedLanes;
-  const int64_t step = (int64_t)gridDim.x * (blockDim.x / kFusedLanes);
-  // the lanes of an atom share i, so they leave the loop together (their shuffles)
-  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kFusedLanes; i < a.n; i += step) {
-    double lam, o[4];
-    int m, T;
-    adj_b1_atom<Real, MULTI, kFusedLanes>(a, t, i, sub, lam, o, m, T);
-    if constexpr (STORE) {
-      if (sub == 0) {
-        a.lam[i] = lam;
-        store_pos(reinterpret_cast<Pos4*>(a.fc), i, Pos4{o[0], o[1], o[2], o[3]});
-        a.fm[i] = m;
+  extern __shared__ double lds[];
+  const AdjAcc acc(lds, W);
+  const int lanes = 1 << lanes_log, sub = threadIdx.x & (lanes - 1);
+  // a contiguous range of atoms per workgroup, neighbouring ranges on one XCD
+  const int64_t per = (a.n + gridDim.x - 1) / gridDim.x;
+  const int64_t first = lblock() * per, end = min(first + per, a.n);
+  for (int64_t i = first + (threadIdx.x >> lanes_log); i < end; i += blockDim.x >> lanes_log) {
+    if (FSUM && sub == 0) adj_embed_add<MULTI>(a, acc, i);
+    const int ti = MULTI ? a.type[i] : 0;
+    const int rep = a.rep ? a.rep[i] : 0;
+    const double* Lb = a.box[rep].L;
+    const Pos4 pi = load_pos(a.pos, i);
+    const Pos4 gi = load_pos(a.gvec, i);
+    const double ge = a.gE[rep];
+    const int cnt = (!MULTI || adj_on(a, ti)) ? a.nnb[i] : 0;
+    const uint32_t base = BLOCK ? a.base[i] : 0;
+    // bit 8 t + u of a lane's mask: place u of its t-th group (BLOCK), or its (8 t + u)-th entry
+    for (int k0 = 0; k0 < cnt; k0 += 64 * lanes) {
+      unsigned long long mask = 0;
+      for (int t = 0; t < 8; t++) {
+        if constexpr (BLOCK) {
+          const int g = (k0 >> 3) + sub + lanes * t;
+          if (8 * g >= cnt) break;
+          const uint4 w = *reinterpret_cast<const uint4*>(a.nbr16 + (((int64_t)g * a.npad + i) << 3));
+          const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int u = 0; u < 8; u++) {
+            const int k = 8 * g + (u < 4 ? 2 * u : 2 * u - 7);
+            const uint32_t slot = u & 1 ? ws[u >> 1] >> 16 : ws[u >> 1] & 0xffffu;
+            const uint32_t j = xsmd_nbr_index(a.stage[base + (k < cnt ? slot : 0u)]);
+            if (k < cnt && (int64_t)j >= i) mask |= 1ull << (8 * t + u);
+          }
+        } else {
+          for (int u = 0; u < 8; u++) {
+            const int k = k0 + sub + lanes * (8 * t + u);
+            if (k < cnt && (int64_t)xsmd_nbr_index(a.nbr[(int64_t)k * a.npad + i]) >= i) mask |= 1ull << (8 * t + u);
+          }
+        }
       }
-    } else {
-      if (sub == 0) lds_add(acc, S, T, m, o);
+      while (mask) {
+        const int bit = __ffsll(mask) - 1;
+        mask &= mask - 1;
+        uint32_t e;
+        if constexpr (BLOCK) {
+          const int g = (k0 >> 3) + sub + lanes * (bit >> 3);
+          e = a.stage[base + a.nbr16[(((int64_t)g * a.npad + i) << 3) + (bit & 7)]];
+        } else {
+          e = a.nbr[(int64_t)(k0 + sub + lanes * bit) * a.npad + i];
+        }
+        const uint32_t j = xsmd_nbr_index(e);
+        const int tj = MULTI ? a.type[j] : 0;
+        if (MULTI && !adj_on(a, tj)) continue;
+        const Pos4 pj = load_pos(a.pos, j);
+        const Pos4 gj = load_pos(a.gvec, j);
+        const int kx = xsmd_nbr_img_x(e), ky = xsmd_nbr_img_y(e), kz = xsmd_nbr_img_z(e);
+        double dx = xsmd_image(pj.x, kx, Lb[0]) - pi.x;
+        double dy = xsmd_image(pj.y, ky, Lb[1]) - pi.y;
+        double dz = xsmd_image(pj.z, kz, Lb[2]) - pi.z;
+        if (a.xf) xsmd_xform_apply(a.xf->m, &dx, &dy, &dz);
+        const double d2 = xsmd_d2(dx, dy, dz);
+        // wi, wj: which of the pair's two entries count; through an image the distance
+        // from j rounds by itself, so a pair at the cutoff may count from one side only
+        double wi = d2 <= a.rc2 ? 1.0 : 0.0, wj = wi;
+        if ((kx | ky | kz) != 0) {
+          double ux = xsmd_image(pi.x, -kx, Lb[0]) - pj.x;
+          double uy = xsmd_image(pi.y, -ky, Lb[1]) - pj.y;
+          double uz = xsmd_image(pi.z, -kz, Lb[2]) - pj.z;
+          if (a.xf) xsmd_xform_apply(a.xf->m, &ux, &uy, &uz);
+          wj = xsmd_d2(ux, uy, uz) <= a.rc2 ? 1.0 : 0.0;
+          if ((int64_t)j == i) {
+            wi *= 0.5;
+            wj *= 0.5;
+          }
+        }
+        const double both = wi + wj;
+        if (both == 0.0) continue;
+        const double r = sqrt(d2), ir = 1.0 / r;
+        // s_ij = u_ij . (g_i - g_j), u_ij = -(dx,dy,dz)/r
+        const double s = (dx * (gj.x - gi.x) + dy * (gj.y - gi.y) + dz * (gj.z - gi.z)) * ir;
+        int m;
+        double p;
+        adj_knot(r, a.rdr, a.nr, m, p);
+        const Hermite h(p);
+        int ri = 0, rj = 0, z = a.nel;
+        if constexpr (MULTI) pm::pair_planes(a.nel, ti, tj, ri, rj, z);
+        const double srdr = s * a.rdr;
+        const double vi = wi * (ge * pi.w - gi.w), vj = wj * (ge * pj.w - gj.w);
+        const double si = -wi * pi.w * srdr, sj = -wj * pj.w * srdr;
+        if (!MULTI || ri == rj) {
+          adj_add(acc, a.nel + ri, m, h, vi + vj, si + sj);
+        } else {
+          adj_add(acc, a.nel + rj, m, h, vi, si);  // rho_j's table at atom i
+          adj_add(acc, a.nel + ri, m, h, vj, sj);
+        }
+        const double c = 0.5 * both * a.conv * ir;
+        adj_add(acc, a.nel + z, m, h, c * (ge + s * ir), -c * srdr);
+      }
     }
-    adj_b2_atom<Real, MULTI, kFusedLanes>(a, t, S, acc, i, sub, lam);
   }
-  lds_out(acc, S, part);
+  acc.out(part);
 }
 
 // Sum of the partials of `groups` workgroups into the gradient rows of this launch's
@@ -326,33 +351,40 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_fused(AdjArgs a, AdjTab<Rea
 // (coalesced), and the 16 sums are added in wave order, so the result does not
 // depend on scheduling.
 constexpr int kRedThreads = 1024;
-__global__ void __launch_bounds__(kRedThreads) k_adj_reduce(AdjSlots S, int groups, const double* __restrict__ part,
-                                                            double* __restrict__ g)
+__global__ void __launch_bounds__(kRedThreads) k_adj_reduce(AdjWindows W, int nel, int nz, int nrho, int nr, int groups,
+                                                            const double* __restrict__ part, double* __restrict__ g)
 {
   __shared__ double red[kRedThreads];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int q = blockIdx.x * 64 + lane;
-  const bool in = q < 4 * S.total;
+  const bool in = q < 2 * W.total;
   double v = 0.0;
   if (in)
-    for (int w = wave; w < groups; w += kRedThreads / 64) v += part[(int64_t)w * S.stride * 4 + q];
+    for (int w = wave; w < groups; w += kRedThreads / 64) v += part[(int64_t)w * 2 * W.total + q];
   red[threadIdx.x] = v;
   __syncthreads();
   if (wave != 0 || !in) return;
   v = red[lane];
   for (int k = 1; k < kRedThreads / 64; k++) v += red[k * 64 + lane];
-  const int row = q >> 2;
-  int k = 0;
-  while (k + 1 < S.n && row >= S.s[k + 1].off) k++;
-  g[(S.s[k].g0 + row - S.s[k].off) * 4 + (q & 3)] = v;
+  const bool slope = q >= W.total;
+  const int row = slope ? q - W.total : q;
+  const int64_t knots = (int64_t)nel * nrho + (int64_t)(nel + nz) * nr;
+  for (int T = 0; T < 2 * nel + nz; T++) {
+    const AdjWin w = W.w[T];
+    if (row < w.off || row >= w.off + w.rows) continue;
+    const int64_t g0 = T < nel ? (int64_t)T * nrho : (int64_t)nel * nrho + (int64_t)(T - nel) * nr;
+    g[(slope ? knots : 0) + g0 + w.lo + row - w.off] = v;
+  }
 }
+
 // g (dL/dF) from id order into cell order as position-like records
-// (and times `scale`); the first nrep threads scale the per-replica dL/dE copy in place
+// (and times `scale`); the first nrep threads scale the per-replica dL/dE
 __global__ void k_gather_g(int64_t n, const int64_t* __restrict__ id, const double* __restrict__ g_id,
-                           Pos4* __restrict__ gvec, double scale, double* __restrict__ gE, int nrep)
+                           Pos4* __restrict__ gvec, double scale, const double* __restrict__ gE_in,
+                           double* __restrict__ gE, int nrep)
 {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nrep) gE[i] *= scale;
+  if (i < nrep) gE[i] = gE_in[i] * scale;
   if (i >= n) return;
   const int64_t q = id[i];
   store_pos(gvec, i, Pos4{g_id[3 * q] * scale, g_id[3 * q + 1] * scale, g_id[3 * q + 2] * scale, 0.0});
@@ -467,120 +499,100 @@ __global__ void __launch_bounds__(kLjAdjThreads) k_lj_adjoint_reduce(int64_t npa
   }
 }
 
-template <class Real>
-AdjTab<Real> adj_tab(Ctx& c);
-
-template <>
-AdjTab<double> adj_tab<double>(Ctx& c)
+// Row windows of every table (F tables have nrho knots, rho and z2r tables nr), packed
+// into launches of at most `limit` LDS rows; `what` selects the F tables (0), the rho and
+// z2r tables (1) or all of them (2).
+std::vector<AdjWindows> adj_launches(int nel, int nz, int nrho, int nr, int what, int limit)
 {
-  AdjTab<double> t;
-  t.frho = c.eam.frho_d.p;
-  t.rhor = c.eam.rhor_d.p;
-  t.z2r = c.eam.z2r_d.p;
-  t.rdr = c.eam.rdr;
-  t.rdrho = c.eam.rdrho;
-  t.rhomax = c.eam.rhomax;
-  t.conv = kEV;
-  t.nr = c.eam.nr;
-  t.nrho = c.eam.nrho;
-  std::memcpy(t.t2rhor, c.eam.t2rhor, sizeof(t.t2rhor));
-  std::memcpy(t.t2z2r, c.eam.t2z2r, sizeof(t.t2z2r));
-  std::memcpy(t.t2frho, c.eam.t2frho, sizeof(t.t2frho));
-  t.types = c.eam_types;
-  return t;
-}
-
-template <>
-AdjTab<float> adj_tab<float>(Ctx& c)
-{
-  AdjTab<float> t;
-  t.frho = c.eam.frho_f.p;
-  t.rhor = c.eam.rhor_f.p;
-  t.z2r = c.eam.z2r_f.p;
-  t.rdr = c.eam.rdr;
-  t.rdrho = c.eam.rdrho;
-  t.rhomax = c.eam.rhomax;
-  t.conv = kEV;
-  t.nr = c.eam.nr;
-  t.nrho = c.eam.nrho;
-  std::memcpy(t.t2rhor, c.eam.t2rhor, sizeof(t.t2rhor));
-  std::memcpy(t.t2z2r, c.eam.t2z2r, sizeof(t.t2z2r));
-  std::memcpy(t.t2frho, c.eam.t2frho, sizeof(t.t2frho));
-  t.types = c.eam_types;
-  return t;
-}
-
-// Row windows of every table (F tables use their rows_f rows, rho and z2r tables
-// rows_r), packed into launches of at most `limit` LDS rows and kAdjSlots windows;
-// `what` selects the F tables (0), the rho and z2r tables (1) or all of them (2).
-std::vector<AdjSlots> adj_launches(int nel, int nz, int64_t rows_f, int64_t rows_r, int what, int limit)
-{
-  std::vector<AdjSlots> out;
-  AdjSlots cur{};
-  cur.stride = limit;
-  auto add = [&](int T, int64_t rows, int64_t g0) {
-    for (int64_t lo = 0; lo < rows; lo += limit) {
-      const int w = (int)std::min<int64_t>(limit, rows - lo);
-      if (cur.n == kAdjSlots || cur.total + w > limit) {
+  std::vector<AdjWindows> out;
+  AdjWindows cur{};
+  const auto add = [&](int T, int rows) {
+    for (int lo = 0; lo < rows;) {
+      if (cur.total == limit) {
         out.push_back(cur);
-        cur = AdjSlots{};
-        cur.stride = limit;
+        cur = AdjWindows{};
       }
-      cur.s[cur.n++] = AdjSlot{T, (int)lo, w, cur.total, g0 + lo};
+      const int w = std::min(limit - cur.total, rows - lo);
+      cur.w[T] = AdjWin{lo, w, cur.total};
       cur.total += w;
+      lo += w;
     }
   };
-  const int64_t f_end = nel * rows_f;
   if (what != 1)
-    for (int t = 0; t < nel; t++) add(t, rows_f, t * rows_f);
-  if (what != 0) {
-    for (int t = 0; t < nel; t++) add(nel + t, rows_r, f_end + t * rows_r);
-    for (int t = 0; t < nz; t++) add(2 * nel + t, rows_r, f_end + (nel + t) * rows_r);
-  }
-  if (cur.n) out.push_back(cur);
+    for (int t = 0; t < nel; t++) add(t, nrho);
+  if (what != 0)
+    for (int t = 0; t < nel + nz; t++) add(nel + t, nr);
+  if (cur.total) out.push_back(cur);
   return out;
 }
 
 template <class Real>
-void adj_run(Ctx& c, const AdjArgs& a)
+void adj_first_sweep(Ctx& c, const AdjArgs& a)
 {
-  const AdjTab<Real> t = adj_tab<Real>(c);
+  const Real* slope;
+  if constexpr (sizeof(Real) == 4) slope = c.eam.slope_f.p;
+  else slope = c.eam.slope_d.p;
+  const auto k = eam_multi(c) ? k_adj_b1<Real, true> : k_adj_b1<Real, false>;
+  k<<<grid_for(a.n * kB1Lanes), 256, 0, c.stream>>>(a, make_eam_tab<Real>(c), slope);
+  XS_HIP(hipGetLastError());
+}
+
+void adj_run(Ctx& c, const AdjArgs& a, double rcut, bool mixed)
+{
   EamHost& e = c.eam;
   const int nel = e.nel, nz = nel * (nel + 1) / 2;
-  const int64_t rows_f = e.nrho + 1, rows_r = e.nr + 1;
-  const bool multi = eam_multi(c);
-  // LDS windows as large as one workgroup may hold; persistent workgroups, as many as
-  // fit on the CUs at the launch's LDS size (1024 threads each, 256 for systems too
-  // small to give every CU 1024 atoms), but no more than the atoms fill
-  const int limit = (int)std::min<size_t>(kAdjRowsMax, c.lds_max / (4 * sizeof(double)));
-  const int cus = std::max(c.num_cu, 1);
-  auto run = [&](auto k, AdjSlots S, int lanes) {
-    const int64_t items = c.n * lanes;
-    const int threads = items >= (int64_t)cus * kAdjThreads ? kAdjThreads : 256;
-    const size_t lds = (size_t)S.total * 4 * sizeof(double);
-    const int64_t per_cu = std::max<int64_t>(1, (int64_t)(c.lds_max / lds));
-    const int groups = (int)std::max<int64_t>(1, std::min<int64_t>(cus * per_cu, (items + threads - 1) / threads));
-    S.stride = S.total;
-    c.adj_part.reserve((size_t)groups * S.stride * 4);
-    XS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)lds));
-    k<<<groups, threads, lds, c.stream>>>(a, t, S, c.adj_part.p);
+  const bool multi = eam_multi(c), block = a.nbr16 != nullptr;
+  if (block) launch_adj_b1_block(c, rcut, mixed);
+  else if (mixed) adj_first_sweep<float>(c, a);
+  else adj_first_sweep<double>(c, a);
+  // LDS windows as large as one workgroup may hold; one persistent workgroup per CU, of
+  // 256 to 1024 threads as the atoms fill them: more of them would each write and have
+  // summed a copy of the rows (864 workgroups of 256 threads at 55 k atoms and 1500 rows
+  // made the sum of the partials 17 us)
+  const int limit = (int)((c.lds_max - adj_lds_bytes(0)) / (2 * sizeof(double)));
+  const int64_t cus = std::max(c.num_cu, 1);
+  const auto shape = [&](int64_t items, int& groups, int& threads) {
+    threads = 256;
+    while (threads < kAdjThreads && items > cus * threads) threads *= 2;
+    groups = (int)std::max<int64_t>(1, std::min<int64_t>(cus, (items + threads - 1) / threads));
+  };
+  const auto reduce = [&](const AdjWindows& W, int groups) {
     XS_HIP(hipGetLastError());
-    k_adj_reduce<<<(unsigned)((4 * S.total + 63) / 64), kRedThreads, 0, c.stream>>>(S, groups, c.adj_part.p,
-                                                                                      c.adj_g.p);
+    k_adj_reduce<<<(unsigned)((2 * W.total + 63) / 64), kRedThreads, 0, c.stream>>>(
+        W, nel, nz, e.nrho, e.nr, groups, c.adj_part.p, c.adj_g.p);
     XS_HIP(hipGetLastError());
   };
-  const std::vector<AdjSlots> all = adj_launches(nel, nz, rows_f, rows_r, 2, limit);
-  if (all.size() == 1) {  // every row fits: one sweep of the list
-    run(multi ? k_adj_fused<Real, true, false> : k_adj_fused<Real, false, false>, all[0], kFusedLanes);
+  const auto launch = [&](auto k, const AdjWindows& W, int64_t items, auto... args) {
+    int groups, threads;
+    shape(items, groups, threads);
+    const size_t lds = adj_lds_bytes(W.total);
+    c.adj_part.reserve((size_t)groups * 2 * W.total);
+    XS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds));
+    k<<<groups, threads, lds, c.stream>>>(a, W, args..., c.adj_part.p);
+    reduce(W, groups);
+  };
+  // lanes per atom: 2, more where the atoms do not fill the CUs
+  int lanes_log = 1;
+  while (lanes_log < 3 && (a.n << lanes_log) < cus * kAdjThreads * 3 / 4) lanes_log++;
+  const auto pairs = [&](const AdjWindows& W, bool fsum) {
+    const auto pick = [&](auto m, auto b) {
+      constexpr bool M = decltype(m)::value, B = decltype(b)::value;
+      launch(fsum ? k_adj_pairs<M, B, true> : k_adj_pairs<M, B, false>, W, a.n << lanes_log, lanes_log);
+    };
+    if (multi && block) pick(std::true_type{}, std::true_type{});
+    else if (multi) pick(std::true_type{}, std::false_type{});
+    else if (block) pick(std::false_type{}, std::true_type{});
+    else pick(std::false_type{}, std::false_type{});
+  };
+  const std::vector<AdjWindows> all = adj_launches(nel, nz, e.nrho, e.nr, 2, limit);
+  if (all.size() == 1) {  // every row fits: one launch
+    pairs(all[0], true);
     return;
   }
-  // B1 with the first window set of the pair tables, then the F tables, then the rest
-  const std::vector<AdjSlots> pairs = adj_launches(nel, nz, rows_f, rows_r, 1, limit);
-  run(multi ? k_adj_fused<Real, true, true> : k_adj_fused<Real, false, true>, pairs[0], kFusedLanes);
-  for (const AdjSlots& S : adj_launches(nel, nz, rows_f, rows_r, 0, limit))
-    run(multi ? k_adj_fsum<Real, true> : k_adj_fsum<Real, false>, S, 1);
-  for (size_t k = 1; k < pairs.size(); k++) run(multi ? k_adj_b2<Real, true> : k_adj_b2<Real, false>, pairs[k], 1);
+  for (const AdjWindows& W : adj_launches(nel, nz, e.nrho, e.nr, 1, limit)) pairs(W, false);
+  for (const AdjWindows& W : adj_launches(nel, nz, e.nrho, e.nr, 0, limit))
+    launch(multi ? k_adj_fsum<true> : k_adj_fsum<false>, W, a.n);
 }
 
 }  // namespace
@@ -629,58 +641,33 @@ void spline_interpolate_adjoint(int n, double delta, const double* G, double* ou
 
 namespace {
 
-// Gather form of spline_interpolate_adjoint for every table at once: one thread per
-// knot k (1-based) of table t sums the rows' value-coefficient gradients G (4 per
-// row, dL/d(c3, c4, c5, c6)) that depend on knot k, directly (c6 = f, and f in
-// c3, c4 of rows k and k - 1) and through the slopes s[m] of rows m = k - 2 .. k + 2.
-__device__ __forceinline__ double adj_gs(const double* __restrict__ G, int n, int m)
-{
-  // dL/ds[m]: c5 of row m, c4 and c3 of row m (s[m]) and of row m - 1 (s[m + 1] there)
-  double v = G[4 * m + 2];
-  if (m <= n - 1) v += -2.0 * G[4 * m + 1] + G[4 * m + 0];
-  if (m >= 2) v += -G[4 * (m - 1) + 1] + G[4 * (m - 1) + 0];
-  return v;
-}
-
+// dL/dknots of every table from the sums over the pairs and atoms: G holds dL/df then
+// dL/ds of every knot.  One thread per knot k (1-based) of its table: f[k] itself, and
+// through the slopes s[m] of the knots m = k - 2 .. k + 2 (the transpose of
+// spline_interpolate's slope map).
 __global__ void k_spline_adjoint(int nel, int nz, int nrho, int nr, const double* __restrict__ G,
                                  double* __restrict__ grad)
 {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t kf = (int64_t)nel * nrho, kr = (int64_t)nel * nr, kz = (int64_t)nz * nr;
-  if (q >= kf + kr + kz) return;
-  int n;
-  int64_t t, k0;
-  const double* g;
-  if (q < kf) {
-    n = nrho;
-    t = q / nrho;
-    k0 = q - t * nrho;
-    g = G + t * (nrho + 1) * 4;
-  } else {
-    const int64_t u = q - kf;
-    n = nr;
-    t = u / nr;
-    k0 = u - t * nr;
-    g = G + (kf + (int64_t)nel) * 4 + t * (nr + 1) * 4;  // the F tables' rows, then nel + nz tables of nr + 1
-  }
-  const int k = (int)k0 + 1;
-  // direct: c6 = f[k]; c4, c3 of row k (-3, +2) and of row k - 1 (+3, -2)
-  double v = g[4 * k + 3];
-  if (k <= n - 1) v += -3.0 * g[4 * k + 1] + 2.0 * g[4 * k + 0];
-  if (k >= 2) v += 3.0 * g[4 * (k - 1) + 1] - 2.0 * g[4 * (k - 1) + 0];
-  // through the slopes
-  if (k == 2) v += adj_gs(g, n, 1);
-  if (k == 1) v -= adj_gs(g, n, 1) + 0.5 * adj_gs(g, n, 2);
-  if (k == 3) v += 0.5 * adj_gs(g, n, 2);
-  if (k == n) v += 0.5 * adj_gs(g, n, n - 1) + adj_gs(g, n, n);
-  if (k == n - 2) v -= 0.5 * adj_gs(g, n, n - 1);
-  if (k == n - 1) v -= adj_gs(g, n, n);
+  const int64_t kf = (int64_t)nel * nrho, knots = kf + (int64_t)(nel + nz) * nr;
+  if (q >= knots) return;
+  const int n = q < kf ? nrho : nr;
+  const int64_t t0 = q < kf ? q / nrho * nrho : kf + (q - kf) / nr * nr;  // the table's first knot
+  const int k = (int)(q - t0) + 1;
+  const double* gs = G + knots + t0 - 1;  // slopes, 1-based
+  double v = G[q];
+  if (k == 2) v += gs[1];
+  if (k == 1) v -= gs[1] + 0.5 * gs[2];
+  if (k == 3) v += 0.5 * gs[2];
+  if (k == n) v += 0.5 * gs[n - 1] + gs[n];
+  if (k == n - 2) v -= 0.5 * gs[n - 1];
+  if (k == n - 1) v -= gs[n];
   // interior slopes m in [3, n - 2]: f[m - 2] +w, f[m + 2] -w, f[m + 1] +8w, f[m - 1] -8w
   const auto interior = [&](int m) { return m >= 3 && m <= n - 2; };
-  if (interior(k + 2)) v += adj_gs(g, n, k + 2) / 12.0;
-  if (interior(k - 2)) v -= adj_gs(g, n, k - 2) / 12.0;
-  if (interior(k - 1)) v += 8.0 * (adj_gs(g, n, k - 1) / 12.0);
-  if (interior(k + 1)) v -= 8.0 * (adj_gs(g, n, k + 1) / 12.0);
+  if (interior(k + 2)) v += gs[k + 2] / 12.0;
+  if (interior(k - 2)) v -= gs[k - 2] / 12.0;
+  if (interior(k - 1)) v += 8.0 * (gs[k - 1] / 12.0);
+  if (interior(k + 1)) v -= 8.0 * (gs[k + 1] / 12.0);
   grad[q] = v;
 }
 
@@ -689,50 +676,59 @@ __global__ void k_spline_adjoint(int nel, int nz, int nrho, int nr, const double
 void eam_adjoint(Ctx& c, double rcut, const double* dLdF_id, const double* dLdE, double scale, double* grad,
                  bool mixed, bool device)
 {
-  ensure_global_list(c);
   EamHost& e = c.eam;
   const int nel = e.nel, nz = nel * (nel + 1) / 2;
-  const size_t rows_r = (size_t)e.nr + 1, rows_f = (size_t)e.nrho + 1;
-  const size_t nF = (size_t)nel * rows_f * 4, nR = (size_t)nel * rows_r * 4, nZ = (size_t)nz * rows_r * 4;
   const size_t nknots = (size_t)nel * e.nrho + (size_t)(nel + nz) * e.nr;
-  c.adj_g.reserve(nF + nR + nZ);
-  c.adj_lam.reserve(c.npad);
+  c.adj_g.reserve(2 * nknots);
   c.adj_gvec.reserve(c.npad);
-  c.adj_in.reserve(3 * (size_t)c.n + c.nrep);
+  c.adj_drho.reserve(c.npad);
+  c.adj_gE.reserve(c.nrep);
   if (!device) c.adj_grad.reserve(nknots);
-  const hipMemcpyKind in_kind = device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-  XS_HIP(hipMemsetAsync(c.adj_g.p, 0, sizeof(double) * (nF + nR + nZ), c.stream));
-  XS_HIP(hipMemcpyAsync(c.adj_in.p, dLdF_id, sizeof(double) * 3 * c.n, in_kind, c.stream));
-  XS_HIP(hipMemcpyAsync(c.adj_in.p + 3 * c.n, dLdE, sizeof(double) * c.nrep, in_kind, c.stream));
+  const double *gF = dLdF_id, *gE = dLdE;  // on the device
+  if (!device) {
+    c.adj_in.reserve(3 * (size_t)c.n + c.nrep);
+    XS_HIP(hipMemcpyAsync(c.adj_in.p, dLdF_id, sizeof(double) * 3 * c.n, hipMemcpyHostToDevice, c.stream));
+    XS_HIP(hipMemcpyAsync(c.adj_in.p + 3 * c.n, dLdE, sizeof(double) * c.nrep, hipMemcpyHostToDevice, c.stream));
+    gF = c.adj_in.p;
+    gE = c.adj_in.p + 3 * c.n;
+  }
   if (c.n > 0) {
     k_gather_g<<<grid_for(std::max<int64_t>(c.n, c.nrep)), kBlock, 0, c.stream>>>(
-        c.n, c.id.p, c.adj_in.p, c.adj_gvec.p, scale, c.adj_in.p + 3 * c.n, c.nrep);
+        c.n, c.id.p, gF, c.adj_gvec.p, scale, gE, c.adj_gE.p, c.nrep);
     XS_HIP(hipGetLastError());
+    const bool block = c.list_kind == ListKind::Block;
     AdjArgs a;
     a.n = c.n;
     a.npad = c.npad;
     a.pos = c.pos.p;
     a.gvec = c.adj_gvec.p;
     a.rho = c.rho.p;
+    a.drho = c.adj_drho.p;
     a.type = c.type.p;
     a.rep = c.has_rep ? c.rep.p : nullptr;
     a.box = c.box_d.p;
-    a.nbr = c.nbr.p;
+    a.nbr = block ? nullptr : c.nbr.p;
+    a.nbr16 = block ? c.nbr16.p : nullptr;
+    a.stage = c.brick_stage.p;
+    a.base = c.atom_stage.p;
     a.nnb = c.nnb.p;
-    a.gE = c.adj_in.p + 3 * c.n;
+    a.gE = c.adj_gE.p;
     a.rc2 = rcut * rcut;
-    a.lam = c.adj_lam.p;
-    c.adj_fc.reserve(4 * (size_t)c.npad);
-    c.adj_fm.reserve(c.npad);
-    a.fc = c.adj_fc.p;
-    a.fm = c.adj_fm.p;
     a.nel = nel;
+    a.nr = e.nr;
+    a.nrho = e.nrho;
+    a.rdr = e.rdr;
+    a.rdrho = e.rdrho;
+    a.rhomax = e.rhomax;
+    a.conv = kEV;
+    a.types = c.eam_types;
     a.xf = c.xf_dev();
     ProfScope prof(c.prof, c.stream, XS_PROF_ADJOINT);
-    if (mixed) adj_run<float>(c, a);
-    else adj_run<double>(c, a);
+    adj_run(c, a, rcut, mixed);
+  } else {
+    XS_HIP(hipMemsetAsync(c.adj_g.p, 0, sizeof(double) * 2 * nknots, c.stream));
   }
-  // dL/dtheta: the transpose of the knot -> coefficient map, on the device
+  // dL/dtheta: the transpose of the knot -> slope map, on the device
   double* out = device ? grad : c.adj_grad.p;
   k_spline_adjoint<<<grid_for((int64_t)nknots), kBlock, 0, c.stream>>>(nel, nz, e.nrho, e.nr, c.adj_g.p, out);
   XS_HIP(hipGetLastError());
@@ -754,7 +750,7 @@ void lj_adjoint(Ctx& c, double eps, double sigma, double rcut, const double* dLd
   XS_HIP(hipMemcpyAsync(c.adj_in.p + 3 * c.n, dLdE, sizeof(double) * c.nrep, hipMemcpyHostToDevice, c.stream));
   double* out = c.adj_part.p + 2 * (size_t)std::max(g, 1u);
   if (c.n > 0) {
-    k_gather_g<<<grid_for(c.n), kBlock, 0, c.stream>>>(c.n, c.id.p, c.adj_in.p, c.adj_gvec.p, 1.0, nullptr, 0);
+    k_gather_g<<<grid_for(c.n), kBlock, 0, c.stream>>>(c.n, c.id.p, c.adj_in.p, c.adj_gvec.p, 1.0, nullptr, nullptr, 0);
     XS_HIP(hipGetLastError());
     LjAdjArgs a;
     a.n = c.n;

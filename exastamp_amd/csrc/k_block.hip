@@ -375,17 +375,6 @@ __device__ __forceinline__ uint32_t wave_radix_sort(uint32_t key, int lo, int nb
 // Lists of at most 64 entries are kept sorted by distance (see k_block_build).
 constexpr int kSortRows = 64;
 
-// Block-list storage.  The entries of atom i come in groups of 8: group q holds
-// entries 8q .. 8q + 7 in the 16 bytes at nbr16 + (q * npad + i) * 8, the even
-// entries first (8q, 8q + 2, 8q + 4, 8q + 6, then 8q + 1, ..., 8q + 7).  The two
-// lanes of an atom walk its even and its odd entries, so each lane reads four of
-// its entries with one 8-byte load and the 32 atoms of a wave read 512 contiguous
-// bytes.  The list capacity (nmax) is a multiple of 8.
-__device__ __forceinline__ int64_t bl_index(int64_t npad, int64_t i, int k)
-{
-  return (((int64_t)(k >> 3) * npad + i) << 3) + ((k & 1) << 2) + ((k & 7) >> 1);
-}
-
 // list order (0, 1), (2, 3), (4, 5), (6, 7) -> the bl_index order (0, 2), (4, 6),
 // (1, 3), (5, 7)
 __device__ __forceinline__ uint4 group_interleave(const uint32_t (&o)[4])
@@ -539,6 +528,7 @@ struct BuildArgs {
   uint32_t* __restrict__ stage;
   uint32_t* __restrict__ cen;
   uint16_t* __restrict__ cen_slot;
+  uint32_t* __restrict__ base;  // per atom: start of its brick's staging entries
   // [0] longest list beyond nmax, [1] halo beyond cap, [2] table space taken (staging
   // entries in units of kStageAlign, central atoms in the lower half)
   unsigned long long* __restrict__ flags;
@@ -610,6 +600,7 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
     P[c] = double3{p.x, p.y, p.z};
     if (total_p[2] >= 0) a.stage[(uint32_t)total_p[2] * kStageAlign + (uint32_t)c] = e;
   });
+  const uint32_t stage0 = (uint32_t)__builtin_amdgcn_readfirstlane(total_p[2]) * kStageAlign;
   const uint32_t cen0 = (uint32_t)__builtin_amdgcn_readfirstlane(total_p[3]);
 
   uint16_t* cand = cand_all + (size_t)wave * a.cand_cap;
@@ -673,6 +664,7 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
     for (int k = lane; k < nat; k += 64) {
       a.cen[q0 + k] = (uint32_t)(g0 + k);
       a.cen_slot[q0 + k] = (uint16_t)(l0 + k);
+      a.base[g0 + k] = stage0;
     }
     double lx = 1e300, ly = 1e300, lz = 1e300, ux = -1e300, uy = -1e300, uz = -1e300;
     if constexpr (!XF) {
@@ -1146,6 +1138,100 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
     if (ln.writes()) {
       if constexpr (DRIFT) pm::write_outputs_drift(o, dr, gi, pi, fx, fy, fz);
       else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, gi, fx, fy, fz, e, v);
+    }
+  }
+}
+
+// First sweep of the EAM adjoint (formulas in k_adjoint.hip): drho_i = sum_j rho'_tj(r_ij) s_ij
+// with s_ij = u_ij . (g_i - g_j), then lambda_i = F''(rho_i) drho_i into the w of g_i's
+// record.  The density pass with the neighbours' loss gradients staged beside their
+// positions (48 bytes a slot, two workgroups per CU at 220-atom bricks); distances, knot
+// fractions and sums FP64, Real is the table's storage.
+struct AdjB1Args {
+  Pos4* gvec;         // g_i (dL/dF_i) in cell order; lambda_i into w
+  double* drho;
+  const double* rho;  // checkpointed rho_i
+  const void* frho;   // rows [c3 c4 c5 c6 | c0 c1 c2 0]
+  const void* slope;  // EamHost::slope_*
+  int nrho;
+  double rdrho, conv;
+};
+
+template <class Real, bool MULTI, bool SPLIT>
+__global__ void __launch_bounds__(kPassThreads, 4) k_block_adj_b1(BlockArgs a, EamTabDev<Real> t, AdjB1Args g)
+{
+  const int64_t b = lblock();
+  if (b >= a.nblocks) return;
+  extern __shared__ __align__(32) unsigned char smem[];
+  LRec rec;
+  const size_t rb = lrec_at(smem, a.cap, false, rec);
+  double* gl = reinterpret_cast<double*>(smem + rb);  // g of slot c at 3 c
+  uint8_t* ltype = MULTI ? smem + 2 * rb : nullptr;
+  const BrickHead hd(a.head[b]);
+  const PassLanes<SPLIT> ln(a);
+  PassAtom<SPLIT> at;
+  if (ln.slot < hd.central) at.index(a, hd, ln.slot);
+  stage<false>(a, hd, rec, ltype);
+  for (int c = threadIdx.x; c < hd.halo; c += kPassThreads) {
+    const double* q = reinterpret_cast<const double*>(g.gvec + xsmd_nbr_index(a.stage[hd.stage + (uint32_t)c]));
+    const double2 xy = *reinterpret_cast<const double2*>(q);
+    gl[3 * c] = xy.x;
+    gl[3 * c + 1] = xy.y;
+    gl[3 * c + 2] = q[2];
+  }
+  if (threadIdx.x < 3) gl[3 * a.cap + threadIdx.x] = 0.0;  // the far record
+  if (ln.slot < hd.central) at.list(a, ln);
+  __syncthreads();
+  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
+    const int64_t gi = at.gi;
+    const int slot = at.slot;
+    const Pos4 pi = rec.get(slot);
+    const double g0 = gl[3 * slot], g1 = gl[3 * slot + 1], g2 = gl[3 * slot + 2];
+    const int ti = MULTI ? ltype[slot] : 0;
+    const bool oni = !MULTI || pm::eam_on(t, ti);
+    const int cnt = oni ? at.cnt : 0;
+    double drho = 0.0;
+    LWords<SPLIT> lw(a, gi, ln);
+    uint2 wnext = at.w;
+    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
+      const uint2 w = wnext;
+      if (k0 + ln.step() < cnt) wnext = lw.next();
+      int c[kBBatch];
+      lslots(w, a.cap, k0, cnt, c);
+      LNb nb[kBBatch];
+      lgather<kBBatch>(a, rec, c, k0, cnt, pi, nb);
+      bool any = false;
+#pragma unroll
+      for (int u = 0; u < kBBatch; u++) {
+        if constexpr (MULTI) nb[u].in = nb[u].in && pm::eam_on(t, ltype[nb[u].c]);
+        any |= nb[u].in;
+      }
+      if (!__any(any)) continue;
+#pragma unroll
+      for (int u = 0; u < kBBatch; u++) {
+        const int tj = MULTI ? ltype[nb[u].c] : 0;
+        const double* gj = gl + 3 * nb[u].c;
+        const double r = sqrt(nb[u].d2);
+        const double s = (nb[u].x * (gj[0] - g0) + nb[u].y * (gj[1] - g1) + nb[u].z * (gj[2] - g2)) / r;
+        double p = fma(r, t.rdr_d, 1.0);
+        const int m = max(0, min((int)p, t.nr - 1));
+        p = fmin(p - (double)m, 1.0);
+        const int plane = MULTI && max(ti, tj) < t.nel ? tj : 0;
+        const pm::Q4<Real> row = pm::load4(pm::pair_row(static_cast<const Real*>(g.slope), t, plane, m));
+        const double dr = ((double)row.a * p + (double)row.b) * p + (double)row.c;
+        drho += nb[u].in ? dr * s : 0.0;
+      }
+    }
+    drho = ln.sum(drho);
+    if (ln.writes()) {
+      // F'' = d/drho of (c0 p + c1) p + c2, zero where p was clamped
+      double p = g.rho[gi] * g.rdrho + 1.0;
+      const int m = max(1, min((int)p, g.nrho - 1));
+      p -= (double)m;
+      const Real* row = static_cast<const Real*>(g.frho) + ((int64_t)t.t2frho[ti + 1] * (g.nrho + 1) + m) * 8;
+      const double fpp = p > 1.0 ? 0.0 : (2.0 * (double)row[4] * p + (double)row[5]) * g.rdrho * g.conv;
+      g.drho[gi] = drho;
+      reinterpret_cast<double*>(g.gvec + gi)[3] = oni ? fpp * drho : 0.0;
     }
   }
 }
@@ -1705,10 +1791,12 @@ bool block_build(Ctx& c, double rl2)
   c.brick_stage.reserve(c.bstage);
   c.brick_cen.reserve(c.n);
   c.brick_cen_slot.reserve(c.n);
+  c.atom_stage.reserve(c.n);
   a.head = c.brick_head.p;
   a.stage = c.brick_stage.p;
   a.cen = c.brick_cen.p;
   a.cen_slot = c.brick_cen_slot.p;
+  a.base = c.atom_stage.p;
   for (int attempt = 0; attempt < 2; attempt++) {
     a.atoms = kBuildAtoms;
     while (a.atoms > 1 && build_lds_bytes(c, a.atoms) > kBlockLdsLimit) a.atoms /= 2;
@@ -1864,6 +1952,38 @@ void launch_johnson_block(Ctx& c, const JohnsonParams& p, double rcut, bool do_e
                          : (vir ? k_block_johnson_force<true, false> : k_block_johnson_force<false, false>);
   k<<<g, kPassThreads, lds, c.stream>>>(a, p, o);
   XS_HIP(hipGetLastError());
+}
+
+void launch_adj_b1_block(Ctx& c, double rcut, bool mixed)
+{
+  const BlockArgs a = block_args(c, rcut);
+  const bool multi = eam_multi(c);
+  // at most 97 KB for the largest halo the brick list allows (kBlockLdsLimit)
+  const size_t lds = ((size_t)c.bcap + 1) * (6 * sizeof(double) + (multi ? 1 : 0));
+  AdjB1Args g;
+  g.gvec = c.adj_gvec.p;
+  g.drho = c.adj_drho.p;
+  g.rho = c.rho.p;
+  g.nrho = c.eam.nrho;
+  g.rdrho = c.eam.rdrho;
+  g.conv = kEV;
+  const auto run = [&](auto zero, auto k) {
+    using Real = decltype(zero);
+    if constexpr (sizeof(Real) == 4) g.frho = c.eam.frho_f.p, g.slope = c.eam.slope_f.p;
+    else g.frho = c.eam.frho_d.p, g.slope = c.eam.slope_d.p;
+    if (lds > kBlockLdsLimit)
+      XS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)lds));
+    k<<<block_grid(c), kPassThreads, lds, c.stream>>>(a, make_eam_tab<Real>(c), g);
+    XS_HIP(hipGetLastError());
+  };
+  const auto pick = [&](auto zero) {
+    using Real = decltype(zero);
+    if (multi) run(zero, a.split ? k_block_adj_b1<Real, true, true> : k_block_adj_b1<Real, true, false>);
+    else run(zero, a.split ? k_block_adj_b1<Real, false, true> : k_block_adj_b1<Real, false, false>);
+  };
+  if (mixed) pick(0.0f);
+  else pick(0.0);
 }
 
 void ensure_global_list(Ctx& c)

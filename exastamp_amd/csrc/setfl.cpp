@@ -233,46 +233,38 @@ std::vector<double> build_all(int ntab, int n, double delta, const std::vector<d
 
 }  // namespace
 
-// Type maps of initialize_types_table (eam_alloy.h:70-133) for nel types mapped
-// to elements in order, then both precisions of every table to the device.
+// Type map of initialize_types_table (eam_alloy.h:70-133) for nel types mapped to
+// elements in order (the pair tables' follow in arithmetic, pair_planes in
+// pair_math.hpp), then both precisions of every table to the device.
 void eam_upload(Ctx& c)
 {
   EamHost& e = c.eam;
   const int nel = e.nel;
-  std::memset(e.t2rhor, 0, sizeof(e.t2rhor));
-  std::memset(e.t2z2r, 0, sizeof(e.t2z2r));
   std::memset(e.t2frho, 0, sizeof(e.t2frho));
-  for (int i = 1; i <= nel; i++) {
-    e.t2frho[i] = (int8_t)(i - 1);
-    for (int j = 1; j <= nel; j++) {
-      e.t2rhor[i][j] = (int8_t)(i - 1);
-      int hiv = i - 1, lov = j - 1;
-      if (hiv < lov) std::swap(hiv, lov);
-      e.t2z2r[i][j] = (int8_t)(hiv * (hiv + 1) / 2 + lov);
-    }
-  }
+  for (int i = 1; i <= nel; i++) e.t2frho[i] = (int8_t)(i - 1);
   const int nz = nel * (nel + 1) / 2;
   const std::vector<double> cf = build_all(nel, e.nrho, e.drho, e.frho_knots);
   const std::vector<double> cr = build_all(nel, e.nr, e.dr, e.rhor_knots);
   const std::vector<double> cz = build_all(nz, e.nr, e.dr, e.z2r_knots);
   upload(c, e.frho_d, cf);
-  upload(c, e.rhor_d, cr);
-  upload(c, e.z2r_d, cz);
   upload(c, e.frho_f, cf);
-  upload(c, e.rhor_f, cr);
-  upload(c, e.z2r_f, cz);
 
   // pair table: the value cubics [c3 c4 c5 c6] of the rho rows, then of the z2r rows
   const size_t rows = (size_t)e.nr + 1, nrows = (nel + nz) * rows;
   std::vector<double> pair(4 * nrows);
   for (size_t q = 0; q < nrows; q++)
     for (int k = 0; k < 4; k++) pair[4 * q + k] = q < nel * rows ? cr[8 * q + 3 + k] : cz[8 * (q - nel * rows) + 3 + k];
+  std::vector<double> slope(4 * (size_t)nel * rows);
+  for (size_t q = 0; q < nel * rows; q++)
+    for (int k = 0; k < 4; k++) slope[4 * q + k] = k < 3 ? cr[8 * q + k] : 0.0;
   auto up = [&](auto& buf, const auto& tmp) {
     buf.reserve(tmp.size());
     XS_HIP(hipMemcpyAsync(buf.p, tmp.data(), tmp.size() * sizeof(tmp[0]), hipMemcpyHostToDevice, c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
   };
   up(e.pair_d, pair);
+  up(e.slope_d, slope);
+  up(e.slope_f, std::vector<float>(slope.begin(), slope.end()));
   // FP32: the same knot planes, then the s = r^2 tables of the mixed passes
   std::vector<float> pf(pair.size());
   for (size_t q = 0; q < pair.size(); q++) pf[q] = (float)pair[q];
@@ -292,64 +284,65 @@ __device__ __forceinline__ double spline_slope_dev(const double* __restrict__ f,
   return ((f[m - 3] - f[m + 1]) + 8.0 * (f[m] - f[m - 2])) / 12.0;
 }
 
-// One coefficient row per thread (row m of table t, rows 0..n): spline_interpolate's
+// The tables of xs_eam_theta_dev: nel F tables of nrho knots, then npair tables (rho, z2r)
+// of nr knots, their knots one after the other.
+struct ThetaRows {
+  int64_t rows_f, rows_r, rows;  // coefficient rows of the F tables, of F and rho, and of all
+  int nrho, nr;
+  double drho, dr;
+  const double* theta;
+  int64_t knots_f;
+  double* frho_d;
+  float* frho_f;
+  double* pair_d;
+  float* pair_f;
+  double* slope_d;
+  float* slope_f;
+};
+
+// One coefficient row per thread (row m of its table, rows 0..n): spline_interpolate's
 // arithmetic in its order, with contraction off in this file, so every coefficient
-// has the host build's bits; written in device order [c3 c4 c5 c6 c0 c1 c2 0] in
-// FP64 and FP32.
-__global__ void k_spline_rows(int ntab, int n, double delta, const double* __restrict__ knots,
-                              double* __restrict__ rows_d, float* __restrict__ rows_f)
+// has the host build's bits.  F rows [c3 c4 c5 c6 c0 c1 c2 0], rows of the pair table
+// [c3 c4 c5 c6], rho' rows [c0 c1 c2 0], in FP64 and FP32.
+__global__ void k_theta_rows(ThetaRows a)
 {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t per = (int64_t)n + 1;
-  if (q >= (int64_t)ntab * per) return;
-  const int t = (int)(q / per), m = (int)(q - t * per);
-  const double* f = knots + (int64_t)t * n;
-  double c[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (q >= a.rows) return;
+  const bool is_f = q < a.rows_f;
+  const int n = is_f ? a.nrho : a.nr;
+  const int64_t u = is_f ? q : q - a.rows_f;
+  const int64_t t = u / (n + 1);
+  const int m = (int)(u - t * (n + 1));
+  const double* f = a.theta + (is_f ? 0 : a.knots_f) + t * n;
+  double c[4] = {0.0, 0.0, 0.0, 0.0};  // c3..c6
   if (m >= 1) {
     const double sm = spline_slope_dev(f, n, m);
-    double a = 0.0, b = 0.0;
     if (m <= n - 1) {
       const double sm1 = spline_slope_dev(f, n, m + 1);
       const double dv = f[m] - f[m - 1];
-      b = 3.0 * dv - 2.0 * sm - sm1;
-      a = sm + sm1 - 2.0 * dv;
+      c[1] = 3.0 * dv - 2.0 * sm - sm1;
+      c[0] = sm + sm1 - 2.0 * dv;
     }
-    c[0] = a;
-    c[1] = b;
     c[2] = sm;
     c[3] = f[m - 1];
-    c[4] = 3.0 * a / delta;
-    c[5] = 2.0 * b / delta;
-    c[6] = sm / delta;
   }
-  double* d = rows_d + 8 * q;
-  float* g = rows_f + 8 * q;
+  double* d = is_f ? a.frho_d + 8 * u : a.pair_d + 4 * u;
+  float* g = is_f ? a.frho_f + 8 * u : a.pair_f + 4 * u;
 #pragma unroll
-  for (int k = 0; k < 8; k++) {
+  for (int k = 0; k < 4; k++) {
     d[k] = c[k];
     g[k] = (float)c[k];
   }
-}
-
-// The knot planes of the pair table (rho and z2r value cubics, eam_upload's layout) from
-// the device rows, both precisions: nr rows of rho tables, nz of z2r tables.
-__global__ void k_pair_planes(int64_t nr, int64_t nz, const double* __restrict__ rhor, const double* __restrict__ z2r,
-                              double* __restrict__ pair_d, float* __restrict__ pair_f)
-{
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= 4 * (nr + nz)) return;
-  const int64_t m = q >> 2, k = q & 3;
-  const double v = m < nr ? rhor[8 * m + k] : z2r[8 * (m - nr) + k];
-  pair_d[q] = v;
-  pair_f[q] = (float)v;
-}
-
-void spline_rows_dev(Ctx& c, int ntab, int n, double delta, const double* knots, DBuf<double>& rows_d,
-                     DBuf<float>& rows_f)
-{
-  const int64_t total = (int64_t)ntab * (n + 1);
-  k_spline_rows<<<grid_for(total), kBlock, 0, c.stream>>>(ntab, n, delta, knots, rows_d.p, rows_f.p);
-  XS_HIP(hipGetLastError());
+  if (q >= a.rows_r) return;
+  const double delta = is_f ? a.drho : a.dr;
+  const double s[4] = {3.0 * c[0] / delta, 2.0 * c[1] / delta, c[2] / delta, 0.0};  // c0..c2
+  d = is_f ? d + 4 : a.slope_d + 4 * u;
+  g = is_f ? g + 4 : a.slope_f + 4 * u;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    d[k] = s[k];
+    g[k] = (float)s[k];
+  }
 }
 
 }  // namespace
@@ -358,15 +351,23 @@ void eam_theta_dev(Ctx& c, const double* theta)
 {
   EamHost& e = c.eam;
   const int nel = e.nel, nz = nel * (nel + 1) / 2;
-  const double* f = theta;
-  const double* r = f + (size_t)nel * e.nrho;
-  const double* z = r + (size_t)nel * e.nr;
-  spline_rows_dev(c, nel, e.nrho, e.drho, f, e.frho_d, e.frho_f);
-  spline_rows_dev(c, nel, e.nr, e.dr, r, e.rhor_d, e.rhor_f);
-  spline_rows_dev(c, nz, e.nr, e.dr, z, e.z2r_d, e.z2r_f);
-  const int64_t rows = (int64_t)e.nr + 1;
-  k_pair_planes<<<grid_for(4 * (nel + nz) * rows), kBlock, 0, c.stream>>>(nel * rows, nz * rows, e.rhor_d.p,
-                                                                          e.z2r_d.p, e.pair_d.p, e.pair_f.p);
+  ThetaRows a;
+  a.rows_f = (int64_t)nel * (e.nrho + 1);
+  a.rows_r = a.rows_f + (int64_t)nel * (e.nr + 1);
+  a.rows = a.rows_r + (int64_t)nz * (e.nr + 1);
+  a.nrho = e.nrho;
+  a.nr = e.nr;
+  a.drho = e.drho;
+  a.dr = e.dr;
+  a.theta = theta;
+  a.knots_f = (int64_t)nel * e.nrho;
+  a.frho_d = e.frho_d.p;
+  a.frho_f = e.frho_f.p;
+  a.pair_d = e.pair_d.p;
+  a.pair_f = e.pair_f.p;
+  a.slope_d = e.slope_d.p;
+  a.slope_f = e.slope_f.p;
+  k_theta_rows<<<grid_for(a.rows), kBlock, 0, c.stream>>>(a);
   XS_HIP(hipGetLastError());
   // the s = r^2 tables were built (and checked) from the previous knots on the host
   e.s_pieces = 0;

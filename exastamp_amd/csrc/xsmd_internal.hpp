@@ -152,6 +152,17 @@ struct StepGate {
   }
 };
 
+// Block-list storage.  The entries of atom i come in groups of 8: group q holds
+// entries 8q .. 8q + 7 in the 16 bytes at nbr16 + (q * npad + i) * 8, the even
+// entries first (8q, 8q + 2, 8q + 4, 8q + 6, then 8q + 1, ..., 8q + 7).  The two
+// lanes of an atom walk its even and its odd entries, so each lane reads four of
+// its entries with one 8-byte load and the 32 atoms of a wave read 512 contiguous
+// bytes.  The list capacity (nmax) is a multiple of 8.
+__device__ __forceinline__ int64_t bl_index(int64_t npad, int64_t i, int k)
+{
+  return (((int64_t)(k >> 3) * npad + i) << 3) + ((k & 1) << 2) + ((k & 7) >> 1);
+}
+
 // Box of one replica, as kernels read it: lo[3], L[3], n/L[3].
 struct BoxDev {
   double lo[3];
@@ -178,9 +189,10 @@ inline double xform_det(const XformDev& x)
 }
 
 // Spline tables on the device.  Each row of the reference's SplineCoeffs
-// (eam_alloy.h:37-42: c0..c2 derivative quadratic, c3..c6 value cubic) is
+// (eam_alloy.h:37-42: c0..c2 derivative quadratic, c3..c6 value cubic) of the F tables is
 // stored as 8 values reordered to [c3 c4 c5 c6 | c0 c1 c2 0] so the value
-// cubic and the derivative quadratic are each one aligned 4-vector load.
+// cubic and the derivative quadratic are each one aligned 4-vector load; the pair table
+// keeps the value cubics of the others (EamHost).
 template <class Real>
 struct EamTabDev {
   const Real* frho = nullptr;  // nel tables of (nrho+1) rows
@@ -202,16 +214,17 @@ struct EamHost {
   int nel = 0, nr = 0, nrho = 0;
   double dr = 0, drho = 0, rdr = 0, rdrho = 0, rc = 0, rhomax = 0;
   std::vector<double> frho_knots, rhor_knots, z2r_knots;
-  int8_t t2rhor[8][8] = {};
-  int8_t t2z2r[8][8] = {};
   int8_t t2frho[8] = {};
-  DBuf<double> frho_d, rhor_d, z2r_d;
-  DBuf<float> frho_f, rhor_f, z2r_f;
+  DBuf<double> frho_d;
+  DBuf<float> frho_f;
   // pair table: nel rho planes, then nel (nel + 1) / 2 z2r planes, row m = [c3 c4 c5 c6]
   // of knot m; the derivative quadratics follow from the value cubics, so the planes
   // serve both EAM passes
   DBuf<double> pair_d;
   DBuf<float> pair_f;
+  // rho'(r) rows [c0 c1 c2 0] of the nel rho tables, nr + 1 each (EAM adjoint)
+  DBuf<double> slope_d;
+  DBuf<float> slope_f;
   // FP32 s = r^2 tables after the knot planes of pair_f (pair_math.hpp): pieces
   // (0 = none), their range [s_lo, s_hi], and their largest FP32 errors against the
   // FP64 spline in FP32 ulps of the largest |rho'/r|, |phi| and |phi'/r|
@@ -390,6 +403,7 @@ struct Ctx {
   DBuf<uint4> brick_head;
   DBuf<uint32_t> brick_stage, brick_cen;
   DBuf<uint16_t> brick_cen_slot;
+  DBuf<uint32_t> atom_stage;
   int bcap = 0;                    // LDS slots per block (max halo atoms, rounded)
   int bcentral = 0;                // max central atoms per block
   int bcand = 0;                   // max atoms in the 27 cells of a central cell
@@ -432,12 +446,11 @@ struct Ctx {
   // bits per species; ~0u = every species (the empty list)
   uint32_t eam_types = ~0u;
 
-  // EAM adjoint scratch: coefficient gradients, lambda_i, dL/dF records, inputs
-  DBuf<double> adj_g, adj_lam, adj_in;
-  DBuf<double> adj_fc, adj_part;  // per-atom F-table contributions; per-workgroup partial rows
+  // EAM adjoint scratch: knot value and slope gradients, drho_i, dL/dE, host inputs,
+  // per-workgroup partial rows; dL/dF records (w = lambda_i)
+  DBuf<double> adj_g, adj_drho, adj_gE, adj_in, adj_part;
   DBuf<double> adj_grad;          // dL/dtheta on the device (host-output adjoint)
   DBuf<double> rep_part;          // per-replica partial energy sums (forces_energies_dev)
-  DBuf<int> adj_fm;               // per-atom F-table row
   DBuf<Pos4> adj_gvec;
 
   Profiler prof;
@@ -463,6 +476,9 @@ bool block_build(Ctx& c, double rl2);
 void block_to_global(Ctx& c);
 void ensure_global_list(Ctx& c);
 double max_displacement2(Ctx& c);
+// first sweep of the EAM adjoint on the brick lists (drho into adj_drho, lambda into
+// adj_gvec's w)
+void launch_adj_b1_block(Ctx& c, double rcut, bool mixed);
 // average ms of the gather-ceiling kernel of the density (force = false) or force pass
 double gather_ceiling(Ctx& c, double rcut, bool force, int level, int reps);
 void pair_count(Ctx& c, double rcut, int64_t& entries, int64_t& within);
