@@ -16,6 +16,7 @@ Ctx::~Ctx()
   if (hscalar) (void)hipHostFree(hscalar);
   if (hthermo) (void)hipHostFree(hthermo);
   if (hflag) (void)hipHostFree(hflag);
+  if (hhalo) (void)hipHostFree(hhalo);
   if (pinned) (void)hipHostFree(pinned);
   for (hipEvent_t e : step_event)
     if (e) (void)hipEventDestroy(e);
@@ -212,6 +213,8 @@ xs_status xs_ctx_create(int device, xs_ctx** out)
     XS_HIP(hipHostMalloc((void**)&c->hthermo, 27 * sizeof(double), hipHostMallocDefault));
     XS_HIP(hipHostMalloc((void**)&c->hflag, sizeof(unsigned long long), hipHostMallocCoherent | hipHostMallocMapped));
     *c->hflag = 0;
+    XS_HIP(hipHostMalloc((void**)&c->hhalo, (4 * kHaloGroups + 1) * sizeof(uint32_t),
+                         hipHostMallocCoherent | hipHostMallocMapped));
     for (hipEvent_t& e : c->step_event) XS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     c->dscalar.reserve(8);
     XS_HIP(hipMemsetAsync(c->dscalar.p, 0, 8 * sizeof(unsigned long long), c->stream));  // flags start clear

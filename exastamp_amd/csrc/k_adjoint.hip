@@ -163,7 +163,7 @@ __device__ __forceinline__ void adj_knot(double x, double rscale, int n, int& m,
 // First sweep on the global list: kB1Lanes lanes per atom gather through it.
 constexpr int kB1Lanes = 4;
 template <class Real, bool MULTI>
-__global__ void __launch_bounds__(256) k_adj_b1(AdjArgs a, EamTabDev<Real> t, const Real* __restrict__ slope)
+__global__ void __launch_bounds__(256) k_adj_b1(AdjArgs a, EamTabDev<Real> t)
 {
   const int sub = threadIdx.x % kB1Lanes;
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kB1Lanes;
@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(256) k_adj_b1(AdjArgs a, EamTabDev<Real> t, co
     int m;
     double p;
     adj_knot(r, a.rdr, a.nr, m, p);
-    const pm::Q4<Real> row = pm::load4(pm::pair_row(slope, t, MULTI && max(ti, tj) < a.nel ? tj : 0, m));
+    const pm::Q4<Real> row = pm::load4(pm::pair_row(t.slope, t, MULTI && max(ti, tj) < a.nel ? tj : 0, m));
     drho += (((double)row.a * p + (double)row.b) * p + (double)row.c) * s;
   }
 #pragma unroll
@@ -529,11 +529,8 @@ std::vector<AdjWindows> adj_launches(int nel, int nz, int nrho, int nr, int what
 template <class Real>
 void adj_first_sweep(Ctx& c, const AdjArgs& a)
 {
-  const Real* slope;
-  if constexpr (sizeof(Real) == 4) slope = c.eam.slope_f.p;
-  else slope = c.eam.slope_d.p;
   const auto k = eam_multi(c) ? k_adj_b1<Real, true> : k_adj_b1<Real, false>;
-  k<<<grid_for(a.n * kB1Lanes), 256, 0, c.stream>>>(a, make_eam_tab<Real>(c), slope);
+  k<<<grid_for(a.n * kB1Lanes), 256, 0, c.stream>>>(a, make_eam_tab<Real>(c));
   XS_HIP(hipGetLastError());
 }
 

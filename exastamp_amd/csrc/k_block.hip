@@ -204,9 +204,11 @@ constexpr int kPassAtoms = kPassThreads / 2;
 // atom at 220-atom bricks) written at the build and read by each pass; the chain of
 // waits it removes was longer: 8.39 M EAM atoms, mixed: density pass 0.907 -> 0.761 ms,
 // force pass 1.350 -> 1.258 ms; 1.05 M argon atoms 0.171 -> 0.141 ms per pass.
-// The bricks' parts of the tables follow one another in the order the build's workgroups
-// took them, so their size goes with the atoms, not with the number of bricks times the
-// densest one.
+// Where the bricks are filled alike, each has room for the densest one; where that would
+// more than double the tables (a cluster in a large vacuum box: gigabytes), the bricks'
+// parts follow one another as the build's workgroups take them, one atomic each (the
+// build of 136 k atoms, whose 700 workgroups start together, takes 86 us so against 80; at
+// 1.05 M atoms there is no difference).
 constexpr uint32_t kStageAlign = 16;  // a brick's staging entries start on 64 bytes
 struct BlockArgs {
   const uint4* __restrict__ head;      // per brick: BrickHead
@@ -529,9 +531,11 @@ struct BuildArgs {
   uint32_t* __restrict__ cen;
   uint16_t* __restrict__ cen_slot;
   uint32_t* __restrict__ base;  // per atom: start of its brick's staging entries
+  int stage_step, cen_step;     // entries per brick; 0: parts handed out through flags[2]
   // [0] longest list beyond nmax, [1] halo beyond cap, [2] table space taken (staging
   // entries in units of kStageAlign, central atoms in the lower half)
   unsigned long long* __restrict__ flags;
+  uint32_t* __restrict__ over;  // host memory: set when [0] or [1] is
 };
 
 // candidate slots of each wave (the staging uses the same bytes first) and the list rows
@@ -559,7 +563,10 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
   const BlockShape s = block_shape(a.g, b);
   const int total = build_halo(a.g, s, a.cell_off, hc, total_p);
   if (total > a.cap) {  // cannot happen when cap = measured maximum; never write past LDS
-    if (threadIdx.x == 0) atomicMax(a.flags + 1, (unsigned long long)total);
+    if (threadIdx.x == 0) {
+      atomicMax(a.flags + 1, (unsigned long long)total);
+      *a.over = 1;
+    }
     return;
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -586,11 +593,16 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
       total_p[2] = -1;
       uint4 head = BrickHead::pack(0, 0, s.r, 0, 0);  // no central atom: nothing to stage
       if (carry > 0) {
-        const unsigned long long need = (unsigned long long)((total + kStageAlign - 1) / kStageAlign) << 32;
-        const unsigned long long at = atomicAdd(a.flags + 2, need | (unsigned long long)carry);
-        total_p[2] = (int)(at >> 32);
-        total_p[3] = (int)(uint32_t)at;
-        head = BrickHead::pack(total, carry, s.r, (uint32_t)(at >> 32), (uint32_t)at);
+        uint32_t at_stage = (uint32_t)b * (uint32_t)(a.stage_step / (int)kStageAlign), at_cen = (uint32_t)b * (uint32_t)a.cen_step;
+        if (a.stage_step == 0) {
+          const unsigned long long need = (unsigned long long)((total + kStageAlign - 1) / kStageAlign) << 32;
+          const unsigned long long at = atomicAdd(a.flags + 2, need | (unsigned long long)carry);
+          at_stage = (uint32_t)(at >> 32);
+          at_cen = (uint32_t)at;
+        }
+        total_p[2] = (int)at_stage;
+        total_p[3] = (int)at_cen;
+        head = BrickHead::pack(total, carry, s.r, at_stage, at_cen);
       }
       a.head[b] = head;
     }
@@ -616,7 +628,10 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
     wave_lds_sync();
     if (lane < nrow) {
       a.nnb[gi] = cnt;
-      if (cnt > a.nmax) atomicMax(a.flags, (unsigned long long)cnt);
+      if (cnt > a.nmax) {
+        atomicMax(a.flags, (unsigned long long)cnt);
+        *a.over = 1;
+      }
     }
     const int la = lane >> 3, j = lane & 7;
     const int ca = la < nrow ? min(__shfl(cnt, la), a.nmax) : 0;
@@ -803,20 +818,24 @@ __global__ void __launch_bounds__(256) k_block_to_global(BlockArgs a, uint32_t* 
   }
 }
 
-// Sizes the LDS of the block kernels and the staging table: out[0..2] the most halo atoms
-// and central atoms of a brick and the most atoms in the 27 cells of a central cell,
-// out[3] the staging entries of the bricks that hold atoms, in units of kStageAlign.  One wave per brick, one lane
+// Sizes the LDS of the block kernels and the staging table: the most halo atoms and
+// central atoms of a brick, the most atoms in the 27 cells of a central cell, and the
+// staging entries of the bricks that hold atoms, in units of kStageAlign.  Each workgroup
+// writes its four to host memory, where they are put together (atomics on four words
+// took 20 us of the kernel's 25 at 700 bricks).  One wave per brick, one lane
 // per halo cell (a thread per brick reads its cells one after the other: 33 us for a
-// single brick of 125 cells, against 4 us).
+// single brick of 125 cells, against 4 us).  Clears the build's flags, which follows.
 constexpr int kHaloMaxWaves = 4;
 __global__ void __launch_bounds__(64 * kHaloMaxWaves) k_block_halo_max(BlockGeom g, const int* __restrict__ cell_off,
-                                                                       unsigned long long* __restrict__ out)
+                                                                       uint32_t* __restrict__ out,
+                                                                       unsigned long long* __restrict__ flags)
 {
+  if (blockIdx.x == 0 && threadIdx.x < 3) flags[threadIdx.x] = 0;
   __shared__ int cnt_all[kHaloMaxWaves][kMaxHaloCells];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   int* cnt = cnt_all[wave];
   int m_total = 0, m_central = 0, m_cand = 0;
-  unsigned long long entries = 0;
+  uint32_t entries = 0;
   for (int64_t b = (int64_t)blockIdx.x * kHaloMaxWaves + wave; b < g.nblocks; b += (int64_t)gridDim.x * kHaloMaxWaves) {
     const BlockShape s = block_shape(g, b);
     const int nh = s.hx * s.hy * s.hz;
@@ -850,24 +869,25 @@ __global__ void __launch_bounds__(64 * kHaloMaxWaves) k_block_halo_max(BlockGeom
       central += __shfl_xor(central, off);
     }
     m_total = max(m_total, total);
-    if (central > 0) entries += (unsigned long long)((total + kStageAlign - 1) / kStageAlign);
+    if (central > 0) entries += (uint32_t)(total + kStageAlign - 1) / kStageAlign;
     m_central = max(m_central, central);
     wave_lds_sync();
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) m_cand = max(m_cand, __shfl_xor(m_cand, off));
-  __shared__ int best[kHaloMaxWaves][3];
+  __shared__ uint32_t best[kHaloMaxWaves][4];
   if (lane == 0) {
-    if (entries) atomicAdd(out + 3, entries);
+    best[wave][3] = entries;
     best[wave][0] = m_total;
     best[wave][1] = m_central;
     best[wave][2] = m_cand;
   }
   __syncthreads();
-  if (threadIdx.x < 3) {
-    int v = best[0][threadIdx.x];
-    for (int w = 1; w < kHaloMaxWaves; w++) v = max(v, best[w][threadIdx.x]);
-    atomicMax(out + threadIdx.x, (unsigned long long)v);
+  if (threadIdx.x < 4) {
+    uint32_t v = best[0][threadIdx.x];
+    for (int w = 1; w < kHaloMaxWaves; w++)
+      v = threadIdx.x == 3 ? v + best[w][3] : max(v, best[w][threadIdx.x]);
+    out[4 * blockIdx.x + threadIdx.x] = v;
   }
 }
 
@@ -1152,7 +1172,6 @@ struct AdjB1Args {
   double* drho;
   const double* rho;  // checkpointed rho_i
   const void* frho;   // rows [c3 c4 c5 c6 | c0 c1 c2 0]
-  const void* slope;  // EamHost::slope_*
   int nrho;
   double rdrho, conv;
 };
@@ -1217,7 +1236,7 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_adj_b1(BlockArgs a, E
         const int m = max(0, min((int)p, t.nr - 1));
         p = fmin(p - (double)m, 1.0);
         const int plane = MULTI && max(ti, tj) < t.nel ? tj : 0;
-        const pm::Q4<Real> row = pm::load4(pm::pair_row(static_cast<const Real*>(g.slope), t, plane, m));
+        const pm::Q4<Real> row = pm::load4(pm::pair_row(t.slope, t, plane, m));
         const double dr = ((double)row.a * p + (double)row.b) * p + (double)row.c;
         drho += nb[u].in ? dr * s : 0.0;
       }
@@ -1729,21 +1748,27 @@ void block_setup(Ctx& c)
   if (!c.block_atoms_set) bound = std::min(bound, std::max(8.0, (double)c.n / (1.5 * std::max(c.num_cu, 1))));
   for (int attempt = 0;; attempt++) {
     block_shape_choose(c, g, bound, per_cell);
-    XS_HIP(hipMemsetAsync(c.dscalar.p + 2, 0, 4 * sizeof(unsigned long long), c.stream));
-    k_block_halo_max<<<(unsigned)std::min<int64_t>(512, (g.nblocks + kHaloMaxWaves - 1) / kHaloMaxWaves),
-                       64 * kHaloMaxWaves, 0, c.stream>>>(g, c.cell_off.p, c.dscalar.p + 2);
+    const unsigned groups = (unsigned)std::min<int64_t>(kHaloGroups, (g.nblocks + kHaloMaxWaves - 1) / kHaloMaxWaves);
+    k_block_halo_max<<<groups, 64 * kHaloMaxWaves, 0, c.stream>>>(g, c.cell_off.p, c.hhalo, c.dscalar.p);
     XS_HIP(hipGetLastError());
-    XS_HIP(hipMemcpyAsync(c.hscalar + 2, c.dscalar.p + 2, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                          c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
-    c.bcap = (int)((c.hscalar[2] + 63) / 64 * 64);
-    c.bcentral = (int)c.hscalar[3];
-    c.bcand = (int)c.hscalar[4];
-    c.bstage = (size_t)c.hscalar[5] * kStageAlign;
+    uint32_t halo = 0, central = 0, cand = 0;
+    size_t entries = 0;
+    for (unsigned k = 0; k < groups; k++) {
+      const uint32_t* h = c.hhalo + 4 * k;
+      halo = std::max(halo, h[0]);
+      central = std::max(central, h[1]);
+      cand = std::max(cand, h[2]);
+      entries += h[3];
+    }
+    c.bcap = (int)((halo + 63) / 64 * 64);
+    c.bcentral = (int)central;
+    c.bcand = (int)cand;
+    c.bstage = entries * kStageAlign;
     const size_t budget = c.block_atoms_set ? kBlockLdsLimit : std::min(kBlockLdsLimit, kLdsPerCu / 3);
     if (block_lds_bytes(c, true, true) <= budget || g.nh_max == 27 || attempt == 6) break;
     // the densest halo set the capacity: size the next shape for that density
-    per_cell = std::max(per_cell, (double)c.hscalar[2] / g.nh_max);
+    per_cell = std::max(per_cell, (double)halo / g.nh_max);
     bound *= 0.75;
   }
 }
@@ -1787,10 +1812,17 @@ bool block_build(Ctx& c, double rl2)
   a.cand_cap = c.bcand;
   a.sort = !c.list_sort_disabled;
   a.flags = c.dscalar.p;
+  a.over = c.hhalo + 4 * kHaloGroups;
   c.brick_head.reserve(c.bgeom.nblocks);
-  c.brick_stage.reserve(c.bstage);
-  c.brick_cen.reserve(c.n);
-  c.brick_cen_slot.reserve(c.n);
+  // bcap is a multiple of kStageAlign
+  const size_t step_total = (size_t)c.bgeom.nblocks * c.bcap;
+  const bool step = step_total <= 2 * c.bstage && step_total < (size_t)1 << 32;
+  a.stage_step = step ? c.bcap : 0;
+  a.cen_step = step ? c.bcentral : 0;
+  c.brick_stage.reserve(step ? step_total : c.bstage);
+  const size_t cen = step ? (size_t)c.bgeom.nblocks * c.bcentral : (size_t)c.n;
+  c.brick_cen.reserve(cen);
+  c.brick_cen_slot.reserve(cen);
   c.atom_stage.reserve(c.n);
   a.head = c.brick_head.p;
   a.stage = c.brick_stage.p;
@@ -1811,15 +1843,18 @@ bool block_build(Ctx& c, double rl2)
     if (lds > kBlockLdsLimit)
       XS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)lds));
-    XS_HIP(hipMemsetAsync(c.dscalar.p, 0, 3 * sizeof(unsigned long long), c.stream));
+    // block_setup's kernel cleared the flags
+    if (attempt > 0) XS_HIP(hipMemsetAsync(c.dscalar.p, 0, 3 * sizeof(unsigned long long), c.stream));
+    *a.over = 0;
     k<<<block_grid(c), kBuildThreads, lds, c.stream>>>(a);
     XS_HIP(hipGetLastError());
+    XS_HIP(hipStreamSynchronize(c.stream));
+    if (*a.over == 0) return true;
     XS_HIP(hipMemcpyAsync(c.hscalar, c.dscalar.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                           c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
     if (c.hscalar[1] != 0) throw Error(XS_E_STATE, "block halo exceeds its measured capacity");
     const unsigned long long need = c.hscalar[0];
-    if (need == 0) return true;
     if (attempt == 1) throw Error(XS_E_STATE, "neighbour list overflow after resize");
     c.nmax = (int)((need + 7) / 8 * 8 + 8);
   }
@@ -1969,8 +2004,8 @@ void launch_adj_b1_block(Ctx& c, double rcut, bool mixed)
   g.conv = kEV;
   const auto run = [&](auto zero, auto k) {
     using Real = decltype(zero);
-    if constexpr (sizeof(Real) == 4) g.frho = c.eam.frho_f.p, g.slope = c.eam.slope_f.p;
-    else g.frho = c.eam.frho_d.p, g.slope = c.eam.slope_d.p;
+    if constexpr (sizeof(Real) == 4) g.frho = c.eam.frho_f.p;
+    else g.frho = c.eam.frho_d.p;
     if (lds > kBlockLdsLimit)
       XS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)lds));

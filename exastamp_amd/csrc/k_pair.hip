@@ -405,6 +405,7 @@ EamTabDev<double> make_eam_tab<double>(Ctx& c)
 {
   EamTabDev<double> t;
   t.frho = c.eam.frho_d.p;
+  t.slope = c.eam.slope_d.p;
   t.nel = c.eam.nel;
   t.nr = c.eam.nr;
   t.nrho = c.eam.nrho;
@@ -423,6 +424,7 @@ EamTabDev<float> make_eam_tab<float>(Ctx& c)
 {
   EamTabDev<float> t;
   t.frho = c.eam.frho_f.p;
+  t.slope = c.eam.slope_f.p;
   t.nel = c.eam.nel;
   t.nr = c.eam.nr;
   t.nrho = c.eam.nrho;

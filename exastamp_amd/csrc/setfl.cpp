@@ -254,9 +254,9 @@ void eam_upload(Ctx& c)
   std::vector<double> pair(4 * nrows);
   for (size_t q = 0; q < nrows; q++)
     for (int k = 0; k < 4; k++) pair[4 * q + k] = q < nel * rows ? cr[8 * q + 3 + k] : cz[8 * (q - nel * rows) + 3 + k];
-  std::vector<double> slope(4 * (size_t)nel * rows);
-  for (size_t q = 0; q < nel * rows; q++)
-    for (int k = 0; k < 4; k++) slope[4 * q + k] = k < 3 ? cr[8 * q + k] : 0.0;
+  std::vector<double> slope(4 * nrows);
+  for (size_t q = 0; q < nrows; q++)
+    for (int k = 0; k < 3; k++) slope[4 * q + k] = q < nel * rows ? cr[8 * q + k] : cz[8 * (q - nel * rows) + k];
   auto up = [&](auto& buf, const auto& tmp) {
     buf.reserve(tmp.size());
     XS_HIP(hipMemcpyAsync(buf.p, tmp.data(), tmp.size() * sizeof(tmp[0]), hipMemcpyHostToDevice, c.stream));
@@ -287,7 +287,7 @@ __device__ __forceinline__ double spline_slope_dev(const double* __restrict__ f,
 // The tables of xs_eam_theta_dev: nel F tables of nrho knots, then npair tables (rho, z2r)
 // of nr knots, their knots one after the other.
 struct ThetaRows {
-  int64_t rows_f, rows_r, rows;  // coefficient rows of the F tables, of F and rho, and of all
+  int64_t rows_f, rows;  // coefficient rows of the F tables, and of all
   int nrho, nr;
   double drho, dr;
   const double* theta;
@@ -303,7 +303,7 @@ struct ThetaRows {
 // One coefficient row per thread (row m of its table, rows 0..n): spline_interpolate's
 // arithmetic in its order, with contraction off in this file, so every coefficient
 // has the host build's bits.  F rows [c3 c4 c5 c6 c0 c1 c2 0], rows of the pair table
-// [c3 c4 c5 c6], rho' rows [c0 c1 c2 0], in FP64 and FP32.
+// [c3 c4 c5 c6] and its derivative rows [c0 c1 c2 0], in FP64 and FP32.
 __global__ void k_theta_rows(ThetaRows a)
 {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -333,7 +333,6 @@ __global__ void k_theta_rows(ThetaRows a)
     d[k] = c[k];
     g[k] = (float)c[k];
   }
-  if (q >= a.rows_r) return;
   const double delta = is_f ? a.drho : a.dr;
   const double s[4] = {3.0 * c[0] / delta, 2.0 * c[1] / delta, c[2] / delta, 0.0};  // c0..c2
   d = is_f ? d + 4 : a.slope_d + 4 * u;
@@ -353,8 +352,7 @@ void eam_theta_dev(Ctx& c, const double* theta)
   const int nel = e.nel, nz = nel * (nel + 1) / 2;
   ThetaRows a;
   a.rows_f = (int64_t)nel * (e.nrho + 1);
-  a.rows_r = a.rows_f + (int64_t)nel * (e.nr + 1);
-  a.rows = a.rows_r + (int64_t)nz * (e.nr + 1);
+  a.rows = a.rows_f + (int64_t)(nel + nz) * (e.nr + 1);
   a.nrho = e.nrho;
   a.nr = e.nr;
   a.drho = e.drho;

@@ -195,7 +195,8 @@ inline double xform_det(const XformDev& x)
 // keeps the value cubics of the others (EamHost).
 template <class Real>
 struct EamTabDev {
-  const Real* frho = nullptr;  // nel tables of (nrho+1) rows
+  const Real* frho = nullptr;   // nel tables of (nrho+1) rows
+  const Real* slope = nullptr;  // EamHost::slope_*
   int nel = 0, nr = 0, nrho = 0;
   Real rdr = 0, rdrho = 0, rhomax = 0, conv = 0;
   double rdr_d = 0;  // 1/dr in FP64 (the knot of r is found in FP64 in both forms)
@@ -222,7 +223,8 @@ struct EamHost {
   // serve both EAM passes
   DBuf<double> pair_d;
   DBuf<float> pair_f;
-  // rho'(r) rows [c0 c1 c2 0] of the nel rho tables, nr + 1 each (EAM adjoint)
+  // derivative rows [c0 c1 c2 0] of the rho and z2r tables, in the pair table's planes (the
+  // EAM adjoint and the FP32 alloy force pass)
   DBuf<double> slope_d;
   DBuf<float> slope_f;
   // FP32 s = r^2 tables after the knot planes of pair_f (pair_math.hpp): pieces
@@ -264,6 +266,7 @@ constexpr double kEV = 1.602176634e-19 / (1.66053906892e-27 * 1.0e4);
 constexpr double kBlockAtoms = 230.0;      // largest expected central atoms per brick
 constexpr size_t kLdsPerCu = 160 * 1024;   // LDS of one CU
 constexpr int kMaxHaloCells = 216;
+constexpr int kHaloGroups = 512;           // workgroups that size the halos
 constexpr size_t kBlockLdsLimit = 64 * 1024;  // default dynamic-LDS limit of a launch
 
 // Event-pair timing per kernel class (see XS_PROF_* in xsmd.h).
@@ -424,9 +427,11 @@ struct Ctx {
   char* pinned = nullptr;
 
   // small device scalars + pinned host mirror
-  DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..5] halo sizes,
-                                     // [6] the MD loop's rebuild flag (StepFlag)
+  DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..3] pair counts
+                                     // (list builds use [0..2]), [6] the MD loop's rebuild flag (StepFlag)
   unsigned long long* hscalar = nullptr;
+  uint32_t* hhalo = nullptr;  // written by kernels: 4 halo sizes of each of kHaloGroups workgroups, the
+                              // build's overflow mark
   DBuf<double> red_part;  // thermo partial sums
   DBuf<double> red_out;
   double* hthermo = nullptr;  // pinned host copy of the 27 results
