@@ -41,13 +41,34 @@ struct BlockShape {
 __device__ __forceinline__ BlockShape block_shape(const BlockGeom& g, int64_t b)
 {
   BlockShape s;
-  const int64_t per = (int64_t)g.nbx * g.nby * g.nbz;
-  s.r = (int)(b / per);
-  int64_t q = b - (int64_t)s.r * per;
-  const int ibx = (int)(q % g.nbx);
-  q /= g.nbx;
-  const int iby = (int)(q % g.nby);
-  const int ibz = (int)(q / g.nby);
+  // full bricks first (fx fy fz of each replica), then those the grid's edge cuts: the
+  // slab of the last brick along x, then along y and z of what is left
+  const int64_t full = (int64_t)g.fx * g.fy * g.fz;
+  const bool whole = b < g.nfull;
+  const int64_t per = whole ? full : (int64_t)g.nbx * g.nby * g.nbz - full;
+  int64_t q = whole ? b : b - g.nfull;
+  s.r = (int)(q / per);
+  q -= (int64_t)s.r * per;
+  int wx = g.fx, wy = g.fy, x0 = 0, y0 = 0, z0 = 0;  // extents of the part q counts in, and its origin
+  if (!whole) {
+    const int64_t sx = (int64_t)(g.nbx - g.fx) * g.nby * g.nbz, sy = (int64_t)(g.nby - g.fy) * g.fx * g.nbz;
+    if (q < sx) {
+      wx = g.nbx - g.fx;
+      wy = g.nby;
+      x0 = g.fx;
+    } else if (q < sx + sy) {
+      q -= sx;
+      wy = g.nby - g.fy;
+      y0 = g.fy;
+    } else {
+      q -= sx + sy;
+      z0 = g.fz;
+    }
+  }
+  const int ibx = x0 + (int)(q % wx);
+  q /= wx;
+  const int iby = y0 + (int)(q % wy);
+  const int ibz = z0 + (int)(q / wy);
   s.cx0 = ibx * g.bx;
   s.cy0 = iby * g.by;
   s.cz0 = ibz * g.bz;
@@ -186,10 +207,18 @@ __device__ void stage_cells(const BlockShape& s, const HaloCell* hc, int total, 
   __syncthreads();
 }
 
-__device__ __forceinline__ int64_t lblock()
+// Brick of this workgroup.  Hardware hands workgroup b to XCD b % 8: each XCD takes a
+// contiguous eighth of the full bricks (one contiguous piece of space for its L2), then
+// an eighth of the cut ones.  The cut ones last: started among the others they leave a
+// last round of full bricks on a mostly idle GPU.  500 k EAM atoms: 2057 full bricks of
+// 768 resident workgroups, 391 cut ones.
+__device__ __forceinline__ int64_t brick_of_block(int64_t nfull, int64_t nblocks)
 {
-  const unsigned b = blockIdx.x, g = gridDim.x;
-  return (int64_t)(b & 7u) * (g >> 3) + (b >> 3);
+  const int64_t k = blockIdx.x & 7u, p = blockIdx.x >> 3;
+  const int64_t f0 = nfull * k >> 3, nf = (nfull * (k + 1) >> 3) - f0;
+  if (p < nf) return f0 + p;
+  const int64_t cut = nblocks - nfull, c0 = cut * k >> 3, c = c0 + p - nf;
+  return c < (cut * (k + 1) >> 3) ? nfull + c : nblocks;
 }
 
 // Two lanes per central atom: the two halves of a wave take the same 32 atoms
@@ -221,7 +250,7 @@ struct BlockArgs {
   const uint16_t* __restrict__ nbr16;
   const int* __restrict__ nnb;
   int64_t npad;
-  int64_t nblocks;
+  int64_t nblocks, nfull;
   int cap;  // halo slots (LDS records)
   double rc2;
   int nmax;            // list capacity
@@ -548,7 +577,7 @@ __host__ __device__ inline size_t build_cand_bytes(int cap, int cand_cap)
 template <bool XF>
 __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
 {
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.g.nfull, a.g.nblocks);
   if (b >= a.g.nblocks) return;
   extern __shared__ __align__(32) unsigned char smem[];
   double3* P = reinterpret_cast<double3*>(smem);
@@ -799,7 +828,7 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
 // entry.  One wave per central atom.
 __global__ void __launch_bounds__(256) k_block_to_global(BlockArgs a, uint32_t* __restrict__ nbr)
 {
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.nfull, a.nblocks);
   if (b >= a.nblocks) return;
   const BrickHead hd(a.head[b]);
   const uint32_t* stage = a.stage + hd.stage;
@@ -1000,7 +1029,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<SPLIT>) k_block_eam_r
                                                                 double* __restrict__ rho_io,
                                                                 double* __restrict__ pos_w, double* __restrict__ ep)
 {
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.nfull, a.nblocks);
   if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, false, ltype);
@@ -1070,7 +1099,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
                                                                   pm::Drift dr)
 {
   static_assert(!DRIFT || (FUSED && !ENERGY && !VIRIAL), "the drift epilogue is the plain MD-loop step");
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.nfull, a.nblocks);
   if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, true, ltype);
@@ -1179,7 +1208,7 @@ struct AdjB1Args {
 template <class Real, bool MULTI, bool SPLIT>
 __global__ void __launch_bounds__(kPassThreads, 4) k_block_adj_b1(BlockArgs a, EamTabDev<Real> t, AdjB1Args g)
 {
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.nfull, a.nblocks);
   if (b >= a.nblocks) return;
   extern __shared__ __align__(32) unsigned char smem[];
   LRec rec;
@@ -1271,7 +1300,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<false>) k_block_gathe
                                                                                             const float* __restrict__ pair,
                                                                                             double* __restrict__ sink)
 {
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.nfull, a.nblocks);
   if (b >= a.nblocks) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, FORCE, ltype);
@@ -1356,7 +1385,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
                                                                            pm::LJMultiDev lm = {})
 {
   static_assert(!DRIFT || (FUSED && !ENERGY && !VIRIAL), "the drift epilogue is the plain MD-loop step");
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.nfull, a.nblocks);
   if (b >= a.nblocks || a.gate.closed()) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, MULTI, false, ltype);
@@ -1439,7 +1468,7 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs
                                                                        double* __restrict__ pos_w,
                                                                        double* __restrict__ ep)
 {
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.nfull, a.nblocks);
   if (b >= a.nblocks) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, false, ltype);
@@ -1488,7 +1517,7 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs
 template <bool VIRIAL, bool SPLIT>
 __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_force(BlockArgs a, JohnsonParams jp, pm::Outputs o)
 {
-  const int64_t b = lblock();
+  const int64_t b = brick_of_block(a.nfull, a.nblocks);
   if (b >= a.nblocks) return;
   uint8_t* ltype;
   const LRec rec = pass_lds(a, false, true, ltype);
@@ -1556,6 +1585,7 @@ BlockArgs block_args(const Ctx& c, double rcut, const StepGate& gate = {})
   a.nnb = c.nnb.p;
   a.npad = c.npad;
   a.nblocks = c.bgeom.nblocks;
+  a.nfull = c.bgeom.nfull;
   a.cap = c.bcap;
   a.rc2 = rcut * rcut;
   a.xf = c.xf_dev();
@@ -1722,6 +1752,10 @@ void block_shape_choose(const Ctx& c, BlockGeom& g, double bound, double per_cel
   g.nby = (g.ny + by - 1) / by;
   g.nbz = (g.nz + bz - 1) / bz;
   g.nblocks = (int64_t)g.nbx * g.nby * g.nbz * c.nrep;
+  g.fx = g.nx / bx;
+  g.fy = g.ny / by;
+  g.fz = g.nz / bz;
+  g.nfull = (int64_t)g.fx * g.fy * g.fz * c.nrep;
   g.nh_max = (bx + 2) * (by + 2) * (bz + 2);
 }
 
@@ -1786,7 +1820,8 @@ bool block_feasible(const Ctx& c)
 
 unsigned block_grid(const Ctx& c)
 {
-  return (unsigned)((c.bgeom.nblocks + 7) / 8 * 8);
+  // every XCD's share of the full and of the cut bricks (brick_of_block)
+  return (unsigned)(8 * ((c.bgeom.nfull + 7) / 8 + (c.bgeom.nblocks - c.bgeom.nfull + 7) / 8));
 }
 
 // LDS of a build launch that collects `atoms` lists per wave

@@ -257,7 +257,9 @@ struct BlockGeom {
   int px, py, pz;
   int nh_max;        // (bx+2)(by+2)(bz+2) halo cells
   int64_t ncell_rep;
+  int fx, fy, fz;    // bricks per axis that the grid's edge does not cut
   int64_t nblocks;   // over all replicas
+  int64_t nfull;     // uncut ones, numbered first (block_shape)
 };
 
 // 1 eV in exaStamp's internal energy unit Da.A^2/ps^2: e / (amu * 1e4 J), exact SI
