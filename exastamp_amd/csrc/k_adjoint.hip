@@ -188,8 +188,9 @@ __global__ void __launch_bounds__(256) k_adj_b1(AdjArgs a, EamTabDev<Real> t)
     const int tj = MULTI ? a.type[j] : 0;
     if (MULTI && !adj_on(a, tj)) continue;
     const double* gj = reinterpret_cast<const double*>(a.gvec + j);
-    const double r = sqrt(d2);
-    const double s = (dx * (gj[0] - gi[0]) + dy * (gj[1] - gi[1]) + dz * (gj[2] - gi[2])) / r;
+    double r, rinv;
+    pm::dist(d2, r, rinv);
+    const double s = (dx * (gj[0] - gi[0]) + dy * (gj[1] - gi[1]) + dz * (gj[2] - gi[2])) * rinv;
     int m;
     double p;
     adj_knot(r, a.rdr, a.nr, m, p);
@@ -319,7 +320,8 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_pairs(AdjArgs a, AdjWindows
         }
         const double both = wi + wj;
         if (both == 0.0) continue;
-        const double r = sqrt(d2), ir = 1.0 / r;
+        double r, ir;
+        pm::dist(d2, r, ir);
         // s_ij = u_ij . (g_i - g_j), u_ij = -(dx,dy,dz)/r
         const double s = (dx * (gj.x - gi.x) + dy * (gj.y - gi.y) + dz * (gj.z - gi.z)) * ir;
         int m;

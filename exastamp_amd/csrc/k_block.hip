@@ -947,25 +947,27 @@ struct LNb {
 // record (a pair longer than any cutoff).  The passes load the next group's word one
 // iteration ahead (none at the end of the list).  In the bl_index layout the word of
 // (gi, half + 8 q) is word 2 gi + half of group q, whose words start q * 2 npad words
-// into the array.  Every lane of a wave is at the same q in a given iteration, so
-// the group's start is one scalar address and each lane adds its own fixed 32-bit
-// offset (the list holds at most 2^26 atoms x 64 entries = 2^30 words).
+// into the array; a lane steps its own pointer, one 64-bit add (from the group's number,
+// which the compiler cannot know to be the same in every lane, it took eight
+// instructions of the 40 to 80 per list word).
 template <bool SPLIT>
 struct LWords {
-  const uint2* base;
-  uint32_t lane;  // this lane's word within a group
-  int64_t step;   // words to the lane's next group
-  int q = 0;
+  const uint2* at;  // this lane's word of its current group
+  int64_t step;     // words to its next group
   __device__ __forceinline__ LWords(const BlockArgs& a, int64_t gi, const PassLanes<SPLIT>& ln)
-      : base(reinterpret_cast<const uint2*>(a.nbr16)), lane((uint32_t)(2 * gi + ln.half)), step(2 * a.npad)
+      : at(reinterpret_cast<const uint2*>(a.nbr16) + 2 * gi + ln.half), step(2 * a.npad)
   {
     if constexpr (SPLIT) {
-      base += ln.part * step;
+      at += ln.part * step;
       step <<= ln.log;
     }
   }
-  __device__ __forceinline__ uint2 first() const { return base[lane]; }
-  __device__ __forceinline__ uint2 next() { return (base + ++q * step)[lane]; }
+  __device__ __forceinline__ uint2 first() const { return *at; }
+  __device__ __forceinline__ uint2 next()
+  {
+    at += step;
+    return *at;
+  }
 };
 // A central atom on its way: its index and slot, then the length of its list and the
 // lane's first list word.  The first atom of each lane is fetched while the halo is
@@ -1259,8 +1261,9 @@ __global__ void __launch_bounds__(kPassThreads, 4) k_block_adj_b1(BlockArgs a, E
       for (int u = 0; u < kBBatch; u++) {
         const int tj = MULTI ? ltype[nb[u].c] : 0;
         const double* gj = gl + 3 * nb[u].c;
-        const double r = sqrt(nb[u].d2);
-        const double s = (nb[u].x * (gj[0] - g0) + nb[u].y * (gj[1] - g1) + nb[u].z * (gj[2] - g2)) / r;
+        double r, rinv;
+        pm::dist(nb[u].d2, r, rinv);
+        const double s = (nb[u].x * (gj[0] - g0) + nb[u].y * (gj[1] - g1) + nb[u].z * (gj[2] - g2)) * rinv;
         double p = fma(r, t.rdr_d, 1.0);
         const int m = max(0, min((int)p, t.nr - 1));
         p = fmin(p - (double)m, 1.0);

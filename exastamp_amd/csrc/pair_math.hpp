@@ -29,14 +29,49 @@ __device__ __forceinline__ Q4<double> load4(const double* __restrict__ p)
   return {u.x, u.y, w.x, w.y};
 }
 
-// sqrt(d2) and 1/sqrt(d2) correctly rounded in FP64 (what plain FP64 code compiles to)
+// Distance from its square, and the reciprocal distance, in FP64.  The compiler's square
+// root and division scale for the ends of the exponent range and fix up special cases: 29
+// instructions of the 79 per list entry of the FP64 force pass.  Squared distances need
+// none of that, so both come from the hardware's reciprocal square root y (about 2^-23) by
+// Goldschmidt's iteration: g -> sqrt, h -> 1 / (2 sqrt), then one residual step each,
+// 11 instructions.  On 8.4 M values from 0.01 to 1e12 r equals sqrt(d2) in every one and
+// rinv is as far from the exact reciprocal as 1 / r (1.50 ulp at most, 0.36 on average);
+// recip equals 1 / x.  d2 = 0 gives NaN where the division gave NaN or infinity.
+__device__ __forceinline__ void dist_steps(double d2, double y, double& g, double& h)
+{
+  g = d2 * y;
+  h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, d2), h, g);
+}
 __device__ __forceinline__ void dist(double d2, double& r, double& rinv)
 {
-  r = sqrt(d2);
-  rinv = 1.0 / r;
+  double h;
+  dist_steps(d2, __builtin_amdgcn_rsq(d2), r, h);
+  const double y = h + h;
+  rinv = fma(fma(-y, r, 1.0), y, y);
+}
+// the distance alone; finite at d2 = 0 (1e-145, the table's first knot)
+__device__ __forceinline__ double dist(double d2)
+{
+  double r, h;
+  // the larger of the two by their upper halves (fmax first quiets NaNs, an instruction more)
+  const unsigned long long b = (unsigned long long)__double_as_longlong(d2);
+  const uint32_t hi = (uint32_t)max((int)(b >> 32), 0x03b90000);
+  const double x = __longlong_as_double((long long)((unsigned long long)hi << 32 | (uint32_t)b));
+  dist_steps(x, __builtin_amdgcn_rsq(x), r, h);
+  return r;
 }
 __device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double recip(double x) { return 1.0 / x; }
+// Newton's iteration on the hardware's reciprocal, without the division's scaling
+__device__ __forceinline__ double recip(double x)
+{
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
 __device__ __forceinline__ float fma_r(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ double fma_r(double a, double b, double c) { return fma(a, b, c); }
 
@@ -151,8 +186,7 @@ template <class Real>
 __device__ __forceinline__ void knot_r(const EamTabDev<Real>& t, Real r, int& m, Real& p)
 {
   p = r * t.rdr + Real(1);
-  m = (int)p;
-  m = max(0, min(m, t.nr - 1));
+  m = min((int)p, t.nr - 1);  // r is not negative, and NaN converts to 0
   p -= (Real)m;
   p = fmin(p, Real(1));
 }
@@ -160,7 +194,6 @@ __device__ __forceinline__ void knot_r(const EamTabDev<Real>& t, Real r, int& m,
 // Distance, 1/r and spline knot of a pair from its FP64 d^2 (the first steps of
 // eam_alloy_rho_noderiv / eam_alloy_mm_force, eam_alloy.h:198-265: p = r rdr + 1,
 // m = min(int p, nr - 1), p -= m, p = min(p, 1)).
-// FP64 form: correctly rounded sqrt and division, as plain FP64 code.
 // Mixed form: the knot fraction of r ~ 5 A at 1000 knots per A needs more than FP32
 // (its ulp at p ~ 5000 is 5e-4 of a knot, which puts ~1e-5 of relative error on the
 // forces of atoms whose pair forces nearly cancel), so 1/sqrt(d2) is the FP32
@@ -173,16 +206,25 @@ __device__ __forceinline__ void knot_dist(const EamTabDev<double>& t, double d2,
   dist(d2, r, rinv);
   knot_r(t, r, m, p);
 }
+// the knot alone
+__device__ __forceinline__ void knot_dist(const EamTabDev<double>& t, double d2, int& m, double& p)
+{
+  knot_r(t, dist(d2), m, p);
+}
 __device__ __forceinline__ void knot_dist(const EamTabDev<float>& t, double d2, int& m, float& p, float& rinv)
 {
   const double y0 = (double)__builtin_amdgcn_rsqf((float)d2);
   const double y = y0 * fma(-0.5 * d2 * y0, y0, 1.5);
   double q = fma(d2 * y, t.rdr_d, 1.0);
-  m = (int)q;
-  m = max(0, min(m, t.nr - 1));
+  m = min((int)q, t.nr - 1);
   q -= (double)m;
   p = (float)fmin(q, 1.0);
   rinv = (float)y;
+}
+__device__ __forceinline__ void knot_dist(const EamTabDev<float>& t, double d2, int& m, float& p)
+{
+  float rinv;
+  knot_dist(t, d2, m, p, rinv);
 }
 
 // Element `i` of a table whose base is the same for every lane: the byte offset is
@@ -383,9 +425,9 @@ template <class Real, bool MULTI>
 __device__ __forceinline__ Real eam_rho_knot(const EamTabDev<Real>& t, const Real* __restrict__ pair, int ti, int tj,
                                              double d2, bool in)
 {
-  Real p, rinv;
+  Real p;
   int m;
-  knot_dist(t, in ? d2 : 1.0, m, p, rinv);
+  knot_dist(t, in ? d2 : 1.0, m, p);
   const Real* row;
   if constexpr (MULTI) row = pair_row(pair, t, max(ti, tj) < t.nel ? tj : 0, m);
   else row = pair_rho_row(pair, m);
@@ -490,7 +532,7 @@ __device__ __forceinline__ void johnson_term(double a, double k, double x, doubl
 __device__ __forceinline__ double johnson_rho(const JohnsonParams& p, double d2)
 {
   double t, dt;
-  johnson_term(p.beta, p.lambda, sqrt(d2) / p.re, t, dt);
+  johnson_term(p.beta, p.lambda, dist(d2) / p.re, t, dt);
   return p.fe * t;
 }
 
@@ -498,12 +540,15 @@ __device__ __forceinline__ double johnson_rho(const JohnsonParams& p, double d2)
 __device__ __forceinline__ void johnson_pair(const JohnsonParams& p, double d2, double fsum, double& de_r,
                                              double& phi)
 {
-  const double r = sqrt(d2), ire = 1.0 / p.re, x = r * ire;
+  const double ire = 1.0 / p.re;
+  double r, rinv;
+  dist(d2, r, rinv);
+  const double x = r * ire;
   double t1, d1, t2, d2x;
   johnson_term(p.alpha, p.kappa, x, t1, d1);
   johnson_term(p.beta, p.lambda, x, t2, d2x);
   phi = p.A * t1 - p.B * t2;
-  de_r = (fma(p.fe, fsum, -p.B) * d2x + p.A * d1) * ire / r;
+  de_r = (fma(p.fe, fsum, -p.B) * d2x + p.A * d1) * ire * rinv;
 }
 
 // F(rho) and F'(rho) (johnson.h:131-167): cubic in rho / (0.85 rhoe) - 1 below
