@@ -991,6 +991,7 @@ struct PassAtom {
   }
   __device__ __forceinline__ void fetch(const BlockArgs& a, const BrickHead& hd, int q, const PassLanes<SPLIT>& ln)
   {
+    cnt = 0;
     if (q >= hd.central) return;
     index(a, hd, q);
     list(a, ln);
@@ -1004,6 +1005,18 @@ __device__ __forceinline__ void lslots(uint2 w, int far_slot, int k0, int cnt, i
   const int fs = far_slot & 0xffff;
 #pragma unroll
   for (int u = 0; u < 4; u++) c[u] = (k0 + 2 * u < cnt) ? raw[u] : fs;
+}
+
+// FP64 table rows are loaded by pairs of neighbouring lanes (pm::RowPair), which hold
+// consecutive atoms: both stay to the end of the longer list, and a lane whose neighbour
+// has the brick's last atom runs along with an empty one.
+template <class Real>
+constexpr bool kPaired = sizeof(Real) == 8;
+template <class Real>
+__device__ __forceinline__ int pair_end(int cnt)
+{
+  if constexpr (kPaired<Real>) return max(cnt, (int)pm::dpp_xor1((uint32_t)cnt));
+  return cnt;
 }
 
 // neighbour records of slots c[0..U-1] (entries k0, k0 + 2, ...)
@@ -1042,7 +1055,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<SPLIT>) k_block_eam_r
   stage<false>(a, hd, rec, ltype);
   if (ln.slot < hd.central) at.list(a, ln);
   __syncthreads();
-  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
+  for (int q = ln.slot; (kPaired<Real> ? q & ~1 : q) < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
     const int64_t gi = at.gi;
     const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
@@ -1052,9 +1065,10 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<SPLIT>) k_block_eam_r
     double rho = 0.0;
     LWords<SPLIT> lw(a, gi, ln);
     uint2 wnext = at.w;
-    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
+    const int end = pair_end<Real>(cnt);
+    for (int k0 = ln.first(); k0 < end; k0 += ln.step()) {
       const uint2 w = wnext;
-      if (k0 + ln.step() < cnt) wnext = lw.next();
+      if (k0 + ln.step() < end) wnext = lw.next();
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
       LNb nb[kBBatch];
@@ -1074,12 +1088,12 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<SPLIT>) k_block_eam_r
         const int tj = MULTI ? ltype[nb[u].c] : 0;
         // every d2 here is finite and positive (entries past the count read the far
         // record), so the knot index needs no guard value; the sum masks by `in`
-        const Real val = pm::eam_rho_knot<Real, MULTI>(t, pair, ti, tj, nb[u].d2, true);
+        const Real val = pm::eam_rho_knot<Real, MULTI, kPaired<Real>>(t, pair, ti, tj, nb[u].d2, true);
         rho += (double)(nb[u].in ? val : Real(0));
       }
     }
     rho = ln.sum(rho);
-    if (ln.writes()) {
+    if (ln.writes() && (!kPaired<Real> || q < hd.central)) {
       rho_io[gi] = rho;
       if constexpr (EMB) {
         Real F, Fp;
@@ -1112,7 +1126,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
   stage<true>(a, hd, rec, ltype);
   if (ln.slot < hd.central) at.list(a, ln);
   __syncthreads();
-  for (int q = ln.slot; q < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
+  for (int q = ln.slot; (kPaired<Real> ? q & ~1 : q) < hd.central; q += ln.atoms(), at.fetch(a, hd, q, ln)) {
     const int64_t gi = at.gi;
     const int slot = at.slot;
     const Pos4 pi = rec.get(slot);
@@ -1123,9 +1137,10 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     LWords<SPLIT> lw(a, gi, ln);
     uint2 wnext = at.w;
-    for (int k0 = ln.first(); k0 < cnt; k0 += ln.step()) {
+    const int end = pair_end<Real>(cnt);
+    for (int k0 = ln.first(); k0 < end; k0 += ln.step()) {
       const uint2 w = wnext;
-      if (k0 + ln.step() < cnt) wnext = lw.next();
+      if (k0 + ln.step() < end) wnext = lw.next();
       int c[kBBatch];
       lslots(w, a.cap, k0, cnt, c);
       // two entries at a time: their four table rows stay in flight together within
@@ -1171,7 +1186,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
           for (int u = 0; u < 2; u++) {
             const int tj = MULTI ? ltype[nb[u].c] : 0;
             Real fp_r, phi;
-            pm::eam_pair_knot<Real, MULTI>(t, pair, ti, tj, fpi, (Real)nb[u].w, nb[u].d2, true, fp_r, phi);
+            pm::eam_pair_knot<Real, MULTI, kPaired<Real>>(t, pair, ti, tj, fpi, (Real)nb[u].w, nb[u].d2, true, fp_r, phi);
             add(nb[u], nb[u].in, fp_r, phi);
           }
         }
@@ -1186,7 +1201,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
 #pragma unroll
       for (int k = 0; k < 9; k++) v[k] = ln.sum(v[k]);
     }
-    if (ln.writes()) {
+    if (ln.writes() && (!kPaired<Real> || q < hd.central)) {
       if constexpr (DRIFT) pm::write_outputs_drift(o, dr, gi, pi, fx, fy, fz);
       else pm::write_outputs<ENERGY, VIRIAL, FUSED>(o, gi, fx, fy, fz, e, v);
     }

@@ -237,6 +237,51 @@ __device__ __forceinline__ const T* at32(const T* base, uint32_t i)
   return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (i * (uint32_t)sizeof(T)));
 }
 
+// A 32-byte row of a table, loaded together with the neighbouring lane's (lane ^ 1, which
+// must be active and do the same): one load takes the two halves of the even lane's row,
+// the next those of the odd lane's, and the halves change lanes in registers.  A lane's load
+// of 16 bytes looks up the cache line of each row it touches; two loads of 64 scattered rows
+// look up about 100 lines, two of 32 rows each, whole, little more than half, and the FP64
+// passes are bound by those lookups (texture address and data units busy 80 % of the time).
+// 500 k EAM atoms, FP64: lookups of the force pass 84 -> 48 million, 118 -> 104 us, density
+// pass 65 -> 56.  The mixed force pass, whose rows are 32 bytes too, pays more for
+// the exchange than it gains (8.39 M atoms: 1139 -> 1346 us).
+__device__ __forceinline__ uint32_t dpp_xor1(uint32_t v)
+{
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppXor1, 0xf, 0xf, true);
+}
+// the rows of a pair of lanes: byte offsets, within a table, of this lane's halves of the
+// even and of the odd lane's row
+struct RowPair {
+  uint32_t even, odd;
+  __device__ __forceinline__ explicit RowPair(uint32_t row)
+  {
+    const bool is_odd = threadIdx.x & 1;
+    const uint32_t half = is_odd ? 16u : 0u, other = dpp_xor1(row);
+    even = (is_odd ? other : row) << 5 | half;
+    odd = (is_odd ? row : other) << 5 | half;
+  }
+};
+__device__ __forceinline__ Q4<double> load_row(const double* base, const RowPair& r)
+{
+  const bool is_odd = threadIdx.x & 1;
+  const uint4 e = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base) + r.even);
+  const uint4 o = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base) + r.odd);
+  // both lanes take part in the exchanges, so they come before the selections
+  const uint4 xe = make_uint4(dpp_xor1(e.x), dpp_xor1(e.y), dpp_xor1(e.z), dpp_xor1(e.w));
+  const uint4 xo = make_uint4(dpp_xor1(o.x), dpp_xor1(o.y), dpp_xor1(o.z), dpp_xor1(o.w));
+  const uint4 lo = is_odd ? xo : e, hi = is_odd ? o : xe;
+  return {__hiloint2double((int)lo.y, (int)lo.x), __hiloint2double((int)lo.w, (int)lo.z),
+          __hiloint2double((int)hi.y, (int)hi.x), __hiloint2double((int)hi.w, (int)hi.z)};
+}
+// Row `row` of four values; PAIRED: with the neighbouring lane (FP64 rows)
+template <bool PAIRED, class Real>
+__device__ __forceinline__ Q4<Real> load_row(const Real* base, uint32_t row)
+{
+  if constexpr (PAIRED && sizeof(Real) == 8) return load_row(base, RowPair(row));
+  else return load4(at32(base, row * 4u));
+}
+
 template <class Real>
 __device__ __forceinline__ Real cubic(const Q4<Real>& c, Real p)
 {
@@ -304,10 +349,15 @@ __device__ __forceinline__ void embed(const EamTabDev<Real>& t, int ti, double r
 // line, so the clustered knots that the lanes of a wave look up touch few lines; the
 // derivative quadratics follow from the value cubics.
 template <class Real>
+__device__ __forceinline__ uint32_t row_index(const EamTabDev<Real>& t, int plane, int m)
+{
+  return (uint32_t)plane * (uint32_t)(t.nr + 1) + (uint32_t)m;
+}
+template <class Real>
 __device__ __forceinline__ const Real* pair_row(const Real* __restrict__ pair, const EamTabDev<Real>& t, int plane,
                                                 int m)
 {
-  return at32(pair, ((uint32_t)plane * (uint32_t)(t.nr + 1) + (uint32_t)m) * 4u);
+  return at32(pair, row_index(t, plane, m) * 4u);
 }
 // Planes of the pair of types ti, tj (type t is element t; initialize_types_table,
 // eam_alloy.h:70-133): rho of each and their z2r, in arithmetic.  A type map is one more
@@ -328,12 +378,6 @@ __device__ __forceinline__ const Real* pair_rho_row(const Real* __restrict__ pai
 {
   return at32(pair, (uint32_t)m * 4u);
 }
-template <class Real>
-__device__ __forceinline__ const Real* pair_z2_row(const Real* __restrict__ pair, const EamTabDev<Real>& t, int m)
-{
-  return at32(pair, (uint32_t)(t.nr + 1 + m) * 4u);
-}
-
 // Single-element psi'(r)/r and phi(r) from the two rows of knot m:
 // rc = rho value cubic, zc = z2r value cubic; the derivative quadratics follow
 // from the value cubics (times 1/dr).
@@ -421,22 +465,20 @@ constexpr bool kSTable = !MULTI && sizeof(Real) == 4;
 // evaluates at d2 = 1 instead (a guard for list padding whose d2 may be 0); the value
 // of a pair that does not count is arbitrary and callers mask it.  Callers whose d2 is
 // always finite and positive pass true.
-template <class Real, bool MULTI>
+template <class Real, bool MULTI, bool PAIRED = false>
 __device__ __forceinline__ Real eam_rho_knot(const EamTabDev<Real>& t, const Real* __restrict__ pair, int ti, int tj,
                                              double d2, bool in)
 {
   Real p;
   int m;
   knot_dist(t, in ? d2 : 1.0, m, p);
-  const Real* row;
-  if constexpr (MULTI) row = pair_row(pair, t, max(ti, tj) < t.nel ? tj : 0, m);
-  else row = pair_rho_row(pair, m);
-  return cubic(load4(row), p);
+  const int plane = MULTI && max(ti, tj) < t.nel ? tj : 0;
+  return cubic(load_row<PAIRED>(pair, row_index(t, plane, m)), p);
 }
 
 // psi'(r)/r and phi(r) of eam_alloy_mm_force (eam_alloy.h:222-265) from the knot
 // rows: psi' = F'_i rho'_j + F'_j rho'_i + phi', phi = z2r / r.
-template <class Real, bool MULTI>
+template <class Real, bool MULTI, bool PAIRED = false>
 __device__ __forceinline__ void eam_pair_knot(const EamTabDev<Real>& t, const Real* __restrict__ pair, int ti, int tj,
                                               Real fpi, Real fpj, double d2, bool in, Real& fpair, Real& phi)
 {
@@ -446,7 +488,7 @@ __device__ __forceinline__ void eam_pair_knot(const EamTabDev<Real>& t, const Re
   if constexpr (MULTI) {
     int pi, pj, pz;
     pair_planes(t.nel, ti, tj, pi, pj, pz);
-    const Q4<Real> zc = load4(pair_row(pair, t, pz, m));
+    const Q4<Real> zc = load_row<PAIRED>(pair, row_index(t, pz, m));
     // FP32: derivative rows of their own; 1/dr and the cubic's coefficients each rounded
     // would add to the forces' error (2.27e-7 of their rms against 2.45e-7)
     Real rhoip, rhojp, z2p;
@@ -455,8 +497,8 @@ __device__ __forceinline__ void eam_pair_knot(const EamTabDev<Real>& t, const Re
       rhojp = quad(load4(pair_row(t.slope, t, pj, m)), p);
       z2p = quad(load4(pair_row(t.slope, t, pz, m)), p);
     } else {
-      rhoip = dcubic(load4(pair_row(pair, t, pi, m)), p) * t.rdr;
-      rhojp = dcubic(load4(pair_row(pair, t, pj, m)), p) * t.rdr;
+      rhoip = dcubic(load_row<PAIRED>(pair, row_index(t, pi, m)), p) * t.rdr;
+      rhojp = dcubic(load_row<PAIRED>(pair, row_index(t, pj, m)), p) * t.rdr;
       z2p = dcubic(zc, p) * t.rdr;
     }
     const Real z2 = cubic(zc, p);
@@ -474,7 +516,14 @@ __device__ __forceinline__ void eam_pair_knot(const EamTabDev<Real>& t, const Re
     phi *= t.conv;
     fpair = psip * rinv;
   } else {
-    eam_pair_rows(t, load4(pair_rho_row(pair, m)), load4(pair_z2_row(pair, t, m)), p, rinv, fpi, fpj, fpair, phi);
+    const Real* z2r = pair + 4 * (t.nr + 1);  // the second plane, at the same offset
+    if constexpr (PAIRED && sizeof(Real) == 8) {
+      const RowPair r((uint32_t)m);
+      eam_pair_rows(t, load_row(pair, r), load_row(z2r, r), p, rinv, fpi, fpj, fpair, phi);
+    } else {
+      eam_pair_rows(t, load4(at32(pair, (uint32_t)m * 4u)), load4(at32(z2r, (uint32_t)m * 4u)), p, rinv, fpi, fpj,
+                    fpair, phi);
+    }
   }
 }
 
