@@ -97,6 +97,10 @@ SIGNATURES = {
     "xs_eam_theta_dev": (C.c_int, [_CTX, C.c_void_p]),
     "xs_forces_energies_dev": (C.c_int, [_CTX, C.c_void_p, C.c_void_p, C.c_double]),
     "xs_lj_adjoint": (C.c_int, [_CTX, C.c_double, C.c_double, C.c_double, _D, _D, _D, C.c_uint]),
+    "xs_fit_loss_dev": (C.c_int, [C.c_int, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p,
+                                  C.c_void_p, C.c_void_p, C.c_double, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "xs_fit_loss_grad_dev": (C.c_int, [C.c_int, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p,
+                                       C.c_void_p, C.c_double, C.c_void_p, C.c_void_p, C.c_void_p]),
     "xs_spline_adjoint": (C.c_int, [C.c_int, C.c_double, _D, _D]),
     "xs_stream_copy": (C.c_int, [_CTX, C.c_size_t, C.c_int, _D]),
     "xs_gather_ceiling": (C.c_int, [_CTX, C.c_double, C.c_int, C.c_int, C.c_int, _D]),

@@ -268,6 +268,17 @@ xs_status xs_eam_adjoint(xs_ctx* ctx, double rcut, const double* dL_dF, const do
  * loss on the device. */
 xs_status xs_eam_adjoint_dev(xs_ctx* ctx, double rcut, const double* dL_dF_dev, const double* dL_dE_dev,
                              double scale, double* grad_dev, unsigned flags);
+/* The fitting loss of device arrays on a caller's stream of `device`, and its gradient; no
+ * context, nothing waits.  rF = F - Ft (nF values), rE = (E - Et) / n (nE), loss =
+ * mean(rF^2) + energy_weight mean(rE^2); partials: scratch of XS_FIT_LOSS_PARTIALS doubles.
+ * Then for dL = *g: gF = dL 2 rF / nF, gE = dL 2 energy_weight rE / (n nE). */
+#define XS_FIT_LOSS_PARTIALS 1024
+xs_status xs_fit_loss_dev(int device, void* stream, int64_t nF, const double* F, const double* Ft, int64_t nE,
+                          const double* E, const double* Et, const double* n, double energy_weight, double* rF,
+                          double* rE, double* partials, double* loss);
+xs_status xs_fit_loss_grad_dev(int device, void* stream, int64_t nF, const double* rF, int64_t nE,
+                               const double* rE, const double* n, double energy_weight, const double* g,
+                               double* gF, double* gE);
 /* No counterpart in exaStamp (the fitting counterpart of eam_alloy_init for new knot
  * values): theta_dev holds knots in xs_eam_adjoint's setfl order, on the grid (nel,
  * nrho, drho, nr, dr, rcut) of the tables loaded last, in device memory.  The spline
