@@ -39,9 +39,9 @@
 // like the density pass (k_block_adj_b1); the second gathers positions and loss gradients
 // through the list, since the accumulators take the LDS a brick's halo would need.
 // Bound by the LDS atomics (8 to 12 per pair) and the gathers (64 bytes per pair).
-// 1.04 M Cu/Ni atoms, 2000 knots: first sweep 233 us, second 532 us, F rows 11 us; walking
+// 1.04 M Cu/Ni atoms, 2000 knots: first sweep 198 us, second 473 us, F rows 11 us; walking
 // every list entry on the global list, with four coefficients per row and so three
-// launches, took 1107 + 2 x 645 us.  55 k atoms, 500 knots: 16 + 36 us against 80.
+// launches, took 1107 + 2 x 645 us.  55 k atoms, 500 knots: 13 + 35 us against 80.
 #include "pair_math.hpp"
 
 #include <algorithm>
@@ -136,9 +136,20 @@ struct Hermite {
   }
 };
 
-// value weight wv and p-derivative weight ws at knot m (1-based) of table T
+// value weight wv and p-derivative weight ws at knot m (1-based) of table T; WHOLE: the
+// launch holds every row of its tables
+template <bool WHOLE>
 __device__ __forceinline__ void adj_add(const AdjAcc& A, int T, int m, const Hermite& h, double wv, double ws)
 {
+  if constexpr (WHOLE) {
+    const double f = wv * h.h01 + ws * h.d01;
+    const int at = A.win[T].off + m - 1;
+    atomicAdd(A.f + at, wv - f);
+    atomicAdd(A.f + at + 1, f);
+    atomicAdd(A.s + at, wv * h.h10 + ws * h.d10);
+    atomicAdd(A.s + at + 1, wv * h.h11 + ws * h.d11);
+    return;
+  }
   const AdjWin w = A.win[T];
   const int row = m - 1 - w.lo;
   const double f1 = wv * h.h01 + ws * h.d01;
@@ -211,7 +222,7 @@ __global__ void __launch_bounds__(256) k_adj_b1(AdjArgs a, EamTabDev<Real> t)
 }
 
 // The F-table weights of atom i (a disabled species has no embedding term)
-template <bool MULTI>
+template <bool MULTI, bool WHOLE>
 __device__ __forceinline__ void adj_embed_add(const AdjArgs& a, const AdjAcc& acc, int64_t i)
 {
   const int ti = MULTI ? a.type[i] : 0;
@@ -221,7 +232,7 @@ __device__ __forceinline__ void adj_embed_add(const AdjArgs& a, const AdjAcc& ac
   double p;
   adj_knot(rho, a.rdrho, a.nrho, m, p);
   const double over = rho > a.rhomax ? rho - a.rhomax : 0.0;
-  adj_add(acc, f_table(a, ti), m, Hermite(p), ge * a.conv, a.conv * (ge * over - a.drho[i]) * a.rdrho);
+  adj_add<WHOLE>(acc, f_table(a, ti), m, Hermite(p), ge * a.conv, a.conv * (ge * over - a.drho[i]) * a.rdrho);
 }
 
 // F-table rows where they have launches of their own
@@ -231,7 +242,7 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_fsum(AdjArgs a, AdjWindows 
   extern __shared__ double lds[];
   const AdjAcc acc(lds, W);
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * blockDim.x)
-    adj_embed_add<MULTI>(a, acc, i);
+    adj_embed_add<MULTI, false>(a, acc, i);
   acc.out(part);
 }
 
@@ -239,8 +250,10 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_fsum(AdjArgs a, AdjWindows 
 // (an atom's own images come as two entries, which take half each), and with FSUM the
 // F-table rows.  1 << lanes_log lanes per atom.  A lane first marks which of its entries
 // are its to take, up to 64 of them, then walks the marked ones, so that lanes whose
-// neighbour had the larger index do not idle through the pair's arithmetic.
-template <bool MULTI, bool BLOCK, bool FSUM>
+// neighbour had the larger index do not idle through the pair's arithmetic; the next pair's
+// records are fetched while one is evaluated (1.04 M atoms: 521 -> 473 us with the rows'
+// window tests left out where the launch holds whole tables).
+template <bool MULTI, bool BLOCK, bool FSUM, bool WHOLE>
 __global__ void __launch_bounds__(kAdjThreads) k_adj_pairs(AdjArgs a, AdjWindows W, int lanes_log,
                                                            double* __restrict__ part)
 {
@@ -251,7 +264,7 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_pairs(AdjArgs a, AdjWindows
   const int64_t per = (a.n + gridDim.x - 1) / gridDim.x;
   const int64_t first = lblock() * per, end = min(first + per, a.n);
   for (int64_t i = first + (threadIdx.x >> lanes_log); i < end; i += blockDim.x >> lanes_log) {
-    if (FSUM && sub == 0) adj_embed_add<MULTI>(a, acc, i);
+    if (FSUM && sub == 0) adj_embed_add<MULTI, WHOLE>(a, acc, i);
     const int ti = MULTI ? a.type[i] : 0;
     const int rep = a.rep ? a.rep[i] : 0;
     const double* Lb = a.box[rep].L;
@@ -260,10 +273,12 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_pairs(AdjArgs a, AdjWindows
     const double ge = a.gE[rep];
     const int cnt = (!MULTI || adj_on(a, ti)) ? a.nnb[i] : 0;
     const uint32_t base = BLOCK ? a.base[i] : 0;
+    const uint32_t iu = (uint32_t)i;
     // bit 8 t + u of a lane's mask: place u of its t-th group (BLOCK), or its (8 t + u)-th entry
     for (int k0 = 0; k0 < cnt; k0 += 64 * lanes) {
       unsigned long long mask = 0;
       for (int t = 0; t < 8; t++) {
+        uint32_t m8 = 0;
         if constexpr (BLOCK) {
           const int g = (k0 >> 3) + sub + lanes * t;
           if (8 * g >= cnt) break;
@@ -274,46 +289,66 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_pairs(AdjArgs a, AdjWindows
             const int k = 8 * g + (u < 4 ? 2 * u : 2 * u - 7);
             const uint32_t slot = u & 1 ? ws[u >> 1] >> 16 : ws[u >> 1] & 0xffffu;
             const uint32_t j = xsmd_nbr_index(a.stage[base + (k < cnt ? slot : 0u)]);
-            if (k < cnt && (int64_t)j >= i) mask |= 1ull << (8 * t + u);
+            m8 |= (k < cnt && j >= iu ? 1u : 0u) << u;
           }
         } else {
           for (int u = 0; u < 8; u++) {
             const int k = k0 + sub + lanes * (8 * t + u);
-            if (k < cnt && (int64_t)xsmd_nbr_index(a.nbr[(int64_t)k * a.npad + i]) >= i) mask |= 1ull << (8 * t + u);
+            m8 |= (k < cnt && xsmd_nbr_index(a.nbr[(int64_t)k * a.npad + i]) >= iu ? 1u : 0u) << u;
           }
         }
+        mask |= (unsigned long long)m8 << (8 * t);
       }
-      while (mask) {
+      // the marked entry with the smallest bit, and the mask without it
+      const auto pop = [&]() {
         const int bit = __ffsll(mask) - 1;
         mask &= mask - 1;
-        uint32_t e;
         if constexpr (BLOCK) {
           const int g = (k0 >> 3) + sub + lanes * (bit >> 3);
-          e = a.stage[base + a.nbr16[(((int64_t)g * a.npad + i) << 3) + (bit & 7)]];
+          return a.stage[base + a.nbr16[(((int64_t)g * a.npad + i) << 3) + (bit & 7)]];
         } else {
-          e = a.nbr[(int64_t)(k0 + sub + lanes * bit) * a.npad + i];
+          return a.nbr[(int64_t)(k0 + sub + lanes * bit) * a.npad + i];
         }
-        const uint32_t j = xsmd_nbr_index(e);
-        const int tj = MULTI ? a.type[j] : 0;
+      };
+      // each pair's records are on their way while the pair before it is evaluated
+      bool more = mask != 0;
+      uint32_t e_next = 0;
+      Pos4 pj_next{}, gj_next{};
+      int tj_next = 0;
+      const auto fetch = [&]() {
+        e_next = pop();
+        const uint32_t j = xsmd_nbr_index(e_next);
+        pj_next = load_pos(a.pos, j);
+        gj_next = load_pos(a.gvec, j);
+        if (MULTI) tj_next = a.type[j];
+      };
+      if (more) fetch();
+      while (more) {
+        const uint32_t e = e_next, j = xsmd_nbr_index(e);
+        const Pos4 pj = pj_next, gj = gj_next;
+        const int tj = tj_next;
+        more = mask != 0;
+        if (more) fetch();
         if (MULTI && !adj_on(a, tj)) continue;
-        const Pos4 pj = load_pos(a.pos, j);
-        const Pos4 gj = load_pos(a.gvec, j);
-        const int kx = xsmd_nbr_img_x(e), ky = xsmd_nbr_img_y(e), kz = xsmd_nbr_img_z(e);
-        double dx = xsmd_image(pj.x, kx, Lb[0]) - pi.x;
-        double dy = xsmd_image(pj.y, ky, Lb[1]) - pi.y;
-        double dz = xsmd_image(pj.z, kz, Lb[2]) - pi.z;
+        double dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+        const bool image = e >> XSMD_NBR_INDEX_BITS;
+        if (image) {
+          dx = xsmd_image(pj.x, xsmd_nbr_img_x(e), Lb[0]) - pi.x;
+          dy = xsmd_image(pj.y, xsmd_nbr_img_y(e), Lb[1]) - pi.y;
+          dz = xsmd_image(pj.z, xsmd_nbr_img_z(e), Lb[2]) - pi.z;
+        }
         if (a.xf) xsmd_xform_apply(a.xf->m, &dx, &dy, &dz);
         const double d2 = xsmd_d2(dx, dy, dz);
         // wi, wj: which of the pair's two entries count; through an image the distance
         // from j rounds by itself, so a pair at the cutoff may count from one side only
         double wi = d2 <= a.rc2 ? 1.0 : 0.0, wj = wi;
-        if ((kx | ky | kz) != 0) {
-          double ux = xsmd_image(pi.x, -kx, Lb[0]) - pj.x;
-          double uy = xsmd_image(pi.y, -ky, Lb[1]) - pj.y;
-          double uz = xsmd_image(pi.z, -kz, Lb[2]) - pj.z;
+        if (image) {
+          double ux = xsmd_image(pi.x, -xsmd_nbr_img_x(e), Lb[0]) - pj.x;
+          double uy = xsmd_image(pi.y, -xsmd_nbr_img_y(e), Lb[1]) - pj.y;
+          double uz = xsmd_image(pi.z, -xsmd_nbr_img_z(e), Lb[2]) - pj.z;
           if (a.xf) xsmd_xform_apply(a.xf->m, &ux, &uy, &uz);
           wj = xsmd_d2(ux, uy, uz) <= a.rc2 ? 1.0 : 0.0;
-          if ((int64_t)j == i) {
+          if (j == iu) {
             wi *= 0.5;
             wj *= 0.5;
           }
@@ -334,13 +369,13 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_pairs(AdjArgs a, AdjWindows
         const double vi = wi * (ge * pi.w - gi.w), vj = wj * (ge * pj.w - gj.w);
         const double si = -wi * pi.w * srdr, sj = -wj * pj.w * srdr;
         if (!MULTI || ri == rj) {
-          adj_add(acc, a.nel + ri, m, h, vi + vj, si + sj);
+          adj_add<WHOLE>(acc, a.nel + ri, m, h, vi + vj, si + sj);
         } else {
-          adj_add(acc, a.nel + rj, m, h, vi, si);  // rho_j's table at atom i
-          adj_add(acc, a.nel + ri, m, h, vj, sj);
+          adj_add<WHOLE>(acc, a.nel + rj, m, h, vi, si);  // rho_j's table at atom i
+          adj_add<WHOLE>(acc, a.nel + ri, m, h, vj, sj);
         }
         const double c = 0.5 * both * a.conv * ir;
-        adj_add(acc, a.nel + z, m, h, c * (ge + s * ir), -c * srdr);
+        adj_add<WHOLE>(acc, a.nel + z, m, h, c * (ge + s * ir), -c * srdr);
       }
     }
   }
@@ -571,13 +606,18 @@ void adj_run(Ctx& c, const AdjArgs& a, double rcut, bool mixed)
     k<<<groups, threads, lds, c.stream>>>(a, W, args..., c.adj_part.p);
     reduce(W, groups);
   };
-  // lanes per atom: 2, more where the atoms do not fill the CUs
+  // lanes per atom: 2, up to 8 where the atoms do not fill the CUs (1.04 M atoms: 589 us
+  // with 1, 473 with 2, 503 with 4, 558 with 8; 55 k: 39.7 with 2, 36.7 with 4, 34.8 with 8)
   int lanes_log = 1;
-  while (lanes_log < 3 && (a.n << lanes_log) < cus * kAdjThreads * 3 / 4) lanes_log++;
+  while (lanes_log < 3 && (a.n << lanes_log) < cus * kAdjThreads) lanes_log++;
   const auto pairs = [&](const AdjWindows& W, bool fsum) {
     const auto pick = [&](auto m, auto b) {
       constexpr bool M = decltype(m)::value, B = decltype(b)::value;
-      launch(fsum ? k_adj_pairs<M, B, true> : k_adj_pairs<M, B, false>, W, a.n << lanes_log, lanes_log);
+      bool whole = true;
+      for (int T = fsum ? 0 : nel; T < 2 * nel + nz; T++) whole = whole && W.w[T].rows == (T < nel ? e.nrho : e.nr);
+      const auto k = whole ? (fsum ? k_adj_pairs<M, B, true, true> : k_adj_pairs<M, B, false, true>)
+                           : (fsum ? k_adj_pairs<M, B, true, false> : k_adj_pairs<M, B, false, false>);
+      launch(k, W, a.n << lanes_log, lanes_log);
     };
     if (multi && block) pick(std::true_type{}, std::true_type{});
     else if (multi) pick(std::true_type{}, std::false_type{});
