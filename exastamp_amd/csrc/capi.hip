@@ -13,10 +13,7 @@ namespace xsmd {
 
 Ctx::~Ctx()
 {
-  if (hscalar) (void)hipHostFree(hscalar);
-  if (hthermo) (void)hipHostFree(hthermo);
-  if (hflag) (void)hipHostFree(hflag);
-  if (hhalo) (void)hipHostFree(hhalo);
+  if (hscalar) (void)hipHostFree(hscalar);  // and the others, which follow it
   if (pinned) (void)hipHostFree(pinned);
   for (hipEvent_t e : step_event)
     if (e) (void)hipEventDestroy(e);
@@ -67,9 +64,18 @@ std::vector<T> from_device(Ctx& c, const DBuf<T>& d, int64_t n)
   return h;
 }
 
-char* pinned_buffer(Ctx& c)
+// at least `bytes` (at most kPinnedBytes) of pinned memory; no transfer uses what it held
+char* pinned_buffer(Ctx& c, size_t bytes)
 {
-  if (!c.pinned) XS_HIP(hipHostMalloc((void**)&c.pinned, kPinnedBytes, hipHostMallocDefault));
+  if (bytes > c.pinned_bytes) {
+    size_t want = 64 << 10;
+    while (want < bytes) want *= 2;
+    if (c.pinned) XS_HIP(hipHostFree(c.pinned));
+    c.pinned = nullptr;
+    c.pinned_bytes = 0;
+    XS_HIP(hipHostMalloc((void**)&c.pinned, want, hipHostMallocDefault));
+    c.pinned_bytes = want;
+  }
   return c.pinned;
 }
 
@@ -95,7 +101,7 @@ void to_id_order(Ctx& c, const double* const* src, int64_t stride, int rows, boo
   c.io_d.reserve((size_t)c.n * r.rows);
   launch_to_id_order(c, r, c.io_d.p);
   if (all <= kPinnedBytes) {
-    char* h = pinned_buffer(c);
+    char* h = pinned_buffer(c, all);
     XS_HIP(hipMemcpyAsync(h, c.io_d.p, all, hipMemcpyDeviceToHost, c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
     if (interleaved) std::memcpy(out[0], h, all);
@@ -209,12 +215,15 @@ xs_status xs_ctx_create(int device, xs_ctx** out)
     thermo_scratch_init(device);
     XS_HIP(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
     c->stream = c->own_stream;
-    XS_HIP(hipHostMalloc((void**)&c->hscalar, 8 * sizeof(unsigned long long), hipHostMallocDefault));
-    XS_HIP(hipHostMalloc((void**)&c->hthermo, 27 * sizeof(double), hipHostMallocDefault));
-    XS_HIP(hipHostMalloc((void**)&c->hflag, sizeof(unsigned long long), hipHostMallocCoherent | hipHostMallocMapped));
-    *c->hflag = 0;
-    XS_HIP(hipHostMalloc((void**)&c->hhalo, (4 * kHaloGroups + 1) * sizeof(uint32_t),
+    // one allocation (each costs tens of microseconds): scalars, thermodynamic results, the
+    // step flag, halo sizes and the overflow mark
+    constexpr size_t words = 8 + 27 + 1 + (4 * kHaloGroups + 1 + 1) / 2;
+    XS_HIP(hipHostMalloc((void**)&c->hscalar, words * sizeof(unsigned long long),
                          hipHostMallocCoherent | hipHostMallocMapped));
+    c->hthermo = reinterpret_cast<double*>(c->hscalar + 8);
+    c->hflag = c->hscalar + 8 + 27;
+    c->hhalo = reinterpret_cast<uint32_t*>(c->hscalar + 8 + 27 + 1);
+    *c->hflag = 0;
     for (hipEvent_t& e : c->step_event) XS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     c->dscalar.reserve(8);
     XS_HIP(hipMemsetAsync(c->dscalar.p, 0, 8 * sizeof(unsigned long long), c->stream));  // flags start clear
@@ -356,7 +365,7 @@ xs_status xs_system_set(xs_ctx* h, int64_t n, const double* rx, const double* ry
       const size_t all = type_at + (size_t)n;
       if (all <= kPinnedBytes) {  // one transfer
         c.io_d.reserve((all + 7) / 8);
-        char* h = pinned_buffer(c);
+        char* h = pinned_buffer(c, all);
         for (int q = 0; q < 6; q++) std::memcpy(h + q * row, rows[q], row);
         if (c.has_rep) std::memcpy(h + rep_at, rep, 2 * (size_t)n);
         std::memcpy(h + type_at, type, (size_t)n);

@@ -427,6 +427,7 @@ struct Ctx {
   DBuf<uint8_t> io_type;
   DBuf<uint16_t> io_rep;
   char* pinned = nullptr;
+  size_t pinned_bytes = 0;
 
   // small device scalars + pinned host mirror
   DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..3] pair counts
