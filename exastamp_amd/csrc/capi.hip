@@ -216,13 +216,14 @@ xs_status xs_ctx_create(int device, xs_ctx** out)
     XS_HIP(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
     c->stream = c->own_stream;
     // one allocation (each costs tens of microseconds): scalars, thermodynamic results, the
-    // step flag, halo sizes and the overflow mark
-    constexpr size_t words = 8 + 27 + 1 + (4 * kHaloGroups + 1 + 1) / 2;
+    // step flag, displacements, halo sizes and the overflow mark
+    constexpr size_t words = 8 + 27 + 1 + kDisplGroups + (4 * kHaloGroups + 1 + 1) / 2;
     XS_HIP(hipHostMalloc((void**)&c->hscalar, words * sizeof(unsigned long long),
                          hipHostMallocCoherent | hipHostMallocMapped));
     c->hthermo = reinterpret_cast<double*>(c->hscalar + 8);
     c->hflag = c->hscalar + 8 + 27;
-    c->hhalo = reinterpret_cast<uint32_t*>(c->hscalar + 8 + 27 + 1);
+    c->hdispl = reinterpret_cast<double*>(c->hscalar + 8 + 27 + 1);
+    c->hhalo = reinterpret_cast<uint32_t*>(c->hscalar + 8 + 27 + 1 + kDisplGroups);
     *c->hflag = 0;
     for (hipEvent_t& e : c->step_event) XS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     c->dscalar.reserve(8);
@@ -350,6 +351,7 @@ xs_status xs_system_set(xs_ctx* h, int64_t n, const double* rx, const double* ry
         c.box_h[r].inv_cs[a] = 1.0 / L;
       }
     for (int a = 0; a < 3; a++) c.periodic[a] = periodic[a] ? 1 : 0;
+    if ((size_t)nrep > c.box_d.n) c.box_up.clear();  // a new device array
     c.box_d.reserve(nrep);
     c.nrep = nrep;
     c.has_rep = nrep > 1;
@@ -363,15 +365,13 @@ xs_status xs_system_set(xs_ctx* h, int64_t n, const double* rx, const double* ry
       const double* rows[6] = {rx, ry, rz, vx, vy, vz};
       const size_t row = sizeof(double) * (size_t)n, rep_at = 6 * row, type_at = rep_at + (c.has_rep ? 2 * (size_t)n : 0);
       const size_t all = type_at + (size_t)n;
-      if (all <= kPinnedBytes) {  // one transfer
-        c.io_d.reserve((all + 7) / 8);
+      if (all <= kPinnedBytes) {  // the kernel reads them from host memory
         char* h = pinned_buffer(c, all);
         for (int q = 0; q < 6; q++) std::memcpy(h + q * row, rows[q], row);
         if (c.has_rep) std::memcpy(h + rep_at, rep, 2 * (size_t)n);
         std::memcpy(h + type_at, type, (size_t)n);
-        XS_HIP(hipMemcpyAsync(c.io_d.p, h, all, hipMemcpyHostToDevice, c.stream));
-        char* d = reinterpret_cast<char*>(c.io_d.p);
-        launch_unpack_atoms(c, c.io_d.p, reinterpret_cast<uint8_t*>(d + type_at), reinterpret_cast<uint16_t*>(d + rep_at));
+        launch_unpack_atoms(c, reinterpret_cast<double*>(h), reinterpret_cast<uint8_t*>(h + type_at),
+                            reinterpret_cast<uint16_t*>(h + rep_at));
       } else {
         c.io_d.reserve(6 * (size_t)n);
         c.io_type.reserve(n);

@@ -245,8 +245,8 @@ __global__ void __launch_bounds__(256) k_build(
   if (cnt > nmax) atomicMax(maxcnt, (unsigned long long)cnt);
 }
 
-// block-wide max of a non-negative double, one atomic per block
-__device__ __forceinline__ void block_max_to(double v, unsigned long long* out)
+// block-wide max of a non-negative double
+__device__ __forceinline__ void block_max_to(double v, double* out)
 {
   for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
   __shared__ double sh[kBlock / 64];
@@ -255,15 +255,17 @@ __device__ __forceinline__ void block_max_to(double v, unsigned long long* out)
   if (threadIdx.x == 0) {
     double m = sh[0];
     for (int w = 1; w < (int)(blockDim.x >> 6); w++) m = fmax(m, sh[w]);
-    if (m > 0.0) atomicMax(out, (unsigned long long)__double_as_longlong(m));
+    *out = m;
   }
 }
 
+// Largest squared displacement since the last build: each workgroup's maximum goes to host
+// memory (out, kDisplGroups values), where they are put together; a clear, an atomic per
+// workgroup on one word and a copy back took as long as the sweep at 130 k atoms.
 __global__ void __launch_bounds__(256) k_max_displ2(int64_t n, const Pos4* __restrict__ pos,
                                                     const double* __restrict__ rrx,
                                                     const double* __restrict__ rry,
-                                                    const double* __restrict__ rrz,
-                                                    unsigned long long* __restrict__ out,
+                                                    const double* __restrict__ rrz, double* __restrict__ out,
                                                     const XformDev* __restrict__ xf)
 {
   double m = 0.0;
@@ -274,7 +276,7 @@ __global__ void __launch_bounds__(256) k_max_displ2(int64_t n, const Pos4* __res
     if (xf) xsmd_xform_apply(xf->m, &ux, &uy, &uz);  // the threshold is a physical distance
     m = fmax(m, xsmd_d2(ux, uy, uz));
   }
-  block_max_to(m, out);
+  block_max_to(m, out + blockIdx.x);
 }
 
 __global__ void k_pair_count(int64_t n, int64_t npad, const Pos4* __restrict__ pos,
@@ -338,8 +340,13 @@ void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block, bo
   }
   for (BoxDev& b : c.box_h)
     for (int a = 0; a < 3; a++) b.inv_cs[a] = c.nc[a] / b.L[a];
-  XS_HIP(hipMemcpyAsync(c.box_d.p, c.box_h.data(), sizeof(BoxDev) * c.box_h.size(),
-                        hipMemcpyHostToDevice, c.stream));
+  // the device's copy, when a box or the cell grid is another than at the last build
+  const size_t box_bytes = sizeof(BoxDev) * c.box_h.size();
+  if (c.box_up.size() != c.box_h.size() || std::memcmp(c.box_up.data(), c.box_h.data(), box_bytes) != 0) {
+    c.box_up.clear();
+    XS_HIP(hipMemcpyAsync(c.box_d.p, c.box_h.data(), box_bytes, hipMemcpyHostToDevice, c.stream));
+    c.box_up = c.box_h;
+  }
   c.ncell_rep = (int64_t)c.nc[0] * c.nc[1] * c.nc[2];
   c.ncell_tot = c.ncell_rep * c.nrep;
   if (c.ncell_tot >= (int64_t)1 << 32) throw Error(XS_E_LIMIT, "too many cells");
@@ -463,16 +470,11 @@ void pair_count(Ctx& c, double rcut, int64_t& entries, int64_t& within)
 double max_displacement2(Ctx& c)
 {
   if (c.n == 0) return 0.0;
-  XS_HIP(hipMemsetAsync(c.dscalar.p + 1, 0, sizeof(unsigned long long), c.stream));
-  const unsigned g = std::min<unsigned>(grid_for(c.n), 2048);
-  k_max_displ2<<<g, kBlock, 0, c.stream>>>(c.n, c.pos.p, c.rrx.p, c.rry.p, c.rrz.p, c.dscalar.p + 1, c.xf_dev());
+  const unsigned g = std::min<unsigned>(grid_for(c.n), kDisplGroups);
+  k_max_displ2<<<g, kBlock, 0, c.stream>>>(c.n, c.pos.p, c.rrx.p, c.rry.p, c.rrz.p, c.hdispl, c.xf_dev());
   XS_HIP(hipGetLastError());
-  XS_HIP(hipMemcpyAsync(c.hscalar + 1, c.dscalar.p + 1, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                        c.stream));
   XS_HIP(hipStreamSynchronize(c.stream));
-  double d;
-  std::memcpy(&d, &c.hscalar[1], sizeof(double));
-  return d;
+  return *std::max_element(c.hdispl, c.hdispl + g);
 }
 
 }  // namespace xsmd

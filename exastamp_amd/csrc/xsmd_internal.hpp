@@ -269,6 +269,7 @@ constexpr double kBlockAtoms = 230.0;      // largest expected central atoms per
 constexpr size_t kLdsPerCu = 160 * 1024;   // LDS of one CU
 constexpr int kMaxHaloCells = 216;
 constexpr int kHaloGroups = 512;           // workgroups that size the halos
+constexpr int kDisplGroups = 1024;         // workgroups of the displacement check
 constexpr size_t kBlockLdsLimit = 64 * 1024;  // default dynamic-LDS limit of a launch
 
 // Event-pair timing per kernel class (see XS_PROF_* in xsmd.h).
@@ -364,6 +365,7 @@ struct Ctx {
   int nrep = 1;
   int periodic[3] = {1, 1, 1};
   std::vector<BoxDev> box_h;
+  std::vector<BoxDev> box_up;  // what box_d holds
   DBuf<BoxDev> box_d;
   XformDev xf = {{1, 0, 0, 0, 1, 0, 0, 0, 1}, {1, 0, 0, 0, 1, 0, 0, 0, 1}, 0};
   DBuf<XformDev> xf_d;  // device copy of xf; kernels get xf_dev(): NULL for the identity
@@ -430,14 +432,14 @@ struct Ctx {
   size_t pinned_bytes = 0;
 
   // small device scalars + pinned host mirror
-  DBuf<unsigned long long> dscalar;  // [0] max count, [1] max displacement^2 bits, [2..3] pair counts
+  DBuf<unsigned long long> dscalar;  // [0] max count, [2..3] pair counts
                                      // (list builds use [0..2]), [6] the MD loop's rebuild flag (StepFlag)
   unsigned long long* hscalar = nullptr;
   uint32_t* hhalo = nullptr;  // written by kernels: 4 halo sizes of each of kHaloGroups workgroups, the
                               // build's overflow mark
   DBuf<double> red_part;  // thermo partial sums
-  DBuf<double> red_out;
-  double* hthermo = nullptr;  // pinned host copy of the 27 results
+  double* hthermo = nullptr;  // xs_thermo's 27 results, written by its last kernel
+  double* hdispl = nullptr;   // largest squared displacement of each of kDisplGroups workgroups
 
   bool has_lj = false;
   double lj_eps = 0, lj_sigma = 0, lj_rcut = 0;
