@@ -428,7 +428,8 @@ def cpu_baseline(cfg, tab, steps, threads, dt, rc, skin):
 
 def operator_forms(sim, rc, reps=5):
     """The eam_alloy_force operator (density, embedding and force passes, mixed) in
-    its plain and its Newton-symmetric form: GPU time per call of each pass class, and the symmetric form's force deviation."""
+    its plain and its Newton-symmetric form: GPU time per call of each pass class, and the
+    symmetric form's force deviation."""
     from exastamp_amd import _lib
     import ctypes as C
     out = {}

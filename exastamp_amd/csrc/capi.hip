@@ -296,7 +296,7 @@ xs_status xs_synchronize(xs_ctx* h)
 {
   return guarded(h, [&](Ctx& c) {
     XS_HIP(hipStreamSynchronize(c.stream));
-    });
+  });
 }
 
 xs_status xs_device_memory(xs_ctx* h, size_t* free_bytes, size_t* total_bytes)

@@ -12,9 +12,8 @@
 // x fastest.  Atoms of one cell are contiguous in HBM (cell-sorted order) and are
 // staged contiguously, cells in enumeration order, so ascending slot order equals
 // the visit order of the global build.  The build finds the same pairs as the
-// global build; k_list_sort then orders each list by distance, and
-// k_block_to_global restores slot order, so a converted block list equals the
-// global list entry for entry.
+// global build and orders short lists by distance; k_block_to_global restores slot
+// order, so a converted block list equals the global list entry for entry.
 #include "pair_math.hpp"
 
 #include <algorithm>
@@ -522,8 +521,9 @@ __device__ __forceinline__ void wave_lds_sync()
 // entries, the tests of 197 candidates, the sort and the candidate search in equal
 // parts) at the three 4-wave workgroups per CU its LDS leaves.  One lane per atom
 // walking its own candidates, with the sort as a second kernel, issued twice as many on
-// diverging lanes.  8.39 M EAM atoms (53 entries): 4.04 -> 2.57 ms, 1.05 M argon atoms
-// (79 entries, unsorted) 0.79 -> 0.38 ms, 4000 argon atoms 112 -> 26 us.  Workgroups of
+// diverging lanes.  8.39 M EAM atoms (53 entries): 4.04 -> 2.65 ms, 1.05 M argon atoms
+// (79 entries, unsorted) 0.79 -> 0.42 ms, 4000 argon atoms 112 -> 15 us, the staging
+// tables included.  Workgroups of
 // 5, 6 or 8 waves measured slower (4.86, 2.84 and 3.70 ms: their waves share the SIMDs
 // unevenly or leave LDS for two workgroups).
 //
@@ -622,7 +622,8 @@ __global__ void __launch_bounds__(kBuildThreads) k_block_build(BuildArgs a)
       total_p[2] = -1;
       uint4 head = BrickHead::pack(0, 0, s.r, 0, 0);  // no central atom: nothing to stage
       if (carry > 0) {
-        uint32_t at_stage = (uint32_t)b * (uint32_t)(a.stage_step / (int)kStageAlign), at_cen = (uint32_t)b * (uint32_t)a.cen_step;
+        uint32_t at_stage = (uint32_t)b * ((uint32_t)a.stage_step / kStageAlign);
+        uint32_t at_cen = (uint32_t)b * (uint32_t)a.cen_step;
         if (a.stage_step == 0) {
           const unsigned long long need = (unsigned long long)((total + kStageAlign - 1) / kStageAlign) << 32;
           const unsigned long long at = atomicAdd(a.flags + 2, need | (unsigned long long)carry);
@@ -1846,7 +1847,8 @@ unsigned block_grid(const Ctx& c)
 static size_t build_lds_bytes(const Ctx& c, int atoms)
 {
   return build_rec_bytes(c.bcap) + (size_t)c.bgeom.nh_max * sizeof(HaloCell) +
-         (4 + (size_t)c.bgeom.bx * c.bgeom.by * c.bgeom.bz) * sizeof(int) + build_cand_bytes(c.bcap, c.bcand) + (size_t)kBuildWaves * atoms * (c.nmax + 1) * sizeof(uint32_t);
+         (4 + (size_t)c.bgeom.bx * c.bgeom.by * c.bgeom.bz) * sizeof(int) + build_cand_bytes(c.bcap, c.bcand) +
+         (size_t)kBuildWaves * atoms * (c.nmax + 1) * sizeof(uint32_t);
 }
 
 // Block list build; false when its LDS does not fit a workgroup (then nothing was

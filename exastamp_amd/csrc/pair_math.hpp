@@ -299,7 +299,7 @@ __device__ __forceinline__ Real dcubic(const Q4<Real>& c, Real p)
   return (Real(3) * c.a * p + Real(2) * c.b) * p + c.c;
 }
 // The FP32 forms spell out their fused multiply-adds, so every kernel that shares
-// them (block and global lists, full and half lists) rounds them alike whatever the
+// them (block and global lists) rounds them alike whatever the
 // compiler's contraction choices around them.
 __device__ __forceinline__ float cubic(const Q4<float>& c, float p) { return fmaf(fmaf(fmaf(c.a, p, c.b), p, c.c), p, c.d); }
 __device__ __forceinline__ float quad(const Q4<float>& c, float p) { return fmaf(fmaf(c.a, p, c.b), p, c.c); }

@@ -30,9 +30,8 @@ config_speculative_verlet.msp) as the trigger and chunk_neighbors as the list
 build, so decks that override any of these nodes run as written.
 
 Differences that a deck cannot see in its results: the Newton-symmetric variants
-(``eam_symmetry: true``, ``lj_compute_force_symetric``) evaluate each pair once
-from a half list and add the partner's share with FP64 atomics (same forces up to
-FP64 summation order, which varies from run to run); ``chunk_size`` is accepted
+(``eam_symmetry: true``, ``lj_compute_force_symetric``) evaluate each pair from both
+of its atoms, with a pair scalar symmetric in them; ``chunk_size`` is accepted
 and does not change the list; the random streams of ``gaussian_noise_r/v`` are
 numpy Philox streams (seed ``--seed``), not exaNBody's.
 
