@@ -23,9 +23,10 @@ namespace {
 // counts were taken in.  That last step reads a cell's members once per atom, which is a
 // small part of the list build's own work per cell.  Four or five launches; a library
 // radix sort of (cell, index) pairs took 8 launches at 4 k atoms and 20 at 1 M
-// (about 150 us there against 57, and 90 against 17 at 4 k).  Leaving the order to k_permute, each atom written to its place,
-// cost more than the launch it saved: its writes lose their coalescing (340 us
-// against 237 + 75 at 8.39 M atoms, 48 against 34 + 16 at 1.05 M).
+// (about 150 us there against 57, and 90 against 17 at 4 k).  Up to kFusedOrder atoms
+// k_order_permute also moves each atom to its place, which saves a launch; above, its
+// writes lose more by their scatter (340 us against 237 + 75 at 8.39 M atoms, 48 against
+// 34 + 16 at 1.05 M).
 
 // Wraps atom i into its box, finds its cell, counts it there: num[i] = its number among
 // the atoms of the cell so far.  Consecutive atoms mostly share a cell (they were sorted
@@ -138,20 +139,30 @@ __global__ void k_cell_place(int64_t n, const uint32_t* __restrict__ keys, const
   if (i < n) members[off[keys[i]] + num[i]] = (uint32_t)i;
 }
 
-// perm[k] = atom at place k of the stable order, and its cell
+// the atom p at place k of `members`, and its place in the stable order; its cell to keys_out
+__device__ __forceinline__ int64_t stable_place(int64_t k, const uint32_t* __restrict__ members,
+                                                const uint32_t* __restrict__ keys, const int* __restrict__ off,
+                                                uint32_t* __restrict__ keys_out, uint32_t& p)
+{
+  p = members[k];
+  const uint32_t key = keys[p];
+  const int o0 = off[key], o1 = off[key + 1];
+  int64_t i = o0;
+  for (int o = o0; o < o1; o++) i += members[o] < p;
+  keys_out[k] = key;  // places k and i are in the same cell
+  return i;
+}
+
+// perm[i] = atom at place i of the stable order
 __global__ void k_cell_order(int64_t n, const uint32_t* __restrict__ members, const uint32_t* __restrict__ keys,
                              const int* __restrict__ off, uint32_t* __restrict__ perm,
                              uint32_t* __restrict__ keys_out)
 {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  const uint32_t p = members[k];
-  const uint32_t key = keys[p];
-  const int o0 = off[key], o1 = off[key + 1];
-  int64_t i = o0;
-  for (int o = o0; o < o1; o++) i += members[o] < p;
+  uint32_t p;
+  const int64_t i = stable_place(k, members, keys, off, keys_out, p);
   perm[i] = p;
-  keys_out[k] = key;  // places k and i are in the same cell
 }
 
 struct PermuteArgs {
@@ -174,11 +185,8 @@ struct PermuteArgs {
 // acceleration components; a caller about to overwrite the accelerations leaves them
 // out); the new positions also become the reference positions of the displacement check.
 template <int ND>
-__global__ void __launch_bounds__(256) k_permute(int64_t n, const uint32_t* __restrict__ perm, PermuteArgs a)
+__device__ __forceinline__ void move_atom(const PermuteArgs& a, uint32_t p, int64_t i)
 {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t p = perm[i];
   const Pos4 q = load_pos(a.pos_src, p);
   store_pos(a.pos_dst, i, q);
   a.rrx[i] = q.x;
@@ -189,6 +197,26 @@ __global__ void __launch_bounds__(256) k_permute(int64_t n, const uint32_t* __re
   a.type_dst[i] = a.type_src[p];
   a.id_dst[i] = a.id_src[p];
   if (a.rep_src) a.rep_dst[i] = a.rep_src[p];
+}
+template <int ND>
+__global__ void __launch_bounds__(256) k_permute(int64_t n, const uint32_t* __restrict__ perm, PermuteArgs a)
+{
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) move_atom<ND>(a, perm[i], i);
+}
+
+// k_cell_order and k_permute in one
+constexpr int64_t kFusedOrder = 1 << 19;
+template <int ND>
+__global__ void __launch_bounds__(256) k_order_permute(int64_t n, const uint32_t* __restrict__ members,
+                                                       const uint32_t* __restrict__ keys, const int* __restrict__ off,
+                                                       uint32_t* __restrict__ keys_out, PermuteArgs a)
+{
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  uint32_t p;
+  const int64_t i = stable_place(k, members, keys, off, keys_out, p);
+  move_atom<ND>(a, p, i);
 }
 
 // One thread per atom; stencil order dz, dy, dx (outer to inner), in-cell order
@@ -376,8 +404,6 @@ void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block, bo
   c.counts_clear = true;
   k_cell_place<<<g, kBlock, 0, c.stream>>>(n, c.keys.p, c.vals.p, c.cell_off.p, c.vals2.p);
   XS_HIP(hipGetLastError());
-  k_cell_order<<<g, kBlock, 0, c.stream>>>(n, c.vals2.p, c.keys.p, c.cell_off.p, c.vals.p, c.keys2.p);
-  XS_HIP(hipGetLastError());
 
   PermuteArgs pa{};
   pa.pos_src = c.pos.p;
@@ -397,7 +423,14 @@ void build_neighbor_list(Ctx& c, double rcut, double skin, bool prefer_block, bo
   pa.id_dst = c.id2.p;
   pa.rep_src = c.has_rep ? c.rep.p : nullptr;
   pa.rep_dst = c.has_rep ? c.rep2.p : nullptr;
-  (keep_accel ? k_permute<6> : k_permute<3>)<<<g, kBlock, 0, c.stream>>>(n, c.vals.p, pa);
+  if (n <= kFusedOrder) {
+    (keep_accel ? k_order_permute<6> : k_order_permute<3>)<<<g, kBlock, 0, c.stream>>>(n, c.vals2.p, c.keys.p,
+                                                                                       c.cell_off.p, c.keys2.p, pa);
+  } else {
+    k_cell_order<<<g, kBlock, 0, c.stream>>>(n, c.vals2.p, c.keys.p, c.cell_off.p, c.vals.p, c.keys2.p);
+    XS_HIP(hipGetLastError());
+    (keep_accel ? k_permute<6> : k_permute<3>)<<<g, kBlock, 0, c.stream>>>(n, c.vals.p, pa);
+  }
   XS_HIP(hipGetLastError());
   c.pos.swap(c.pos2);
   c.vx.swap(c.vx2);

@@ -122,6 +122,7 @@ class LjForcesEnergies(torch.autograd.Function):
 
 
 _LOSS_PARTIALS = 1024  # XS_FIT_LOSS_PARTIALS
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 0)
 
 
 def _plain(*tensors):
@@ -129,7 +130,7 @@ def _plain(*tensors):
     records the operations on them, so that a kernel may read them by address."""
     d = tensors[0].device
     return (d.type == "cuda" and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and torch._C._len_torch_dispatch_stack() == 0
+            and _dispatch_modes() == 0
             and all(type(t) is torch.Tensor and t.dtype is torch.float64 and t.device == d and t.is_contiguous()
                     and t.numel() > 0 for t in tensors))
 
