@@ -127,12 +127,13 @@ _dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 0)
 
 def _plain(*tensors):
     """Whether the tensors are ordinary, contiguous FP64 tensors of one GPU and nothing
-    records the operations on them, so that a kernel may read them by address."""
+    records the operations on them, so that a kernel may read them by address.  (The memory
+    of a negated view, ``z.conj().imag``, holds what it negates.)"""
     d = tensors[0].device
     return (d.type == "cuda" and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and _dispatch_modes() == 0
             and all(type(t) is torch.Tensor and t.dtype is torch.float64 and t.device == d and t.is_contiguous()
-                    and t.numel() > 0 for t in tensors))
+                    and t.numel() > 0 and not t.is_neg() for t in tensors))
 
 
 def _launch(f, device, *args):
