@@ -125,15 +125,29 @@ _LOSS_PARTIALS = 1024  # XS_FIT_LOSS_PARTIALS
 _dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 0)
 
 
-def _plain(*tensors):
-    """Whether the tensors are ordinary, contiguous FP64 tensors of one GPU and nothing
-    records the operations on them, so that a kernel may read them by address.  (The memory
-    of a negated view, ``z.conj().imag``, holds what it negates.)"""
+def _addresses(*tensors):
+    """The addresses of ordinary, contiguous FP64 tensors of one device, whose memory holds
+    their values; None for any other.  A negated view (``z.conj().imag``) has the memory of
+    what it negates, a tensor of zeros from autograd has none (address 0), and that of a
+    batched backward (``is_grads_batched``) has no address to give."""
     d = tensors[0].device
-    return (d.type == "cuda" and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and _dispatch_modes() == 0
-            and all(type(t) is torch.Tensor and t.dtype is torch.float64 and t.device == d and t.is_contiguous()
-                    and t.numel() > 0 and not t.is_neg() for t in tensors))
+    if not all(type(t) is torch.Tensor and t.dtype is torch.float64 and t.device == d and t.is_contiguous()
+               and t.numel() > 0 and not t.is_neg() for t in tensors):
+        return None
+    try:
+        at = [t.data_ptr() for t in tensors]
+    except RuntimeError:
+        return None
+    return at if all(at) else None
+
+
+def _kernel_addresses(*tensors):
+    """_addresses of tensors on a GPU, unless something records the operations on them;
+    None: the operations have to run as tensor operations."""
+    if (tensors[0].device.type != "cuda" or torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or _dispatch_modes() != 0):
+        return None
+    return _addresses(*tensors)
 
 
 def _launch(f, device, *args):
@@ -153,13 +167,16 @@ class _FitLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, F, E, F_target, E_target, n, energy_weight):
         ctx.energy_weight = energy_weight
-        if (isinstance(energy_weight, (int, float)) and F.shape == F_target.shape and E.shape == E_target.shape == n.shape
-                and _plain(F, F_target, E, E_target, n)):
+        at = None
+        if (isinstance(energy_weight, (int, float)) and F.shape == F_target.shape
+                and E.shape == E_target.shape == n.shape):
+            at = _kernel_addresses(F, F_target, E, E_target, n)
+        if at:
+            pF, pFt, pE, pEt, pn = at
             rF, rE = torch.empty_like(F), torch.empty_like(E)
             partials, loss = F.new_empty(_LOSS_PARTIALS), F.new_empty(())
-            _launch(_lib.load().xs_fit_loss_dev, F.device, F.numel(), F.data_ptr(), F_target.data_ptr(), E.numel(),
-                    E.data_ptr(), E_target.data_ptr(), n.data_ptr(), energy_weight, rF.data_ptr(), rE.data_ptr(),
-                    partials.data_ptr(), loss.data_ptr())
+            _launch(_lib.load().xs_fit_loss_dev, F.device, F.numel(), pF, pFt, E.numel(), pE, pEt, pn, energy_weight,
+                    rF.data_ptr(), rE.data_ptr(), partials.data_ptr(), loss.data_ptr())
             ctx.save_for_backward(rF, rE, n)
             return loss
         rF = F - F_target
@@ -170,11 +187,15 @@ class _FitLoss(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         rF, rE, n = ctx.saved_tensors
+        at = None
         if (not torch.is_grad_enabled() and isinstance(ctx.energy_weight, (int, float)) and g.numel() == 1
-                and rE.shape == n.shape and _plain(rF, rE, n, g)):
+                and rE.shape == n.shape):
+            at = _kernel_addresses(rF, rE, n, g)
+        if at:
+            pF, pE, pn, pg = at
             gF, gE = torch.empty_like(rF), torch.empty_like(rE)
-            _launch(_lib.load().xs_fit_loss_grad_dev, rF.device, rF.numel(), rF.data_ptr(), rE.numel(), rE.data_ptr(),
-                    n.data_ptr(), ctx.energy_weight, g.data_ptr(), gF.data_ptr(), gE.data_ptr())
+            _launch(_lib.load().xs_fit_loss_grad_dev, rF.device, rF.numel(), pF, rE.numel(), pE, pn, ctx.energy_weight,
+                    pg, gF.data_ptr(), gE.data_ptr())
             return gF, gE, None, None, None, None
         gF = rF * (g * (2.0 / rF.numel()))
         gE = rE / n * (g * (2.0 * ctx.energy_weight / rE.numel()))

@@ -51,3 +51,33 @@ def test_fit_loss_imaginary_part_of_a_conjugate():
     assert Et.is_neg() and Et.item() == -200.0
     L, L0 = fit_loss(F, E, Ft, Et, n, 0.1).item(), _loss(F, E, Ft, torch.full_like(E, -200.0), n, 0.1).item()
     assert abs(L - L0) <= 1e-14 * abs(L0)
+
+
+def test_fit_loss_batched_backward():
+    """Several incoming gradients at once: the gradient that reaches the node is a batched
+    tensor, which has no address."""
+    import torch
+    from exastamp_amd.fitting import fit_loss
+    case = _inputs(reps=4)
+    scales = torch.tensor([1.0, -2.5, 0.0], dtype=torch.float64)
+    ref = [t.clone().requires_grad_(k < 2) for k, t in enumerate(case)]
+    gF0, gE0 = torch.autograd.grad(_loss(*ref, 0.1), ref[:2])
+    args = [t.cuda().requires_grad_(k < 2) for k, t in enumerate(case)]
+    gF, gE = torch.autograd.grad(fit_loss(*args, 0.1), args[:2], scales.cuda(), is_grads_batched=True)
+    for g, g0 in ((gF, gF0), (gE, gE0)):
+        want = torch.stack([s * g0 for s in scales])
+        assert g.shape == want.shape and (g.cpu() - want).abs().max() <= 2e-15 * want.abs().max()
+
+
+@pytest.mark.parametrize("which", ["Ft", "Et"])
+def test_fit_loss_zero_tensors(which):
+    """Autograd's tensors of zeros, which have no memory"""
+    import torch
+    from exastamp_amd.fitting import fit_loss
+    case = dict(zip(("F", "E", "Ft", "Et", "n"), _inputs(reps=4)))
+    case[which] = torch.zeros_like(case[which])
+    L0 = _loss(*case.values(), 0.1).item()
+    used = {k: t.cuda() for k, t in case.items()}
+    used[which] = torch._efficientzerotensor(case[which].shape, dtype=torch.float64, device="cuda")
+    L = fit_loss(*used.values(), 0.1).item()
+    assert abs(L - L0) <= 1e-14 * abs(L0)
