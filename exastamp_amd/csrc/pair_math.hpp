@@ -36,7 +36,8 @@ __device__ __forceinline__ Q4<double> load4(const double* __restrict__ p)
 // Goldschmidt's iteration: g -> sqrt, h -> 1 / (2 sqrt), then one residual step each,
 // 11 instructions.  On 8.4 M values from 0.01 to 1e12 r equals sqrt(d2) in every one and
 // rinv is as far from the exact reciprocal as 1 / r (1.50 ulp at most, 0.36 on average);
-// recip equals 1 / x.  d2 = 0 gives NaN where the division gave NaN or infinity.
+// recip equals 1 / x.  For d2 = 0 (coincident atoms) the steps give NaN: the minimum makes
+// rinv the infinity that the division gives, r stays NaN (knot_r takes it as 0).
 __device__ __forceinline__ void dist_steps(double d2, double y, double& g, double& h)
 {
   g = d2 * y;
@@ -51,7 +52,7 @@ __device__ __forceinline__ void dist(double d2, double& r, double& rinv)
   double h;
   dist_steps(d2, __builtin_amdgcn_rsq(d2), r, h);
   const double y = h + h;
-  rinv = fma(fma(-y, r, 1.0), y, y);
+  rinv = fmin(fma(fma(-y, r, 1.0), y, y), HUGE_VAL);
 }
 // the distance alone; finite at d2 = 0 (1e-145, the table's first knot)
 __device__ __forceinline__ double dist(double d2)
@@ -186,9 +187,9 @@ template <class Real>
 __device__ __forceinline__ void knot_r(const EamTabDev<Real>& t, Real r, int& m, Real& p)
 {
   p = r * t.rdr + Real(1);
-  m = min((int)p, t.nr - 1);  // r is not negative, and NaN converts to 0
+  m = max(1, min((int)p, t.nr - 1));  // NaN, the distance of coincident atoms, converts to 0
   p -= (Real)m;
-  p = fmin(p, Real(1));
+  p = fmin(fmax(p, Real(0)), Real(1));  // one instruction's clamp, which takes NaN as 0
 }
 
 // Distance, 1/r and spline knot of a pair from its FP64 d^2 (the first steps of
@@ -592,7 +593,7 @@ __device__ __forceinline__ void johnson_pair(const JohnsonParams& p, double d2, 
   const double ire = 1.0 / p.re;
   double r, rinv;
   dist(d2, r, rinv);
-  const double x = r * ire;
+  const double x = fmax(r, 0.0) * ire;  // coincident atoms: 0
   double t1, d1, t2, d2x;
   johnson_term(p.alpha, p.kappa, x, t1, d1);
   johnson_term(p.beta, p.lambda, x, t2, d2x);
