@@ -504,16 +504,10 @@ __device__ __forceinline__ void eam_pair_knot(const EamTabDev<Real>& t, const Re
     }
     const Real z2 = cubic(zc, p);
     phi = z2 * rinv;
-    Real phip, psip;
-    if constexpr (sizeof(Real) == 4) {
-      phip = fmaf(z2p, rinv, -(phi * rinv)) * t.conv;
-      // in an order that both atoms of the pair agree on, so that their forces cancel
-      const bool first = fpi <= fpj;
-      psip = fmaf(first ? fpi : fpj, first ? rhojp : rhoip, fmaf(first ? fpj : fpi, first ? rhoip : rhojp, phip));
-    } else {
-      phip = (z2p * rinv - phi * rinv) * t.conv;
-      psip = fpi * rhojp + fpj * rhoip + phip;
-    }
+    // half of phi' to each embedding term: the sum of the two is the same from either atom,
+    // so the forces of a pair are opposite to the last bit
+    const Real hp = fma_r(z2p, rinv, -(phi * rinv)) * (Real(0.5) * t.conv);
+    const Real psip = fma_r(fpi, rhojp, hp) + fma_r(fpj, rhoip, hp);
     phi *= t.conv;
     fpair = psip * rinv;
   } else {

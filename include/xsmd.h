@@ -52,8 +52,9 @@ typedef enum {
                           accelerations): skip the initial build and force step */
 #define XS_SYMMETRIC 16u /* Newton-symmetric evaluation (eam_symmetry: true,
                             lj_compute_force_symetric): the two atoms of a pair get
-                            opposite forces from the same pair scalar.  Operators only
-                            (not xs_md_run). */
+                            opposite forces from the same pair scalar, to the last bit
+                            inside the box; through a periodic image to the rounding of
+                            the image's coordinates.  Operators only (not xs_md_run). */
 
 /* potentials for xs_md_run */
 #define XS_POT_LJ 0
