@@ -82,7 +82,9 @@ char* pinned_buffer(Ctx& c, size_t bytes)
 // Rows of the device's cell order to the caller's arrays, in id order: the order is
 // restored on the device, and the host copies what it asked for.  `out` receives the
 // rows one after the other, row q at out[q] (NULL: not wanted); with one array of all
-// rows (interleaved), out[0].  Small results cross in one transfer through pinned memory.
+// rows (interleaved), out[0].  Small results cross in one transfer through pinned memory;
+// others by way of the second position array, which holds four rows of all atoms and
+// nothing between two calls, one range of ids after the other.
 void to_id_order(Ctx& c, const double* const* src, int64_t stride, int rows, bool interleaved, double* const* out)
 {
   if (c.n == 0) return;
@@ -95,12 +97,17 @@ void to_id_order(Ctx& c, const double* const* src, int64_t stride, int rows, boo
     }
   if (r.rows == 0) return;
   r.stride = stride;
-  r.atom_step = interleaved ? r.rows : 1;
-  r.row_step = interleaved ? 1 : c.n;
+  const auto launch = [&](int64_t first, int64_t count, double* dst) {
+    r.first = first;
+    r.count = count;
+    r.atom_step = interleaved ? r.rows : 1;
+    r.row_step = interleaved ? 1 : count;
+    launch_to_id_order(c, r, dst);
+  };
   const size_t row = sizeof(double) * (size_t)c.n, all = row * r.rows;
-  c.io_d.reserve((size_t)c.n * r.rows);
-  launch_to_id_order(c, r, c.io_d.p);
   if (all <= kPinnedBytes) {
+    c.io_d.reserve((size_t)c.n * r.rows);
+    launch(0, c.n, c.io_d.p);
     char* h = pinned_buffer(c, all);
     XS_HIP(hipMemcpyAsync(h, c.io_d.p, all, hipMemcpyDeviceToHost, c.stream));
     XS_HIP(hipStreamSynchronize(c.stream));
@@ -109,10 +116,18 @@ void to_id_order(Ctx& c, const double* const* src, int64_t stride, int rows, boo
       for (int q = 0; q < r.rows; q++) std::memcpy(to[q], h + q * row, row);
     return;
   }
-  if (interleaved) XS_HIP(hipMemcpyAsync(out[0], c.io_d.p, all, hipMemcpyDeviceToHost, c.stream));
-  else
-    for (int q = 0; q < r.rows; q++)
-      XS_HIP(hipMemcpyAsync(to[q], c.io_d.p + (size_t)q * c.n, row, hipMemcpyDeviceToHost, c.stream));
+  double* buf = reinterpret_cast<double*>(c.pos2.p);
+  const int64_t range = 4 * c.npad / r.rows;
+  for (int64_t first = 0; first < c.n; first += range) {
+    const int64_t count = std::min(range, c.n - first);
+    const size_t part = sizeof(double) * (size_t)count;
+    launch(first, count, buf);
+    if (interleaved)
+      XS_HIP(hipMemcpyAsync(out[0] + first * r.rows, buf, part * r.rows, hipMemcpyDeviceToHost, c.stream));
+    else
+      for (int q = 0; q < r.rows; q++)
+        XS_HIP(hipMemcpyAsync(to[q] + first, buf + q * count, part, hipMemcpyDeviceToHost, c.stream));
+  }
   XS_HIP(hipStreamSynchronize(c.stream));
 }
 
@@ -365,24 +380,25 @@ xs_status xs_system_set(xs_ctx* h, int64_t n, const double* rx, const double* ry
       const double* rows[6] = {rx, ry, rz, vx, vy, vz};
       const size_t row = sizeof(double) * (size_t)n, rep_at = 6 * row, type_at = rep_at + (c.has_rep ? 2 * (size_t)n : 0);
       const size_t all = type_at + (size_t)n;
+      AtomRows in;
       if (all <= kPinnedBytes) {  // the kernel reads them from host memory
         char* h = pinned_buffer(c, all);
-        for (int q = 0; q < 6; q++) std::memcpy(h + q * row, rows[q], row);
+        for (int q = 0; q < 6; q++) {
+          std::memcpy(h + q * row, rows[q], row);
+          in.row[q] = reinterpret_cast<double*>(h + q * row);
+        }
         if (c.has_rep) std::memcpy(h + rep_at, rep, 2 * (size_t)n);
         std::memcpy(h + type_at, type, (size_t)n);
-        launch_unpack_atoms(c, reinterpret_cast<double*>(h), reinterpret_cast<uint8_t*>(h + type_at),
-                            reinterpret_cast<uint16_t*>(h + rep_at));
-      } else {
-        c.io_d.reserve(6 * (size_t)n);
-        c.io_type.reserve(n);
-        for (int q = 0; q < 6; q++)
-          XS_HIP(hipMemcpyAsync(c.io_d.p + (size_t)q * n, rows[q], row, hipMemcpyHostToDevice, c.stream));
-        to_device(c, c.io_type, type, n);
-        if (c.has_rep) {
-          c.io_rep.reserve(n);
-          to_device(c, c.io_rep, rep, n);
+        launch_unpack_atoms(c, in, reinterpret_cast<uint8_t*>(h + type_at), reinterpret_cast<uint16_t*>(h + rep_at));
+      } else {  // by way of the arrays that the next list build sorts into
+        DBuf<double>* const via[6] = {&c.vx2, &c.vy2, &c.vz2, &c.ax2, &c.ay2, &c.az2};
+        for (int q = 0; q < 6; q++) {
+          to_device(c, *via[q], rows[q], n);
+          in.row[q] = via[q]->p;
         }
-        launch_unpack_atoms(c, c.io_d.p, c.io_type.p, c.io_rep.p);
+        to_device(c, c.type2, type, n);
+        if (c.has_rep) to_device(c, c.rep2, rep, n);
+        launch_unpack_atoms(c, in, c.type2.p, c.rep2.p);
       }
     }
     XS_HIP(hipStreamSynchronize(c.stream));
@@ -424,11 +440,10 @@ xs_status xs_velocity_set(xs_ctx* h, const double* vx, const double* vy, const d
   return guarded(h, [&](Ctx& c) {
     require(vx && vy && vz, XS_E_ARG, "null velocity array");
     if (c.n == 0) return;
-    c.io_d.reserve(3 * (size_t)c.n);
-    const double* rows[3] = {vx, vy, vz};
-    for (int q = 0; q < 3; q++)
-      XS_HIP(hipMemcpyAsync(c.io_d.p + (size_t)q * c.n, rows[q], sizeof(double) * c.n, hipMemcpyHostToDevice, c.stream));
-    launch_velocities_in(c, c.io_d.p);
+    to_device(c, c.vx2, vx, c.n);
+    to_device(c, c.vy2, vy, c.n);
+    to_device(c, c.vz2, vz, c.n);
+    launch_velocities_in(c, c.vx2.p, c.vy2.p, c.vz2.p);
     XS_HIP(hipStreamSynchronize(c.stream));
   });
 }

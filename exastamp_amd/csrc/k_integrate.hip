@@ -97,9 +97,9 @@ __global__ void __launch_bounds__(256) k_drift_kick(
   if (far) over.raise();
 }
 
-// Atoms as the caller gave them -- x, y, z, vx, vy, vz in rows of n, types, replicas --
+// Atoms as the caller gave them -- rows x, y, z, vx, vy, vz, types, replicas --
 // into the per-atom arrays, accelerations, energies and virials zeroed
-__global__ void k_unpack_atoms(int64_t n, int64_t npad, const double* __restrict__ in,
+__global__ void k_unpack_atoms(int64_t n, int64_t npad, AtomRows in,
                                const uint8_t* __restrict__ type_in, const uint16_t* __restrict__ rep_in,
                                Pos4* __restrict__ pos, double* __restrict__ rrx, double* __restrict__ rry,
                                double* __restrict__ rrz, double* __restrict__ vx, double* __restrict__ vy,
@@ -109,14 +109,14 @@ __global__ void k_unpack_atoms(int64_t n, int64_t npad, const double* __restrict
 {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const double x = in[i], y = in[n + i], z = in[2 * n + i];
+  const double x = in.row[0][i], y = in.row[1][i], z = in.row[2][i];
   store_pos(pos, i, Pos4{x, y, z, 0.0});
   rrx[i] = x;
   rry[i] = y;
   rrz[i] = z;
-  vx[i] = in[3 * n + i];
-  vy[i] = in[4 * n + i];
-  vz[i] = in[5 * n + i];
+  vx[i] = in.row[3][i];
+  vy[i] = in.row[4][i];
+  vz[i] = in.row[5][i];
   ax[i] = ay[i] = az[i] = ep[i] = 0.0;
 #pragma unroll
   for (int q = 0; q < 9; q++) vir[q * npad + i] = 0.0;
@@ -125,26 +125,29 @@ __global__ void k_unpack_atoms(int64_t n, int64_t npad, const double* __restrict
   id[i] = i;
 }
 
-// `rows` per-atom arrays in id order: row q of atom k from src[q][stride k] to
-// out[os id[k] + oq q] (os, oq: the caller's layout)
+// `rows` per-atom arrays in id order, of the `count` ids from `first` on: row q of atom k
+// from src[q][stride k] to out[os (id[k] - first) + oq q] (os, oq: the caller's layout)
 __global__ void k_to_id_order(int64_t n, const int64_t* __restrict__ id, IdRows r, double* __restrict__ out)
 {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  double* o = out + r.atom_step * id[k];
+  const int64_t i = id[k] - r.first;
+  if (i < 0 || i >= r.count) return;
+  double* o = out + r.atom_step * i;
   for (int q = 0; q < r.rows; q++) o[q * r.row_step] = r.src[q][r.stride * k];
 }
 
-// v (id order, rows of n) into the cell order
-__global__ void k_velocities_in(int64_t n, const int64_t* __restrict__ id, const double* __restrict__ in,
+// v (id order) into the cell order
+__global__ void k_velocities_in(int64_t n, const int64_t* __restrict__ id, const double* __restrict__ in_x,
+                                const double* __restrict__ in_y, const double* __restrict__ in_z,
                                 double* __restrict__ vx, double* __restrict__ vy, double* __restrict__ vz)
 {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const int64_t i = id[k];
-  vx[k] = in[i];
-  vy[k] = in[n + i];
-  vz[k] = in[2 * n + i];
+  vx[k] = in_x[i];
+  vy[k] = in_y[i];
+  vz[k] = in_z[i];
 }
 
 // Plain streaming copy, 16 bytes per lane per iteration.
@@ -285,7 +288,7 @@ double* g_scratch_ptr[kMaxDevices] = {};
 
 }  // namespace
 
-void launch_unpack_atoms(Ctx& c, const double* in, const uint8_t* type, const uint16_t* rep)
+void launch_unpack_atoms(Ctx& c, const AtomRows& in, const uint8_t* type, const uint16_t* rep)
 {
   k_unpack_atoms<<<grid_for(c.n), kBlock, 0, c.stream>>>(
       c.n, c.npad, in, type, rep, c.pos.p, c.rrx.p, c.rry.p, c.rrz.p, c.vx.p, c.vy.p, c.vz.p, c.ax.p, c.ay.p, c.az.p,
@@ -299,9 +302,9 @@ void launch_to_id_order(Ctx& c, const IdRows& r, double* out)
   XS_HIP(hipGetLastError());
 }
 
-void launch_velocities_in(Ctx& c, const double* in)
+void launch_velocities_in(Ctx& c, const double* vx, const double* vy, const double* vz)
 {
-  k_velocities_in<<<grid_for(c.n), kBlock, 0, c.stream>>>(c.n, c.id.p, in, c.vx.p, c.vy.p, c.vz.p);
+  k_velocities_in<<<grid_for(c.n), kBlock, 0, c.stream>>>(c.n, c.id.p, vx, vy, vz, c.vx.p, c.vy.p, c.vz.p);
   XS_HIP(hipGetLastError());
 }
 

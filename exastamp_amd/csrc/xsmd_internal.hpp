@@ -423,11 +423,10 @@ struct Ctx {
   unsigned long long* hflag = nullptr;  // pinned host copy of the loop's flag dscalar[6] (StepFlag)
   hipEvent_t step_event[2] = {nullptr, nullptr};  // ends of the MD loop's queued steps
   DBuf<double> thermo_log;              // the loop's thermodynamic samples
-  // atoms on their way in and out: device buffers, and pinned host memory that small
-  // transfers go through in one piece (kPinnedBytes)
+  // atoms on their way in and out: a device buffer and pinned host memory that small
+  // transfers go through in one piece (at most kPinnedBytes each); others go by way of the
+  // list build's second arrays
   DBuf<double> io_d;
-  DBuf<uint8_t> io_type;
-  DBuf<uint16_t> io_rep;
   char* pinned = nullptr;
   size_t pinned_bytes = 0;
 
@@ -494,17 +493,20 @@ double gather_ceiling(Ctx& c, double rcut, bool force, int level, int reps);
 void pair_count(Ctx& c, double rcut, int64_t& entries, int64_t& within);
 
 // ---- launches (k_integrate.hip) ----
-// x, y, z, vx, vy, vz (rows of n), types and replicas in device memory into the context
-void launch_unpack_atoms(Ctx& c, const double* in, const uint8_t* type, const uint16_t* rep);
+// x, y, z, vx, vy, vz, types and replicas in memory the device reads into the context
+struct AtomRows {
+  const double* row[6];
+};
+void launch_unpack_atoms(Ctx& c, const AtomRows& in, const uint8_t* type, const uint16_t* rep);
 // per-atom rows of the cell order, element k of row q at src[q][stride k], and where they
-// go in id order: atom i, row q at atom_step i + row_step q
+// go in id order: atom first + i, row q at atom_step i + row_step q, for i < count
 struct IdRows {
   const double* src[9];
   int rows;
-  int64_t stride, atom_step, row_step;
+  int64_t stride, atom_step, row_step, first, count;
 };
 void launch_to_id_order(Ctx& c, const IdRows& r, double* out);
-void launch_velocities_in(Ctx& c, const double* in);
+void launch_velocities_in(Ctx& c, const double* vx, const double* vy, const double* vz);
 void launch_zero(Ctx& c);
 void launch_force_to_accel(Ctx& c);
 // inv_xform: xform_mode INV_XFORM (the step is mapped to grid space by the xform's
