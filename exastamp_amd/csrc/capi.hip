@@ -616,14 +616,12 @@ xs_status xs_lj_multi_force(xs_ctx* h, int ntypes, const double* epsilon, const 
     std::vector<double> d(4 * (size_t)np);
     std::vector<float> f(4 * (size_t)np);
     std::vector<double> rc2(np, -1.0);
-    double reach = 0.0;
     for (int k = 0; k < np; k++) {
       if (epsilon[k] != 0.0) {  // the largest number whose square root is at most rcut
         double x = rcut[k] * rcut[k];
         while (std::sqrt(x) > rcut[k]) x = std::nextafter(x, 0.0);
         for (double y; std::sqrt(y = std::nextafter(x, HUGE_VAL)) <= rcut[k];) x = y;
         rc2[k] = x;
-        reach = std::max(reach, rcut[k]);
       }
       const double row[4] = {sigma[k] * sigma[k], 4.0 * epsilon[k], 24.0 * epsilon[k],
                              lj_energy_cutoff(epsilon[k], sigma[k], rcut[k])};
@@ -641,7 +639,7 @@ xs_status xs_lj_multi_force(xs_ctx* h, int ntypes, const double* epsilon, const 
     XS_HIP(hipStreamSynchronize(c.stream));  // the host rows go out of scope
     c.has_ljm = true;
     c.ljm_ntypes = ntypes;
-    c.ljm_reach = reach;
+    c.ljm_rc2 = *std::max_element(rc2.begin(), rc2.end());
     launch_lj_multi(c, flags);
   });
 }

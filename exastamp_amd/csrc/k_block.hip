@@ -1998,7 +1998,8 @@ void launch_lj_block(Ctx& c, double eps, double sigma, double rcut, unsigned fla
 
 void launch_lj_multi_block(Ctx& c, unsigned flags)
 {
-  const BlockArgs a = block_args(c, c.ljm_reach);
+  BlockArgs a = block_args(c, 0.0);
+  a.rc2 = c.ljm_rc2;
   const size_t lds = block_lds_bytes(c, true, false);
   const unsigned g = block_grid(c);
   const pm::Outputs o = make_outputs(c, ForceEpilogue{});

@@ -381,7 +381,8 @@ void lj_dispatch(Ctx& c, double eps, double sigma, double rcut, unsigned flags, 
 template <class Real>
 void lj_multi_dispatch(Ctx& c, unsigned flags)
 {
-  const PairCommon pc = make_common(c, c.ljm_reach);
+  PairCommon pc = make_common(c, 0.0);
+  pc.rc2 = c.ljm_rc2;
   const Outputs o = make_outputs(c, ForceEpilogue{});
   const pm::LJMultiDev lm = ljm_dev<Real>(c);
   const unsigned g = pair_grid(c.n);

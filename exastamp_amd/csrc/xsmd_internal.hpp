@@ -446,7 +446,7 @@ struct Ctx {
   // {sigma^2, 4 eps, 24 eps, E(rcut)} and the pairs' squared cutoffs
   bool has_ljm = false;
   int ljm_ntypes = 0;
-  double ljm_reach = 0;  // largest cutoff of a pair that interacts
+  double ljm_rc2 = -1.0;  // largest of ljm_rcut2 (below 0: nothing interacts)
   DBuf<float> ljm_f;
   DBuf<double> ljm_d, ljm_rcut2;
   bool has_eam = false;
