@@ -637,7 +637,6 @@ xs_status xs_lj_multi_force(xs_ctx* h, int ntypes, const double* epsilon, const 
     to_device(c, c.ljm_f, f.data(), (int64_t)f.size());
     to_device(c, c.ljm_rcut2, rc2.data(), np);
     XS_HIP(hipStreamSynchronize(c.stream));  // the host rows go out of scope
-    c.has_ljm = true;
     c.ljm_ntypes = ntypes;
     c.ljm_rc2 = *std::max_element(rc2.begin(), rc2.end());
     launch_lj_multi(c, flags);

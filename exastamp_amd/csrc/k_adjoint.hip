@@ -636,12 +636,14 @@ void adj_run(Ctx& c, const AdjArgs& a, double rcut, bool mixed)
 
 }  // namespace
 
-// Transpose of the knot -> coefficient map of spline_interpolate for one table:
+// Transpose of the knot -> value cubic map of spline_interpolate for one table, on the
+// host (xs_spline_adjoint, for programs that hold gradients of the coefficients; the
+// adjoint's own sweeps sum values and slopes, whose transpose is k_spline_adjoint):
 // G holds dL/d(c3,c4,c5,c6) per row (rows 0..n), out receives dL/df for the n knots.
 void spline_interpolate_adjoint(int n, double delta, const double* G, double* out)
 {
   std::vector<double> gf(n + 2, 0.0), gs(n + 2, 0.0);
-  (void)delta;  // slope coefficients were folded into c3..c5 on the device
+  (void)delta;  // the value cubics are in units of the knot spacing
   for (int m = 1; m <= n; m++) {
     const double* g = G + 4 * (size_t)m;
     gf[m] += g[3];  // c6 = f

@@ -439,13 +439,6 @@ __device__ __forceinline__ void s_knot(const EamTabDev<float>& t, double d2, int
   p = (float)(x - (double)m);
 }
 
-// d^2 outside the s-table's range [s_lo, s_hi]
-__device__ __forceinline__ bool s_out(const EamTabDev<float>& t, double d2)
-{
-  const double x = fma(d2, t.s_rds, t.s_off);
-  return !(x >= 0.0 && x <= t.s_xmax);
-}
-
 // the slope quadratic [A B C] of an s-table force row (its fourth value is padding)
 struct Q3 {
   float a, b, c;

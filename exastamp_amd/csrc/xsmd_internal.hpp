@@ -357,7 +357,6 @@ struct Ctx {
 
   int nspecies = 0;
   double mass[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  DBuf<double> inv_mass_d;  // unused slots 0
   DBuf<double> mass_d;
 
   int64_t n = 0;
@@ -444,7 +443,6 @@ struct Ctx {
   double lj_eps = 0, lj_sigma = 0, lj_rcut = 0;
   // lj_multi_force: per type pair (packed triangle) FP32 and FP64 rows
   // {sigma^2, 4 eps, 24 eps, E(rcut)} and the pairs' squared cutoffs
-  bool has_ljm = false;
   int ljm_ntypes = 0;
   double ljm_rc2 = -1.0;  // largest of ljm_rcut2 (below 0: nothing interacts)
   DBuf<float> ljm_f;

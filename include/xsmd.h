@@ -310,7 +310,8 @@ xs_status xs_forces_energies_dev(xs_ctx* ctx, double* F_dev, double* E_dev, doub
 xs_status xs_lj_adjoint(xs_ctx* ctx, double epsilon, double sigma, double rcut, const double* dL_dF,
                         const double* dL_dE, double grad[2], unsigned flags);
 /* Knot-gradient of the spline construction alone (transpose of the knot -> c3..c6
- * map): G has (n+1) rows of 4 coefficient gradients, out n knots.  Host only. */
+ * map), for gradients of the coefficients from elsewhere: G has (n+1) rows of 4
+ * coefficient gradients, out n knots.  Host only; xs_eam_adjoint does not go through it. */
 xs_status xs_spline_adjoint(int n, double delta, const double* G, double* out);
 
 /* --- fused NVE loop ---------------------------------------------------------------- */
