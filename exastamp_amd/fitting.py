@@ -130,12 +130,14 @@ def _addresses(*tensors):
     their values; None for any other.  A negated view (``z.conj().imag``) has the memory of
     what it negates, a tensor of zeros from autograd has none (address 0), and that of a
     batched backward (``is_grads_batched``) has no address to give."""
-    d = tensors[0].device
-    if not all(type(t) is torch.Tensor and t.dtype is torch.float64 and t.device == d and t.is_contiguous()
-               and t.numel() > 0 and not t.is_neg() for t in tensors):
-        return None
+    at = []
     try:
-        at = [t.data_ptr() for t in tensors]
+        device = tensors[0].get_device()
+        for t in tensors:
+            if (type(t) is not torch.Tensor or t.dtype is not torch.float64 or t.get_device() != device
+                    or not t.is_contiguous() or t.is_neg() or t.numel() == 0):
+                return None
+            at.append(t.data_ptr())
     except RuntimeError:
         return None
     return at if all(at) else None
@@ -144,8 +146,7 @@ def _addresses(*tensors):
 def _kernel_addresses(*tensors):
     """_addresses of tensors on a GPU, unless something records the operations on them;
     None: the operations have to run as tensor operations."""
-    if (tensors[0].device.type != "cuda" or torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or _dispatch_modes() != 0):
+    if (not tensors[0].is_cuda or torch.compiler.is_compiling() or torch._C._is_tracing() or _dispatch_modes() != 0):
         return None
     return _addresses(*tensors)
 
