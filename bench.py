@@ -192,7 +192,7 @@ def gather_ceiling(sim, rc, kernels):
 def force_kernel_name(list_info):
     if list_info["kind"] != "block":
         return "k_eam_force<float, false, false, false, true>"
-    return "k_block_eam_force<float, false, false, false, true, true>"
+    return "k_block_eam_force<float, false, false, false, true, true, false>"
 
 
 def measured_traffic(kernel):

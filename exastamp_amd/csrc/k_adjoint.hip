@@ -39,7 +39,7 @@
 // like the density pass (k_block_adj_b1); the second gathers positions and loss gradients
 // through the list, since the accumulators take the LDS a brick's halo would need.
 // Bound by the LDS atomics (8 to 12 per pair) and the gathers (64 bytes per pair).
-// 1.04 M Cu/Ni atoms, 2000 knots: first sweep 198 us, second 473 us, F rows 11 us; walking
+// 1.04 M Cu/Ni atoms, 2000 knots: first sweep 201 us, second 473 us, F rows 12 us; walking
 // every list entry on the global list, with four coefficients per row and so three
 // launches, took 1107 + 2 x 645 us.  55 k atoms, 500 knots: 13 + 35 us against 80.
 #include "pair_math.hpp"

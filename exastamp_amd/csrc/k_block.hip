@@ -1479,7 +1479,7 @@ __global__ void __launch_bounds__(kPassThreads, kPassWaves<VIRIAL || SPLIT>) k_b
 // rho_i, F'(rho_i) into the position record's w and F(rho_i) added to ep.
 // Bound by the FP64 arithmetic of the pairs (one or two exponentials, divisions and a
 // square root each).  128 k Ta atoms (83 entries, 53 in rc), both passes with energy and
-// virial: 134 us, against 338 us, and 115 us to convert the list, on the global list with
+// virial: 121 us, against 338 us, and 115 us to convert the list, on the global list with
 // the general power function and every term evaluated for itself.
 template <bool SPLIT>
 __global__ void __launch_bounds__(kPassThreads, 4) k_block_johnson_rho(BlockArgs a, JohnsonParams jp,

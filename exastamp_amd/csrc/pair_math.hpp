@@ -34,7 +34,7 @@ __device__ __forceinline__ Q4<double> load4(const double* __restrict__ p)
 // instructions of the 79 per list entry of the FP64 force pass.  Squared distances need
 // none of that, so both come from the hardware's reciprocal square root y (about 2^-23) by
 // Goldschmidt's iteration: g -> sqrt, h -> 1 / (2 sqrt), then one residual step each,
-// 11 instructions.  On 8.4 M values from 0.01 to 1e12 r equals sqrt(d2) in every one and
+// 12 instructions with the minimum.  On 8.4 M values from 0.01 to 1e12 r equals sqrt(d2) in every one and
 // rinv is as far from the exact reciprocal as 1 / r (1.50 ulp at most, 0.36 on average);
 // recip equals 1 / x.  For d2 = 0 (coincident atoms) the steps give NaN: the minimum makes
 // rinv the infinity that the division gives, r stays NaN (knot_r takes it as 0).
@@ -244,7 +244,7 @@ __device__ __forceinline__ const T* at32(const T* base, uint32_t i)
 // of 16 bytes looks up the cache line of each row it touches; two loads of 64 scattered rows
 // look up about 100 lines, two of 32 rows each, whole, little more than half, and the FP64
 // passes are bound by those lookups (texture address and data units busy 80 % of the time).
-// 500 k EAM atoms, FP64: lookups of the force pass 84 -> 48 million, 118 -> 104 us, density
+// 500 k EAM atoms, FP64: lookups of the force pass 84 -> 48 million, 118 -> 102 us, density
 // pass 65 -> 56.  The mixed force pass, whose rows are 32 bytes too, pays more for
 // the exchange than it gains (8.39 M atoms: 1139 -> 1346 us).
 __device__ __forceinline__ uint32_t dpp_xor1(uint32_t v)
@@ -364,8 +364,8 @@ __device__ __forceinline__ const Real* pair_row(const Real* __restrict__ pair, c
 // eam_alloy.h:70-133): rho of each and their z2r, in arithmetic.  A type map is one more
 // gather ahead of every row's, and rows that also hold the derivative quadratic cost four
 // 32-byte gathers per pair instead of three: the alloy force pass of 130 k atoms (FP64,
-// energy and virial) took 134 us with both, 80 us without, the density pass 42 and 35.
-// Types past the last element take the first planes.
+// energy and virial) took 134 us with both, 80 us without (73 with rows loaded in pairs),
+// the density pass 42 and 35 (32).  Types past the last element take the first planes.
 __device__ __forceinline__ void pair_planes(int nel, int ti, int tj, int& rho_i, int& rho_j, int& z2r)
 {
   const int hi = max(ti, tj), lo = min(ti, tj);
